@@ -160,3 +160,30 @@ def test_device_array_checks(gpu_available):
                 s.get(A.FIELD_MASS)
         finally:
             bad.free()
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (1, 1, 85), (5, 51, 1), (4, 8, 8), (1, 1, 257)])
+def test_transfer_at_block_edges(gpu_available, n):
+    """Element tensors, two-value and sixteen-value states and node vectors at 1, 85, 255, 256
+    and 257 elements (the transfer kernels work on blocks of 256 entities or values): the
+    device arrays hold exactly what the host path returns."""
+    X, conn = M.hex_lattice(*n)
+    rng = np.random.default_rng(sum(n))
+    u = 1e-2 / max(n) * rng.uniform(-1, 1, X.shape)
+    for per_qp in (0, 1):
+        with A.Solver() as s:
+            s.set_mesh(A.HEX8, X, conn)
+            s.set_material(A.NEO_HOOKEAN_DAMAGE, 1000.0, 1e9, 0.3, state_per_qp=per_qp,
+                           damage=dict(I1_critical=3.0001, I1_failure=3.1, alpha=1.0))
+            state = 0.5 * rng.uniform(0, 1, s.field_shape(A.FIELD_STATE))
+            dev = DeviceArray(state.size).upload(state)
+            try:
+                s.set_field_device(A.FIELD_STATE, dev.address)
+                s.synchronize()
+            finally:
+                dev.free()
+            assert np.array_equal(s.get(A.FIELD_STATE), state)
+            s.set_field(A.FIELD_U, u)
+            s.internal_force()
+            for f in (A.FIELD_U, A.FIELD_F, A.FIELD_H, A.FIELD_P, A.FIELD_STATE, A.FIELD_VOLUME):
+                assert np.array_equal(_get_device(s, f), s.get(f)), (n, per_qp, f)
