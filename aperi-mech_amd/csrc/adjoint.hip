@@ -609,7 +609,7 @@ void adjoint_forward(Ctx &c, double dt, int n_steps, int interval) {
     D.final_state.alloc(9 * c.nn);
     for (int s = 0; s < n_steps; ++s) {
         if (s % interval == 0) copy_state(c, D.ckpt[s / interval]->p);
-        step_once_tiles(c, dt);
+        step_once_tiles(c, dt, s + 1 == n_steps);
     }
     copy_state(c, D.final_state.p);
     APHIP_HIP(hipStreamSynchronize(c.stream));
@@ -643,7 +643,7 @@ void adjoint_backward(Ctx &c, const double *ub_T, const double *vb_T, double *E_
         const int s0 = sg * K, len = std::min(K, D.n_steps - s0);
         restore_state(c, D.ckpt[sg]->p);
         for (int k = 0; k < len; ++k) {
-            step_once_tiles(c, D.dt);
+            step_once_tiles(c, D.dt, false);
             APHIP_HIP(hipMemcpyAsync(D.seg_u.p + (size_t)k * n3, c.u.p, sizeof(double) * n3, hipMemcpyDeviceToDevice,
                                      c.stream));
         }

@@ -450,7 +450,7 @@ static void force_pass(Ctx &c) {
     prof_end(c, 1);
 }
 
-static void step_once(Ctx &c, double dt, bool pred_in = false, bool pred_out = false);
+static void step_once(Ctx &c, double dt, bool pred_in = false, bool pred_out = false, bool keep = true);
 
 static void node_pass(Ctx &c, double dt, int mode) {
     prof_begin(c, 2);
@@ -459,19 +459,18 @@ static void node_pass(Ctx &c, double dt, int mode) {
     prof_end(c, 2);
 }
 
-void step_once_tiles(Ctx &c, double dt);
-
 // one step of the explicit loop body (src/Solvers/Explicit.cpp:391-452).  On the tile
 // path, pred_out has the shared-node pass also store the shared nodes' predicted
 // displacement for the next step, and pred_in has the tile kernel take it instead of
 // predicting from u, v and a (the same arithmetic on the same values: bitwise the same
 // step, 57 B less per shared tile-node row).  Only steps of one aphip_step call pass a
-// prediction on, so nothing between calls can leave it stale.
-static void step_once(Ctx &c, double dt, bool pred_in, bool pred_out) {
+// prediction on, so nothing between calls can leave it stale.  keep = false on the tile
+// path: H, P and f are not stored, for the steps of a call after which another follows.
+static void step_once(Ctx &c, double dt, bool pred_in, bool pred_out, bool keep) {
     c.state_np1 = 1 - c.state_np1;  // UpdateFieldStates (Explicit.cpp:393)
     c.rate_dt = dt;                 // SetTimeIncrement (ElementTetrahedron4.h:187)
     if (use_tiles(c)) {
-        tile_run(c, dt, 2, nullptr, nullptr, pred_in, pred_out);
+        tile_run(c, dt, 2, nullptr, nullptr, pred_in, pred_out, keep);
     } else {
         fem_predict(c, dt);
         force_pass(c);
@@ -479,12 +478,13 @@ static void step_once(Ctx &c, double dt, bool pred_in, bool pred_out) {
     }
 }
 
-void step_once_tiles(Ctx &c, double dt) { step_once(c, dt); }
+void step_once_tiles(Ctx &c, double dt, bool keep) { step_once(c, dt, false, false, keep); }
 
-// f, H, P and the NP1 state from the current u (ComputeInternalForceAllElements).
-static void internal_force_eval(Ctx &c) {
+// f, H, P and the NP1 state from the current u (ComputeInternalForceAllElements).  With
+// keep = false H and P may be left unwritten (the power method reads f alone).
+static void internal_force_eval(Ctx &c, bool keep = true) {
     if (use_tiles(c)) {
-        tile_run(c, 0.0, 0);
+        tile_run(c, 0.0, 0, nullptr, nullptr, false, false, keep);
     } else {
         force_pass(c);
         node_pass(c, 0.0, 0);
@@ -574,7 +574,7 @@ static PowerMethodResult power_method(Ctx &c, const PowerMethodWork &w, double p
         APHIP_HIP(hipMemcpyAsync(w.v, c.pm_eig.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
     else
         pm_start(c, c.d_node_iperm.p, seed, eps, l, w.v);
-    internal_force_eval(c);  // F(u)
+    internal_force_eval(c, false);  // F(u)
     APHIP_HIP(hipMemcpyAsync(w.f0, c.f.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
 
     constexpr int window = 5;
@@ -585,7 +585,7 @@ static PowerMethodResult power_method(Ctx &c, const PowerMethodWork &w, double p
     for (int k = 0; k < n_iter; ++k) {
         dt_n = dt_np1;
         pm_perturb(c, w.u_in, w.v, l, eps);
-        internal_force_eval(c);
+        internal_force_eval(c, false);
         const double lambda = pm_next(c, w.f0, l, eps, w.v, w.partial);
         pm_scale(c, lambda, w.v);
         dt_np1 = 2.0 / std::sqrt(lambda);
@@ -1236,8 +1236,8 @@ int aphip_step(aphip_ctx *c, double dt, int32_t n_steps) {
             hipGraph_t g = nullptr;
             APHIP_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             try {  // the second step takes the first one's prediction
-                step_once(*c, dt, false, true);
-                step_once(*c, dt, true, false);
+                step_once(*c, dt, false, true, false);
+                step_once(*c, dt, true, false, true);
             } catch (...) {
                 (void)hipStreamEndCapture(c->stream, &g);
                 if (g) (void)hipGraphDestroy(g);
@@ -1256,7 +1256,7 @@ int aphip_step(aphip_ctx *c, double dt, int32_t n_steps) {
     for (bool pred = false; done < n_steps; ++done) {
         const bool more = done + 1 < n_steps && c->formulation != APHIP_SEMI_LAGRANGIAN;
         prof_begin(*c, 0);
-        step_once(*c, dt, pred, more);
+        step_once(*c, dt, pred, more, !more);
         prof_end(*c, 0);
         pred = more;
         // the reference's StepScheduler(interval, interval) after step n (Explicit.cpp:195-212)

@@ -381,15 +381,19 @@ void renumber_nodes(Ctx &c, const std::vector<int32_t> &old_of_new);
 // pred_in (mode 2): shared nodes take the displacement predicted by the previous step's
 // shared-node pass (it must have run with pred_out and the same dt in this same call);
 // pred_out (mode 2): the shared-node pass stores that prediction for the next step.
+// keep = false: H, P (and in mode 2 f) of this evaluation are not stored: an inner step of
+// one call, whose values the next step overwrites before anything can read them, or a
+// force evaluation whose stress nobody reads (ignored for the rate-form materials).
 void tile_run(Ctx &c, double dt, int mode, const double *u_in = nullptr, double *f_out = nullptr,
-              bool pred_in = false, bool pred_out = false);
+              bool pred_in = false, bool pred_out = false, bool keep = true);
 
 // ---- adjoint (adjoint.hip) ----
 void adjoint_forward(Ctx &c, double dt, int n_steps, int interval);
 void adjoint_backward(Ctx &c, const double *ub_T, const double *vb_T, double *E_bar, double *nu_bar,
                       double *v0_bar);
 void force_vjp(Ctx &c, const double *f_bar, double *u_bar, double *E_bar, double *nu_bar);
-void step_once_tiles(Ctx &c, double dt);
+// keep: as tile_run's, for every step but the last of a call
+void step_once_tiles(Ctx &c, double dt, bool keep);
 
 // ---- RK (rk.hip) ----
 // nodal_subdomains >= 0: nodal smoothing cells of a thex mesh (0: every hex a subcell,

@@ -89,6 +89,8 @@ struct TileArgs {
     // pass (row first_shared + b at upred[3 b]), or null: predicted here from u, v, a
     const double *upred;
     int64_t first_shared;
+    // 0: an inner step of one call, whose H, P and f the next step overwrites unread
+    int keep;
 };
 
 // LDS carve-up (bytes), sized on the host (tile_lds_bytes) from maxtn, max_nint, te
@@ -167,7 +169,7 @@ __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L,
                                             const double (&f)[3]) {
     if (ln < nint) {
         const int64_t g = ibase + ln;
-        st3(A.f, g, f);
+        if (MODE != 2 || A.keep) st3(A.f, g, f);
         if constexpr (MODE == 1) {
             const double mm = L.M[ln];
             const double acc[3] = {f[0] / mm, f[1] / mm, f[2] / mm};
@@ -371,7 +373,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
             double H[9], P[9];
             hex8_qp_lane<KIND, PER_QP>(q, lc, L.X, L.U, m, A.gauss_a, state_width<KIND>() ? A.state_n + so : nullptr,
                                        state_width<KIND>() ? A.state_np1 + so : nullptr, H, P, fe[0], &rin);
-            if (q == 7) {
+            if (q == 7 && A.keep) {
 #pragma unroll
                 for (int i = 0; i < 9; ++i) {
                     store_once(A.H + i * A.ne + e, H[i]);
@@ -397,11 +399,16 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
             hex8_element<KIND, PER_QP>(X, U, m, A.gauss_a, state_width<KIND>() ? A.state_n + so : nullptr,
                                        state_width<KIND>() ? A.state_np1 + so : nullptr, H, P, fe, &rin);
         }
+        if constexpr (NPE == 4) {
 #pragma unroll
-        for (int i = 0; i < 9; ++i) {
-            store_once(A.H + i * A.ne + e, H[i]);
-            if constexpr (NPE == 4) pdef[i] = P[i];
-            else store_once(A.P + i * A.ne + e, P[i]);
+            for (int i = 0; i < 9; ++i) pdef[i] = P[i];
+        }
+        if (A.keep) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i) {
+                store_once(A.H + i * A.ne + e, H[i]);
+                if constexpr (NPE != 4) store_once(A.P + i * A.ne + e, P[i]);
+            }
         }
         if (my_round == 0) {
 #pragma unroll
@@ -410,7 +417,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
     }
     __syncthreads();
     if constexpr (NPE == 4) {
-        if (has_elem) {
+        if (has_elem && A.keep) {
 #pragma unroll
             for (int i = 0; i < 9; ++i) store_once(A.P + i * A.ne + e, pdef[i]);
         }
@@ -670,9 +677,11 @@ __global__ __launch_bounds__(256) void k_tile_stream(TileArgs A, int nblk) {
     // every prefetch is unconditional, on tile ids clamped to the block's range: a
     // branch around a load would make the compiler wait for it at the join
     const int64_t tlast = tend - 1;
-    const __amdgpu_buffer_rsrc_t rH = buffer_rsrc(A.H, 72 * A.ne), rP = buffer_rsrc(A.P, 72 * A.ne);
+    // (an inner step's H, P and f stores are dropped by empty resources)
+    const int64_t hp_bytes = A.keep ? 72 * A.ne : 0;
+    const __amdgpu_buffer_rsrc_t rH = buffer_rsrc(A.H, hp_bytes), rP = buffer_rsrc(A.P, hp_bytes);
     const __amdgpu_buffer_rsrc_t rS = buffer_rsrc(A.state_np1, KIND == APHIP_J2 ? 8 * A.ne : 0);
-    const __amdgpu_buffer_rsrc_t rF = buffer_rsrc(A.f, 24 * A.nn), rU = buffer_rsrc(A.u, 24 * A.nn);
+    const __amdgpu_buffer_rsrc_t rF = buffer_rsrc(A.f, A.keep ? 24 * A.nn : 0), rU = buffer_rsrc(A.u, 24 * A.nn);
     const __amdgpu_buffer_rsrc_t rV = buffer_rsrc(A.v, 24 * A.nn), rA = buffer_rsrc(A.a, 24 * A.nn);
     const __amdgpu_buffer_rsrc_t rB = buffer_rsrc(A.bpart, 24 * A.nslot);
 
@@ -791,6 +800,7 @@ struct BoundArgs {
     const double *zero;  // 8 zero doubles: stands in for an absent optional array
     double dt;
     double *upred;  // mode 2: store the next step's predicted displacement (same dt), or null
+    int keep;       // 0: an inner step, f is not stored
 };
 
 template <int MODE>
@@ -830,7 +840,7 @@ __global__ __launch_bounds__(256) void k_boundary(BoundArgs A) {
         }
     }
     if (!live) return;
-    st3(A.f, g, f);
+    if (MODE != 2 || A.keep) st3(A.f, g, f);
     if constexpr (MODE == 1) {
         const double acc[3] = {f[0] / m, f[1] / m, f[2] / m};
         st3(A.a, g, acc);
@@ -1134,7 +1144,8 @@ void tile_build(Ctx &c, int te, int threads) {
     APHIP_HIP(hipStreamSynchronize(c.stream));
 }
 
-void tile_run(Ctx &c, double dt, int mode, const double *u_in, double *f_out, bool pred_in, bool pred_out) {
+void tile_run(Ctx &c, double dt, int mode, const double *u_in, double *f_out, bool pred_in, bool pred_out,
+              bool keep) {
     TilePlan &P = c.tiles;
     APHIP_REQUIRE(P.ready, "tile plan not built");
     APHIP_REQUIRE(mode == 0 || (u_in == nullptr && f_out == nullptr), "displacement / force arrays only in force mode");
@@ -1190,6 +1201,7 @@ void tile_run(Ctx &c, double dt, int mode, const double *u_in, double *f_out, bo
     A.dt = dt;
     A.upred = pred_in ? P.upred.p : nullptr;
     A.first_shared = P.n_interior;
+    A.keep = keep || c.mat.rate_form();  // (the rate-form materials read the previous H and P)
     prof_begin(c, 1);
     if (c.npe == 4) {
         if (mode == 0) dispatch_kind<4, 0>(c, A, P.lds_bytes);
@@ -1205,7 +1217,7 @@ void tile_run(Ctx &c, double dt, int mode, const double *u_in, double *f_out, bo
     if (P.nb > 0) {
         BoundArgs B{P.nb, P.n_interior, P.bstart.p, P.bpart.p, c.u.p, c.v.p, c.a.p, A.f, c.mass.p,
                     c.has_fixed ? c.fixed.p : nullptr, c.node_dt.p, P.zero.p, dt,
-                    pred_out ? P.upred.p : nullptr};
+                    pred_out ? P.upred.p : nullptr, A.keep};
         const dim3 grid((unsigned)((P.nb + 255) / 256));
         prof_begin(c, 2);
         if (mode == 0) hipLaunchKernelGGL(k_boundary<0>, grid, dim3(256), 0, c.stream, B);

@@ -22,16 +22,21 @@ import numpy as np  # noqa: E402
 
 METRIC = "FP64 element-updates/s + % HBM roofline; batched & adjoint vs plain, 1 GPU"
 HBM_PEAK_GBS = 8000.0
-# Algorithmic bytes per element-update of the full-output step: element streams
-# conn 16 B + H 72 B + P 72 B; node streams 200 B per node (read X, u, v, a as
-# 4 x 24 B and the mass 8 B; write u, v, a, f as 4 x 24 B).
-ELEM_BYTES_TET4 = 4 * 4 + 72 + 72
-NODE_BYTES = 200
+# Algorithmic bytes per element-update of one step of a call of `steps` steps: element
+# connectivity (4 B per corner), the node streams (176 B per node: read X, u, v, a as 4 x 24 B
+# and the mass 8 B; write u, v, a as 3 x 24 B) and, once per call, H, P (144 B per element) and
+# f (24 B per node): the steps of a call before its last do not store what the next overwrites.
+
+
+def step_bytes(npe, nn, ne, steps, material_fields=False):
+    return 4 * npe + (16 if material_fields else 0) + 176 * nn / ne + (144 + 24 * nn / ne) / steps
+
+
 # HBM bytes per step measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (one run each),
 # scaled by the same counters on a 1 GiB device copy (fetch x 2.0, write x 1.0); summed
 # over the step's two launches.  profiles/tile_step_tet4_6M_neohookean_hbm_traffic.txt
 # holds the commands and per-kernel figures.  Keyed by (material, hexes per edge).
-MEASURED_TRAFFIC = {("nh", 100): 1339.7e6, ("le", 100): 1337.9e6}
+MEASURED_TRAFFIC = {}
 # FP64 flops per step of the same workload from rocprofv3 --pmc SQ_INSTS_VALU_{FMA,MUL,ADD,
 # TRANS}_F64 on the tile kernel (64 lanes x (2 FMA + MUL + ADD + TRANS) per wave
 # instruction) on the tile and shared-node kernels; profiles/tile_step_tet4_6M_neohookean_
@@ -92,13 +97,6 @@ def run_gpu(w, kind, steps, warmup):
     return dict(wall=walls[best], mode=best, walls=walls, wall_prof=wall, step_ms=ms_step / max(n_step, 1),
                 force_ms=ms_force / max(n_force, 1), node_ms=ms_node / max(n_node, 1),
                 n_step=n_step, finite=ok, dt=dt)
-
-
-def hex8_bytes_per_update(nn, ne, material_fields=True):
-    """Algorithmic bytes per Hex8 element-update: connectivity 32 B, H 72 B, P 72 B, the
-    per-element E and nu 16 B when the material varies per element, and the node streams
-    (200 B per node) spread over the elements."""
-    return 8 * 4 + 72 + 72 + (16 if material_fields else 0) + NODE_BYTES * nn / ne
 
 
 def roofline(bytes_per_update, updates_per_launch, ms_per_launch, kernel):
@@ -190,7 +188,7 @@ def bench_batched(n_specimens=256, steps=50, tune=True):
     t_loop = run_loop()
     identical, _ = compare(True)
     step_ms, tile_ms = kernel_ms()
-    bpu = hex8_bytes_per_update(nn, ne, material_fields=True)
+    bpu = step_bytes(8, nn, ne, 10, material_fields=True)
     out = {"workload": f"{n_specimens} Hex8 cubes, edges log-uniform in [8,48] ({ne} Hex8, {nn} nodes), "
                        f"neo-Hookean, per-specimen E, nu and dt, {steps} steps",
            "elements": ne, "nodes": nn, "steps": steps,
@@ -341,7 +339,7 @@ def bench_adjoint(n=64, steps=200, interval=20, n_check=32, h=1e-6):
     s.close()
     errs, errs10 = np.array(errs), np.array(errs10)
     ne, nn = len(conn), len(X)
-    bpu_fwd = hex8_bytes_per_update(nn, ne, material_fields=True)
+    bpu_fwd = step_bytes(8, nn, ne, 20, material_fields=True)
     # reverse sweep per element-update: the forward's streams again (segment recompute), the
     # adjoint node vectors lambda_u and lambda_v read and written (4 x 24 B per node) and the
     # per-element E / nu sensitivities read and written (32 B)
@@ -399,7 +397,7 @@ def bench_hex8_forward(n=64, steps=20):
     step_ms = m0 / max(n0, 1)
     return {"workload": f"{n}^3 Hex8 ({ne} el), neo-Hookean with per-element E/nu, {steps} steps",
             "kernels_ms": {"step": step_ms, "tile_kernel": m1 / max(n1, 1)},
-            "roofline": roofline(hex8_bytes_per_update(nn, ne, True), ne, step_ms, "step, HIP events")}
+            "roofline": roofline(step_bytes(8, nn, ne, steps, True), ne, step_ms, "step, HIP events")}
 
 
 def bench_rkpm(n_nodes_edge=64, steps=100, scale=1.5, one_pass=True):
@@ -697,7 +695,7 @@ def main():
     r = run_gpu(w, kind, args.steps, args.warmup)
     ne, nn = w["conn"].shape[0], w["X"].shape[0]
     value = ne * args.steps / r["wall"]
-    bytes_per_update = ELEM_BYTES_TET4 + NODE_BYTES * nn / ne
+    bytes_per_update = step_bytes(4, nn, ne, args.steps)
     achieved = bytes_per_update * ne / (r["step_ms"] * 1e-3) / 1e9
     line = {
         "metric": METRIC,
@@ -714,7 +712,7 @@ def main():
         "data": "synthetic (seeded jittered lattice, counter-based splitmix64)",
         "config": {"workload": f"large Tet4 block {args.n}^3x6 = {ne} Tet4, {nn} nodes, "
                                f"{'neo-Hookean' if kind == A.NEO_HOOKEAN else 'linear elastic'} FP64, "
-                               f"full-output central-difference step",
+                               f"central-difference steps, {args.steps} per call, H, P and f stored by a call's last step",
                    "elements": ne, "nodes": nn, "material": args.material},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": MEASURED_TRAFFIC.get((args.material, args.n)),
