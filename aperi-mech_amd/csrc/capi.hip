@@ -326,8 +326,9 @@ void renumber_nodes(Ctx &c, const std::vector<int32_t> &old_of_new) {
 }
 
 static bool use_tiles(const Ctx &c) {
-    return !c.cells.ready && c.tiles.ready && !(c.flags & APHIP_FLAG_TWO_PASS) &&
-           c.formulation == APHIP_TOTAL_LAGRANGIAN;
+    // finite-element smoothed Tet4 cells are the elements themselves
+    if (c.cells.ready) return c.cells.fe && c.tiles.ready && !c.node_dt.p;
+    return c.tiles.ready && !(c.flags & APHIP_FLAG_TWO_PASS) && c.formulation == APHIP_TOTAL_LAGRANGIAN;
 }
 
 static void default_tiling(Ctx &c) {
@@ -443,38 +444,45 @@ static void setup_mesh(Ctx &c, int32_t elem_type, int64_t n_nodes, const double 
     APHIP_HIP(hipStreamSynchronize(c.stream));
 }
 
-static void force_pass(Ctx &c) {
+static void force_pass(Ctx &c, bool keep = true) {
     prof_begin(c, 1);
-    if (c.cells.ready) rk_cell_force(c);
+    if (c.cells.ready) rk_cell_force(c, keep);
     else fem_element_force(c);
     prof_end(c, 1);
 }
 
 static void step_once(Ctx &c, double dt, bool pred_in = false, bool pred_out = false, bool keep = true);
 
-static void node_pass(Ctx &c, double dt, int mode) {
+static void node_pass(Ctx &c, double dt, int mode, bool more = false) {
     prof_begin(c, 2);
-    if (c.cells.ready) rk_node_update(c, dt, mode);
+    if (c.cells.ready) rk_node_update(c, dt, mode, more);
     else fem_node_update(c, dt, mode);
     prof_end(c, 2);
 }
 
-// one step of the explicit loop body (src/Solvers/Explicit.cpp:391-452).  On the tile
-// path, pred_out has the shared-node pass also store the shared nodes' predicted
-// displacement for the next step, and pred_in has the tile kernel take it instead of
-// predicting from u, v and a (the same arithmetic on the same values: bitwise the same
-// step, 57 B less per shared tile-node row).  Only steps of one aphip_step call pass a
-// prediction on, so nothing between calls can leave it stale.  keep = false on the tile
-// path: H, P and f are not stored, for the steps of a call after which another follows.
+// one step of the explicit loop body (src/Solvers/Explicit.cpp:391-452).  Steps of one
+// aphip_step call hand the next one's predictor on, so nothing between calls can leave it
+// stale (the same arithmetic on the same values: bitwise the same steps).  On the tile path,
+// pred_out has the shared-node pass also store the shared nodes' predicted displacement for
+// the next step, and pred_in has the tile kernel take it instead of predicting from u, v and
+// a (57 B less per shared tile-node row); on smoothed cells the node pass leaves u and v as
+// the next step's predictor would.  keep = false: H, P and f (smoothed cells: a too) are not
+// stored, for the steps of a call after which another follows.
 static void step_once(Ctx &c, double dt, bool pred_in, bool pred_out, bool keep) {
     c.state_np1 = 1 - c.state_np1;  // UpdateFieldStates (Explicit.cpp:393)
     c.rate_dt = dt;                 // SetTimeIncrement (ElementTetrahedron4.h:187)
     if (use_tiles(c)) {
-        tile_run(c, dt, 2, nullptr, nullptr, pred_in, pred_out, keep);
+        TileRun run;
+        run.pred_in = pred_in;
+        run.pred_out = pred_out;
+        run.keep = keep;
+        tile_run(c, dt, 2, run);
     } else {
-        fem_predict(c, dt);
-        force_pass(c);
-        node_pass(c, dt, 2);
+        // (ensembles keep their own increment per node, which only the predictor kernel reads)
+        const bool chain = c.cells.ready && !c.node_dt.p;
+        if (!(chain && pred_in)) fem_predict(c, dt);
+        force_pass(c, keep);
+        node_pass(c, dt, 2, chain && pred_out);
     }
 }
 
@@ -484,9 +492,11 @@ void step_once_tiles(Ctx &c, double dt, bool keep) { step_once(c, dt, false, fal
 // keep = false H and P may be left unwritten (the power method reads f alone).
 static void internal_force_eval(Ctx &c, bool keep = true) {
     if (use_tiles(c)) {
-        tile_run(c, 0.0, 0, nullptr, nullptr, false, false, keep);
+        TileRun run;
+        run.keep = keep;
+        tile_run(c, 0.0, 0, run);
     } else {
-        force_pass(c);
+        force_pass(c, keep);
         node_pass(c, 0.0, 0);
     }
 }

@@ -361,4 +361,115 @@ APHIP_DEV void hex8_qp_lane(int q, const int (&lc)[8], const double *sX, const d
     }
 }
 
+// Smoothed Tet4 B and volume from the faces (include/QuadratureSmoothed.h:32-62)
+__host__ __device__ inline void smoothed_tet4(const double (&X)[4][3], double (&B)[4][3], double &V) {
+    const int faces[4][3] = {{0, 1, 3}, {1, 2, 3}, {0, 3, 2}, {0, 2, 1}};
+    double vol = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) B[k][0] = B[k][1] = B[k][2] = 0.0;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        double e1[3], e2[3], n[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            e1[d] = X[faces[f][1]][d] - X[faces[f][0]][d];
+            e2[d] = X[faces[f][2]][d] - X[faces[f][0]][d];
+        }
+        n[0] = (e1[1] * e2[2] - e1[2] * e2[1]) / 2.0;
+        n[1] = (e1[2] * e2[0] - e1[0] * e2[2]) / 2.0;
+        n[2] = (e1[0] * e2[1] - e1[1] * e2[0]) / 2.0;
+        const double *x0 = X[faces[f][0]];
+        vol += x0[0] * n[0] + x0[1] * n[1] + x0[2] * n[2];
+#pragma unroll
+        for (int l = 0; l < 3; ++l)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) B[faces[f][l]][d] += n[d] / 3.0;
+    }
+    vol /= 3.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) B[k][d] /= vol;
+    V = vol;
+}
+
+// Smoothed Hex8 B and volume from the faces, each split into four triangles about
+// its centroid (include/QuadratureSmoothed.h:96-150)
+__host__ __device__ inline void smoothed_hex8(const double (&X)[8][3], double (&B)[8][3], double &V) {
+    const int faces[6][4] = {{0, 1, 5, 4}, {1, 2, 6, 5}, {2, 3, 7, 6}, {0, 4, 7, 3}, {0, 3, 2, 1}, {4, 5, 6, 7}};
+    double vol = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) B[k][0] = B[k][1] = B[k][2] = 0.0;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+        double mid[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) mid[d] += X[faces[f][k]][d];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) mid[d] /= 4.0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int km1 = (k + 3) & 3;
+            double e1[3], e2[3], n[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                e1[d] = X[faces[f][km1]][d] - mid[d];
+                e2[d] = X[faces[f][k]][d] - mid[d];
+            }
+            n[0] = (e1[1] * e2[2] - e1[2] * e2[1]) / 2.0;
+            n[1] = (e1[2] * e2[0] - e1[0] * e2[2]) / 2.0;
+            n[2] = (e1[0] * e2[1] - e1[1] * e2[0]) / 2.0;
+            vol += mid[0] * n[0] + mid[1] * n[1] + mid[2] * n[2];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                const double cw = (l == k || l == km1) ? 5.0 / 12.0 : 1.0 / 12.0;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) B[faces[f][l]][d] += n[d] * cw;
+            }
+        }
+    }
+    vol /= 3.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) B[k][d] /= vol;
+    V = vol;
+}
+
+template <int NPE>
+__host__ __device__ __forceinline__ void smoothed_cell(const double (&X)[NPE][3], double (&B)[NPE][3], double &V) {
+    if constexpr (NPE == 4) smoothed_tet4(X, B, V);
+    else smoothed_hex8(X, B, V);
+}
+
+// Smoothed Hex8 cell (one subcell per hex, include/ComputeInternalForceSmoothedCell.h:86-117,
+// :186-224, :325-349): H = sum_k u_k (x) B_k and fe[k] = -V P B_k with the face-smoothed B,
+// recomputed from the coordinates (192 B a cell less to read, some 600 flops).
+template <int KIND>
+APHIP_DEV void hex8_cell(const double (&X)[8][3], const double (&U)[8][3], const MatParams &m, const double *state_n,
+                         double *state_np1, double *H, double *P, double (&fe)[8][3], const RateIn *r = nullptr) {
+#pragma clang fp contract(off)
+    double B[8][3], V;
+    smoothed_hex8(X, B, V);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) H[i] = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) H[3 * i + j] = __fma_rn(U[k][i], B[k][j], H[3 * i + j]);
+    double snp1 = 0.0, aux = 0.0;
+    stress<KIND>(H, m, load_state<KIND>(state_n, 0), snp1, aux, P, r, load_state2<KIND>(state_n, 0));
+    store_state<KIND>(state_np1, 0, cell_damage_marker<KIND>(snp1, m), aux);
+    const double mv = -V;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            fe[k][i] = mv * dot3(P[3 * i], B[k][0], P[3 * i + 1], B[k][1], P[3 * i + 2], B[k][2]);
+}
+
 }  // namespace aphip

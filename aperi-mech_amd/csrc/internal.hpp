@@ -127,11 +127,6 @@ struct CellData {
     DevBuf<int32_t> nodes;      // [nnz] internal node ids
     DevBuf<double> dphi;        // [nnz * 3]
     DevBuf<double> volume;      // [ne]
-    DevBuf<int32_t> inc_cell;   // [nnz] cell owning each entry
-    DevBuf<int64_t> node_start; // [nn + 1] node -> entries naming it
-    DevBuf<int32_t> node_inc;   // unused (kept for layout stability)
-    DevBuf<int32_t> entry_pos;  // [nnz] position of each entry in node order (by node, then ascending entry)
-    DevBuf<double> g;           // [nnz * 3] two-pass: per-entry force contributions of the last evaluation, node order
     DevBuf<int64_t> rstart;     // [nn + 1] reverse neighbor lists: points i that list node J
     DevBuf<int32_t> rsrc;       // [nrev] i, ascending per node
     DevBuf<double> rphi;        // [nrev] phi_iJ
@@ -148,13 +143,14 @@ struct CellData {
     std::vector<int32_t> sub_of_elem;     // [ne] subcell of each internal element (nodal cells)
     std::vector<int32_t> sub_first_elem;  // [ncells] first internal element of each subcell
     std::vector<int64_t> fcell_sub_h;     // host copy of fcell_sub
-    // two-pass method: cells list the element's own nodes; the cell force acts on
-    // u_phys = Phi d and f = Phi^T f_local
+    // two-pass method: cells list the element's own nodes, u_phys and f_local can be read
     bool two_pass = false;
+    // finite-element strain smoothing: Phi is the identity, the step is the element tiles' own
+    bool fe = false;
+    // element cells (one-pass too): the cell force acts on u_phys = Phi d and f = Phi^T f_local
     DevBuf<double> u_phys;      // [nn * 3] physical displacement of the last evaluation
     DevBuf<double> f_local;     // [nn * 3] cell force before the scatter
-    // one-pass method on cell tiles (runs of consecutive cells, one wave each)
-    bool tiled = false;
+    // nodal cells on cell tiles (runs of consecutive cells, one wave each)
     int tile_cells = 0;             // cells per tile
     int tile_maxtn = 0;             // largest tile node set
     int tile_lpc = 8;               // lanes per cell of the tile kernel
@@ -171,7 +167,7 @@ struct CellData {
     void reset() {
         ready = false;
         two_pass = false;
-        tiled = false;
+        fe = false;
         tile_cells = tile_maxtn = 0;
         ntiles = tile_total = 0;
         lidx.release(); t_nstart.release(); t_node.release(); nslot_start.release(); nslot.release(); slots.release();
@@ -184,8 +180,7 @@ struct CellData {
         fcell_sub.release(); fcell_volume.release(); evol.release(); sub_fcell.release();
         sub_of_elem.clear(); sub_first_elem.clear(); fcell_sub_h.clear();
         num_nbr.release(); nbr.release(); phi.release(); radius.release(); start.release();
-        nodes.release(); dphi.release(); volume.release(); inc_cell.release(); node_start.release();
-        node_inc.release(); entry_pos.release(); g.release();
+        nodes.release(); dphi.release(); volume.release();
     }
 };
 
@@ -375,17 +370,22 @@ void tile_build(Ctx &c, int te, int threads);
 // Reorders the internal nodes (old_of_new[i] = current id of new node i) and every
 // node-indexed array of the context (capi.hip).
 void renumber_nodes(Ctx &c, const std::vector<int32_t> &old_of_new);
-// One tiled pass (MODE 0 force only, 1 force and a = f/m, 2 the full step).  In MODE 0 the
-// displacement read and the force written may be other arrays than the context's u and f
-// (the two-pass RKPM force: physical displacement in, local force out).
-// pred_in (mode 2): shared nodes take the displacement predicted by the previous step's
-// shared-node pass (it must have run with pred_out and the same dt in this same call);
-// pred_out (mode 2): the shared-node pass stores that prediction for the next step.
-// keep = false: H, P (and in mode 2 f) of this evaluation are not stored: an inner step of
-// one call, whose values the next step overwrites before anything can read them, or a
-// force evaluation whose stress nobody reads (ignored for the rate-form materials).
-void tile_run(Ctx &c, double dt, int mode, const double *u_in = nullptr, double *f_out = nullptr,
-              bool pred_in = false, bool pred_out = false, bool keep = true);
+// One tiled pass (MODE 0 force only, 1 force and a = f/m, 2 the full step).
+struct TileRun {
+    // MODE 0: displacement read and force written when not the context's u and f (RKPM
+    // element cells: physical displacement in, local force out)
+    const double *u_in = nullptr;
+    double *f_out = nullptr;
+    // MODE 2: shared nodes take the displacement predicted by the previous step's shared-node
+    // pass (it must have run with pred_out and the same dt in this same call); pred_out: the
+    // shared-node pass stores that prediction for the next step
+    bool pred_in = false, pred_out = false;
+    // false: H, P (and in MODE 2 f) of this evaluation are not stored: an inner step of one
+    // call, whose values the next step overwrites before anything can read them, or a force
+    // evaluation whose stress nobody reads (ignored for the rate-form materials)
+    bool keep = true;
+};
+void tile_run(Ctx &c, double dt, int mode, const TileRun &run = TileRun());
 
 // ---- adjoint (adjoint.hip) ----
 void adjoint_forward(Ctx &c, double dt, int n_steps, int interval);
@@ -400,8 +400,11 @@ void step_once_tiles(Ctx &c, double dt, bool keep);
 // 1: every cell one subcell), with F-bar over the subcells when fbar
 void rk_setup(Ctx &c, double scale, bool two_pass, bool fe_cells = false, int nodal_subdomains = -1,
               bool fbar = false);
-void rk_cell_force(Ctx &c);
-void rk_node_update(Ctx &c, double dt, int mode);
+// keep = false: H and P may be left unwritten (see TileRun)
+void rk_cell_force(Ctx &c, bool keep);
+// more (mode 2): another step of the same call with the same dt follows; its predictor is
+// taken here and fem_predict is not called for it
+void rk_node_update(Ctx &c, double dt, int mode, bool more);
 void rk_mass(Ctx &c, double *total);
 
 // ---- profiling helpers (capi.hip) ----

@@ -51,9 +51,6 @@
 
 namespace aphip {
 
-void stable_sort_pairs(Ctx &c, const int32_t *keys_in, int32_t *keys_out, const int32_t *vals_in, int32_t *vals_out,
-                       int64_t n, int key_bits);
-
 namespace {
 
 constexpr int kMaxNbr = 40;  // include/Constants.h:15
@@ -403,89 +400,6 @@ __global__ __launch_bounds__(cell_block<NPE>()) void k_cell_count(int64_t ne, co
     len_out[e] = cell_union<NPE>(en, num, nbr, list + threadIdx.x, BLK);
 }
 
-// Smoothed Tet4 B and volume from the faces (include/QuadratureSmoothed.h:32-62)
-__host__ __device__ void smoothed_tet4(const double (&X)[4][3], double (&B)[4][3], double &V) {
-    const int faces[4][3] = {{0, 1, 3}, {1, 2, 3}, {0, 3, 2}, {0, 2, 1}};
-    double vol = 0.0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) B[k][0] = B[k][1] = B[k][2] = 0.0;
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        double e1[3], e2[3], n[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            e1[d] = X[faces[f][1]][d] - X[faces[f][0]][d];
-            e2[d] = X[faces[f][2]][d] - X[faces[f][0]][d];
-        }
-        n[0] = (e1[1] * e2[2] - e1[2] * e2[1]) / 2.0;
-        n[1] = (e1[2] * e2[0] - e1[0] * e2[2]) / 2.0;
-        n[2] = (e1[0] * e2[1] - e1[1] * e2[0]) / 2.0;
-        const double *x0 = X[faces[f][0]];
-        vol += x0[0] * n[0] + x0[1] * n[1] + x0[2] * n[2];
-#pragma unroll
-        for (int l = 0; l < 3; ++l)
-#pragma unroll
-            for (int d = 0; d < 3; ++d) B[faces[f][l]][d] += n[d] / 3.0;
-    }
-    vol /= 3.0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) B[k][d] /= vol;
-    V = vol;
-}
-
-// Smoothed Hex8 B and volume from the faces, each split into four triangles about
-// its centroid (include/QuadratureSmoothed.h:96-150)
-__host__ __device__ void smoothed_hex8(const double (&X)[8][3], double (&B)[8][3], double &V) {
-    const int faces[6][4] = {{0, 1, 5, 4}, {1, 2, 6, 5}, {2, 3, 7, 6}, {0, 4, 7, 3}, {0, 3, 2, 1}, {4, 5, 6, 7}};
-    double vol = 0.0;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) B[k][0] = B[k][1] = B[k][2] = 0.0;
-#pragma unroll
-    for (int f = 0; f < 6; ++f) {
-        double mid[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int d = 0; d < 3; ++d) mid[d] += X[faces[f][k]][d];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) mid[d] /= 4.0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int km1 = (k + 3) & 3;
-            double e1[3], e2[3], n[3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                e1[d] = X[faces[f][km1]][d] - mid[d];
-                e2[d] = X[faces[f][k]][d] - mid[d];
-            }
-            n[0] = (e1[1] * e2[2] - e1[2] * e2[1]) / 2.0;
-            n[1] = (e1[2] * e2[0] - e1[0] * e2[2]) / 2.0;
-            n[2] = (e1[0] * e2[1] - e1[1] * e2[0]) / 2.0;
-            vol += mid[0] * n[0] + mid[1] * n[1] + mid[2] * n[2];
-#pragma unroll
-            for (int l = 0; l < 4; ++l) {
-                const double cw = (l == k || l == km1) ? 5.0 / 12.0 : 1.0 / 12.0;
-#pragma unroll
-                for (int d = 0; d < 3; ++d) B[faces[f][l]][d] += n[d] * cw;
-            }
-        }
-    }
-    vol /= 3.0;
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) B[k][d] /= vol;
-    V = vol;
-}
-
-template <int NPE>
-__host__ __device__ __forceinline__ void smoothed_cell(const double (&X)[NPE][3], double (&B)[NPE][3], double &V) {
-    if constexpr (NPE == 4) smoothed_tet4(X, B, V);
-    else smoothed_hex8(X, B, V);
-}
-
 struct CellFillArgs {
     int64_t ne;
     const int32_t *conn;
@@ -497,7 +411,6 @@ struct CellFillArgs {
     int32_t *nodes;
     double *dphi;
     double *volume;
-    int32_t *entry_cell;
 };
 
 template <int NPE>
@@ -520,7 +433,6 @@ __global__ __launch_bounds__(cell_block<NPE>()) void k_cell_fill(CellFillArgs A)
     double *dp = A.dphi + 3 * s0;
     for (int t = 0; t < len; ++t) {
         A.nodes[s0 + t] = my[t * BLK];
-        A.entry_cell[s0 + t] = (int32_t)e;
         dp[3 * t] = dp[3 * t + 1] = dp[3 * t + 2] = 0.0;
     }
     // grad phi_J = sum_k B_k V phi_{k,J} / V_sub (SmoothedCellDataProcessor.h:623-662)
@@ -548,8 +460,7 @@ __global__ __launch_bounds__(cell_block<NPE>()) void k_cell_fill(CellFillArgs A)
 // Two-pass cells: entry 4e + k is node k of element e with derivative (B_k V) / V.
 template <int NPE>
 __global__ __launch_bounds__(256) void k_cell_two_pass(int64_t ne, const int32_t *conn, const double *X,
-                                                       int32_t *nodes, double *dphi, double *volume,
-                                                       int32_t *entry_cell) {
+                                                       int32_t *nodes, double *dphi, double *volume) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= ne) return;
     int32_t en[NPE];
@@ -562,7 +473,6 @@ __global__ __launch_bounds__(256) void k_cell_two_pass(int64_t ne, const int32_t
 #pragma unroll
     for (int k = 0; k < NPE; ++k) {
         nodes[NPE * e + k] = en[k];
-        entry_cell[NPE * e + k] = (int32_t)e;
 #pragma unroll
         for (int m = 0; m < 3; ++m) dphi[3 * (NPE * e + k) + m] = (B[k][m] * V) / V;
     }
@@ -580,49 +490,24 @@ __global__ __launch_bounds__(256) void k_identity_functions(int64_t nn, int32_t 
     }
 }
 
-__global__ __launch_bounds__(256) void k_iota(int64_t n, int32_t *v) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) v[i] = (int32_t)i;
-}
-
-// pos[perm[k]] = k
-__global__ __launch_bounds__(256) void k_invert_perm(int64_t n, const int32_t *perm, int32_t *pos) {
-    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (k < n) pos[perm[k]] = (int32_t)k;
-}
-
-__global__ __launch_bounds__(256) void k_count_keys(int64_t n, const int32_t *keys, int32_t *count) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) atomicAdd(&count[keys[i]], 1);
-}
-
 // ---- smoothed-cell force step --------------------------------------------
-// Cell and node kernels of the smoothed-cell force.  Lanes in groups of 16 stride over
-// a cell's (or node's) entries, accumulate their share of the sum and combine the 16
-// partial sums with a xor butterfly; addition is commutative, so every lane ends with
-// the same bits.  The one-pass force runs on cell tiles (below); the two-pass cells
-// (four entries) keep their entry forces in node order (g) for the plain node sum.
+// The derivative of a smoothed cell is a product, grad phi_J = sum_k B_k phi_J(x_k) over the
+// nodes k of its elements, and so are the cell's gradient and force:
+//   H = sum_J d_J (x) grad phi_J = sum_k (Phi d)_k (x) B_k,
+//   f = -sum_c V_c P_c grad phi^T = Phi^T (-sum_c V_c P_c B_k^T).
+// Element cells (one- and two-pass method alike) therefore apply the factors: a gather
+// u = Phi d over the nodes' neighbor rows, the cell force on u by the element tile plan (the
+// cell of a Tet4 is the element itself with its own gradient), and a scatter Phi^T over the
+// reverse neighbor lists.  Applying the product instead (the CSR of about 77 derivatives a
+// Tet4 cell at kernel scale 1.5, 26 B each, in wave-sized cell tiles) took 0.92 ms a step on
+// the 64^3-node lattice where the factors take 0.2 ms; the CSR is kept for aphip_rk_get_cells.
+// Nodal cells (several hexes each, F-bar over their subcells) run on cell tiles over the CSR.
+// Lanes in groups stride over a node's (or cell's) entries, accumulate their share of the sum
+// and combine the partial sums with a xor butterfly; addition is commutative, so every lane
+// ends with the same bits.
 constexpr int kCellLanes = 16;
+constexpr int kSlotLanes = 8;  // lanes per node of the nodal cells' slot sum
 
-struct CellForceArgs {
-    int64_t ne, nblocks;
-    const int64_t *start;
-    const int32_t *nodes;
-    const double *dphi;
-    const double *volume;
-    const double *u;
-    double *H, *P;
-    double *g;  // [nnz * 3] per-entry force contributions, node order
-    const int32_t *pos;  // [nnz] node-order position of each entry
-    const double *state_n;
-    double *state_np1;
-    MatParams mat;
-    const double *elem_lambda, *elem_mu;
-    const double *Hn, *Pn;  // rate-form materials: H and P of the previous step
-    double rate_dt;
-};
-
-constexpr int kNodeBatch = 4;  // incidences per lane whose loads are issued together
 // lanes per node of the two-pass gather (u = Phi d)
 constexpr int kGsLanes = 8;
 constexpr int kNumXcd = 8;
@@ -643,134 +528,49 @@ __device__ __forceinline__ double group_sum(double x) {
     return x;
 }
 
-__device__ __forceinline__ double group_sum16(double x) { return group_sum<kCellLanes>(x); }
-
-// Two-pass cells, one thread per cell: the element's four nodes, their derivative
-// (B_k V) / V recomputed from the coordinates by the set-up's formula (instead of
-// streaming the stored 96 B per cell), H, stress and the four entry forces
-// -V P grad N_k at their node-order positions.
-template <int KIND, int NPE>
-__global__ __launch_bounds__(256) void k_rk_cells_two_pass(CellForceArgs A, const double *X) {
-#pragma clang fp contract(off)
-    const int64_t c_raw = xcd_block(A.nblocks) * 256 + threadIdx.x;
-    const bool live = c_raw < A.ne;
-    const int64_t c = live ? c_raw : A.ne - 1;
-    int32_t en[NPE], ps[NPE];
-#pragma unroll
-    for (int k = 0; k < NPE; ++k) {
-        en[k] = A.nodes[NPE * c + k];
-        ps[k] = A.pos[NPE * c + k];
-    }
-    double Xe[NPE][3], uj[NPE][3];
-#pragma unroll
-    for (int k = 0; k < NPE; ++k) {
-        ld3(X, en[k], Xe[k]);
-        ld3(A.u, en[k], uj[k]);
-    }
-    double snp1 = 0.0, aux = 0.0;
-    const double sn = load_state<KIND>(A.state_n, c), sn2 = load_state2<KIND>(A.state_n, c);
-    MatParams m = A.mat;
-    if (A.elem_lambda) {
-        m.lambda = A.elem_lambda[c];
-        m.mu = A.elem_mu[c];
-    }
-    double B[NPE][3], V;
-    smoothed_cell<NPE>(Xe, B, V);
-    double gc[NPE][3];
-#pragma unroll
-    for (int k = 0; k < NPE; ++k)
-#pragma unroll
-        for (int b = 0; b < 3; ++b) gc[k][b] = (B[k][b] * V) / V;
-    double H[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, P[9];
-#pragma unroll
-    for (int k = 0; k < NPE; ++k)
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int b = 0; b < 3; ++b) H[3 * a + b] = __fma_rn(uj[k][a], gc[k][b], H[3 * a + b]);
-    RateIn rin;
-    load_rate<KIND>(rin, A.Hn, A.Pn, A.ne, c, A.rate_dt);
-    stress<KIND>(H, m, sn, snp1, aux, P, &rin, sn2);
-    snp1 = cell_damage_marker<KIND>(snp1, m);
-    if (!live) return;
-    store_state<KIND>(A.state_np1, c, snp1, aux);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        store_once(A.H + i * A.ne + c, H[i]);
-        store_once(A.P + i * A.ne + c, P[i]);
-    }
-    const double mv = -V;
-#pragma unroll
-    for (int k = 0; k < NPE; ++k) {
-        double f[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) f[a] = mv * dot3(P[3 * a], gc[k][0], P[3 * a + 1], gc[k][1], P[3 * a + 2], gc[k][2]);
-        st3(A.g, ps[k], f);
-    }
-}
-
 struct RkNodeArgs {
     int64_t nn, nblocks;
-    const int64_t *inc_start;
-    const double *g;  // node order
     const double *mass;
     const uint8_t *fixed;
-    double *f, *a, *v;
+    double *f, *a, *v, *u;
     double dt;
+    // mode 2, 1: another step of the same call follows with the same dt.  The node then
+    // also takes that step's predictor (u and v are what k_predict would leave) and stores
+    // neither f nor a, which that step overwrites unread
+    int more;
 };
 
 // Node i's force f is complete: store it and finish the node (MODE 0: force only,
 // 1: a = f/m, 2: central-difference corrector).
 template <int MODE>
 __device__ __forceinline__ void rk_finish(const RkNodeArgs &A, int64_t i, const double (&f)[3]) {
-    A.f[3 * i] = f[0];
-    A.f[3 * i + 1] = f[1];
-    A.f[3 * i + 2] = f[2];
-    if constexpr (MODE == 1) {
-        const double m = A.mass[i];
-        A.a[3 * i] = f[0] / m;
-        A.a[3 * i + 1] = f[1] / m;
-        A.a[3 * i + 2] = f[2] / m;
-    } else if constexpr (MODE == 2) {
+    if constexpr (MODE == 2) {
         double vh[3], a1[3], v1[3];
         ld3(A.v, i, vh);
-        cd_correct(f, A.mass[i], A.fixed ? A.fixed[i] : 0u, A.dt, vh, a1, v1);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            A.a[3 * i + d] = a1[d];
-            A.v[3 * i + d] = v1[d];
+        const unsigned fx = A.fixed ? A.fixed[i] : 0u;
+        cd_correct(f, A.mass[i], fx, A.dt, vh, a1, v1);
+        if (A.more) {
+            double u[3], u1[3];
+            ld3(A.u, i, u);
+            cd_predict(u, v1, a1, fx, A.dt, vh, u1);
+            st3(A.u, i, u1);
+            st3(A.v, i, vh);
+        } else {
+            st3(A.f, i, f);
+            st3(A.a, i, a1);
+            st3(A.v, i, v1);
+        }
+    } else {
+        st3(A.f, i, f);
+        if constexpr (MODE == 1) {
+            const double m = A.mass[i];
+            const double a1[3] = {f[0] / m, f[1] / m, f[2] / m};
+            st3(A.a, i, a1);
         }
     }
 }
 
-template <int MODE>
-__global__ __launch_bounds__(256) void k_rk_nodes(RkNodeArgs A) {
-    const int l = threadIdx.x & (kCellLanes - 1);
-    const int64_t i_raw = xcd_block(A.nblocks) * (256 / kCellLanes) + (threadIdx.x / kCellLanes);
-    const bool live = i_raw < A.nn;
-    const int64_t i = live ? i_raw : A.nn - 1;
-    double f[3] = {0.0, 0.0, 0.0};
-    const int64_t t0 = A.inc_start[i], t1 = A.inc_start[i + 1];
-    // kNodeBatch incidences at a time, all loads issued before the first sum (clamped
-    // indices, absent incidences add zero); ascending order.
-    for (int64_t tb = t0 + l; tb < t1; tb += kNodeBatch * kCellLanes) {
-        double g[kNodeBatch][3];
-#pragma unroll
-        for (int r = 0; r < kNodeBatch; ++r) ld3(A.g, min(tb + r * kCellLanes, t1 - 1), g[r]);
-#pragma unroll
-        for (int r = 0; r < kNodeBatch; ++r) {
-            const bool in = tb + r * kCellLanes < t1;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) f[d] += in ? g[r][d] : 0.0;
-        }
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) f[d] = group_sum16(f[d]);
-    if (!live || l != 0) return;
-    rk_finish<MODE>(A, i, f);
-}
-
-// ---- one-pass method on cell tiles -------------------------------------------
+// ---- nodal cells on cell tiles -------------------------------------------
 // A tile is a run of consecutive (Morton-ordered) cells; its node set is the sorted
 // union of their node lists and every entry carries its node's index in that set
 // (uint16).  One wave per tile:
@@ -1172,11 +972,12 @@ struct RkGatherArgs {
     const double *phi;
     const double *src;  // coefficients [nn * 3]
     double *dst;        // physical values [nn * 3]
+    int copy_lonely;    // two-pass: a node without neighbors copies its coefficient (one-pass: zero)
 };
 
 // dst_i = sum_k phi_ik src_(nbr_ik): LANES lanes per node, lane l takes entries
 // l, l + LANES, ... of the node's row (contiguous across the lanes), the partial
-// sums are combined by the xor butterfly.  A node without neighbors copies src_i.
+// sums are combined by the xor butterfly.
 // (8 lanes, five entries each for a full row of 40: 3 % faster than 16 lanes.)
 template <int LANES>
 __global__ __launch_bounds__(256) void k_rk_gather(RkGatherArgs A) {
@@ -1209,7 +1010,7 @@ __global__ __launch_bounds__(256) void k_rk_gather(RkGatherArgs A) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) s[d] = group_sum<LANES>(s[d]);
     if (!live || l != 0) return;
-    if (n == 0) ld3(A.src, i, s);
+    if (n == 0 && A.copy_lonely) ld3(A.src, i, s);
     A.dst[3 * i] = s[0];
     A.dst[3 * i + 1] = s[1];
     A.dst[3 * i + 2] = s[2];
@@ -1222,13 +1023,13 @@ struct RkScatterArgs {
     const int32_t *rsrc;     // points i listing the node, ascending
     const double *rphi;      // phi_iJ of each reverse entry
     const double *src;       // local (physical) force [nn * 3]
+    int copy_lonely;         // two-pass: a node without neighbors takes src_J
 };
 
 // f_J = sum over points i that list J of phi_iJ src_i (the transpose of the
 // gather), LANES lanes per node over its contiguous reverse entries, NB per lane at a
 // time (16 x 3: a reverse list of about 40 entries in one round with little padding;
-// 6 % faster than 16 x 4, and than 8 x 5), then the node update.  A node without
-// neighbors takes src_J.
+// 6 % faster than 16 x 4, and than 8 x 5), then the node update.
 template <int MODE, int LANES, int NB>
 __global__ __launch_bounds__(256) void k_rk_scatter(RkScatterArgs A) {
     const int l = threadIdx.x & (LANES - 1);
@@ -1256,7 +1057,7 @@ __global__ __launch_bounds__(256) void k_rk_scatter(RkScatterArgs A) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) f[d] = group_sum<LANES>(f[d]);
     if (!live || l != 0) return;
-    if (A.num[i] == 0) ld3(A.src, i, f);
+    if (A.copy_lonely && A.num[i] == 0) ld3(A.src, i, f);
     rk_finish<MODE>(A.out, i, f);
 }
 
@@ -1311,7 +1112,7 @@ void scan_counts(Ctx &c, const DevBuf<int32_t> &counts, int64_t n, DevBuf<T> &st
 
 void fe_smoothing_setup(Ctx &c);
 void rk_cells_and_order(Ctx &c, bool two_pass, bool elem_cells);
-void rk_cells_order(Ctx &c, bool two_pass);
+void rk_cells_order(Ctx &c);
 
 // Nodal cells of a thex mesh (MeshLabelerProcessor.h:227-330, :690-827): marks each hex's
 // node of lowest caller id active, checks that every hex then holds exactly one active
@@ -1398,7 +1199,7 @@ static void nodal_subcells(Ctx &c, const std::vector<int64_t> &sub_start, const 
     c.X.download(hX.data(), hX.size(), c.stream);
     APHIP_HIP(hipStreamSynchronize(c.stream));
     std::vector<int64_t> start(ns + 1, 0);
-    std::vector<int32_t> nodes, inc_cell;
+    std::vector<int32_t> nodes;
     std::vector<double> dphi, vsub(ns, 0.0), evol(ne, 0.0);
     std::vector<int64_t> stamp(nn, -1);
     std::vector<int32_t> pos(nn, 0);
@@ -1419,7 +1220,6 @@ static void nodal_subcells(Ctx &c, const std::vector<int64_t> &sub_start, const 
                         stamp[j] = sc;
                         pos[j] = (int32_t)((int64_t)nodes.size() - t0);
                         nodes.push_back(j);
-                        inc_cell.push_back((int32_t)sc);
                     }
                 }
             }
@@ -1453,7 +1253,6 @@ static void nodal_subcells(Ctx &c, const std::vector<int64_t> &sub_start, const 
     APHIP_REQUIRE(D.nnz < (int64_t)INT32_MAX, "too many cell entries for int32 incidences");
     D.start.upload(start.data(), start.size(), c.stream);
     D.nodes.upload(nodes.data(), std::max<size_t>(nodes.size(), 1), c.stream);
-    D.inc_cell.upload(inc_cell.data(), std::max<size_t>(inc_cell.size(), 1), c.stream);
     D.dphi.upload(dphi.data(), std::max<size_t>(dphi.size(), 1), c.stream);
     D.volume.upload(vsub.data(), std::max<int64_t>(ns, 1), c.stream);
     D.evol.upload(evol.data(), std::max<int64_t>(ne, 1), c.stream);
@@ -1473,11 +1272,27 @@ static void nodal_subcells(Ctx &c, const std::vector<int64_t> &sub_start, const 
     APHIP_HIP(hipStreamSynchronize(c.stream));
 }
 
+// The element cells' force runs on the element tile plan, one element per thread: built
+// here when the context has none (APHIP_FLAG_TWO_PASS, a nodal set-up before this one) or
+// has the eight-lanes-per-Hex8 shape.  64 elements always fit a CU's LDS.
+static void ensure_element_tiles(Ctx &c) {
+    if (c.ne == 0 || (c.tiles.ready && c.tiles.threads == c.tiles.te)) return;
+    for (int te = c.npe == 4 ? 1024 : 128;; te /= 2) {
+        try {
+            tile_build(c, te, te);
+            return;
+        } catch (const Error &e) {
+            if (te == 64 || e.code != APHIP_ERR_INVALID) throw;
+        }
+    }
+}
+
 void rk_setup(Ctx &c, double scale, bool two_pass, bool fe_cells, int nodal_subdomains, bool fbar) {
     CellData &D = c.cells;
     D.reset();
     c.n_dof = c.nn;
     const int64_t nn = c.nn;
+    if (nodal_subdomains < 0) ensure_element_tiles(c);  // (renumbers the nodes: before anything refers to them)
     if (fe_cells) {
         fe_smoothing_setup(c);
         return;
@@ -1574,7 +1389,7 @@ void rk_setup(Ctx &c, double scale, bool two_pass, bool fe_cells, int nodal_subd
 
     if (nodal) {
         nodal_subcells(c, sub_start, sub_elems);
-        rk_cells_order(c, false);
+        rk_cells_order(c);
     } else {
         rk_cells_and_order(c, two_pass, two_pass);
     }
@@ -1584,9 +1399,11 @@ void rk_setup(Ctx &c, double scale, bool two_pass, bool fe_cells, int nodal_subd
 // include/ElementSmoothedTetrahedron4.h): the element's own shape functions, i.e. every
 // node its own only "neighbor" with value 1, and the cells of the element's nodes with
 // derivative (B_k V) / V (SmoothedCellDataProcessor.h:623-668 with unit function values).
-// The force runs on the one-pass kernels; the mass scatter is the identity.
+// Phi is the identity, so a step is the fused element tile step; the mass scatter is the
+// identity too.
 void fe_smoothing_setup(Ctx &c) {
     CellData &D = c.cells;
+    D.fe = true;
     const int64_t nn = c.nn;
     D.radius.alloc(nn);
     D.radius.zero(c.stream);
@@ -1600,8 +1417,9 @@ void fe_smoothing_setup(Ctx &c) {
     rk_cells_and_order(c, false, true);
 }
 
-// Cells (element-node cells when elem_cells), reverse neighbor lists and the node
-// order of the cell entries; two_pass selects the force method.
+// Cells (element-node cells when elem_cells) and reverse neighbor lists; two_pass selects
+// the reference's force method, which fixes what a node without neighbors contributes and
+// whether the physical displacement and local force can be read.
 void rk_cells_and_order(Ctx &c, bool two_pass, bool elem_cells) {
     CellData &D = c.cells;
     const int64_t nn = c.nn, ne = c.ne;
@@ -1619,17 +1437,10 @@ void rk_cells_and_order(Ctx &c, bool two_pass, bool elem_cells) {
         D.nodes.alloc(std::max<int64_t>(D.nnz, 1));
         D.dphi.alloc(3 * std::max<int64_t>(D.nnz, 1));
         D.volume.alloc(std::max<int64_t>(ne, 1));
-        D.inc_cell.alloc(std::max<int64_t>(D.nnz, 1));
         if (ne) {
             hipLaunchKernelGGL(hex ? k_cell_two_pass<8> : k_cell_two_pass<4>, grid1(ne, 256), dim3(256), 0, c.stream, ne, c.conn.p, c.X.p,
-                               D.nodes.p, D.dphi.p, D.volume.p, D.inc_cell.p);
+                               D.nodes.p, D.dphi.p, D.volume.p);
             APHIP_HIP(hipGetLastError());
-        }
-        if (two_pass) {
-            D.u_phys.alloc(3 * nn);
-            D.u_phys.zero(c.stream);
-            D.f_local.alloc(3 * nn);
-            D.f_local.zero(c.stream);
         }
     } else {
         DevBuf<int32_t> clen;
@@ -1645,18 +1456,21 @@ void rk_cells_and_order(Ctx &c, bool two_pass, bool elem_cells) {
         D.nodes.alloc(std::max<int64_t>(D.nnz, 1));
         D.dphi.alloc(3 * std::max<int64_t>(D.nnz, 1));
         D.volume.alloc(std::max<int64_t>(ne, 1));
-        D.inc_cell.alloc(std::max<int64_t>(D.nnz, 1));
         if (ne) {
             CellFillArgs F{ne, c.conn.p, c.X.p, D.num_nbr.p, D.nbr.p, D.phi.p, D.start.p, D.nodes.p, D.dphi.p,
-                           D.volume.p, D.inc_cell.p};
+                           D.volume.p};
             const int blk = hex ? cell_block<8>() : cell_block<4>();
             hipLaunchKernelGGL(hex ? k_cell_fill<8> : k_cell_fill<4>, grid1(ne, blk), dim3(blk), 0, c.stream, F);
             APHIP_HIP(hipGetLastError());
         }
     }
 
+    D.u_phys.alloc(3 * nn);
+    D.u_phys.zero(c.stream);
+    D.f_local.alloc(3 * nn);
+    D.f_local.zero(c.stream);
     D.ncells = ne;
-    rk_cells_order(c, two_pass);
+    rk_cells_order(c);
 }
 
 // LDS of one tile-kernel workgroup (u and force rows of the tile nodes; F-bar also the
@@ -1788,11 +1602,10 @@ static void rk_tile_plan(Ctx &c) {
     D.slots.alloc(3 * std::max<int64_t>(total, 1));
     D.slots.zero(c.stream);
     APHIP_HIP(hipStreamSynchronize(c.stream));
-    D.tiled = true;
 }
 
-// Reverse neighbor lists and the node order of the cell entries (after the cell CSR).
-void rk_cells_order(Ctx &c, bool two_pass) {
+// Reverse neighbor lists (after the cell CSR) and, for nodal cells, the cell tiles.
+void rk_cells_order(Ctx &c) {
     CellData &D = c.cells;
     const int64_t nn = c.nn;
     // reverse neighbor lists: for node J the points i that list it, ascending i,
@@ -1824,34 +1637,7 @@ void rk_cells_order(Ctx &c, bool two_pass) {
         APHIP_HIP(hipStreamSynchronize(c.stream));
     }
 
-    // the one-pass force (F-bar included) runs on cell tiles; the two-pass force keeps
-    // its entry forces in node order
-    const bool tiled = !two_pass;
-    if (tiled) {
-        rk_tile_plan(c);
-        D.inc_cell.release();
-    }
-    // node -> entries naming it, ascending entry (stable radix sort by node)
-    if (!tiled) {
-        DevBuf<int32_t> vals, keys_sorted, ccount;
-        vals.alloc(std::max<int64_t>(D.nnz, 1));
-        keys_sorted.alloc(std::max<int64_t>(D.nnz, 1));
-        D.node_inc.release();
-        DevBuf<int32_t> inc;
-        inc.alloc(std::max<int64_t>(D.nnz, 1));
-        hipLaunchKernelGGL(k_iota, grid1(D.nnz, 256), dim3(256), 0, c.stream, D.nnz, vals.p);
-        int bits = 1;
-        while (((int64_t)1 << bits) < nn) ++bits;
-        stable_sort_pairs(c, D.nodes.p, keys_sorted.p, vals.p, inc.p, D.nnz, bits);
-        ccount.alloc(nn);
-        ccount.zero(c.stream);
-        hipLaunchKernelGGL(k_count_keys, grid1(D.nnz, 256), dim3(256), 0, c.stream, D.nnz, D.nodes.p, ccount.p);
-        scan_counts(c, ccount, nn, D.node_start, nullptr);
-        D.entry_pos.alloc(std::max<int64_t>(D.nnz, 1));
-        hipLaunchKernelGGL(k_invert_perm, grid1(D.nnz, 256), dim3(256), 0, c.stream, D.nnz, inc.p, D.entry_pos.p);
-        APHIP_HIP(hipGetLastError());
-    }
-    if (two_pass) D.g.alloc(3 * std::max<int64_t>(D.nnz, 1));
+    if (D.nodal) rk_tile_plan(c);  // nodal cells run on cell tiles, element cells on the element tile plan
     APHIP_HIP(hipStreamSynchronize(c.stream));
     D.ready = true;
 }
@@ -1918,117 +1704,54 @@ static void rk_tile_force(Ctx &c) {
     APHIP_HIP(hipGetLastError());
 }
 
-// The two-pass cells of a Tet4 background are the elements themselves with the
-// element's own gradient (the smoothed gradient of a linear tet), so their force is the
-// Gauss Tet4 element force on the physical displacement: the element tile plan computes it
-// with the deterministic LDS gather and no per-entry force array.  Not for the damage
-// material, whose smoothed-cell update marks new failures differently
-// (ComputeInternalForceSmoothedCell.h:219-223).
-static bool two_pass_on_tiles(const Ctx &c) {
-    return c.cells.two_pass && c.etype == APHIP_TET4 && c.tiles.ready && c.mat.kind != APHIP_NEO_HOOKEAN_DAMAGE;
-}
-
-void rk_cell_force(Ctx &c) {
+void rk_cell_force(Ctx &c, bool keep) {
     CellData &D = c.cells;
-    if (D.two_pass) {  // physical displacement = Phi d (ExplicitSolver::ComputeForce, Explicit.cpp:148-152)
-        const int64_t nbg = padded_groups(c.nn, kGsLanes);
-        RkGatherArgs G{c.nn, nbg, D.num_nbr.p, D.nbr.p, D.phi.p, c.u.p, D.u_phys.p};
-        hipLaunchKernelGGL(k_rk_gather<kGsLanes>, dim3((unsigned)nbg), dim3(256), 0, c.stream, G);
-        APHIP_HIP(hipGetLastError());
-        if (two_pass_on_tiles(c)) {
-            const bool prof = c.prof.enabled;  // timed as this force pass, not as tile launches
-            c.prof.enabled = false;
-            tile_run(c, 0.0, 0, D.u_phys.p, D.f_local.p);
-            c.prof.enabled = prof;
-            return;
-        }
-    }
-    if (D.ncells == 0) return;
-    if (D.tiled && !D.fbar) {
-        rk_tile_force(c);
-        return;
-    }
-    const int64_t nbc = padded_groups(D.ncells, D.two_pass ? 1 : kCellLanes);
-    CellForceArgs A{D.ncells, nbc, D.start.p, D.nodes.p, D.dphi.p, D.volume.p, D.two_pass ? D.u_phys.p : c.u.p,
-                    c.Hnp1().p, c.Pnp1().p, D.g.p, D.entry_pos.p,
-                    c.state[1 - c.state_np1].p, c.state[c.state_np1].p,
-                    c.mat.params(),
-                    c.has_fields ? c.elem_lambda.p : nullptr, c.has_fields ? c.elem_mu.p : nullptr,
-                    c.mat.rate_form() ? c.Hn().p : nullptr, c.mat.rate_form() ? c.Pn().p : nullptr, c.rate_dt};
-    const dim3 g((unsigned)nbc);
+    if (D.ncells == 0) return;  // no cells: f_local stays zero
     if (D.fbar) {
         rk_fbar_tiles(c);
         return;
     }
-    if (D.two_pass) {
-        const double *X = c.X.p;
-        const bool hex = c.etype == APHIP_HEX8;
-        auto go = [&](auto k4, auto k8) {
-            hipLaunchKernelGGL(hex ? k8 : k4, g, dim3(256), 0, c.stream, A, X);
-        };
-        switch (c.mat.kind) {
-            case APHIP_LINEAR_ELASTIC:
-                go(k_rk_cells_two_pass<APHIP_LINEAR_ELASTIC, 4>, k_rk_cells_two_pass<APHIP_LINEAR_ELASTIC, 8>);
-                break;
-            case APHIP_NEO_HOOKEAN:
-                go(k_rk_cells_two_pass<APHIP_NEO_HOOKEAN, 4>, k_rk_cells_two_pass<APHIP_NEO_HOOKEAN, 8>);
-                break;
-            case APHIP_J2: go(k_rk_cells_two_pass<APHIP_J2, 4>, k_rk_cells_two_pass<APHIP_J2, 8>); break;
-            case APHIP_SVK: go(k_rk_cells_two_pass<APHIP_SVK, 4>, k_rk_cells_two_pass<APHIP_SVK, 8>); break;
-            case APHIP_NEO_HOOKEAN_DAMAGE:
-                go(k_rk_cells_two_pass<APHIP_NEO_HOOKEAN_DAMAGE, 4>, k_rk_cells_two_pass<APHIP_NEO_HOOKEAN_DAMAGE, 8>);
-                break;
-            case APHIP_POWER_LAW_CREEP:
-                go(k_rk_cells_two_pass<APHIP_POWER_LAW_CREEP, 4>, k_rk_cells_two_pass<APHIP_POWER_LAW_CREEP, 8>);
-                break;
-            case APHIP_DRUCKER_PRAGER:
-                go(k_rk_cells_two_pass<APHIP_DRUCKER_PRAGER, 4>, k_rk_cells_two_pass<APHIP_DRUCKER_PRAGER, 8>);
-                break;
-            default: throw Error(APHIP_ERR_INVALID, "material not set");
-        }
+    if (D.nodal) {
+        rk_tile_force(c);
+        return;
     }
+    // physical displacement = Phi d (ExplicitSolver::ComputeForce, Explicit.cpp:148-152), then
+    // the element tiles
+    const int64_t nbg = padded_groups(c.nn, kGsLanes);
+    RkGatherArgs G{c.nn, nbg, D.num_nbr.p, D.nbr.p, D.phi.p, c.u.p, D.u_phys.p, D.two_pass};
+    hipLaunchKernelGGL(k_rk_gather<kGsLanes>, dim3((unsigned)nbg), dim3(256), 0, c.stream, G);
     APHIP_HIP(hipGetLastError());
+    const bool prof = c.prof.enabled;  // timed as this force pass, not as tile launches
+    c.prof.enabled = false;
+    TileRun run;
+    run.u_in = D.u_phys.p;
+    run.f_out = D.f_local.p;
+    run.keep = keep;
+    tile_run(c, 0.0, 0, run);
+    c.prof.enabled = prof;
 }
 
-void rk_node_update(Ctx &c, double dt, int mode) {
+void rk_node_update(Ctx &c, double dt, int mode, bool more) {
     CellData &D = c.cells;
-    const int64_t nbn = padded_groups(c.nn);
-    const dim3 g((unsigned)nbn);
-    RkNodeArgs A{c.nn, nbn, D.node_start.p, D.g.p, c.mass.p,
-                 c.has_fixed ? c.fixed.p : nullptr, c.f.p, c.a.p, c.v.p, dt};
-    if (D.two_pass) {
-        // cell entries -> local force (unless the element tiles assembled it), then
-        // f = Phi^T f_local with the node update (ScatterValues, Explicit.cpp:181-186)
-        if (!two_pass_on_tiles(c)) {
-            RkNodeArgs L = A;
-            L.f = D.f_local.p;
-            hipLaunchKernelGGL(k_rk_nodes<0>, g, dim3(256), 0, c.stream, L);
-            APHIP_HIP(hipGetLastError());
-        }
-        RkScatterArgs S{A, D.num_nbr.p, D.rstart.p, D.rsrc.p, D.rphi.p, D.f_local.p};
+    // nodes with degrees of freedom only (nodal cells put them first; the others keep
+    // their values, as the reference's integrator runs over the active part)
+    const int lanes = D.nodal ? kSlotLanes : kCellLanes;
+    const int64_t nb = padded_groups(c.n_dof, lanes);
+    const dim3 g((unsigned)nb);
+    const RkNodeArgs A{c.n_dof, nb, c.mass.p, c.has_fixed ? c.fixed.p : nullptr, c.f.p, c.a.p, c.v.p, c.u.p, dt, more};
+    if (D.nodal) {
+        const RkSlotNodeArgs N{A, D.nslot_start.p, D.nslot.p, D.slots.p};
+        if (mode == 0) hipLaunchKernelGGL((k_rk_slot_nodes<0, kSlotLanes>), g, dim3(256), 0, c.stream, N);
+        else if (mode == 1) hipLaunchKernelGGL((k_rk_slot_nodes<1, kSlotLanes>), g, dim3(256), 0, c.stream, N);
+        else hipLaunchKernelGGL((k_rk_slot_nodes<2, kSlotLanes>), g, dim3(256), 0, c.stream, N);
+    } else {  // f = Phi^T f_local with the node update (ScatterValues, Explicit.cpp:181-186)
+        const RkScatterArgs S{A, D.num_nbr.p, D.rstart.p, D.rsrc.p, D.rphi.p, D.f_local.p, D.two_pass};
         constexpr int NB = (kMaxNbr + kCellLanes - 1) / kCellLanes;
         if (mode == 0) hipLaunchKernelGGL((k_rk_scatter<0, kCellLanes, NB>), g, dim3(256), 0, c.stream, S);
         else if (mode == 1) hipLaunchKernelGGL((k_rk_scatter<1, kCellLanes, NB>), g, dim3(256), 0, c.stream, S);
         else hipLaunchKernelGGL((k_rk_scatter<2, kCellLanes, NB>), g, dim3(256), 0, c.stream, S);
-        APHIP_HIP(hipGetLastError());
-        return;
     }
-    // nodes with degrees of freedom only (nodal cells put them first; the others keep
-    // their values, as the reference's integrator runs over the active part)
-    if (D.tiled) {
-        constexpr int kSlotLanes = 8;
-        const int64_t nbs = padded_groups(c.n_dof, kSlotLanes);
-        RkSlotNodeArgs N{A, D.nslot_start.p, D.nslot.p, D.slots.p};
-        N.out.nn = c.n_dof;
-        N.out.nblocks = nbs;
-        const dim3 gs((unsigned)nbs);
-        if (mode == 0) hipLaunchKernelGGL((k_rk_slot_nodes<0, kSlotLanes>), gs, dim3(256), 0, c.stream, N);
-        else if (mode == 1) hipLaunchKernelGGL((k_rk_slot_nodes<1, kSlotLanes>), gs, dim3(256), 0, c.stream, N);
-        else hipLaunchKernelGGL((k_rk_slot_nodes<2, kSlotLanes>), gs, dim3(256), 0, c.stream, N);
-        APHIP_HIP(hipGetLastError());
-        return;
-    }
-    throw Error(APHIP_ERR_INVALID, "one-pass cells without a tile plan");
+    APHIP_HIP(hipGetLastError());
 }
 
 void rk_mass(Ctx &c, double *total) {

@@ -91,6 +91,7 @@ struct TileArgs {
     int64_t first_shared;
     // 0: an inner step of one call, whose H, P and f the next step overwrites unread
     int keep;
+    int cell_marker;  // smoothed cells turn a new failure's marker into the maximum damage
 };
 
 // LDS carve-up (bytes), sized on the host (tile_lds_bytes) from maxtn, max_nint, te
@@ -190,7 +191,8 @@ __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L,
 
 // MODE 0: force only; 1: force + a = f/m (initial); 2: full central-difference step.
 // QPAR (Hex8 only): eight lanes per element, one per Gauss point.
-template <int NPE, int KIND, bool PER_QP, int MODE, bool QPAR>
+// CELL (Hex8 only): smoothed Hex8 cells instead of 2x2x2 Gauss elements.
+template <int NPE, int KIND, bool PER_QP, int MODE, bool QPAR, bool CELL = false>
 __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !QPAR ? 2 : 1) void k_tile(TileArgs A) {
     extern __shared__ __align__(16) char lds_raw[];
     const int64_t t = xcd_tile(A.nblocks);
@@ -393,11 +395,14 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
         if constexpr (NPE == 4) {
             double snp1 = 0.0, aux = 0.0;
             tet4_element<KIND>(X, U, m, sn, snp1, aux, H, P, fe, &rin, sn2);
+            if (A.cell_marker) snp1 = cell_damage_marker<KIND>(snp1, m);
             store_state<KIND>(A.state_np1, e, snp1, aux);
         } else {
             const int64_t so = state_width<KIND>() * (PER_QP ? e * 8 : e);
-            hex8_element<KIND, PER_QP>(X, U, m, A.gauss_a, state_width<KIND>() ? A.state_n + so : nullptr,
-                                       state_width<KIND>() ? A.state_np1 + so : nullptr, H, P, fe, &rin);
+            const double *sn_p = state_width<KIND>() ? A.state_n + so : nullptr;
+            double *snp1_p = state_width<KIND>() ? A.state_np1 + so : nullptr;
+            if constexpr (CELL) hex8_cell<KIND>(X, U, m, sn_p, snp1_p, H, P, fe, &rin);
+            else hex8_element<KIND, PER_QP>(X, U, m, A.gauss_a, sn_p, snp1_p, H, P, fe, &rin);
         }
         if constexpr (NPE == 4) {
 #pragma unroll
@@ -863,19 +868,24 @@ inline int64_t padded(int64_t n) { return ((n + kNumXcd - 1) / kNumXcd) * kNumXc
 
 template <int NPE, int KIND, bool PER_QP, int MODE>
 void launch_tile(Ctx &c, const TileArgs &A, size_t lds) {
+    auto go = [&](auto kern) {
+        if (lds > 65536)
+            APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(c.tiles.threads), lds, c.stream, A);
+    };
     if constexpr (NPE == 8) {
         if (c.tiles.threads == 8 * c.tiles.te) {
-            auto kq = k_tile<NPE, KIND, PER_QP, MODE, true>;
-            if (lds > 65536)
-                APHIP_HIP(hipFuncSetAttribute((const void *)kq, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(kq, dim3((unsigned)A.nblocks), dim3(c.tiles.threads), lds, c.stream, A);
+            go(k_tile<NPE, KIND, PER_QP, MODE, true>);
             return;
         }
+        if constexpr (MODE == 0 && !PER_QP) {
+            if (c.cells.ready) {
+                go(k_tile<NPE, KIND, false, 0, false, true>);
+                return;
+            }
+        }
     }
-    auto kern = k_tile<NPE, KIND, PER_QP, MODE, false>;
-    if (lds > 65536)
-        APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(c.tiles.threads), lds, c.stream, A);
+    go(k_tile<NPE, KIND, PER_QP, MODE, false>);
 }
 
 template <int KIND>
@@ -1144,21 +1154,23 @@ void tile_build(Ctx &c, int te, int threads) {
     APHIP_HIP(hipStreamSynchronize(c.stream));
 }
 
-void tile_run(Ctx &c, double dt, int mode, const double *u_in, double *f_out, bool pred_in, bool pred_out,
-              bool keep) {
+void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     TilePlan &P = c.tiles;
     APHIP_REQUIRE(P.ready, "tile plan not built");
-    APHIP_REQUIRE(mode == 0 || (u_in == nullptr && f_out == nullptr), "displacement / force arrays only in force mode");
-    APHIP_REQUIRE(mode == 2 || !(pred_in || pred_out), "predicted displacements only in step mode");
-    pred_in = pred_in && P.nb > 0;
-    pred_out = pred_out && P.nb > 0;
+    APHIP_REQUIRE(mode == 0 || (run.u_in == nullptr && run.f_out == nullptr),
+                  "displacement / force arrays only in force mode");
+    APHIP_REQUIRE(mode == 2 || !(run.pred_in || run.pred_out), "predicted displacements only in step mode");
+    const bool pred_in = run.pred_in && P.nb > 0, pred_out = run.pred_out && P.nb > 0;
+    // smoothed Hex8 cells have a B of their own (a smoothed Tet4's is its gradient)
+    const bool cells8 = c.npe == 8 && c.cells.ready;
+    APHIP_REQUIRE(!cells8 || (mode == 0 && P.threads == P.te), "Hex8 cells: force mode, one cell per thread");
     if (c.ne == 0) return;
     TileArgs A;
     A.X = c.X.p;
-    A.u = u_in ? const_cast<double *>(u_in) : c.u.p;
+    A.u = run.u_in ? const_cast<double *>(run.u_in) : c.u.p;
     A.v = c.v.p;
     A.a = c.a.p;
-    A.f = f_out ? f_out : c.f.p;
+    A.f = run.f_out ? run.f_out : c.f.p;
     A.mass = c.mass.p;
     A.fixed = c.has_fixed ? c.fixed.p : nullptr;
     A.tn_start = P.tn_start.p;
@@ -1201,7 +1213,8 @@ void tile_run(Ctx &c, double dt, int mode, const double *u_in, double *f_out, bo
     A.dt = dt;
     A.upred = pred_in ? P.upred.p : nullptr;
     A.first_shared = P.n_interior;
-    A.keep = keep || c.mat.rate_form();  // (the rate-form materials read the previous H and P)
+    A.cell_marker = c.cells.ready;
+    A.keep = run.keep || c.mat.rate_form();  // (the rate-form materials read the previous H and P)
     prof_begin(c, 1);
     if (c.npe == 4) {
         if (mode == 0) dispatch_kind<4, 0>(c, A, P.lds_bytes);

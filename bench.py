@@ -437,16 +437,12 @@ def bench_rkpm(n_nodes_edge=64, steps=100, scale=1.5, one_pass=True):
     yielded = int((s.get(A.FIELD_STATE) > 0).sum())
     s.close()
     lc = nnz / ne
-    # one-pass, per cell: entries (4 B id + 24 B grad) + H, P, volume, J2 state N/NP1;
-    # per node: the node streams.  Two-pass, per cell: the four node ids + H, P, J2 state
-    # (the derivatives and volume follow from X, part of the node streams); per node: the
-    # node streams, the neighbor rows of the gather and of the scatter (4 B id + 8 B phi
-    # per neighbor each) and the physical displacement and local force, each written
-    # once and read once
-    if one_pass:
-        bytes_per_update = 28.0 * lc + 168.0 + 200.0 * nn / ne
-    else:
-        bytes_per_update = 16.0 + 160.0 + (200.0 + 96.0 + 24.0 * float(num.mean())) * nn / ne
+    # both methods apply the factors of the cell derivatives.  Per cell: the four node ids and
+    # the J2 state read and written; H and P once per call.  Per node: the neighbor rows of the
+    # gather and of the scatter (4 B id + 8 B phi per neighbor each); u, the physical
+    # displacement and the local force written and read, X, v and the mass read, u and v
+    # written; f and a once per call
+    bytes_per_update = 16.0 + 16.0 + (248.0 + 24.0 * float(num.mean())) * nn / ne + (144.0 + 48.0 * nn / ne) / steps
     step_ms = m0 / max(n0, 1)
     achieved = bytes_per_update * ne / (step_ms * 1e-3) / 1e9
     method = "one-pass" if one_pass else "two-pass"
@@ -455,8 +451,8 @@ def bench_rkpm(n_nodes_edge=64, steps=100, scale=1.5, one_pass=True):
             "setup_s": t_setup, "mean_neighbors": float(num.mean()), "max_neighbors": int(num.max()),
             "extra_neighbors": int(truncated), "cell_list_mean": lc,
             "cell_updates_per_s": ne * steps / wall, "ms_per_step": 1e3 * wall / steps,
-            "kernels_ms": {"step": step_ms, "cell_force" if one_pass else "gather_and_cell_force": m1 / max(n1, 1),
-                           "node_gather" if one_pass else "node_sum_and_scatter": m2 / max(n2, 1)},
+            "kernels_ms": {"step": step_ms, "gather_and_cell_force": m1 / max(n1, 1),
+                           "scatter": m2 / max(n2, 1)},
             "roofline": {"bound": "hbm", "bytes_per_update": bytes_per_update, "achieved": achieved,
                          "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS},
             "yielded_cells": yielded}

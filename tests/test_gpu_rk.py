@@ -420,3 +420,83 @@ def test_one_pass_tiles_are_deterministic_and_size_independent(gpu_available, mo
     assert ref.state.max() > 0.0
     for g, rf in ((u, ref.u), (v, ref.v), (f, ref.f), (P, ref.P), (st, ref.state)):
         assert rel_err(g, rf) < 1e-10
+
+
+# ---- element cells on the element tile plan -------------------------------------
+
+@pytest.mark.parametrize("etype", [A.TET4, A.HEX8])
+@pytest.mark.parametrize("route", ["default", "two-pass flag", "eight lanes or 64 tiles", "after nodal cells"])
+@pytest.mark.parametrize("one_pass", [True, False])
+def test_element_cells_force_from_every_plan(gpu_available, etype, route, one_pass):
+    """The factored cell force (u = Phi d, element tiles, Phi^T) against the oracle's cell
+    forces for every state of the context's tile plan before the RK set-up: the default
+    plan, none (APHIP_FLAG_TWO_PASS, or dropped by an earlier nodal set-up), another shape."""
+    if route == "after nodal cells":
+        if etype == A.TET4:
+            pytest.skip("nodal cells need a Hex8 mesh")
+        X, conn = M.thex_block(2, 5)
+    else:
+        X, hc = M.hex_lattice(5, 6, 7, 5 / 7, 6 / 7, 1.0)
+        X = M.jitter(X, 1 / 7, 0.1, 3, 1)
+        conn = M.split_tets(X, hc) if etype == A.TET4 else hc
+    scale = 1.3
+    r = O.kernel_radius(O.max_edge_length(X, conn), scale)
+    num, nbr, _ = O.neighbor_search(X, r)
+    phi = O.rk_function_values(X, r, num, nbr)
+    cells = O.rk_cells(X, conn, num, nbr, phi)
+    lam, mu = O.lame(J2["E"], J2["nu"])
+    u = 4e-3 * (2 * M.uniform01(8, 7, X.size).reshape(X.shape) - 1)
+    f, H, P, st = O.cell_internal_force(len(X), cells, O.J2, lam, mu, u, yield_stress=J2["yield_stress"],
+                                        hardening=J2["hardening"])
+    print(f"element cells etype={etype} {route} one_pass={one_pass}: {len(X)} nodes, {len(conn)} cells", flush=True)
+    with A.Solver(flags=A.FLAG_TWO_PASS if route == "two-pass flag" else 0) as s:
+        s.set_mesh(etype, X, conn)
+        s.set_material(A.J2, J2["rho"], J2["E"], J2["nu"], J2["yield_stress"], J2["hardening"])
+        if route == "eight lanes or 64 tiles":
+            s.set_tiling(*((16, 128) if etype == A.HEX8 else (64, 64)))
+        if route == "after nodal cells":
+            s.rk_nodal_setup(0.9, 0, True)
+        s.rk_setup(scale, one_pass=one_pass)
+        s.set_field(A.FIELD_U, u)
+        s.internal_force()
+        for fld, ref in ((A.FIELD_F, f), (A.FIELD_H, H), (A.FIELD_P, P), (A.FIELD_STATE, st)):
+            assert rel_err(s.get(fld), ref) < 1e-12, fld
+
+
+@pytest.mark.parametrize("cells", ["one-pass", "two-pass", "fe", "nodal", "f-bar"])
+def test_cell_steps_of_one_call_match_single_steps(gpu_available, cells):
+    """A call's steps hand the next step's predictor on and store H, P, f and a at the last
+    step only: calls of 1, 2 and 5 steps, and graph replay, give the same bits (fixed DOFs)."""
+    if cells in ("nodal", "f-bar"):
+        X, conn = M.thex_block(2, 5)
+    else:
+        X, hc = M.hex_lattice(4, 5, 3, 4 / 5, 1.0, 3 / 5)
+        X = M.jitter(X, 1 / 5, 0.1, 3, 1)
+        conn = M.split_tets(X, hc)
+    kind = A.SVK if cells == "f-bar" else A.J2
+    fixed = np.zeros(X.shape, dtype=np.uint8)
+    fixed[X[:, 2] < 0.05] = (1, 0, 1)
+    v0 = 40.0 * (2 * M.uniform01(9, 4, X.size).reshape(X.shape) - 1)
+    dt = 0.2 * M.stable_dt_estimate(X, conn, J2["E"], J2["nu"], J2["rho"])
+    out = []
+    for calls, graph in (([1] * 10, False), ([2] * 5, False), ([5, 5], False), ([4, 6], True)):
+        with A.Solver() as s:
+            s.set_mesh(A.HEX8 if conn.shape[1] == 8 else A.TET4, X, conn)
+            s.set_material(kind, J2["rho"], J2["E"], J2["nu"], J2["yield_stress"], J2["hardening"])
+            if cells == "fe":
+                s.strain_smoothing_setup()
+            elif cells in ("nodal", "f-bar"):
+                s.rk_nodal_setup(0.9, 0, cells == "f-bar")
+            else:
+                s.rk_setup(1.5, one_pass=cells == "one-pass")
+            s.compute_mass()
+            s.set_fixed(fixed)
+            s.set_field(A.FIELD_V, v0)
+            s.set_graph(graph)
+            s.initialize()
+            for n in calls:
+                s.step(dt, n)
+            out.append([s.get(f) for f in (A.FIELD_U, A.FIELD_V, A.FIELD_A, A.FIELD_F, A.FIELD_H, A.FIELD_P)])
+    for o in out[1:]:
+        for a, b in zip(out[0], o):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
