@@ -331,6 +331,11 @@ static bool use_tiles(const Ctx &c) {
     return c.tiles.ready && !(c.flags & APHIP_FLAG_TWO_PASS) && c.formulation == APHIP_TOTAL_LAGRANGIAN;
 }
 
+// Graph replay keeps the tile kernels: a patch launch exchanges the buffers of u, v and a.
+static bool steps_on_patches(Ctx &c) {
+    return use_tiles(c) && !c.cells.ready && !c.graph_enabled && patch_eligible(c);
+}
+
 static void default_tiling(Ctx &c) {
     if (c.ne == 0 || (c.flags & APHIP_FLAG_TWO_PASS)) return;
     if (c.etype == APHIP_TET4) {
@@ -370,6 +375,7 @@ static void setup_mesh(Ctx &c, int32_t elem_type, int64_t n_nodes, const double 
     c.pm_l_valid = false;
     for (DevBuf<double> &b : c.pm_work) b.release();
     c.tiles.reset();
+    c.patch.reset();
     c.graph_reset();
     c.etype = elem_type;
     c.npe = npe;
@@ -1221,6 +1227,7 @@ int aphip_initialize(aphip_ctx *c) {
     c->steps_done = 0;
     APHIP_HIP(hipSetDevice(c->device));
     if (use_tiles(*c)) {
+        (void)steps_on_patches(*c);  // builds the steps' plan before the first of them
         tile_run(*c, 0.0, 1);
     } else {
         force_pass(*c);
@@ -1262,6 +1269,19 @@ int aphip_step(aphip_ctx *c, double dt, int32_t n_steps) {
             c->graph_parity = parity;
         }
         for (; done + 2 <= n_steps; done += 2) APHIP_HIP(hipGraphLaunch(c->graph_exec, c->stream));
+    }
+    if (steps_on_patches(*c)) {  // small meshes: several steps per launch
+        while (done < n_steps) {
+            const int k = patch_steps(*c, n_steps - done);
+            prof_begin(*c, 0);
+            c->state_np1 = 1 - c->state_np1;
+            c->rate_dt = dt;
+            prof_begin(*c, 1);
+            patch_run(*c, dt, k, done + k == n_steps);
+            prof_end(*c, 1);
+            prof_end(*c, 0);
+            done += k;
+        }
     }
     for (bool pred = false; done < n_steps; ++done) {
         const bool more = done + 1 < n_steps && c->formulation != APHIP_SEMI_LAGRANGIAN;

@@ -18,30 +18,32 @@ namespace aphip {
 // bit-identical arithmetic.
 //   predictor  v1/2 = v + dt/2 a, velocity BC, u1 = u + dt v1/2  (ExplicitTimeIntegrator.h:116-126, :348-357)
 //   corrector  a = f/m, acceleration BC, v = v1/2 + dt/2 a       (ExplicitTimeIntegrator.h:267-276, :308-318)
+APHIP_DEV void cd_predict1(double u, double v, double a, bool fixed, double dt, double &vh, double &u1) {
+#pragma clang fp contract(off)
+    double w = __fma_rn(0.5 * dt, a, v);
+    if (fixed) w = 0.0;
+    vh = w;
+    u1 = __fma_rn(dt, w, u);
+}
+
+APHIP_DEV void cd_correct1(double f, double m, bool fixed, double dt, double vh, double &a1, double &v1) {
+#pragma clang fp contract(off)
+    double acc = f / m;
+    if (fixed) acc = 0.0;
+    a1 = acc;
+    v1 = __fma_rn(0.5 * dt, acc, vh);
+}
+
 APHIP_DEV void cd_predict(const double *u, const double *v, const double *a, unsigned fixed, double dt, double *vh,
                           double *u1) {
-#pragma clang fp contract(off)
-    const double h = 0.5 * dt;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        double w = __fma_rn(h, a[d], v[d]);
-        if (fixed & (1u << d)) w = 0.0;
-        vh[d] = w;
-        u1[d] = __fma_rn(dt, w, u[d]);
-    }
+    for (int d = 0; d < 3; ++d) cd_predict1(u[d], v[d], a[d], fixed & (1u << d), dt, vh[d], u1[d]);
 }
 
 APHIP_DEV void cd_correct(const double *f, double m, unsigned fixed, double dt, const double *vh, double *a1,
                           double *v1) {
-#pragma clang fp contract(off)
-    const double h = 0.5 * dt;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        double acc = f[d] / m;
-        if (fixed & (1u << d)) acc = 0.0;
-        a1[d] = acc;
-        v1[d] = __fma_rn(h, acc, vh[d]);
-    }
+    for (int d = 0; d < 3; ++d) cd_correct1(f[d], m, fixed & (1u << d), dt, vh[d], a1[d], v1[d]);
 }
 
 // H, P and the state are written once per step and not read again in it: a

@@ -237,6 +237,34 @@ struct TilePlan {
     }
 };
 
+// Node patches of the small-mesh step (patch.hip), internal numbering.
+struct PatchPlan {
+    static constexpr int kRings = 4;  // most rings of a plan
+    bool ready = false;
+    bool tried = false;               // built, or found not to apply, for the current tile plan
+    int rings = 0;                    // rings of this plan: most steps per launch
+    int threads = 0;
+    int64_t npatch = 0;
+    int npad = 0, cpad = 0, epad = 0, entpad = 0;  // row counts of the padded lists below
+    size_t lds_bytes = 0;
+    DevBuf<unsigned char> lists;      // the lists below
+    const int32_t *meta = nullptr, *node = nullptr, *elem = nullptr;  // [npatch * 16 / npad / epad]
+    const uint32_t *csr = nullptr;                                    // [npatch * cpad]
+    const uint16_t *conn = nullptr, *ent = nullptr;                   // [npatch * epad * npe / entpad]
+    DevBuf<double> u, v, a;           // [nn * 3] the buffers the next launch writes
+    void reset() {
+        ready = tried = false;
+        rings = threads = npad = cpad = epad = entpad = 0;
+        npatch = 0;
+        lds_bytes = 0;
+        lists.release();
+        meta = node = elem = nullptr;
+        csr = nullptr;
+        conn = ent = nullptr;
+        u.release(); v.release(); a.release();
+    }
+};
+
 struct Profile {
     bool enabled = false;
     std::vector<hipEvent_t> ev;   // pairs (start, stop) tagged by which
@@ -345,6 +373,7 @@ struct Ctx {
 
     CellData cells;
     TilePlan tiles;
+    PatchPlan patch;
     AdjointData adj;
     Profile prof;
 
@@ -386,6 +415,15 @@ struct TileRun {
     bool keep = true;
 };
 void tile_run(Ctx &c, double dt, int mode, const TileRun &run = TileRun());
+
+// ---- small-mesh step on node patches (patch.hip) ----
+// Whether this context's total-Lagrangian steps run on patches (builds the plan on first use:
+// aphip_initialize, or the first step without it).
+bool patch_eligible(Ctx &c);
+int patch_steps(const Ctx &c, int left);
+// `steps` steps in one launch (the state buffers' roles were swapped once by the caller);
+// keep: store H, P and f of the last one
+void patch_run(Ctx &c, double dt, int steps, bool keep);
 
 // ---- adjoint (adjoint.hip) ----
 void adjoint_forward(Ctx &c, double dt, int n_steps, int interval);

@@ -1,0 +1,496 @@
+// Small meshes: several central-difference steps of a node patch per launch.
+//
+// A mesh of some thousand elements fills a few of the tile plan's workgroups and leaves most of
+// the chip idle, and a step is two dependent launches (about 3.4 us of host time each, 12 us of
+// device time a step on 6,174 Tet4).  Here a workgroup owns a patch of neighbouring nodes and
+// recomputes what it needs from its neighbours instead of exchanging it: with K rings,
+//   N_0 = the owned nodes, E_r = the elements around N_{r-1}, N_r = the nodes of E_r
+// (E_1 also holds the elements the patch owns, a run of the element order; a node belongs to
+// the patch of its lowest element),
+// it stages N_k (k <= K), and step s = 1..k evaluates E_{k-s+1} and finishes N_{k-s} in LDS;
+// after the last step it writes its owned nodes, and, of the elements it owns, the state (and H
+// and P if the call ends here).  No workgroup waits for another and nothing is exchanged: u, v
+// and a are read from one set of buffers and written to another, which the host exchanges.
+//
+// The price is the elements evaluated by several patches, so the plan is for small meshes only
+// (the rule is at patch_build).  What bounds it is latency: the launch, two dependent loads,
+// and per step the element's arithmetic and LDS reads (6,174 SVK Tet4, 50 steps in one call:
+// 338 -> about 115 us with three meshes in turn, 595 -> 290 us alone; 49,392 Tet4, one step a
+// call: 7.6 -> 5.2 us a step in turn, 14 -> 11 us alone).  Results are the tile path's, bit for bit: the element
+// arithmetic is the same and a node's sum is grouped by the plan's tiles (partial sums of the
+// node's elements in ascending order, added in ascending tile order).
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <thread>
+#include <vector>
+
+#include "element.hpp"
+#include "internal.hpp"
+
+namespace aphip {
+
+namespace {
+
+constexpr int kNumXcd = 8;
+constexpr int kRings = PatchPlan::kRings;
+constexpr uint16_t kNewTile = 0x8000;   // entry flag: the node's first element of another tile
+constexpr int kBatch = 8;               // entries of a node are padded to a multiple of this
+
+__device__ __forceinline__ void ld3(const double *p, int64_t i, double *o) {
+    o[0] = p[3 * i];
+    o[1] = p[3 * i + 1];
+    o[2] = p[3 * i + 2];
+}
+
+__device__ __forceinline__ void st3(double *p, int64_t i, const double *o) {
+    p[3 * i] = o[0];
+    p[3 * i + 1] = o[1];
+    p[3 * i + 2] = o[2];
+}
+
+struct PatchArgs {
+    const double *X;
+    const double *u, *v, *a;     // state read
+    double *u1, *v1, *a1, *f;    // state written (other buffers)
+    const double *mass;
+    const uint8_t *fixed;
+    const double *zero;          // 8 zero doubles: stands in for an absent optional array
+    const int32_t *meta;         // [npatch * 16] nodes per ring at 0, elements per ring at 8 (owned: at 8)
+    const int32_t *node;         // [npatch * npad] node ids, ring by ring
+    const uint32_t *csr;         // [npatch * cpad] (start << 16) | count of the nodes N_{K-1}
+    const int32_t *elem;         // [npatch * epad] element ids, owned ones first, ring by ring
+    const uint16_t *conn;        // [npatch * epad * npe] local nodes
+    const uint16_t *ent;         // [npatch * entpad] force row of the entry (| kNewTile)
+    double *H, *P;
+    const double *state_n;
+    double *state_np1;
+    MatParams mat;
+    const double *elem_lambda, *elem_mu;
+    double dt;
+    int64_t ne, npatch, nblocks;
+    int npad, cpad, epad, entpad;
+    int steps, keep;
+};
+
+// LDS carve-up (bytes), sized on the host with the same function
+struct PatchLds {
+    double *X, *U, *V, *M, *S, *F;
+    uint32_t *csr;
+    uint16_t *conn, *ent;
+    uint8_t *fx;
+    size_t bytes;
+};
+
+// rows between the slot blocks of the force rows (as in the tile kernel: the slots of one
+// element sit 24 banks apart)
+__host__ __device__ __forceinline__ int f_stride(int n) { return n + ((4 - n) & 31); }
+
+__host__ __device__ __forceinline__ PatchLds carve(char *base, int npe, int npad, int cpad, int epad, int entpad) {
+    PatchLds L;
+    char *p = base;
+    auto take = [&](size_t n) {
+        char *q = p;
+        p += (n + 15) & ~(size_t)15;
+        return q;
+    };
+    L.X = reinterpret_cast<double *>(take(24 * (size_t)npad));
+    L.U = reinterpret_cast<double *>(take(24 * (size_t)npad));
+    L.V = reinterpret_cast<double *>(take(24 * (size_t)npad));
+    L.M = reinterpret_cast<double *>(take(8 * (size_t)cpad));
+    L.S = reinterpret_cast<double *>(take(8 * (size_t)epad));
+    L.F = reinterpret_cast<double *>(take(24 * (size_t)npe * f_stride(epad)));
+    L.csr = reinterpret_cast<uint32_t *>(take(4 * (size_t)cpad));
+    L.conn = reinterpret_cast<uint16_t *>(take(2 * (size_t)npe * epad));
+    L.ent = reinterpret_cast<uint16_t *>(take(2 * (size_t)entpad));
+    L.fx = reinterpret_cast<uint8_t *>(take((size_t)npad));
+    L.bytes = (size_t)(p - base);
+    return L;
+}
+
+template <int NPE, int KIND>
+__global__ __launch_bounds__(1024) void k_patch(PatchArgs A) {
+    extern __shared__ __align__(16) char lds_raw[];
+    const int64_t b = blockIdx.x;
+    const int64_t p = (b % kNumXcd) * (A.nblocks / kNumXcd) + b / kNumXcd;  // neighbours share an XCD's L2
+    if (p >= A.npatch) return;
+    const PatchLds L = carve(lds_raw, NPE, A.npad, A.cpad, A.epad, A.entpad);
+    const int tid = threadIdx.x, nt = blockDim.x;
+    // the first row of every list needs the patch id alone (the lists are padded to a fixed
+    // stride, rows past the end repeat the last one), so that staging is two memory latencies
+    const int32_t *node = A.node + p * A.npad;
+    const int32_t *elem = A.elem + p * A.epad;
+    const int32_t *meta = A.meta + 16 * p;
+    const int nN = meta[A.steps], nE = meta[8 + A.steps], nC = meta[A.steps - 1], nown = meta[8];
+    for (int i = tid; i < A.npad; i += nt) {
+        const int64_t g = node[i];
+        double x[3], u[3], v[3], a[3], vh[3], up[3];
+        ld3(A.X, g, x);
+        ld3(A.u, g, u);
+        ld3(A.v, g, v);
+        ld3(A.a, g, a);
+        const uint8_t *pf = A.fixed ? A.fixed : reinterpret_cast<const uint8_t *>(A.zero);
+        const unsigned f8 = pf[A.fixed ? g : 0], fx = A.fixed ? f8 : 0u;
+        const double m = A.mass[g];
+        cd_predict(u, v, a, fx, A.dt, vh, up);
+        if (i < nN) {
+            st3(L.X, i, x);
+            st3(L.U, i, up);
+            st3(L.V, i, vh);
+            L.fx[i] = (uint8_t)fx;
+            if (i < A.cpad) L.M[i] = m;
+        }
+    }
+    for (int i = tid; i < A.cpad; i += nt) L.csr[i] = A.csr[p * A.cpad + i];
+    {
+        const uint4 *src = reinterpret_cast<const uint4 *>(A.ent + p * A.entpad);
+        uint4 *dst = reinterpret_cast<uint4 *>(L.ent);
+        for (int i = tid; i < A.entpad / kBatch; i += nt) dst[i] = src[i];
+    }
+    for (int i = tid; i < A.epad; i += nt) {
+        reinterpret_cast<ushort4 *>(L.conn)[i] = reinterpret_cast<const ushort4 *>(A.conn + p * A.epad * NPE)[i];
+        if constexpr (state_width<KIND>() > 0) L.S[i] = load_state<KIND>(A.state_n, elem[i]);
+    }
+    __syncthreads();
+    const int fs = f_stride(A.epad);
+    int ne_now = nE, nn_now = nC;
+    for (int s = 1;; ++s) {
+        const bool last = s == A.steps;
+        for (int le = tid; le < ne_now; le += nt) {
+            const ushort4 c = reinterpret_cast<const ushort4 *>(L.conn)[le];
+            const int lc[4] = {c.x, c.y, c.z, c.w};
+            double X[NPE][3], U[NPE][3], fe[NPE][3], H[9], P[9];
+#pragma unroll
+            for (int k = 0; k < NPE; ++k) {
+                ld3(L.X, lc[k], X[k]);
+                ld3(L.U, lc[k], U[k]);
+            }
+            MatParams m = A.mat;
+            if (A.elem_lambda) {
+                const int64_t e = elem[le];
+                m.lambda = A.elem_lambda[e];
+                m.mu = A.elem_mu[e];
+            }
+            double sn = 0.0, snp1 = 0.0, aux = 0.0;
+            if constexpr (state_width<KIND>() > 0) sn = L.S[le];
+            tet4_element<KIND>(X, U, m, sn, snp1, aux, H, P, fe);
+#pragma unroll
+            for (int k = 0; k < NPE; ++k) st3(L.F, k * fs + le, fe[k]);
+            if (last) {
+                if (le < nown && (A.keep || state_width<KIND>() > 0)) {
+                    const int64_t e = elem[le];
+                    store_state<KIND>(A.state_np1, e, snp1, aux);
+                    if (A.keep) {
+#pragma unroll
+                        for (int i = 0; i < 9; ++i) {
+                            store_once(A.H + i * A.ne + e, H[i]);
+                            store_once(A.P + i * A.ne + e, P[i]);
+                        }
+                    }
+                }
+            } else if constexpr (state_width<KIND>() > 0) {
+                L.S[le] = snp1;
+            }
+        }
+        __syncthreads();
+        // four lanes per node, one per component (the fourth idles): the sums stay in order and
+        // the LDS latency is paid once per kBatch entries
+        for (int t4 = tid; t4 < 4 * nn_now; t4 += nt) {
+            const int ln = t4 >> 2, d = t4 & 3;
+            if (d == 3) continue;
+            const uint32_t pk = L.csr[ln];
+            const int st = (int)(pk >> 16) * kBatch, cnt = (int)(pk & 0xffffu);
+            const double *F = L.F + d;
+            double f = 0.0, t = 0.0;
+            for (int j = 0; j < cnt; j += kBatch) {
+                const uint4 w = *reinterpret_cast<const uint4 *>(L.ent + st + j);
+                const unsigned en[kBatch] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16,
+                                             w.z & 0xffffu, w.z >> 16, w.w & 0xffffu, w.w >> 16};
+                double r[kBatch];
+#pragma unroll
+                for (int q = 0; q < kBatch; ++q) r[q] = F[3 * (en[q] & 0x7fffu)];
+#pragma unroll
+                for (int q = 0; q < kBatch; ++q) {
+                    const bool fresh = en[q] & kNewTile;
+                    f = fresh ? f + t : f;
+                    t = fresh ? 0.0 : t;
+                    t = j + q < cnt ? t + r[q] : t;
+                }
+            }
+            f += t;
+            const bool fx = L.fx[ln] & (1u << d);
+            double a1, v1;
+            const double u1 = L.U[3 * ln + d];
+            cd_correct1(f, L.M[ln], fx, A.dt, L.V[3 * ln + d], a1, v1);
+            if (last) {
+                const int64_t g = 3 * (int64_t)node[ln] + d;
+                A.u1[g] = u1;
+                A.v1[g] = v1;
+                A.a1[g] = a1;
+                if (A.keep) A.f[g] = f;
+            } else {
+                cd_predict1(u1, v1, a1, fx, A.dt, L.V[3 * ln + d], L.U[3 * ln + d]);
+            }
+        }
+        if (last) return;
+        __syncthreads();
+        ne_now = meta[8 + A.steps - s];
+        nn_now = meta[A.steps - s - 1];
+    }
+}
+
+template <int NPE>
+void launch(Ctx &c, const PatchArgs &A) {
+    const PatchPlan &P = c.patch;
+    auto go = [&](auto kern) {
+        if (P.lds_bytes > 65536)
+            APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)P.lds_bytes));
+        hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(P.threads), P.lds_bytes, c.stream, A);
+        APHIP_HIP(hipGetLastError());
+    };
+    switch (c.mat.kind) {
+        case APHIP_LINEAR_ELASTIC: go(k_patch<NPE, APHIP_LINEAR_ELASTIC>); break;
+        case APHIP_NEO_HOOKEAN: go(k_patch<NPE, APHIP_NEO_HOOKEAN>); break;
+        case APHIP_J2: go(k_patch<NPE, APHIP_J2>); break;
+        case APHIP_SVK: go(k_patch<NPE, APHIP_SVK>); break;
+        default: throw Error(APHIP_ERR_INVALID, "material without a patch kernel");
+    }
+}
+
+}  // namespace
+
+// Steps that the next launch of a call with `left` steps to go takes.  A material with state
+// ends a call with a launch of one step: the N buffer must hold the state before the last step.
+int patch_steps(const Ctx &c, int left) {
+    const int k = std::min(left, c.patch.rings);
+    return c.mat.state_width() > 0 && left > 1 && k == left ? left - 1 : k;
+}
+
+// Plan for the current tile plan and numbering; none when the mesh is too large for it.
+static void patch_build(Ctx &c) {
+    PatchPlan &P = c.patch;
+    P.tried = true;
+    const int64_t nn = c.nn, ne = c.ne;
+    const int npe = c.npe;
+    // The lines, from calls of 20 steps on n^3 x 6 Tet4 lattices (neo-Hookean; us a call, three
+    // meshes in turn / one alone; T the tile path, k x s: k rings, s owned elements):
+    //     750 T 71/177  2x64 59/149          24,576 T 119/275  1x128 70/174  2x128 88/169
+    //   3,072 T 169/294 2x64 46/137  1x64 95/203   48,000 T 168/280  1x256 114/211  1x128 119/229
+    //  10,368 T 120/264 2x128 54/165 2x64 69/146   93,750 T 167/288  1x256 209/344
+    // A second ring pays while the chip idles (it evaluates some four times the elements), the
+    // whole scheme until the elements evaluated twice cost what a launch does.
+    if (npe != 4 || ne == 0 || ne > 64000 || c.tiles.threads != c.tiles.te || c.elem_seg.size() != 2) return;
+    const int K = ne <= 16000 ? 2 : 1;
+    const int64_t target = ne <= 6500 ? 64 : ne <= 32000 ? 128 : 256;
+    const std::vector<int32_t> &conn = c.conn_h;
+    // node -> (element, slot), ascending
+    std::vector<int32_t> start(nn + 1, 0), inc((size_t)ne * npe);
+    for (int64_t t = 0; t < ne * npe; ++t) start[conn[t] + 1]++;
+    for (int64_t i = 0; i < nn; ++i) start[i + 1] += start[i];
+    {
+        std::vector<int32_t> fill(start.begin(), start.end() - 1);
+        for (int64_t t = 0; t < ne * npe; ++t) inc[fill[conn[t]]++] = (int32_t)t;
+    }
+    // patch of every node: that of its lowest element; nodes of no element go round
+    const int64_t np = (ne + target - 1) / target;
+    std::vector<std::vector<int32_t>> own(np);
+    for (int64_t i = 0; i < nn; ++i)
+        own[start[i] < start[i + 1] ? (inc[start[i]] / npe) / target : i % np].push_back((int32_t)i);
+    // tile of every element (the grouping of the sums)
+    const int te = c.tiles.te;
+    struct Patch {
+        std::vector<int32_t> nodes, elems;
+        int nn[kRings + 1] = {0}, ne[kRings + 1] = {0};
+        std::vector<uint32_t> csr;
+        std::vector<uint16_t> conn, ent;
+    };
+    std::vector<Patch> pt(np);
+    std::atomic<bool> fits{true};
+    auto work = [&](int w, int nw) {
+        std::vector<int32_t> nloc(nn, -1), eloc(ne, -1);
+        for (int64_t p = w; p < np; p += nw) {
+            Patch &q = pt[p];
+            q.nodes = own[p];
+            for (int64_t e = p * target; e < std::min(ne, (p + 1) * target); ++e) {
+                eloc[e] = 0;
+                q.elems.push_back((int32_t)e);
+            }
+            q.ne[0] = (int)q.elems.size();
+            for (size_t i = 0; i < q.nodes.size(); ++i) nloc[q.nodes[i]] = (int32_t)i;
+            q.nn[0] = (int)q.nodes.size();
+            size_t n_from = 0;
+            for (int r = 1; r <= K; ++r) {
+                const size_t n_to = q.nodes.size(), e_from = q.elems.size(), e_new = r == 1 ? 0 : e_from;
+                for (size_t i = n_from; i < n_to; ++i)
+                    for (int32_t t = start[q.nodes[i]]; t < start[q.nodes[i] + 1]; ++t) {
+                        const int32_t e = inc[t] / npe;
+                        if (eloc[e] < 0) {
+                            eloc[e] = 0;
+                            q.elems.push_back(e);
+                        }
+                    }
+                std::sort(q.elems.begin() + e_from, q.elems.end());
+                for (size_t i = e_new; i < q.elems.size(); ++i) {  // ring 1: the owned elements too
+                    eloc[q.elems[i]] = (int32_t)i;
+                    for (int k = 0; k < npe; ++k) {
+                        const int32_t n = conn[(int64_t)q.elems[i] * npe + k];
+                        if (nloc[n] < 0) {
+                            nloc[n] = 0;
+                            q.nodes.push_back(n);
+                        }
+                    }
+                }
+                std::sort(q.nodes.begin() + n_to, q.nodes.end());
+                for (size_t i = n_to; i < q.nodes.size(); ++i) nloc[q.nodes[i]] = (int32_t)i;
+                n_from = n_to;
+                q.nn[r] = (int)q.nodes.size();
+                q.ne[r] = (int)q.elems.size();
+            }
+            for (int i = 0; i < q.nn[K - 1]; ++i) {
+                const size_t s0 = q.ent.size();
+                int32_t tile = -1;
+                for (int32_t t = start[q.nodes[i]]; t < start[q.nodes[i] + 1]; ++t) {
+                    const int32_t e = inc[t] / npe, k = inc[t] % npe;
+                    const bool fresh = tile >= 0 && e / te != tile;
+                    tile = e / te;
+                    // (local element and slot; the force row once the row stride is known)
+                    q.ent.push_back((uint16_t)(eloc[e] * npe + k) | (fresh ? kNewTile : 0));
+                }
+                const size_t cnt = q.ent.size() - s0;
+                if (s0 / kBatch > 0xffff || cnt > 0xffff) fits = false;
+                q.csr.push_back((uint32_t)((s0 / kBatch) << 16) | (uint32_t)cnt);
+                while (q.ent.size() % kBatch) q.ent.push_back(0);
+            }
+            for (int32_t e : q.elems)
+                for (int k = 0; k < npe; ++k) q.conn.push_back((uint16_t)nloc[conn[(int64_t)e * npe + k]]);
+            if (npe * f_stride((int)q.elems.size()) > 0x7fff || q.nodes.size() > 0xffff) fits = false;
+            for (int32_t n : q.nodes) nloc[n] = -1;
+            for (int32_t e : q.elems) eloc[e] = -1;
+        }
+    };
+    {
+        const int nw = (int)std::max<int64_t>(1, std::min<int64_t>({16, (int64_t)std::thread::hardware_concurrency(), np / 6}));
+        std::vector<std::thread> pool;
+        for (int w = 1; w < nw; ++w) pool.emplace_back(work, w, nw);
+        work(0, nw);
+        for (auto &t : pool) t.join();
+    }
+    if (!fits) return;
+    size_t npad = 1, cpad = 1, epad = 1, entpad = kBatch;
+    for (const Patch &q : pt) {
+        npad = std::max(npad, q.nodes.size());
+        cpad = std::max(cpad, q.csr.size());
+        epad = std::max(epad, q.elems.size());
+        entpad = std::max(entpad, q.ent.size());
+    }
+    const int fs = f_stride((int)epad);
+    if (npe * fs > 0x7fff) return;
+    const size_t lds = carve(nullptr, npe, (int)npad, (int)cpad, (int)epad, (int)entpad).bytes;
+    if (lds > 160 * 1024) return;
+    std::vector<int32_t> meta((size_t)np * 16, 0), node(np * npad);
+    std::vector<int32_t> elem(np * epad);
+    std::vector<uint32_t> csr(np * cpad, 0);
+    std::vector<uint16_t> lconn(np * epad * npe), ent(np * entpad, 0);
+    for (int64_t p = 0; p < np; ++p) {
+        const Patch &q = pt[p];
+        for (int r = 0; r <= K; ++r) {
+            meta[16 * p + r] = q.nn[r];
+            meta[16 * p + 8 + r] = q.ne[r];
+        }
+        for (size_t i = 0; i < npad; ++i) node[p * npad + i] = q.nodes[std::min(i, q.nodes.size() - 1)];
+        std::copy(q.csr.begin(), q.csr.end(), csr.begin() + p * cpad);
+        for (size_t i = 0; i < q.ent.size(); ++i) {
+            const int le = q.ent[i] & ~kNewTile;
+            ent[p * entpad + i] = (uint16_t)((le % npe) * fs + le / npe) | (q.ent[i] & kNewTile);
+        }
+        for (size_t i = 0; i < epad; ++i) {
+            const size_t j = std::min(i, q.elems.size() - 1);
+            elem[p * epad + i] = q.elems[j];
+            for (int k = 0; k < npe; ++k) lconn[(p * epad + i) * npe + k] = q.conn[j * npe + k];
+        }
+    }
+    // one allocation and one copy for the six lists (each on a 16-byte boundary)
+    std::vector<unsigned char> bytes;
+    auto put = [&](const auto &v) {
+        const size_t at = (bytes.size() + 15) & ~(size_t)15;
+        bytes.resize(at + sizeof(v[0]) * v.size());
+        std::memcpy(bytes.data() + at, v.data(), sizeof(v[0]) * v.size());
+        return at;
+    };
+    const size_t o_meta = put(meta), o_node = put(node), o_csr = put(csr), o_elem = put(elem), o_conn = put(lconn),
+                 o_ent = put(ent);
+    P.lists.upload(bytes.data(), bytes.size(), c.stream);
+    P.meta = reinterpret_cast<const int32_t *>(P.lists.p + o_meta);
+    P.node = reinterpret_cast<const int32_t *>(P.lists.p + o_node);
+    P.csr = reinterpret_cast<const uint32_t *>(P.lists.p + o_csr);
+    P.elem = reinterpret_cast<const int32_t *>(P.lists.p + o_elem);
+    P.conn = reinterpret_cast<const uint16_t *>(P.lists.p + o_conn);
+    P.ent = reinterpret_cast<const uint16_t *>(P.lists.p + o_ent);
+    P.u.alloc(3 * nn);
+    P.v.alloc(3 * nn);
+    P.a.alloc(3 * nn);
+    APHIP_HIP(hipStreamSynchronize(c.stream));
+    P.rings = K;
+    P.npatch = np;
+    P.npad = (int)npad;
+    P.cpad = (int)cpad;
+    P.epad = (int)epad;
+    P.entpad = (int)entpad;
+    P.lds_bytes = lds;
+    P.threads = std::max(128, std::min(1024, (int)(epad + 63) / 64 * 64));
+    P.ready = true;
+}
+
+bool patch_eligible(Ctx &c) {
+    if (c.tiles.ready && !c.patch.tried) patch_build(c);
+    return c.patch.ready && !c.node_dt.p && !c.tiles.use_stream &&
+           (c.mat.kind == APHIP_LINEAR_ELASTIC || c.mat.kind == APHIP_NEO_HOOKEAN || c.mat.kind == APHIP_J2 ||
+            c.mat.kind == APHIP_SVK);
+}
+
+void patch_run(Ctx &c, double dt, int steps, bool keep) {
+    PatchPlan &P = c.patch;
+    APHIP_REQUIRE(P.ready && steps >= 1 && steps <= P.rings, "patch plan does not cover these steps");
+    PatchArgs A;
+    A.X = c.X.p;
+    A.u = c.u.p;
+    A.v = c.v.p;
+    A.a = c.a.p;
+    A.u1 = P.u.p;
+    A.v1 = P.v.p;
+    A.a1 = P.a.p;
+    A.f = c.f.p;
+    A.mass = c.mass.p;
+    A.fixed = c.has_fixed ? c.fixed.p : nullptr;
+    A.zero = c.tiles.zero.p;
+    A.meta = P.meta;
+    A.node = P.node;
+    A.csr = P.csr;
+    A.elem = P.elem;
+    A.conn = P.conn;
+    A.ent = P.ent;
+    A.H = c.H.p;
+    A.P = c.P.p;
+    A.state_n = c.state[1 - c.state_np1].p;
+    A.state_np1 = c.state[c.state_np1].p;
+    A.mat = c.mat.params();
+    A.elem_lambda = c.has_fields ? c.elem_lambda.p : nullptr;
+    A.elem_mu = c.has_fields ? c.elem_mu.p : nullptr;
+    A.dt = dt;
+    A.ne = c.ne;
+    A.npatch = P.npatch;
+    A.nblocks = ((P.npatch + kNumXcd - 1) / kNumXcd) * kNumXcd;
+    A.npad = P.npad;
+    A.cpad = P.cpad;
+    A.epad = P.epad;
+    A.entpad = P.entpad;
+    A.steps = steps;
+    A.keep = keep;
+    launch<4>(c, A);
+    std::swap(c.u.p, P.u.p);
+    std::swap(c.v.p, P.v.p);
+    std::swap(c.a.p, P.a.p);
+}
+
+}  // namespace aphip

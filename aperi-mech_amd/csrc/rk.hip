@@ -1151,6 +1151,7 @@ static void nodal_label(Ctx &c, int subdomains, std::vector<int64_t> &sub_start,
         if (!act[i]) old_of_new.push_back((int32_t)i);
     renumber_nodes(c, old_of_new);
     c.tiles.reset();  // the tile plan's node groups are void after the renumbering
+    c.patch.reset();
     c.n_dof = n_act;
     // cells: active nodes by caller id; hexes by caller element id
     std::vector<int32_t> act_nodes(n_act);

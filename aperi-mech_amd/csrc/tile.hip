@@ -1151,6 +1151,7 @@ void tile_build(Ctx &c, int te, int threads) {
     P.use_stream = (c.flags & APHIP_FLAG_PIPELINED) != 0;
     for (int &g : P.stream_grid) g = 0;  // sized (and LDS attribute set) at the first launch
     P.ready = true;
+    c.patch.reset();
     APHIP_HIP(hipStreamSynchronize(c.stream));
 }
 

@@ -1,0 +1,55 @@
+"""Small meshes step on node patches (several steps a launch, neighbours' elements
+recomputed); graph replay keeps the tile kernels.  Both must give the same bits: the element
+arithmetic is the same and the patches group a node's sum by the plan's tiles."""
+import numpy as np
+import pytest
+
+import aperi_hip as A
+from aperi_hip import meshgen as M
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = (A.FIELD_U, A.FIELD_V, A.FIELD_A, A.FIELD_F, A.FIELD_H, A.FIELD_P)
+
+
+def _run(X, conn, kind, calls, graph, fields, tiling):
+    rho, E, nu = 2700.0, 70e9, 0.33
+    fixed = np.zeros(X.shape, dtype=np.uint8)
+    fixed[X[:, 2] < 0.01] = (1, 1, 0)
+    with A.Solver() as s:
+        s.set_mesh(A.TET4, X, conn)
+        s.set_material(kind, rho, E, nu, 30e6, 1e9)
+        if tiling:
+            s.set_tiling(tiling, tiling)
+        if fields:
+            r = M.uniform01(3, 5, 2 * len(conn))
+            s.set_material_fields(E * (0.8 + 0.4 * r[:len(conn)]), 0.2 + 0.2 * r[len(conn):])
+        s.compute_mass()
+        s.set_fixed(fixed)
+        s.set_field(A.FIELD_V, 30.0 * (2 * M.uniform01(9, 4, X.size).reshape(X.shape) - 1))
+        s.set_graph(graph)
+        s.initialize()
+        dt = 0.3 * M.stable_dt_estimate(X, conn, E, nu, rho)
+        for n in calls:
+            s.step(dt, n)
+        out = [s.get(f) for f in FIELDS]
+        if kind == A.J2:
+            out.append(s.get(A.FIELD_STATE))
+            s.internal_force(0.0, dt)  # reads the state before the last step
+            out += [s.get(A.FIELD_F), s.get(A.FIELD_STATE)]
+        return out
+
+
+# one hex; two rings of 64 and of 128 owned elements; one ring of 128 and of 256; the tile path
+@pytest.mark.parametrize("n", [(1, 1, 1), (3, 4, 5), (9, 9, 9), (11, 12, 13), (15, 14, 16), (20, 18, 20), (22, 22, 23)])
+@pytest.mark.parametrize("kind,fields,tiling", [(A.NEO_HOOKEAN, False, 0), (A.J2, True, 256), (A.SVK, False, 64)])
+def test_patches_match_tiles(gpu_available, n, kind, fields, tiling):
+    X, hc = M.hex_lattice(*n, *(k / max(n) for k in n))
+    X = M.jitter(X, 1.0 / max(n), 0.1, 7, 1)
+    conn = M.split_tets(X, hc)
+    print(f"patches {len(conn)} Tet4 kind={kind} tiling={tiling}", flush=True)
+    want = _run(X, conn, kind, [2, 2, 2], True, fields, tiling)
+    for calls in ([1] * 6, [6], [3, 3]):
+        got = _run(X, conn, kind, calls, False, fields, tiling)
+        for a, b in zip(want, got):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
