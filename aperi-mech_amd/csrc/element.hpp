@@ -110,9 +110,9 @@ APHIP_DEV void hex8_sign(int k, int &s0, int &s1, int &s2) {
 //   8 dX/dxi0 = M[s0] + p1 M[s0s1] + p2 M[s0s2] + p1 p2 M[s0s1s2]   (and cyclically),
 // which replaces the 8-corner sums of J and grad u by 3 multiply-adds per entry.
 // The nodal force f_k = -sum_q dN_k(q) Q_q is accumulated in the same seven modes
-// and returned to the corners by one inverse transform.  The 1/8 of the shape
-// function derivatives is carried as exact powers of two (J and grad u scaled by 8,
-// J^-1 by 1/8, w = det / 512), which leaves every rounding unchanged.
+// and returned to the corners by one inverse transform.  The 1/8 of the shape function
+// derivatives is carried as exact powers of two (J and grad u scaled by 8, the force by
+// 1/512), and w J^-1 = det J J^-1 is the adjugate.
 // Gauss points in the order of include/ElementHexahedron8.h:107-115, w = detJ;
 // stored H / P are those of the last point (ComputeInternalForceGaussian.h:89, :99-107).
 
@@ -195,11 +195,7 @@ APHIP_DEV void hex8_element(const double (&X)[8][3], const double (&U)[8][3], co
         sn = load_state<KIND>(state_n, 0);
         sn2 = load_state2<KIND>(state_n, 0);
     }
-    // Two Gauss points in flight where the registers allow it without spilling (the
-    // neo-Hookean and SVK updates; measured -3 % on the neo-Hookean step); one otherwise.
-    // The order of the force accumulation is the same either way.
-    constexpr int kQUnroll = (KIND == APHIP_NEO_HOOKEAN || KIND == APHIP_SVK) && !UL ? 2 : 1;
-#pragma unroll kQUnroll
+#pragma unroll 1
     for (int q = 0; q < 8; ++q) {
         int sq0, sq1, sq2;
         hex8_sign(q, sq0, sq1, sq2);
@@ -217,13 +213,13 @@ APHIP_DEV void hex8_element(const double (&X)[8][3], const double (&U)[8][3], co
                 G[3 * i + d] = gu[d];
             }
         }
-        double Ji[9];  // (8 J)^-1 = J^-1 / 8
-        const double w = inverse3(J, Ji) * (-1.0 / 512.0);  // -detJ
+        double Ad[9];  // adj(8 J): w J^-1 up to exact powers of two
+        const double id = 1.0 / adjugate3(J, Ad);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 3; ++j)
-                H[3 * i + j] = dot3(G[3 * i], Ji[j], G[3 * i + 1], Ji[3 + j], G[3 * i + 2], Ji[6 + j]);
+                H[3 * i + j] = dot3(G[3 * i], Ad[j], G[3 * i + 1], Ad[3 + j], G[3 * i + 2], Ad[6 + j]) * id;
         double snp1 = 0.0, aux = 0.0;
         if constexpr (PER_QP) {
             sn = load_state<KIND>(state_n, q);
@@ -242,10 +238,10 @@ APHIP_DEV void hex8_element(const double (&X)[8][3], const double (&U)[8][3], co
         }
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            // Q[n] = -(w / 8) (J^-1 P^T)[n][j]: the force of axis n's derivative
+            // Q[n] = (w J^-1 P^T)[n][j] up to exact powers of two: the force of axis n's derivative
             double Q[3];
 #pragma unroll
-            for (int n = 0; n < 3; ++n) Q[n] = w * dot3(Ji[3 * n], Pf[3 * j], Ji[3 * n + 1], Pf[3 * j + 1], Ji[3 * n + 2], Pf[3 * j + 2]);
+            for (int n = 0; n < 3; ++n) Q[n] = dot3(Ad[3 * n], Pf[3 * j], Ad[3 * n + 1], Pf[3 * j + 1], Ad[3 * n + 2], Pf[3 * j + 2]);
             R[j][1] += Q[0];
             R[j][2] += Q[1];
             R[j][4] += Q[2];
@@ -260,107 +256,141 @@ APHIP_DEV void hex8_element(const double (&X)[8][3], const double (&U)[8][3], co
         double v[8];
         hex8_corners(R[j], v);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) fe[k][j] = v[k];
+        for (int k = 0; k < 8; ++k) fe[k][j] = v[k] * (-1.0 / 512.0);  // (exact: -w det^-1 of the scaled J)
     }
 }
 
-// Hex8 with one lane per Gauss point: lane q (= lane id mod 8) evaluates point q
-// and the eight lanes of an element combine their nodal contributions with a
-// three-step exchange, after which lane k holds node k's force (summed as
-// ((q0+q4)+(q2+q6)) + ((q1+q5)+(q3+q7)), a fixed order).  Node coordinates and
-// displacements are streamed from LDS (sX/sU, 3 doubles per local node, lc =
-// local node of each corner), so no lane keeps the 48-double element state.
-// H, P and a per-element J2 state are those of Gauss point 7 (the last point,
-// ComputeInternalForceGaussian.h:89, :99-107); with per-point state each lane
-// owns its slot.
-template <int KIND, bool PER_QP>
-APHIP_DEV void hex8_qp_lane(int q, const int (&lc)[8], const double *sX, const double *sU, const MatParams &m,
-                            double ga, const double *state_n, double *state_np1, double *H, double *P,
-                            double (&fk)[3], const RateIn *r = nullptr) {
+// Hex8 with one lane per Gauss point, in the modal form of hex8_element.  Eight lanes share
+// an element: one field's corner values per lane (six of the eight) go through the transform
+// and its seven modes into the element's LDS row, every lane evaluates its Gauss point from
+// the row, and the three vectors Q_n of the force are summed over the points, combined into
+// the modes and returned to the corners by transforms across the lanes (DPP moves, no LDS).
+//
+// A lane's label x = (x0, x1, x2) says which point (axis a at + if x_a), mode (the axes with
+// x_a) and corner (s_a = + if x_a) it holds.  Labels are chosen so that the partner along every
+// axis is one DPP move away: axis 0 lane ^ 1, axis 1 lane ^ 2, axis 2 lane ^ 7 (the mirror in a
+// half row; xor 4 is not a DPP pattern), i.e. x2 = bit 2, x1 = bit 1 ^ x2, x0 = bit 0 ^ x2.
+constexpr int kHexRow = 42;  // doubles of an element's LDS row: 6 fields x 7 modes, then 8 x 3 forces
+
+template <int CTRL>
+APHIP_DEV double dpp_move(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// the value of the partner lane along axis a
+template <int AXIS>
+APHIP_DEV double hex8_partner(double v) {
+    constexpr int ctrl = AXIS == 0 ? 0xb1 /* quad_perm 1,0,3,2 */ : AXIS == 1 ? 0x4e /* 2,3,0,1 */ : 0x141 /* half-row mirror */;
+    return dpp_move<ctrl>(v);
+}
+
+APHIP_DEV int hex8_lane_label(int lane) {
+    const int x2 = (lane >> 2) & 1, x1 = ((lane >> 1) & 1) ^ x2, x0 = (lane & 1) ^ x2;
+    return x0 | (x1 << 1) | (x2 << 2);
+}
+
+// lane: 0..7 within the element (all eight active); cn: the offsets (3 x local node) of corners
+// 2 i and 2 i + 1 in cn[i]; sX, sU: 3 doubles per local node; row: the element's kHexRow doubles, on
+// return the corner forces (corner k at 3 k).  H, P and the state of the last point are valid
+// in the lane for which the function returns true; with PER_QP every lane stores its state.
+// LEAN: the lane's signs are derived again after the stress update instead of held across it
+// (12 VGPRs less, for callers that would spill).
+template <int KIND, bool PER_QP, bool LEAN = false>
+APHIP_DEV bool hex8_lanes(int lane, const uint32_t (&cn)[4], const double *sX, const double *sU, double *row,
+                          const MatParams &m, double ga, const double *state_n, double *state_np1, double *H,
+                          double *P, const RateIn *r = nullptr) {
 #pragma clang fp contract(off)
-    int sq0, sq1, sq2;
-    hex8_sign(q, sq0, sq1, sq2);
-    const double p0 = sq0 * ga, p1 = sq1 * ga, p2 = sq2 * ga;
-    // parametric derivatives of node k at this lane's Gauss point
-    auto dn = [&](int k, double (&d)[3]) {
-        int s0, s1, s2;
-        hex8_sign(k, s0, s1, s2);
-        const double f0 = s0 < 0 ? (1.0 - p0) : (1.0 + p0);
-        const double f1 = s1 < 0 ? (1.0 - p1) : (1.0 + p1);
-        const double f2 = s2 < 0 ? (1.0 - p2) : (1.0 + p2);
-        d[0] = (s0 * 0.125) * f1 * f2;
-        d[1] = (s1 * 0.125) * f0 * f2;
-        d[2] = (s2 * 0.125) * f0 * f1;
-    };
-    double J[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, G[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    int x = hex8_lane_label(lane);
+    bool b0 = x & 1, b1 = x & 2, b2 = x & 4;
+    const int q = x == 2 ? 3 : x == 3 ? 2 : x == 6 ? 7 : x == 7 ? 6 : x;  // point (and corner) index
+    if (lane < 6) {
+        const double *src = (lane < 3 ? sX : sU) + (lane < 3 ? lane : lane - 3);
+        double v[8], w[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        double d[3];
-        dn(k, d);
-        const double *x = sX + 3 * lc[k];
-        const double *u = sU + 3 * lc[k];
+        for (int k = 0; k < 8; ++k) v[k] = src[k & 1 ? cn[k >> 1] >> 16 : cn[k >> 1] & 0xffffu];
+        hex8_modes(v, w);
+        // a mode of |S| axes is only ever used times ga^(|S| - 1) and signs
+        w[3] *= ga;
+        w[5] *= ga;
+        w[6] *= ga;
+        w[7] *= ga * ga;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const double xi = x[i], ui = u[i];
-#pragma unroll
-            for (int dd = 0; dd < 3; ++dd) {
-                J[3 * i + dd] = __fma_rn(xi, d[dd], J[3 * i + dd]);
-                G[3 * i + dd] = __fma_rn(ui, d[dd], G[3 * i + dd]);
-            }
-        }
+        for (int S = 1; S < 8; ++S) row[7 * lane + S - 1] = w[S];
     }
-    double Ji[9];
-    const double w = inverse3(J, Ji);
+    __builtin_amdgcn_wave_barrier();  // (LDS operations of a wave stay in order)
+    double s0 = b0 ? -1.0 : 1.0, s1 = b1 ? -1.0 : 1.0, s2 = b2 ? -1.0 : 1.0;
+    const double s01 = s0 * s1, s02 = s0 * s2, s12 = s1 * s2;
+    double J[9], G[9];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        double wx[8], wu[8], g[3];
+        wx[0] = wu[0] = 0.0;
+#pragma unroll
+        for (int S = 1; S < 8; ++S) {
+            wx[S] = row[7 * i + S - 1];
+            wu[S] = row[7 * (i + 3) + S - 1];
+        }
+        hex8_grad(wx, -s0, -s1, -s2, s01, s02, s12, g);
+        J[3 * i] = g[0];
+        J[3 * i + 1] = g[1];
+        J[3 * i + 2] = g[2];
+        hex8_grad(wu, -s0, -s1, -s2, s01, s02, s12, g);
+        G[3 * i] = g[0];
+        G[3 * i + 1] = g[1];
+        G[3 * i + 2] = g[2];
+    }
+    // w J^-1 = adj(J) up to exact powers of two, so the force takes the adjugate itself
+    double Ad[9];
+    const double id = 1.0 / adjugate3(J, Ad);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-            H[3 * i + j] = dot3(G[3 * i], Ji[j], G[3 * i + 1], Ji[3 + j], G[3 * i + 2], Ji[6 + j]);
-    double sn = 0.0, snp1 = 0.0, aux = 0.0;
-    sn = load_state<KIND>(state_n, PER_QP ? q : 0);
-    const double sn2 = load_state2<KIND>(state_n, PER_QP ? q : 0);
+            H[3 * i + j] = dot3(G[3 * i], Ad[j], G[3 * i + 1], Ad[3 + j], G[3 * i + 2], Ad[6 + j]) * id;
+    const bool last = q == 7;
+    double snp1 = 0.0, aux = 0.0;
+    const double sn = load_state<KIND>(state_n, PER_QP ? q : 0), sn2 = load_state2<KIND>(state_n, PER_QP ? q : 0);
     stress<KIND>(H, m, sn, snp1, aux, P, r, sn2);
     if constexpr (PER_QP) store_state<KIND>(state_np1, q, snp1, aux);
-    else if (q == 7) store_state<KIND>(state_np1, 0, snp1, aux);
-    double Q[9];
+    else if (last) store_state<KIND>(state_np1, 0, snp1, aux);
+    if constexpr (LEAN) {
+        asm volatile("" : "+v"(x));  // (a value the compiler cannot match with the earlier one)
+        b0 = x & 1;
+        b1 = x & 2;
+        b2 = x & 4;
+        s0 = b0 ? -1.0 : 1.0;
+        s1 = b1 ? -1.0 : 1.0;
+        s2 = b2 ? -1.0 : 1.0;
+    }
+    // W_nj[x] = sum over the points of sign_(x without n)(point) Q_nj by butterflies: lane x keeps
+    // pattern x of the other axes, along axis n both partners take the plain sum
+    double W[3][3];
 #pragma unroll
     for (int n = 0; n < 3; ++n)
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-            Q[3 * n + j] = w * dot3(Ji[3 * n], P[3 * j], Ji[3 * n + 1], P[3 * j + 1], Ji[3 * n + 2], P[3 * j + 2]);
-    // reduce-scatter over the 8 lanes: at each step keep the half of the nodes whose
-    // index bit matches this lane's bit and add the partner's copy of that half
-    const bool b2 = (q >> 2) & 1, b1 = (q >> 1) & 1, b0 = q & 1;
-    double r4[4][3];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        double dl[3], dh[3];
-        dn(k, dl);
-        dn(k + 4, dh);
-#pragma unroll
         for (int j = 0; j < 3; ++j) {
-            const double cl = -dot3(dl[0], Q[j], dl[1], Q[3 + j], dl[2], Q[6 + j]);
-            const double ch = -dot3(dh[0], Q[j], dh[1], Q[3 + j], dh[2], Q[6 + j]);
-            const double keep = b2 ? ch : cl;
-            const double send = b2 ? cl : ch;
-            r4[k][j] = keep + __shfl_xor(send, 4, 8);
+            double v = dot3(Ad[3 * n], P[3 * j], Ad[3 * n + 1], P[3 * j + 1], Ad[3 * n + 2], P[3 * j + 2]);
+            v = n == 0 ? v + hex8_partner<0>(v) : __fma_rn(s0, hex8_partner<0>(v), v);
+            v = n == 1 ? v + hex8_partner<1>(v) : __fma_rn(s1, hex8_partner<1>(v), v);
+            W[n][j] = n == 2 ? v + hex8_partner<2>(v) : __fma_rn(s2, hex8_partner<2>(v), v);
         }
-    }
-    double r2[2][3];
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const double keep = b1 ? r4[k + 2][j] : r4[k][j];
-            const double send = b1 ? r4[k][j] : r4[k + 2][j];
-            r2[k][j] = keep + __shfl_xor(send, 2, 8);
-        }
+    // mode x: R_xj = c sum_{n in x} W_nj, c = ga^(|x| - 1); then to the corners
+    const int nx = (x & 1) + ((x >> 1) & 1) + (x >> 2);
+    const double c = (nx == 3 ? ga * ga : nx == 2 ? ga : 1.0) * (-1.0 / 512.0);  // (-1/512 = -w det^-1, exact)
+    const double c0 = b0 ? c : 0.0, c1 = b1 ? c : 0.0, c2 = b2 ? c : 0.0;
+    double f[3];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-        const double keep = b0 ? r2[1][j] : r2[0][j];
-        const double send = b0 ? r2[0][j] : r2[1][j];
-        fk[j] = keep + __shfl_xor(send, 1, 8);
+        double v = __fma_rn(c2, W[2][j], __fma_rn(c1, W[1][j], c0 * W[0][j]));
+        v = __fma_rn(-s0, hex8_partner<0>(v), v);
+        v = __fma_rn(-s1, hex8_partner<1>(v), v);
+        f[j] = __fma_rn(-s2, hex8_partner<2>(v), v);
     }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) row[3 * q + j] = f[j];
+    return last;
 }
 
 // Smoothed Tet4 B and volume from the faces (include/QuadratureSmoothed.h:32-62)

@@ -193,7 +193,6 @@ struct TilePlan {
     int64_t ntiles = 0;
     int maxtn = 0;                    // most nodes in one tile
     int max_nint = 0;                 // most interior nodes in one tile
-    int f_rounds = 1;                 // LDS rounds of the element forces (tile kernel)
     int64_t nb = 0;                   // shared nodes (finished by the second launch)
     int64_t n_interior = 0;           // first shared node id
     int64_t total_tile_nodes = 0;
@@ -222,10 +221,16 @@ struct TilePlan {
     DevBuf<uint32_t> tnp_csr;         // [ntiles * tpad]
     DevBuf<int32_t> tnp_bdst;         // [ntiles * tpad]
     DevBuf<uint16_t> lconn_p;         // [ntiles * te * npe]
+    // the Gauss Hex8 kernel's forms of the corners and the entries (k_hex_tile)
+    int hx_rounds = 1;                // LDS rounds of a tile's elements
+    DevBuf<uint16_t> hx_conn;         // [ntiles * te * 8] 3 x local node
+    DevBuf<uint4> hx_first, hx_more;  // [ntiles * rounds * tpad] first eight entries of a row; the rest
+    DevBuf<uint32_t> hx_csr;          // [ntiles * rounds * tpad] (first further batch << 16) | batches
+    DevBuf<int32_t> hx_base;          // [ntiles * rounds] origin of the batches in hx_more
+    size_t cell_lds_bytes = 0;        // LDS of the smoothed Hex8 cell kernel
     void reset() {
         ready = false;
         te = threads = maxtn = max_nint = 0;
-        f_rounds = 1;
         ntiles = nb = n_interior = total_tile_nodes = nslot = 0;
         lds_bytes = 0;
         for (int &g : stream_grid) g = 0;
@@ -234,6 +239,9 @@ struct TilePlan {
         zero.release(); meta.release();
         tpad = 0;
         tnp_node.release(); tnp_csr.release(); tnp_bdst.release(); lconn_p.release();
+        hx_conn.release(); hx_first.release(); hx_more.release(); hx_csr.release(); hx_base.release();
+        hx_rounds = 1;
+        cell_lds_bytes = 0;
     }
 };
 

@@ -1277,13 +1277,16 @@ static void nodal_subcells(Ctx &c, const std::vector<int64_t> &sub_start, const 
 // here when the context has none (APHIP_FLAG_TWO_PASS, a nodal set-up before this one) or
 // has the eight-lanes-per-Hex8 shape.  64 elements always fit a CU's LDS.
 static void ensure_element_tiles(Ctx &c) {
-    if (c.ne == 0 || (c.tiles.ready && c.tiles.threads == c.tiles.te)) return;
+    auto fits = [&] {
+        return c.tiles.ready && c.tiles.threads == c.tiles.te && c.tiles.cell_lds_bytes <= 160 * 1024;
+    };
+    if (c.ne == 0 || fits()) return;
     for (int te = c.npe == 4 ? 1024 : 128;; te /= 2) {
         try {
             tile_build(c, te, te);
-            return;
+            if (fits()) return;
         } catch (const Error &e) {
-            if (te == 64 || e.code != APHIP_ERR_INVALID) throw;
+            if (te <= 64 || e.code != APHIP_ERR_INVALID) throw;
         }
     }
 }

@@ -68,6 +68,14 @@ struct TileArgs {
     const int32_t *tnp_bdst;
     const uint16_t *lconn_p;
     int tpad;
+    // k_hex_tile's forms (TilePlan::hx_*): corners as 3 x local node; per round and node row the
+    // first eight entries as force-row offsets (padded with the zero row) and the further
+    // batches (first << 16) | count in hx_more, from hx_base[tile * rounds + round] on
+    const uint16_t *hx_conn;
+    const uint4 *hx_first, *hx_more;
+    const uint32_t *hx_csr;
+    const int32_t *hx_base;
+    int hx_rounds;
     double *bpart;
     double *H, *P;
     const double *Hn, *Pn;  // rate-form materials: H and P of the previous step
@@ -94,11 +102,10 @@ struct TileArgs {
     int cell_marker;  // smoothed cells turn a new failure's marker into the maximum damage
 };
 
-// LDS carve-up (bytes), sized on the host (tile_lds_bytes) from maxtn, max_nint, te
-// and the number of force rounds.  X and U (the predicted displacement) are kept for
-// every tile node; v_half, m, dt and the fixed mask for max_nint rows (Hex8: the
-// interior nodes, the only ones the kernel finishes; Tet4: every tile node); F holds
-// the element forces of one round.
+// LDS carve-up (bytes), sized on the host (tile_lds_bytes) from the tile's rows.  X and U (the
+// predicted displacement) are kept for every tile node; v_half, m, dt and the fixed mask for
+// max_nint rows (Hex8: the interior nodes, the only ones the kernel finishes; Tet4: every
+// tile node); F holds nf doubles: the element forces of one round or the Hex8 element rows.
 struct TileLds {
     double *X, *U, *V, *F, *M, *DT;
     uint32_t *csr;
@@ -113,8 +120,7 @@ struct TileLds {
 // read at the same time in the gather, never share a bank.
 __host__ __device__ __forceinline__ int f_stride(int te_round) { return te_round + ((4 - te_round) & 31); }
 
-__host__ __device__ __forceinline__ TileLds carve(char *base, int maxtn, int max_nint, int te, int f_rounds,
-                                                  int npe) {
+__host__ __device__ __forceinline__ TileLds carve(char *base, int maxtn, int max_nint, int nent, size_t nf) {
     TileLds L;
     L.X = reinterpret_cast<double *>(base);
     L.U = L.X + 3 * maxtn;
@@ -122,16 +128,38 @@ __host__ __device__ __forceinline__ TileLds carve(char *base, int maxtn, int max
     L.M = L.V + 3 * max_nint;
     L.DT = L.M + max_nint;
     L.F = L.DT + max_nint;
-    L.csr = reinterpret_cast<uint32_t *>(L.F + 3 * (size_t)f_stride(te / f_rounds) * npe);
+    L.csr = reinterpret_cast<uint32_t *>(L.F + nf);
     L.bdst = reinterpret_cast<int32_t *>(L.csr + maxtn);
-    L.ent = reinterpret_cast<uint16_t *>(L.bdst + maxtn);
-    L.fx = reinterpret_cast<uint8_t *>(L.ent + te * npe);
+    // (16-byte aligned: entries are read eight at a time)
+    L.ent = reinterpret_cast<uint16_t *>((reinterpret_cast<uintptr_t>(L.bdst + maxtn) + 15) & ~(uintptr_t)15);
+    L.fx = reinterpret_cast<uint8_t *>(L.ent + nent);
     return L;
 }
 
-__host__ inline size_t tile_lds_bytes(int maxtn, int max_nint, int te, int f_rounds, int npe) {
-    return sizeof(double) * (6 * (size_t)maxtn + 5 * (size_t)max_nint + 3 * (size_t)f_stride(te / f_rounds) * npe) +
-           8 * (size_t)maxtn + 2 * (size_t)te * npe + (size_t)max_nint + 16;
+// F doubles of a tile: Tet4 one round of slot-major force rows, smoothed Hex8 cells two rounds
+// of half the tile (half the rows: twice the workgroups fit a CU), Gauss Hex8 kHexRow a row and
+// a zero row
+__host__ __device__ __forceinline__ size_t tile_f_doubles(int npe, int te, bool cell) {
+    return npe == 4 ? 12 * (size_t)f_stride(te) : cell ? 24 * (size_t)f_stride(te / 2) : kHexRow * (size_t)te + 4;
+}
+
+// nent: entries kept in LDS
+__host__ inline size_t tile_lds_bytes(int maxtn, int max_nint, int te, int npe, int nent, bool cell) {
+    return sizeof(double) * (6 * (size_t)maxtn + 5 * (size_t)max_nint + tile_f_doubles(npe, te, cell)) +
+           8 * (size_t)maxtn + 2 * (size_t)nent + (size_t)max_nint + 16 + 16;
+}
+
+// Materials whose Hex8 kernel needs more than the 128 VGPRs of four waves per SIMD (it would
+// spill 117 for creep, 78 for Drucker-Prager, 10 for damage).
+template <int KIND>
+constexpr bool hex_wide() {
+    return rate_form<KIND>() || KIND == APHIP_NEO_HOOKEAN_DAMAGE;
+}
+// Workgroup of the Hex8 kernel: eight lanes per element, at most 512 lanes up to 128 elements
+// (two passes: two workgroups fit a CU) and in rounds, else 1024 (wide materials 512).
+template <int KIND>
+__host__ int hex_threads(int te, int rounds) {
+    return std::min(te <= 128 || rounds > 1 || hex_wide<KIND>() ? 512 : 1024, 8 * (te / rounds));
 }
 
 // Optional arrays are read without branches: an absent array is replaced by the
@@ -190,20 +218,21 @@ __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L,
 }
 
 // MODE 0: force only; 1: force + a = f/m (initial); 2: full central-difference step.
-// QPAR (Hex8 only): eight lanes per element, one per Gauss point.
-// CELL (Hex8 only): smoothed Hex8 cells instead of 2x2x2 Gauss elements.
-template <int NPE, int KIND, bool PER_QP, int MODE, bool QPAR, bool CELL = false>
-__global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !QPAR ? 2 : 1) void k_tile(TileArgs A) {
+// One element per thread: Tet4 (NPE 4), or smoothed Hex8 cells (NPE 8, MODE 0); the 2x2x2 Gauss
+// Hex8 has k_hex_tile.
+template <int NPE, int KIND, int MODE>
+__global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_tile(TileArgs A) {
+    static_assert(NPE == 4 || MODE == 0, "smoothed Hex8 cells are evaluated in force mode");
     extern __shared__ __align__(16) char lds_raw[];
     const int64_t t = xcd_tile(A.nblocks);
     if (t >= A.ntiles) return;
-    // One-element-per-thread Hex8 tiles pass their forces through LDS in two rounds
-    // (24 doubles per element otherwise keep a 128-element tile at one wave per SIMD);
-    // Tet4 and QPAR tiles in one.  The host sizes the LDS with the same counts.
-    constexpr int ROUNDS = (NPE == 8 && !QPAR) ? 2 : 1;
-    const TileLds L = carve(lds_raw, A.maxtn, NPE == 4 ? A.maxtn : A.max_nint, A.te, ROUNDS, NPE);
+    // Smoothed Hex8 cells pass their forces through LDS in two rounds (24 doubles per element
+    // otherwise keep a 128-element tile at one wave per SIMD); Tet4 tiles in one.
+    constexpr int ROUNDS = NPE == 8 ? 2 : 1;
+    const TileLds L = carve(lds_raw, A.maxtn, NPE == 4 ? A.maxtn : A.max_nint, A.te * NPE,
+                            tile_f_doubles(NPE, A.te, true));
     const int tid = threadIdx.x;
-    const int le = QPAR ? (tid >> 3) : tid;
+    const int le = tid;
     int lc[NPE];
     // (le < te always; the fixed-stride copy needs no per-tile scalar)
     const int64_t ep = t * (int64_t)A.te + le;
@@ -222,8 +251,8 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
     // together, then the node data of the first NPT node rows of each thread.  (A load
     // followed by its LDS write in a loop waits for that load, and vmcnt counts in
     // order, so each iteration would add a full memory latency.)
-    constexpr int EW = NPE == 4 ? 2 : (QPAR ? 1 : 4);  // CSR words per thread: nent / 2 <= EW x blockDim
-    constexpr int NPT = NPE == 4 ? 1 : (QPAR ? 1 : 2); // node rows per thread loaded together
+    constexpr int EW = NPE == 4 ? 2 : 4;  // CSR words per thread: nent / 2 <= EW x blockDim
+    constexpr int NPT = NPE == 4 ? 1 : 2; // node rows per thread loaded together
     const int nw = A.te * NPE / 2;  // words of a full tile; a partial tile reads zeros past its end
     const uint32_t *ent_src = reinterpret_cast<const uint32_t *>(A.lcsr) + t * (int64_t)nw;
     uint32_t ew[EW];
@@ -348,10 +377,9 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
     wait_vmem_loads();
     __syncthreads();
 
-    // B: one element per thread, or one Gauss point per lane.  The element's nodal
-    // forces (QPAR: this lane's node) stay in registers until their round's LDS pass.
-    constexpr int KF = (QPAR && NPE == 8) ? 1 : NPE;
-    double fe[KF][3];
+    // B: one element per thread.  The element's nodal forces stay in registers until their
+    // round's LDS pass.
+    double fe[NPE][3];
     // Tet4: the element phase stores H and keeps P for the start of the gather phase.
     // The 144 B per element of H and P, all issued during the element phase, leave a CU
     // faster than the memory takes them while many CUs are in that phase; split between
@@ -361,30 +389,13 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
     double pdef[NPE == 4 ? 9 : 1];
     const int te_round = ROUNDS == 1 ? A.te : A.te / ROUNDS;
     const int my_round = ROUNDS == 1 ? 0 : le / te_round;
-    // LDS row of entry (element j of the round, slot k).  One element per thread:
-    // slot-major with padded slot blocks, so a wave's writes of one slot are
-    // consecutive 24-byte rows (no bank conflicts; element-major rows 96 bytes apart
-    // hit 16 of the 64 banks) and the slots of one element sit in distinct banks for
-    // the gather.  One Gauss point per lane: element-major, consecutive for those lanes.
+    // LDS row of entry (element j of the round, slot k): slot-major with padded slot blocks, so
+    // a wave's writes of one slot are consecutive 24-byte rows (no bank conflicts;
+    // element-major rows 96 bytes apart hit 16 of the 64 banks) and the slots of one element
+    // sit in distinct banks for the gather.
     const int fs = f_stride(te_round);
-    auto frow = [fs](int j, int k) { return QPAR ? j * NPE + k : k * fs + j; };
-    if constexpr (QPAR && NPE == 8) {
-        if (has_elem) {
-            const int q = tid & 7;
-            const int64_t so = state_width<KIND>() * (PER_QP ? e * 8 : e);
-            double H[9], P[9];
-            hex8_qp_lane<KIND, PER_QP>(q, lc, L.X, L.U, m, A.gauss_a, state_width<KIND>() ? A.state_n + so : nullptr,
-                                       state_width<KIND>() ? A.state_np1 + so : nullptr, H, P, fe[0], &rin);
-            if (q == 7 && A.keep) {
-#pragma unroll
-                for (int i = 0; i < 9; ++i) {
-                    store_once(A.H + i * A.ne + e, H[i]);
-                    store_once(A.P + i * A.ne + e, P[i]);
-                }
-            }
-            if (my_round == 0) st3(L.F, frow(le, q), fe[0]);
-        }
-    } else if (has_elem) {
+    auto frow = [fs](int j, int k) { return k * fs + j; };
+    if (has_elem) {
         double X[NPE][3], U[NPE][3];
 #pragma unroll
         for (int k = 0; k < NPE; ++k) {
@@ -398,11 +409,9 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
             if (A.cell_marker) snp1 = cell_damage_marker<KIND>(snp1, m);
             store_state<KIND>(A.state_np1, e, snp1, aux);
         } else {
-            const int64_t so = state_width<KIND>() * (PER_QP ? e * 8 : e);
-            const double *sn_p = state_width<KIND>() ? A.state_n + so : nullptr;
-            double *snp1_p = state_width<KIND>() ? A.state_np1 + so : nullptr;
-            if constexpr (CELL) hex8_cell<KIND>(X, U, m, sn_p, snp1_p, H, P, fe, &rin);
-            else hex8_element<KIND, PER_QP>(X, U, m, A.gauss_a, sn_p, snp1_p, H, P, fe, &rin);
+            const int64_t so = state_width<KIND>() * e;
+            hex8_cell<KIND>(X, U, m, state_width<KIND>() ? A.state_n + so : nullptr,
+                            state_width<KIND>() ? A.state_np1 + so : nullptr, H, P, fe, &rin);
         }
         if constexpr (NPE == 4) {
 #pragma unroll
@@ -461,12 +470,8 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
         if (r > 0) {
             __syncthreads();  // the previous round's gather is done with F
             if (has_elem && my_round == r) {
-                if constexpr (QPAR && NPE == 8) {
-                    st3(L.F, frow(le - r * te_round, tid & 7), fe[0]);
-                } else {
 #pragma unroll
-                    for (int k = 0; k < NPE; ++k) st3(L.F, frow(le - r * te_round, k), fe[k]);
-                }
+                for (int k = 0; k < NPE; ++k) st3(L.F, frow(le - r * te_round, k), fe[k]);
             }
             __syncthreads();
         }
@@ -497,8 +502,195 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : (QPAR ? 512 : 256), NPE == 8 && !
     }
 }
 
+// Gauss Hex8 tile step: the phases of k_tile with eight lanes per element (hex8_lanes).  Bound
+// by VALU issue (340 FP64 and about 230 other instructions a Gauss point; 77 % of the issue
+// slots busy on the uneven ensemble).  One element per thread held 246 VGPRs, two waves per
+// SIMD, and gave a 128-element tile two waves in all; the lanes' kernel fits the 128 VGPRs of
+// four waves per SIMD (the wide materials two).  20^3 Hex8, a step: 21.6 -> 12.5 us alone; the
+// 1.3M-Hex8 ensemble, where issue slots alone count, 0.20 ms of tile kernel either way.  The
+// elements' forces and, before them, the modes share the element's LDS row; a tile whose rows
+// do not fit the LDS passes them through in rounds (MULTI), whose sums a node's thread adds up
+// in an LDS row: the same sequence for every number of rounds.
+template <int KIND, bool PER_QP, int MODE, bool MULTI>
+__global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KIND>() ? 2 : 4) void k_hex_tile(TileArgs A) {
+    extern __shared__ __align__(16) char lds_raw[];
+    const int64_t t = xcd_tile(A.nblocks);
+    if (t >= A.ntiles) return;
+    const int rounds = MULTI ? A.hx_rounds : 1, rw = A.te / rounds;
+    // (MULTI: 12 entry halves a row are the 24 bytes of its partial sum)
+    const TileLds L = carve(lds_raw, A.maxtn, A.max_nint, (MULTI ? 12 : 8) * A.maxtn, tile_f_doubles(8, rw, false));
+    double *acc = reinterpret_cast<double *>(L.ent);
+    const int tid = threadIdx.x, nt = blockDim.x;
+    // A: every global load of the stage before the first LDS write (see k_tile)
+    constexpr int PASSES = hex_wide<KIND>() ? 4 : 2;  // te <= PASSES * blockDim / 8
+    const uint4 *conn = reinterpret_cast<const uint4 *>(A.hx_conn) + t * (int64_t)A.te;
+    uint4 cq[PASSES];
+    if constexpr (!MULTI) {
+#pragma unroll
+        for (int q = 0; q < PASSES; ++q) cq[q] = conn[min((tid + q * nt) >> 3, rw - 1)];
+    }
+    const int wave0 = tid & ~63;  // waves past the last node row load none
+    double x0[3], u0[3], v0[3], a0[3], m0 = 1.0, d0 = A.dt;
+    unsigned f0 = 0u;
+    int32_t bd0 = 0;
+    bool pre0 = false;
+    uint4 en0{};
+    uint32_t csr0 = 0;
+    if (wave0 < A.tpad) {
+        const int64_t row = t * (int64_t)A.tpad + min(tid, A.tpad - 1);
+        const int64_t g0 = A.tnp_node[row];
+        bd0 = A.tnp_bdst[row];
+        if constexpr (!MULTI) {
+            en0 = A.hx_first[row];
+            csr0 = A.hx_csr[row];
+        }
+        pre0 = MODE == 2 && A.upred != nullptr && bd0 >= 0;  // X and the predicted u only
+        ld3(A.X, g0, x0);
+        if (pre0) {
+            ld3(A.upred, g0 - A.first_shared, u0);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) v0[d] = a0[d] = 0.0;
+        } else {
+            ld3(A.u, g0, u0);
+            f0 = load_fixed(A, g0);
+            if constexpr (MODE >= 1) m0 = A.mass[g0];
+            if constexpr (MODE == 2) {
+                ld3(A.v, g0, v0);
+                ld3(A.a, g0, a0);
+                d0 = load_node_dt(A, g0);
+            }
+        }
+    }
+    const int tn = A.tn_start[t + 1] - A.tn_start[t];
+    const int nint = A.tn_ninterior[t];
+    const int64_t ibase = A.int_base[t];
+    const int64_t te0 = A.tile_e0[t];
+    const int nel = A.tile_e0[t + 1] - (int)te0;
+    if (tid < 3) L.F[kHexRow * rw + tid] = 0.0;  // the row of padding entries
+    auto stage = [&](int ln, uint4 en, uint32_t csr, int32_t bdst, const double *x, const double *u, const double *v,
+                     const double *a, unsigned fx, double mm, double nd, bool pre) {
+        if constexpr (!MULTI) {
+            reinterpret_cast<uint4 *>(L.ent)[ln] = en;
+            L.csr[ln] = csr;
+        }
+        L.bdst[ln] = bdst;
+        st3(L.X, ln, x);
+        if (ln < nint) {
+            L.fx[ln] = (uint8_t)fx;
+            L.M[ln] = mm;
+            L.DT[ln] = nd;
+        }
+        if constexpr (MODE == 2) {
+            double vh[3] = {0.0, 0.0, 0.0}, u1[3] = {u[0], u[1], u[2]};
+            if (!pre) cd_predict(u, v, a, fx, nd, vh, u1);
+            st3(L.U, ln, u1);
+            if (ln < nint) st3(L.V, ln, vh);
+        } else {
+            st3(L.U, ln, u);
+        }
+    };
+    if (tid < tn) stage(tid, en0, csr0, bd0, x0, u0, v0, a0, f0, m0, d0, pre0);
+    for (int ln = tid + nt; ln < tn; ln += nt) {  // tiles with more nodes than threads
+        const int64_t row = t * (int64_t)A.tpad + ln, g = A.tnp_node[row];
+        double x[3], u[3], v[3], a[3], mm = 1.0, nd = A.dt;
+        ld3(A.X, g, x);
+        ld3(A.u, g, u);
+        const unsigned fx = load_fixed(A, g);
+        if constexpr (MODE >= 1) mm = A.mass[g];
+        if constexpr (MODE == 2) {
+            ld3(A.v, g, v);
+            ld3(A.a, g, a);
+            nd = load_node_dt(A, g);
+        }
+        stage(ln, MULTI ? uint4{} : A.hx_first[row], MULTI ? 0u : A.hx_csr[row], A.tnp_bdst[row], x, u, v, a, fx, mm,
+              nd, false);
+    }
+    __syncthreads();
+
+    // node sums: eight entries' rows in flight (padding entries add zero), in ascending order
+    auto add8 = [&](const uint4 &w, double (&f)[3]) {
+        const unsigned en[8] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16,
+                                w.z & 0xffffu, w.z >> 16, w.w & 0xffffu, w.w >> 16};
+        double r[8][3];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) ld3(L.F + en[k], 0, r[k]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) f[d] += r[k][d];
+    };
+    auto add_more = [&](uint32_t csr, int32_t base, double (&f)[3]) {
+        for (uint32_t k = 0; k < (csr & 0xffffu); ++k) add8(A.hx_more[base + (csr >> 16) + k], f);
+    };
+    for (int r = 0; r < rounds; ++r) {
+        // B: eight lanes per element; a group of eight is active or idle together
+        auto element = [&](int lr, const uint4 &cw) {
+            const int le = r * rw + lr;
+            const int64_t e = te0 + le;
+            MatParams m = A.mat;
+            {  // (a uniform base and a 32-bit lane offset)
+                const double *pl = A.elem_lambda ? A.elem_lambda + te0 : A.zero;
+                const double *pm = A.elem_lambda ? A.elem_mu + te0 : A.zero;
+                const unsigned i = A.elem_lambda ? (unsigned)le : 0u;
+                const double lam = pl[i], mu = pm[i];
+                m.lambda = A.elem_lambda ? lam : m.lambda;
+                m.mu = A.elem_lambda ? mu : m.mu;
+            }
+            RateIn rin;
+            load_rate<KIND>(rin, A.Hn, A.Pn, A.ne, e, A.rate_dt);
+            const uint32_t cn[4] = {cw.x, cw.y, cw.z, cw.w};
+            const int64_t so = state_width<KIND>() * (PER_QP ? e * 8 : e);
+            double H[9], P[9];
+            const bool last = hex8_lanes<KIND, PER_QP, MULTI>(tid & 7, cn, L.X, L.U, L.F + kHexRow * lr, m, A.gauss_a,
+                                                       state_width<KIND>() ? A.state_n + so : nullptr,
+                                                       state_width<KIND>() ? A.state_np1 + so : nullptr, H, P, &rin);
+            if (last && A.keep) {
+#pragma unroll
+                for (int i = 0; i < 9; ++i) {
+                    store_once(A.H + i * A.ne + e, H[i]);
+                    store_once(A.P + i * A.ne + e, P[i]);
+                }
+            }
+        };
+        if constexpr (!MULTI) {
+#pragma unroll
+            for (int q = 0; q < PASSES; ++q) {
+                const int lr = (tid + q * nt) >> 3;
+                if (lr >= rw || lr >= nel) break;
+                element(lr, cq[q]);
+            }
+        } else {
+#pragma unroll 1
+            for (int lr = tid >> 3; lr < min(rw, nel - r * rw); lr += nt >> 3) element(lr, conn[r * rw + lr]);
+        }
+        __syncthreads();
+        // C: gather
+        if constexpr (!MULTI) {
+            for (int ln = tid; ln < tn; ln += nt) {
+                double f[3] = {0.0, 0.0, 0.0};
+                add8(reinterpret_cast<const uint4 *>(L.ent)[ln], f);
+                const uint32_t csr = L.csr[ln];
+                if (csr & 0xffffu) add_more(csr, A.hx_base[t], f);
+                finish_node<MODE>(A, L, ln, nint, ibase, f);
+            }
+        } else {
+            const int64_t tr = t * (int64_t)rounds + r;
+            for (int ln = tid; ln < tn; ln += nt) {
+                double f[3] = {0.0, 0.0, 0.0};
+                if (r > 0) ld3(acc, ln, f);
+                add8(A.hx_first[tr * A.tpad + ln], f);
+                const uint32_t csr = A.hx_csr[tr * A.tpad + ln];
+                if (csr & 0xffffu) add_more(csr, A.hx_base[tr], f);
+                if (r + 1 < rounds) st3(acc, ln, f);
+                else finish_node<MODE>(A, L, ln, nint, ibase, f);
+            }
+            if (r + 1 < rounds) __syncthreads();
+        }
+    }
+}
+
 // ---- persistent, software-pipelined Tet4 step -------------------------------
-// Same arithmetic and summation order as k_tile<4, KIND, false, 2, false>, so the
+// Same arithmetic and summation order as k_tile<4, KIND, 2>, so the
 // results are bitwise identical.  A block owns the tile sequence
 //   tbeg(xcd) + kx, + bx, + 2 bx, ...   (xcd = block % 8, kx = block / 8)
 // inside the Morton range of its XCD and overlaps the global loads of the next
@@ -867,29 +1059,29 @@ __global__ __launch_bounds__(256) void k_boundary(BoundArgs A) {
 inline int64_t padded(int64_t n) { return ((n + kNumXcd - 1) / kNumXcd) * kNumXcd; }
 
 template <int NPE, int KIND, bool PER_QP, int MODE>
-void launch_tile(Ctx &c, const TileArgs &A, size_t lds) {
-    auto go = [&](auto kern) {
+void launch_tile(Ctx &c, const TileArgs &A) {
+    const TilePlan &P = c.tiles;
+    auto go = [&](auto kern, int threads, size_t lds) {
         if (lds > 65536)
             APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(c.tiles.threads), lds, c.stream, A);
+        hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(threads), lds, c.stream, A);
     };
-    if constexpr (NPE == 8) {
-        if (c.tiles.threads == 8 * c.tiles.te) {
-            go(k_tile<NPE, KIND, PER_QP, MODE, true>);
-            return;
-        }
+    if constexpr (NPE == 4) {
+        go(k_tile<4, KIND, MODE>, P.threads, P.lds_bytes);
+    } else {
         if constexpr (MODE == 0 && !PER_QP) {
             if (c.cells.ready) {
-                go(k_tile<NPE, KIND, false, 0, false, true>);
+                go(k_tile<8, KIND, 0>, P.te, P.cell_lds_bytes);
                 return;
             }
         }
+        if (P.hx_rounds == 1) go(k_hex_tile<KIND, PER_QP, MODE, false>, hex_threads<KIND>(P.te, 1), P.lds_bytes);
+        else go(k_hex_tile<KIND, PER_QP, MODE, true>, hex_threads<KIND>(P.te, P.hx_rounds), P.lds_bytes);
     }
-    go(k_tile<NPE, KIND, PER_QP, MODE, false>);
 }
 
 template <int KIND>
-void launch_stream(Ctx &c, const TileArgs &A, size_t) {
+void launch_stream(Ctx &c, const TileArgs &A) {
     auto kern = k_tile_stream<KIND>;
     TilePlan &P = c.tiles;
     const size_t lds = stream_lds_bytes(P.te, P.maxtn);
@@ -917,38 +1109,38 @@ bool stream_eligible(const Ctx &c) {
 }
 
 template <int NPE, int MODE>
-void dispatch_kind(Ctx &c, const TileArgs &A, size_t lds) {
+void dispatch_kind(Ctx &c, const TileArgs &A) {
     if constexpr (NPE == 4 && MODE == 2) {
         if (stream_eligible(c)) {
             switch (c.mat.kind) {
-                case APHIP_LINEAR_ELASTIC: launch_stream<APHIP_LINEAR_ELASTIC>(c, A, lds); return;
-                case APHIP_NEO_HOOKEAN: launch_stream<APHIP_NEO_HOOKEAN>(c, A, lds); return;
-                case APHIP_J2: launch_stream<APHIP_J2>(c, A, lds); return;
-                case APHIP_SVK: launch_stream<APHIP_SVK>(c, A, lds); return;
+                case APHIP_LINEAR_ELASTIC: launch_stream<APHIP_LINEAR_ELASTIC>(c, A); return;
+                case APHIP_NEO_HOOKEAN: launch_stream<APHIP_NEO_HOOKEAN>(c, A); return;
+                case APHIP_J2: launch_stream<APHIP_J2>(c, A); return;
+                case APHIP_SVK: launch_stream<APHIP_SVK>(c, A); return;
                 default: break;
             }
         }
     }
     const bool pq = c.mat.state_per_qp && NPE == 8;
     switch (c.mat.kind) {
-        case APHIP_LINEAR_ELASTIC: launch_tile<NPE, APHIP_LINEAR_ELASTIC, false, MODE>(c, A, lds); break;
-        case APHIP_NEO_HOOKEAN: launch_tile<NPE, APHIP_NEO_HOOKEAN, false, MODE>(c, A, lds); break;
+        case APHIP_LINEAR_ELASTIC: launch_tile<NPE, APHIP_LINEAR_ELASTIC, false, MODE>(c, A); break;
+        case APHIP_NEO_HOOKEAN: launch_tile<NPE, APHIP_NEO_HOOKEAN, false, MODE>(c, A); break;
         case APHIP_J2:
-            if (pq) launch_tile<NPE, APHIP_J2, true, MODE>(c, A, lds);
-            else launch_tile<NPE, APHIP_J2, false, MODE>(c, A, lds);
+            if (pq) launch_tile<NPE, APHIP_J2, true, MODE>(c, A);
+            else launch_tile<NPE, APHIP_J2, false, MODE>(c, A);
             break;
-        case APHIP_SVK: launch_tile<NPE, APHIP_SVK, false, MODE>(c, A, lds); break;
+        case APHIP_SVK: launch_tile<NPE, APHIP_SVK, false, MODE>(c, A); break;
         case APHIP_NEO_HOOKEAN_DAMAGE:
-            if (pq) launch_tile<NPE, APHIP_NEO_HOOKEAN_DAMAGE, true, MODE>(c, A, lds);
-            else launch_tile<NPE, APHIP_NEO_HOOKEAN_DAMAGE, false, MODE>(c, A, lds);
+            if (pq) launch_tile<NPE, APHIP_NEO_HOOKEAN_DAMAGE, true, MODE>(c, A);
+            else launch_tile<NPE, APHIP_NEO_HOOKEAN_DAMAGE, false, MODE>(c, A);
             break;
         case APHIP_POWER_LAW_CREEP:
-            if (pq) launch_tile<NPE, APHIP_POWER_LAW_CREEP, true, MODE>(c, A, lds);
-            else launch_tile<NPE, APHIP_POWER_LAW_CREEP, false, MODE>(c, A, lds);
+            if (pq) launch_tile<NPE, APHIP_POWER_LAW_CREEP, true, MODE>(c, A);
+            else launch_tile<NPE, APHIP_POWER_LAW_CREEP, false, MODE>(c, A);
             break;
         case APHIP_DRUCKER_PRAGER:
-            if (pq) launch_tile<NPE, APHIP_DRUCKER_PRAGER, true, MODE>(c, A, lds);
-            else launch_tile<NPE, APHIP_DRUCKER_PRAGER, false, MODE>(c, A, lds);
+            if (pq) launch_tile<NPE, APHIP_DRUCKER_PRAGER, true, MODE>(c, A);
+            else launch_tile<NPE, APHIP_DRUCKER_PRAGER, false, MODE>(c, A);
             break;
         default: throw Error(APHIP_ERR_INVALID, "material not set");
     }
@@ -1109,6 +1301,51 @@ void tile_build(Ctx &c, int te, int threads) {
         P.tnp_csr.upload(pc.data(), pc.size(), c.stream);
         P.tnp_bdst.upload(pb.data(), pb.size(), c.stream);
         P.lconn_p.upload(pl.data(), pl.size(), c.stream);
+        if (npe == 8) {  // k_hex_tile's forms
+            std::vector<uint16_t> hc(pl.size());
+            for (size_t i = 0; i < pl.size(); ++i) hc[i] = (uint16_t)(3 * (int)pl[i]);
+            P.hx_conn.upload(hc.data(), hc.size(), c.stream);
+            // one round unless the rows do not fit the LDS beside the tile's nodes
+            int max_int = 0;
+            for (int64_t t = 0; t < nt; ++t) max_int = std::max(max_int, ninterior[t]);
+            auto lds_of = [&](int r) { return tile_lds_bytes(maxtn, max_int, te / r, 8, (r == 1 ? 8 : 12) * maxtn, false); };
+            int R = 1;
+            while (te / R > 16 && lds_of(R) > 160 * 1024) R *= 2;
+            const int rw = te / R;
+            P.hx_rounds = R;
+            P.lds_bytes = lds_of(R);
+            std::vector<uint16_t> first((size_t)nt * R * P.tpad * 8, (uint16_t)(kHexRow * rw)), more;
+            std::vector<uint32_t> hcsr((size_t)nt * R * P.tpad, 0);
+            std::vector<int32_t> base((size_t)nt * R, 0);
+            for (int64_t t = 0; t < nt; ++t)
+                for (int r = 0; r < R; ++r) {
+                    const int64_t tr = t * R + r;
+                    base[tr] = (int32_t)(more.size() / 8);
+                    for (int ln = 0; ln < tstart[t + 1] - tstart[t]; ++ln) {
+                        const uint32_t pk = tcsr[tstart[t] + ln];
+                        const uint16_t *es = &lcsr[(size_t)t * te * npe + (pk >> 16)];
+                        int k = 0, n = 0, cnt = (int)(pk & 0xffffu);
+                        while (k < cnt && es[k] < r * rw * 8) ++k;
+                        const uint32_t m0 = (uint32_t)(more.size() / 8 - base[tr]);
+                        for (; k < cnt && es[k] < (r + 1) * rw * 8; ++k, ++n) {
+                            const int s = es[k] - r * rw * 8;
+                            const uint16_t off = (uint16_t)(kHexRow * (s / 8) + 3 * (s % 8));
+                            if (n < 8) {
+                                first[((size_t)tr * P.tpad + ln) * 8 + n] = off;
+                            } else {
+                                if (n % 8 == 0) more.resize(more.size() + 8, (uint16_t)(kHexRow * rw));
+                                more[more.size() - 8 + n % 8] = off;
+                            }
+                        }
+                        hcsr[(size_t)tr * P.tpad + ln] = (m0 << 16) | (n > 8 ? (uint32_t)(n - 1) / 8 : 0u);
+                    }
+                }
+            APHIP_REQUIRE(more.size() / 8 < (size_t)INT32_MAX, "too many tile entries");
+            P.hx_first.upload(reinterpret_cast<const uint4 *>(first.data()), first.size() / 8, c.stream);
+            P.hx_more.upload(reinterpret_cast<const uint4 *>(more.data()), more.size() / 8, c.stream);
+            P.hx_csr.upload(hcsr.data(), hcsr.size(), c.stream);
+            P.hx_base.upload(base.data(), base.size(), c.stream);
+        }
     }
     P.nslot = bstart[nb];
     P.bpart.alloc(3 * std::max<int64_t>(1, (int64_t)bstart[nb]));
@@ -1133,21 +1370,21 @@ void tile_build(Ctx &c, int te, int threads) {
     int max_nint = 0;
     for (int64_t t = 0; t < nt; ++t) max_nint = std::max(max_nint, ninterior[t]);
     P.max_nint = npe == 4 ? maxtn : max_nint;  // LDS rows of the corrector data (the kernel's choice)
-    // One-element-per-thread Hex8 tiles pass their forces through LDS in two rounds of
-    // te / 2 elements: half the F rows, so twice the workgroups fit per CU.
-    P.f_rounds = (npe == 8 && te == threads) ? 2 : 1;  // the kernel's ROUNDS
-    P.lds_bytes = tile_lds_bytes(P.maxtn, P.max_nint, te, P.f_rounds, npe);  // the kernel carves with these
+    if (npe == 4) P.lds_bytes = tile_lds_bytes(P.maxtn, P.max_nint, te, npe, te * npe, false);
+    P.cell_lds_bytes = tile_lds_bytes(P.maxtn, P.max_nint, te, npe, te * npe, true);
+    // (smoothed Hex8 cells check their own at launch)
     APHIP_REQUIRE(P.lds_bytes <= 160 * 1024, "tile needs more LDS than a CU has; use a smaller tile");
-    {  // the kernel's carve-up must end inside the allocation
-        const TileLds L = carve(nullptr, P.maxtn, P.max_nint, te, P.f_rounds, npe);
+    for (const bool cell : {false, true}) {  // the kernels' carve-up must end inside the allocation
+        const int R = npe == 8 && !cell ? P.hx_rounds : 1;
+        const int nent = npe == 8 && !cell ? (R == 1 ? 8 : 12) * P.maxtn : te * npe;
+        const TileLds L = carve(nullptr, P.maxtn, P.max_nint, nent, tile_f_doubles(npe, te / R, cell));
         APHIP_REQUIRE((size_t)(reinterpret_cast<const char *>(L.fx + P.max_nint) - static_cast<const char *>(nullptr)) <=
-                          P.lds_bytes,
+                          (cell ? P.cell_lds_bytes : P.lds_bytes),
                       "tile LDS layout exceeds its allocation");
     }
-    APHIP_REQUIRE(maxtn <= npe * threads, "tile has more nodes than its gather covers");
-    // the staging loads te * npe / 2 CSR words with at most 2 (Tet4), 4 (Hex8, one element
-    // per thread) or 1 (Hex8, eight lanes per element) per thread
-    APHIP_REQUIRE(te * npe / 2 <= (npe == 4 ? 2 : (threads == te ? 4 : 1)) * threads, "tile CSR exceeds the staging");
+    // the one-element-per-thread gather covers npe x te nodes; its staging loads te * npe / 2
+    // CSR words with at most 2 (Tet4) or 4 (Hex8 cells) per thread.
+    APHIP_REQUIRE(maxtn <= npe * te, "tile has more nodes than its gather covers");
     P.use_stream = (c.flags & APHIP_FLAG_PIPELINED) != 0;
     for (int &g : P.stream_grid) g = 0;  // sized (and LDS attribute set) at the first launch
     P.ready = true;
@@ -1188,6 +1425,12 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     A.tnp_bdst = P.tnp_bdst.p;
     A.lconn_p = P.lconn_p.p;
     A.tpad = P.tpad;
+    A.hx_conn = P.hx_conn.p;
+    A.hx_first = P.hx_first.p;
+    A.hx_more = P.hx_more.p;
+    A.hx_csr = P.hx_csr.p;
+    A.hx_base = P.hx_base.p;
+    A.hx_rounds = P.hx_rounds;
     A.bpart = P.bpart.p;
     A.H = c.Hnp1().p;
     A.P = c.Pnp1().p;
@@ -1218,13 +1461,13 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     A.keep = run.keep || c.mat.rate_form();  // (the rate-form materials read the previous H and P)
     prof_begin(c, 1);
     if (c.npe == 4) {
-        if (mode == 0) dispatch_kind<4, 0>(c, A, P.lds_bytes);
-        else if (mode == 1) dispatch_kind<4, 1>(c, A, P.lds_bytes);
-        else dispatch_kind<4, 2>(c, A, P.lds_bytes);
+        if (mode == 0) dispatch_kind<4, 0>(c, A);
+        else if (mode == 1) dispatch_kind<4, 1>(c, A);
+        else dispatch_kind<4, 2>(c, A);
     } else {
-        if (mode == 0) dispatch_kind<8, 0>(c, A, P.lds_bytes);
-        else if (mode == 1) dispatch_kind<8, 1>(c, A, P.lds_bytes);
-        else dispatch_kind<8, 2>(c, A, P.lds_bytes);
+        if (mode == 0) dispatch_kind<8, 0>(c, A);
+        else if (mode == 1) dispatch_kind<8, 1>(c, A);
+        else dispatch_kind<8, 2>(c, A);
     }
     APHIP_HIP(hipGetLastError());
     prof_end(c, 1);
