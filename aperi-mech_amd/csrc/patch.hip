@@ -16,11 +16,13 @@
 // (the rule is at patch_build).  What bounds it is latency: the launch, two dependent loads,
 // and per step the element's arithmetic and LDS reads (6,174 SVK Tet4, 50 steps in one call:
 // 338 -> about 115 us with three meshes in turn, 595 -> 290 us alone; 49,392 Tet4, one step a
-// call: 7.6 -> 5.2 us a step in turn, 14 -> 11 us alone).  Results are the tile path's, bit for bit: the element
+// call: 7.6 -> 5.2 us a step in turn, 14 -> 11 us alone; 8,000 neo-Hookean Hex8, 50 steps:
+// 276 -> 216 us in turn, 626 -> 550 us alone).  Results are the tile path's, bit for bit: the element
 // arithmetic is the same and a node's sum is grouped by the plan's tiles (partial sums of the
 // node's elements in ascending order, added in ascending tile order).
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstring>
 #include <thread>
 #include <vector>
@@ -60,13 +62,14 @@ struct PatchArgs {
     const int32_t *node;         // [npatch * npad] node ids, ring by ring
     const uint32_t *csr;         // [npatch * cpad] (start << 16) | count of the nodes N_{K-1}
     const int32_t *elem;         // [npatch * epad] element ids, owned ones first, ring by ring
-    const uint16_t *conn;        // [npatch * epad * npe] local nodes
-    const uint16_t *ent;         // [npatch * entpad] force row of the entry (| kNewTile)
+    const uint16_t *conn;        // [npatch * epad * npe] local nodes (Hex8: 3 x local node)
+    const uint16_t *ent;         // [npatch * entpad] offset of the entry's force row / 3 (| kNewTile)
     double *H, *P;
     const double *state_n;
     double *state_np1;
     MatParams mat;
     const double *elem_lambda, *elem_mu;
+    double gauss_a;
     double dt;
     int64_t ne, npatch, nblocks;
     int npad, cpad, epad, entpad;
@@ -86,6 +89,12 @@ struct PatchLds {
 // element sit 24 banks apart)
 __host__ __device__ __forceinline__ int f_stride(int n) { return n + ((4 - n) & 31); }
 
+// force row of (local element, slot), in rows of three doubles: Tet4 slot-major, Hex8 in the
+// element's LDS row
+__host__ __device__ __forceinline__ int force_row(int npe, int epad, int le, int k) {
+    return npe == 4 ? k * f_stride(epad) + le : (kHexRow / 3) * le + k;
+}
+
 __host__ __device__ __forceinline__ PatchLds carve(char *base, int npe, int npad, int cpad, int epad, int entpad) {
     PatchLds L;
     char *p = base;
@@ -99,7 +108,7 @@ __host__ __device__ __forceinline__ PatchLds carve(char *base, int npe, int npad
     L.V = reinterpret_cast<double *>(take(24 * (size_t)npad));
     L.M = reinterpret_cast<double *>(take(8 * (size_t)cpad));
     L.S = reinterpret_cast<double *>(take(8 * (size_t)epad));
-    L.F = reinterpret_cast<double *>(take(24 * (size_t)npe * f_stride(epad)));
+    L.F = reinterpret_cast<double *>(take(npe == 4 ? 96 * (size_t)f_stride(epad) : 8 * kHexRow * (size_t)epad));
     L.csr = reinterpret_cast<uint32_t *>(take(4 * (size_t)cpad));
     L.conn = reinterpret_cast<uint16_t *>(take(2 * (size_t)npe * epad));
     L.ent = reinterpret_cast<uint16_t *>(take(2 * (size_t)entpad));
@@ -109,7 +118,7 @@ __host__ __device__ __forceinline__ PatchLds carve(char *base, int npe, int npad
 }
 
 template <int NPE, int KIND>
-__global__ __launch_bounds__(1024) void k_patch(PatchArgs A) {
+__global__ __launch_bounds__(NPE == 4 ? 1024 : 512, NPE == 4 ? 1 : 3) void k_patch(PatchArgs A) {
     extern __shared__ __align__(16) char lds_raw[];
     const int64_t b = blockIdx.x;
     const int64_t p = (b % kNumXcd) * (A.nblocks / kNumXcd) + b / kNumXcd;  // neighbours share an XCD's L2
@@ -148,7 +157,10 @@ __global__ __launch_bounds__(1024) void k_patch(PatchArgs A) {
         for (int i = tid; i < A.entpad / kBatch; i += nt) dst[i] = src[i];
     }
     for (int i = tid; i < A.epad; i += nt) {
-        reinterpret_cast<ushort4 *>(L.conn)[i] = reinterpret_cast<const ushort4 *>(A.conn + p * A.epad * NPE)[i];
+#pragma unroll
+        for (int k = 0; k < NPE / 4; ++k)
+            reinterpret_cast<ushort4 *>(L.conn)[NPE / 4 * i + k] =
+                reinterpret_cast<const ushort4 *>(A.conn + p * A.epad * NPE)[NPE / 4 * i + k];
         if constexpr (state_width<KIND>() > 0) L.S[i] = load_state<KIND>(A.state_n, elem[i]);
     }
     __syncthreads();
@@ -156,30 +168,22 @@ __global__ __launch_bounds__(1024) void k_patch(PatchArgs A) {
     int ne_now = nE, nn_now = nC;
     for (int s = 1;; ++s) {
         const bool last = s == A.steps;
-        for (int le = tid; le < ne_now; le += nt) {
-            const ushort4 c = reinterpret_cast<const ushort4 *>(L.conn)[le];
-            const int lc[4] = {c.x, c.y, c.z, c.w};
-            double X[NPE][3], U[NPE][3], fe[NPE][3], H[9], P[9];
-#pragma unroll
-            for (int k = 0; k < NPE; ++k) {
-                ld3(L.X, lc[k], X[k]);
-                ld3(L.U, lc[k], U[k]);
-            }
-            MatParams m = A.mat;
-            if (A.elem_lambda) {
-                const int64_t e = elem[le];
-                m.lambda = A.elem_lambda[e];
-                m.mu = A.elem_mu[e];
-            }
-            double sn = 0.0, snp1 = 0.0, aux = 0.0;
-            if constexpr (state_width<KIND>() > 0) sn = L.S[le];
-            tet4_element<KIND>(X, U, m, sn, snp1, aux, H, P, fe);
-#pragma unroll
-            for (int k = 0; k < NPE; ++k) st3(L.F, k * fs + le, fe[k]);
-            if (last) {
-                if (le < nown && (A.keep || state_width<KIND>() > 0)) {
+        if constexpr (NPE == 8) {  // eight lanes per element
+            for (int le = tid >> 3; le < ne_now; le += nt >> 3) {
+                const uint4 c = reinterpret_cast<const uint4 *>(L.conn)[le];
+                const uint32_t cn[4] = {c.x, c.y, c.z, c.w};
+                MatParams m = A.mat;
+                if (A.elem_lambda) {
                     const int64_t e = elem[le];
-                    store_state<KIND>(A.state_np1, e, snp1, aux);
+                    m.lambda = A.elem_lambda[e];
+                    m.mu = A.elem_mu[e];
+                }
+                double H[9], P[9];
+                if (hex8_lanes<KIND, false>(tid & 7, cn, L.X, L.U, L.F + kHexRow * le, m, A.gauss_a, L.S + le, L.S + le,
+                                            H, P) &&
+                    last && le < nown) {
+                    const int64_t e = elem[le];
+                    if constexpr (state_width<KIND>() > 0) A.state_np1[e] = L.S[le];
                     if (A.keep) {
 #pragma unroll
                         for (int i = 0; i < 9; ++i) {
@@ -188,8 +192,43 @@ __global__ __launch_bounds__(1024) void k_patch(PatchArgs A) {
                         }
                     }
                 }
-            } else if constexpr (state_width<KIND>() > 0) {
-                L.S[le] = snp1;
+            }
+        } else {
+            for (int le = tid; le < ne_now; le += nt) {
+                const ushort4 c = reinterpret_cast<const ushort4 *>(L.conn)[le];
+                const int lc[4] = {c.x, c.y, c.z, c.w};
+                double X[NPE][3], U[NPE][3], fe[NPE][3], H[9], P[9];
+#pragma unroll
+                for (int k = 0; k < NPE; ++k) {
+                    ld3(L.X, lc[k], X[k]);
+                    ld3(L.U, lc[k], U[k]);
+                }
+                MatParams m = A.mat;
+                if (A.elem_lambda) {
+                    const int64_t e = elem[le];
+                    m.lambda = A.elem_lambda[e];
+                    m.mu = A.elem_mu[e];
+                }
+                double sn = 0.0, snp1 = 0.0, aux = 0.0;
+                if constexpr (state_width<KIND>() > 0) sn = L.S[le];
+                tet4_element<KIND>(X, U, m, sn, snp1, aux, H, P, fe);
+#pragma unroll
+                for (int k = 0; k < NPE; ++k) st3(L.F, k * fs + le, fe[k]);
+                if (last) {
+                    if (le < nown && (A.keep || state_width<KIND>() > 0)) {
+                        const int64_t e = elem[le];
+                        store_state<KIND>(A.state_np1, e, snp1, aux);
+                        if (A.keep) {
+#pragma unroll
+                            for (int i = 0; i < 9; ++i) {
+                                store_once(A.H + i * A.ne + e, H[i]);
+                                store_once(A.P + i * A.ne + e, P[i]);
+                            }
+                        }
+                    }
+                } else if constexpr (state_width<KIND>() > 0) {
+                    L.S[le] = snp1;
+                }
             }
         }
         __syncthreads();
@@ -239,6 +278,8 @@ __global__ __launch_bounds__(1024) void k_patch(PatchArgs A) {
     }
 }
 
+static_assert(state_width<APHIP_J2>() == 1, "patches keep one state value per element");
+
 template <int NPE>
 void launch(Ctx &c, const PatchArgs &A) {
     const PatchPlan &P = c.patch;
@@ -278,11 +319,15 @@ static void patch_build(Ctx &c) {
     //     750 T 71/177  2x64 59/149          24,576 T 119/275  1x128 70/174  2x128 88/169
     //   3,072 T 169/294 2x64 46/137  1x64 95/203   48,000 T 168/280  1x256 114/211  1x128 119/229
     //  10,368 T 120/264 2x128 54/165 2x64 69/146   93,750 T 167/288  1x256 209/344
+    // n^3 Hex8 (the tile path costs 163-175 in turn from launches alone, on this host):
+    //     125 T 96/192  2x8 59/171  1x16 94/181    8,000 T 175/286  1x32 103/248  1x64 138/336
+    //   1,000 T 172/265 1x16 93/178 2x8 74/216    17,576 T 168/337  1x32 153/322
+    //   2,744 T 175/267 1x16 97/181 1x32 92/211   32,768 T 163/292  1x64 231/340
     // A second ring pays while the chip idles (it evaluates some four times the elements), the
     // whole scheme until the elements evaluated twice cost what a launch does.
-    if (npe != 4 || ne == 0 || ne > 64000 || c.tiles.threads != c.tiles.te || c.elem_seg.size() != 2) return;
-    const int K = ne <= 16000 ? 2 : 1;
-    const int64_t target = ne <= 6500 ? 64 : ne <= 32000 ? 128 : 256;
+    if (ne == 0 || ne > (npe == 4 ? 64000 : 20000) || c.tiles.threads != c.tiles.te || c.elem_seg.size() != 2) return;
+    const int K = ne <= (npe == 4 ? 16000 : 500) ? 2 : 1;
+    const int64_t target = npe == 4 ? (ne <= 6500 ? 64 : ne <= 32000 ? 128 : 256) : (ne <= 500 ? 8 : ne <= 4000 ? 16 : 32);
     const std::vector<int32_t> &conn = c.conn_h;
     // node -> (element, slot), ascending
     std::vector<int32_t> start(nn + 1, 0), inc((size_t)ne * npe);
@@ -364,7 +409,8 @@ static void patch_build(Ctx &c) {
             }
             for (int32_t e : q.elems)
                 for (int k = 0; k < npe; ++k) q.conn.push_back((uint16_t)nloc[conn[(int64_t)e * npe + k]]);
-            if (npe * f_stride((int)q.elems.size()) > 0x7fff || q.nodes.size() > 0xffff) fits = false;
+            if (force_row(npe, (int)q.elems.size(), (int)q.elems.size(), npe) > 0x7fff || 3 * q.nodes.size() > 0xffff)
+                fits = false;
             for (int32_t n : q.nodes) nloc[n] = -1;
             for (int32_t e : q.elems) eloc[e] = -1;
         }
@@ -384,8 +430,7 @@ static void patch_build(Ctx &c) {
         epad = std::max(epad, q.elems.size());
         entpad = std::max(entpad, q.ent.size());
     }
-    const int fs = f_stride((int)epad);
-    if (npe * fs > 0x7fff) return;
+    if (force_row(npe, (int)epad, (int)epad, npe) > 0x7fff) return;
     const size_t lds = carve(nullptr, npe, (int)npad, (int)cpad, (int)epad, (int)entpad).bytes;
     if (lds > 160 * 1024) return;
     std::vector<int32_t> meta((size_t)np * 16, 0), node(np * npad);
@@ -402,12 +447,12 @@ static void patch_build(Ctx &c) {
         std::copy(q.csr.begin(), q.csr.end(), csr.begin() + p * cpad);
         for (size_t i = 0; i < q.ent.size(); ++i) {
             const int le = q.ent[i] & ~kNewTile;
-            ent[p * entpad + i] = (uint16_t)((le % npe) * fs + le / npe) | (q.ent[i] & kNewTile);
+            ent[p * entpad + i] = (uint16_t)force_row(npe, (int)epad, le / npe, le % npe) | (q.ent[i] & kNewTile);
         }
         for (size_t i = 0; i < epad; ++i) {
             const size_t j = std::min(i, q.elems.size() - 1);
             elem[p * epad + i] = q.elems[j];
-            for (int k = 0; k < npe; ++k) lconn[(p * epad + i) * npe + k] = q.conn[j * npe + k];
+            for (int k = 0; k < npe; ++k) lconn[(p * epad + i) * npe + k] = (uint16_t)((npe == 8 ? 3 : 1) * q.conn[j * npe + k]);
         }
     }
     // one allocation and one copy for the six lists (each on a 16-byte boundary)
@@ -438,13 +483,15 @@ static void patch_build(Ctx &c) {
     P.epad = (int)epad;
     P.entpad = (int)entpad;
     P.lds_bytes = lds;
-    P.threads = std::max(128, std::min(1024, (int)(epad + 63) / 64 * 64));
+    // Tet4: one element per thread where 1024 reach; Hex8 (eight lanes per element) 256, so that
+    // several patches share a CU (8,000 Hex8, 50 steps: 216 us in turn, 312 us with 512)
+    P.threads = npe == 4 ? std::max(128, std::min(1024, (int)(epad + 63) / 64 * 64)) : 256;
     P.ready = true;
 }
 
 bool patch_eligible(Ctx &c) {
     if (c.tiles.ready && !c.patch.tried) patch_build(c);
-    return c.patch.ready && !c.node_dt.p && !c.tiles.use_stream &&
+    return c.patch.ready && !c.node_dt.p && !c.tiles.use_stream && !c.mat.state_per_qp &&
            (c.mat.kind == APHIP_LINEAR_ELASTIC || c.mat.kind == APHIP_NEO_HOOKEAN || c.mat.kind == APHIP_J2 ||
             c.mat.kind == APHIP_SVK);
 }
@@ -477,6 +524,7 @@ void patch_run(Ctx &c, double dt, int steps, bool keep) {
     A.mat = c.mat.params();
     A.elem_lambda = c.has_fields ? c.elem_lambda.p : nullptr;
     A.elem_mu = c.has_fields ? c.elem_mu.p : nullptr;
+    A.gauss_a = 1.0 / std::sqrt(3.0);
     A.dt = dt;
     A.ne = c.ne;
     A.npatch = P.npatch;
@@ -487,7 +535,8 @@ void patch_run(Ctx &c, double dt, int steps, bool keep) {
     A.entpad = P.entpad;
     A.steps = steps;
     A.keep = keep;
-    launch<4>(c, A);
+    if (c.npe == 4) launch<4>(c, A);
+    else launch<8>(c, A);
     std::swap(c.u.p, P.u.p);
     std::swap(c.v.p, P.v.p);
     std::swap(c.a.p, P.a.p);

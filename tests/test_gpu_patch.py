@@ -12,12 +12,12 @@ pytestmark = pytest.mark.gpu
 FIELDS = (A.FIELD_U, A.FIELD_V, A.FIELD_A, A.FIELD_F, A.FIELD_H, A.FIELD_P)
 
 
-def _run(X, conn, kind, calls, graph, fields, tiling):
+def _run(X, conn, kind, calls, graph, fields, tiling, etype=A.TET4):
     rho, E, nu = 2700.0, 70e9, 0.33
     fixed = np.zeros(X.shape, dtype=np.uint8)
     fixed[X[:, 2] < 0.01] = (1, 1, 0)
     with A.Solver() as s:
-        s.set_mesh(A.TET4, X, conn)
+        s.set_mesh(etype, X, conn)
         s.set_material(kind, rho, E, nu, 30e6, 1e9)
         if tiling:
             s.set_tiling(tiling, tiling)
@@ -51,5 +51,19 @@ def test_patches_match_tiles(gpu_available, n, kind, fields, tiling):
     want = _run(X, conn, kind, [2, 2, 2], True, fields, tiling)
     for calls in ([1] * 6, [6], [3, 3]):
         got = _run(X, conn, kind, calls, False, fields, tiling)
+        for a, b in zip(want, got):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+# two rings of 8 owned elements; one ring of 16 and of 32 (the last tile partial); the tile path
+@pytest.mark.parametrize("n", [(1, 1, 1), (7, 8, 9), (11, 12, 13), (17, 19, 18), (26, 27, 29)])
+@pytest.mark.parametrize("kind,fields,tiling", [(A.NEO_HOOKEAN, True, 0), (A.J2, False, 256), (A.LINEAR_ELASTIC, False, 64)])
+def test_hex8_patches_match_tiles(gpu_available, n, kind, fields, tiling):
+    X, conn = M.hex_lattice(*n, *(k / max(n) for k in n))
+    X = M.jitter(X, 1.0 / max(n), 0.1, 7, 1)
+    print(f"patches {len(conn)} Hex8 kind={kind} tiling={tiling}", flush=True)
+    want = _run(X, conn, kind, [2, 2, 2], True, fields, tiling, A.HEX8)
+    for calls in ([1] * 6, [6], [3, 3]):
+        got = _run(X, conn, kind, calls, False, fields, tiling, A.HEX8)
         for a, b in zip(want, got):
             assert np.isfinite(a).all() and np.array_equal(a, b)
