@@ -331,6 +331,15 @@ static bool use_tiles(const Ctx &c) {
     return c.tiles.ready && !(c.flags & APHIP_FLAG_TWO_PASS) && c.formulation == APHIP_TOTAL_LAGRANGIAN;
 }
 
+// Updated and semi-Lagrangian steps on the tile plan: two launches a step, element forces
+// through LDS, where the element-partial kernels take three and pass 24 B per element node
+// through memory (20 steps of 33k J2 Hex8: 279 -> 200 us with three streams in turn).  Their
+// force evaluations, and a Hex8 plan that needs several LDS rounds, keep the partials.
+static bool ul_steps_on_tiles(const Ctx &c) {
+    return c.formulation != APHIP_TOTAL_LAGRANGIAN && !c.cells.ready && c.tiles.ready && c.tiles.hx_rounds == 1 &&
+           !(c.flags & APHIP_FLAG_TWO_PASS);
+}
+
 // Graph replay keeps the tile kernels: a patch launch exchanges the buffers of u, v and a.
 static bool steps_on_patches(Ctx &c) {
     return use_tiles(c) && !c.cells.ready && !c.graph_enabled && patch_eligible(c);
@@ -477,10 +486,11 @@ static void node_pass(Ctx &c, double dt, int mode, bool more = false) {
 static void step_once(Ctx &c, double dt, bool pred_in, bool pred_out, bool keep) {
     c.state_np1 = 1 - c.state_np1;  // UpdateFieldStates (Explicit.cpp:393)
     c.rate_dt = dt;                 // SetTimeIncrement (ElementTetrahedron4.h:187)
-    if (use_tiles(c)) {
+    if (use_tiles(c) || ul_steps_on_tiles(c)) {
+        const bool total = c.formulation == APHIP_TOTAL_LAGRANGIAN;
         TileRun run;
-        run.pred_in = pred_in;
-        run.pred_out = pred_out;
+        run.pred_in = pred_in && total;
+        run.pred_out = pred_out && total;
         run.keep = keep;
         tile_run(c, dt, 2, run);
     } else {
@@ -1284,9 +1294,11 @@ int aphip_step(aphip_ctx *c, double dt, int32_t n_steps) {
         }
     }
     for (bool pred = false; done < n_steps; ++done) {
-        const bool more = done + 1 < n_steps && c->formulation != APHIP_SEMI_LAGRANGIAN;
+        const bool more = done + 1 < n_steps;
+        // (a semi-Lagrangian reference update after this step reads H)
+        const bool update = c->formulation == APHIP_SEMI_LAGRANGIAN && (c->steps_done + 1) % c->semi_interval == 0;
         prof_begin(*c, 0);
-        step_once(*c, dt, pred, more, !more);
+        step_once(*c, dt, pred, more, !more || update);
         prof_end(*c, 0);
         pred = more;
         // the reference's StepScheduler(interval, interval) after step n (Explicit.cpp:195-212)

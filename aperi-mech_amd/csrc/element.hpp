@@ -297,7 +297,8 @@ APHIP_DEV int hex8_lane_label(int lane) {
 // in the lane for which the function returns true; with PER_QP every lane stores its state.
 // LEAN: the lane's signs are derived again after the stress update instead of held across it
 // (12 VGPRs less, for callers that would spill).
-template <int KIND, bool PER_QP, bool LEAN = false>
+// UL: updated / semi-Lagrangian, as hex8_element's.
+template <int KIND, bool PER_QP, bool LEAN = false, bool UL = false>
 APHIP_DEV bool hex8_lanes(int lane, const uint32_t (&cn)[4], const double *sX, const double *sU, double *row,
                           const MatParams &m, double ga, const double *state_n, double *state_np1, double *H,
                           double *P, const RateIn *r = nullptr) {
@@ -352,9 +353,17 @@ APHIP_DEV bool hex8_lanes(int lane, const uint32_t (&cn)[4], const double *sX, c
     const bool last = q == 7;
     double snp1 = 0.0, aux = 0.0;
     const double sn = load_state<KIND>(state_n, PER_QP ? q : 0), sn2 = load_state2<KIND>(state_n, PER_QP ? q : 0);
+    if constexpr (UL) ul_gradient(H, r->Hn);
     stress<KIND>(H, m, sn, snp1, aux, P, r, sn2);
     if constexpr (PER_QP) store_state<KIND>(state_np1, q, snp1, aux);
     else if (last) store_state<KIND>(state_np1, 0, snp1, aux);
+    double Pf[9];
+    if constexpr (UL) {
+        ul_force_stress(P, r->Hn, Pf);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 9; ++i) Pf[i] = P[i];
+    }
     if constexpr (LEAN) {
         asm volatile("" : "+v"(x));  // (a value the compiler cannot match with the earlier one)
         b0 = x & 1;
@@ -371,7 +380,7 @@ APHIP_DEV bool hex8_lanes(int lane, const uint32_t (&cn)[4], const double *sX, c
     for (int n = 0; n < 3; ++n)
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            double v = dot3(Ad[3 * n], P[3 * j], Ad[3 * n + 1], P[3 * j + 1], Ad[3 * n + 2], P[3 * j + 2]);
+            double v = dot3(Ad[3 * n], Pf[3 * j], Ad[3 * n + 1], Pf[3 * j + 1], Ad[3 * n + 2], Pf[3 * j + 2]);
             v = n == 0 ? v + hex8_partner<0>(v) : __fma_rn(s0, hex8_partner<0>(v), v);
             v = n == 1 ? v + hex8_partner<1>(v) : __fma_rn(s1, hex8_partner<1>(v), v);
             W[n][j] = n == 2 ? v + hex8_partner<2>(v) : __fma_rn(s2, hex8_partner<2>(v), v);

@@ -99,6 +99,11 @@ struct TileArgs {
     int64_t first_shared;
     // 0: an inner step of one call, whose H, P and f the next step overwrites unread
     int keep;
+    int keep_h;  // H alone (the updated formulation reads it in the next step)
+    // updated / semi-Lagrangian steps (X: the configuration integrated over): the increments
+    // written, the next coordinates (updated), 1 when the increments accumulate (semi)
+    double *dinc, *xnp1;
+    int semi;
     int cell_marker;  // smoothed cells turn a new failure's marker into the maximum damage
 };
 
@@ -151,15 +156,15 @@ __host__ inline size_t tile_lds_bytes(int maxtn, int max_nint, int te, int npe, 
 
 // Materials whose Hex8 kernel needs more than the 128 VGPRs of four waves per SIMD (it would
 // spill 117 for creep, 78 for Drucker-Prager, 10 for damage).
-template <int KIND>
+template <int KIND, bool UL = false>
 constexpr bool hex_wide() {
-    return rate_form<KIND>() || KIND == APHIP_NEO_HOOKEAN_DAMAGE;
+    return UL || rate_form<KIND>() || KIND == APHIP_NEO_HOOKEAN_DAMAGE;
 }
 // Workgroup of the Hex8 kernel: eight lanes per element, at most 512 lanes up to 128 elements
 // (two passes: two workgroups fit a CU) and in rounds, else 1024 (wide materials 512).
-template <int KIND>
+template <int KIND, bool UL = false>
 __host__ int hex_threads(int te, int rounds) {
-    return std::min(te <= 128 || rounds > 1 || hex_wide<KIND>() ? 512 : 1024, 8 * (te / rounds));
+    return std::min(te <= 128 || rounds > 1 || hex_wide<KIND, UL>() ? 512 : 1024, 8 * (te / rounds));
 }
 
 // Optional arrays are read without branches: an absent array is replaced by the
@@ -186,14 +191,48 @@ __device__ __forceinline__ void load_elem_lame(const TileArgs &A, int64_t e, Mat
     m.mu = A.elem_lambda ? mu : m.mu;
 }
 
+// MODE 2 staging of a node: v1/2 and what the element gradients are taken of, the predicted
+// displacement or (UL, u then being the semi-Lagrangian increments so far) the increment
+// since the configuration integrated over.
+template <bool UL>
+__device__ __forceinline__ void stage_predict(const TileArgs &A, const double *u, const double *v, const double *a,
+                                              unsigned fx, double dt, double *vh, double *u1) {
+#pragma clang fp contract(off)
+    cd_predict(u, v, a, fx, dt, vh, u1);
+    if constexpr (UL) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double inc = dt * vh[d];
+            u1[d] = A.semi ? u[d] + inc : inc;
+        }
+    }
+}
+
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt at their maxima: not waited on).  At a
 // point where no store is outstanding this costs nothing beyond the loads' latency.
 __device__ __forceinline__ void wait_vmem_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
+// Updated / semi-Lagrangian node update (ExplicitTimeIntegrator.h:193-226): with the step's
+// increment inc = dt v1/2, u += inc; updated: x_{n+1} = x_n + inc and the increment itself is
+// kept; semi: the accumulated increment acc.
+__device__ __forceinline__ void ul_store(double *u, double *dinc, double *xnp1, int semi, int64_t g, double dt,
+                                         const double *vh, const double *x, const double *acc) {
+#pragma clang fp contract(off)
+    double un[3];
+    ld3(u, g, un);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double inc = dt * vh[d];
+        u[3 * g + d] = un[d] + inc;
+        dinc[3 * g + d] = semi ? acc[d] : inc;
+        if (!semi) xnp1[3 * g + d] = x[d] + inc;
+    }
+}
+
 // Node ln's force f is complete: an interior node is finished and written (MODE 0: f;
 // 1: f and a = f/m; 2: the corrector); a shared node parks f in its slot for the
 // shared-node pass.
-template <int MODE>
+template <int MODE, bool UL = false>
 __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L, int ln, int nint, int64_t ibase,
                                             const double (&f)[3]) {
     if (ln < nint) {
@@ -208,7 +247,13 @@ __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L,
             ld3(L.V, ln, vh);
             ld3(L.U, ln, u1);
             cd_correct(f, L.M[ln], L.fx[ln], L.DT[ln], vh, a1, v1);
-            st3(A.u, g, u1);
+            if constexpr (UL) {
+                double x[3];
+                ld3(L.X, ln, x);
+                ul_store(A.u, A.dinc, A.xnp1, A.semi, g, A.dt, vh, x, u1);
+            } else {
+                st3(A.u, g, u1);
+            }
             st3(A.v, g, v1);
             st3(A.a, g, a1);
         }
@@ -220,7 +265,8 @@ __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L,
 // MODE 0: force only; 1: force + a = f/m (initial); 2: full central-difference step.
 // One element per thread: Tet4 (NPE 4), or smoothed Hex8 cells (NPE 8, MODE 0); the 2x2x2 Gauss
 // Hex8 has k_hex_tile.
-template <int NPE, int KIND, int MODE>
+// UL: updated / semi-Lagrangian step.
+template <int NPE, int KIND, int MODE, bool UL = false>
 __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_tile(TileArgs A) {
     static_assert(NPE == 4 || MODE == 0, "smoothed Hex8 cells are evaluated in force mode");
     extern __shared__ __align__(16) char lds_raw[];
@@ -285,7 +331,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
 #pragma unroll
             for (int d = 0; d < 3; ++d) vq[q][d] = aq[q][d] = 0.0;
         } else {
-            ld3(A.u, g, uq[q]);
+            ld3(UL ? A.dinc : A.u, g, uq[q]);
             fq[q] = load_fixed(A, g);
             if constexpr (MODE >= 1) mq[q] = A.mass[g];
             if constexpr (MODE == 2) {
@@ -314,7 +360,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
         sn2 = load_state2<KIND>(A.state_n, ec);
     }
     RateIn rin;
-    load_rate<KIND>(rin, A.Hn, A.Pn, A.ne, ec, A.rate_dt);
+    load_rate<KIND, UL>(rin, A.Hn, A.Pn, A.ne, ec, A.rate_dt);
 
     {
         uint32_t *dst = reinterpret_cast<uint32_t *>(L.ent);
@@ -341,7 +387,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
         }
         if constexpr (MODE == 2) {
             double vh[3] = {0.0, 0.0, 0.0}, u1[3] = {u[0], u[1], u[2]};
-            if (!pre) cd_predict(u, v, a, fx, nd, vh, u1);
+            if (!pre) stage_predict<UL>(A, u, v, a, fx, nd, vh, u1);
             st3(L.U, ln, u1);
             if (interior) st3(L.V, ln, vh);
         } else {
@@ -358,7 +404,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
         const int64_t g = A.tn_node[tb + ln];
         double x[3], u[3], v[3], a[3];
         ld3(A.X, g, x);
-        ld3(A.u, g, u);
+        ld3(UL ? A.dinc : A.u, g, u);
         const unsigned fx = load_fixed(A, g);
         double mm = 1.0, nd = A.dt;
         if constexpr (MODE >= 1) mm = A.mass[g];
@@ -405,7 +451,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
         double H[9], P[9];
         if constexpr (NPE == 4) {
             double snp1 = 0.0, aux = 0.0;
-            tet4_element<KIND>(X, U, m, sn, snp1, aux, H, P, fe, &rin, sn2);
+            tet4_element<KIND, UL>(X, U, m, sn, snp1, aux, H, P, fe, &rin, sn2);
             if (A.cell_marker) snp1 = cell_damage_marker<KIND>(snp1, m);
             store_state<KIND>(A.state_np1, e, snp1, aux);
         } else {
@@ -417,7 +463,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
 #pragma unroll
             for (int i = 0; i < 9; ++i) pdef[i] = P[i];
         }
-        if (A.keep) {
+        if (A.keep_h) {
 #pragma unroll
             for (int i = 0; i < 9; ++i) {
                 store_once(A.H + i * A.ne + e, H[i]);
@@ -453,7 +499,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
                 f[1] += L.F[rw + 1];
                 f[2] += L.F[rw + 2];
             }
-            finish_node<MODE>(A, L, ln, nint, ibase, f);
+            finish_node<MODE, UL>(A, L, ln, nint, ibase, f);
         }
         return;
     }
@@ -511,8 +557,8 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
 // elements' forces and, before them, the modes share the element's LDS row; a tile whose rows
 // do not fit the LDS passes them through in rounds (MULTI), whose sums a node's thread adds up
 // in an LDS row: the same sequence for every number of rounds.
-template <int KIND, bool PER_QP, int MODE, bool MULTI>
-__global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KIND>() ? 2 : 4) void k_hex_tile(TileArgs A) {
+template <int KIND, bool PER_QP, int MODE, bool MULTI, bool UL = false>
+__global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_wide<KIND, UL>()) ? 2 : 4) void k_hex_tile(TileArgs A) {
     extern __shared__ __align__(16) char lds_raw[];
     const int64_t t = xcd_tile(A.nblocks);
     if (t >= A.ntiles) return;
@@ -522,7 +568,7 @@ __global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KI
     double *acc = reinterpret_cast<double *>(L.ent);
     const int tid = threadIdx.x, nt = blockDim.x;
     // A: every global load of the stage before the first LDS write (see k_tile)
-    constexpr int PASSES = hex_wide<KIND>() ? 4 : 2;  // te <= PASSES * blockDim / 8
+    constexpr int PASSES = hex_wide<KIND, UL>() ? 4 : 2;  // te <= PASSES * blockDim / 8
     const uint4 *conn = reinterpret_cast<const uint4 *>(A.hx_conn) + t * (int64_t)A.te;
     uint4 cq[PASSES];
     if constexpr (!MULTI) {
@@ -551,7 +597,7 @@ __global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KI
 #pragma unroll
             for (int d = 0; d < 3; ++d) v0[d] = a0[d] = 0.0;
         } else {
-            ld3(A.u, g0, u0);
+            ld3(UL ? A.dinc : A.u, g0, u0);
             f0 = load_fixed(A, g0);
             if constexpr (MODE >= 1) m0 = A.mass[g0];
             if constexpr (MODE == 2) {
@@ -582,7 +628,7 @@ __global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KI
         }
         if constexpr (MODE == 2) {
             double vh[3] = {0.0, 0.0, 0.0}, u1[3] = {u[0], u[1], u[2]};
-            if (!pre) cd_predict(u, v, a, fx, nd, vh, u1);
+            if (!pre) stage_predict<UL>(A, u, v, a, fx, nd, vh, u1);
             st3(L.U, ln, u1);
             if (ln < nint) st3(L.V, ln, vh);
         } else {
@@ -594,7 +640,7 @@ __global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KI
         const int64_t row = t * (int64_t)A.tpad + ln, g = A.tnp_node[row];
         double x[3], u[3], v[3], a[3], mm = 1.0, nd = A.dt;
         ld3(A.X, g, x);
-        ld3(A.u, g, u);
+        ld3(UL ? A.dinc : A.u, g, u);
         const unsigned fx = load_fixed(A, g);
         if constexpr (MODE >= 1) mm = A.mass[g];
         if constexpr (MODE == 2) {
@@ -637,18 +683,18 @@ __global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KI
                 m.mu = A.elem_lambda ? mu : m.mu;
             }
             RateIn rin;
-            load_rate<KIND>(rin, A.Hn, A.Pn, A.ne, e, A.rate_dt);
+            load_rate<KIND, UL>(rin, A.Hn, A.Pn, A.ne, e, A.rate_dt);
             const uint32_t cn[4] = {cw.x, cw.y, cw.z, cw.w};
             const int64_t so = state_width<KIND>() * (PER_QP ? e * 8 : e);
             double H[9], P[9];
-            const bool last = hex8_lanes<KIND, PER_QP, MULTI>(tid & 7, cn, L.X, L.U, L.F + kHexRow * lr, m, A.gauss_a,
+            const bool last = hex8_lanes<KIND, PER_QP, MULTI, UL>(tid & 7, cn, L.X, L.U, L.F + kHexRow * lr, m, A.gauss_a,
                                                        state_width<KIND>() ? A.state_n + so : nullptr,
                                                        state_width<KIND>() ? A.state_np1 + so : nullptr, H, P, &rin);
-            if (last && A.keep) {
+            if (last && A.keep_h) {
 #pragma unroll
                 for (int i = 0; i < 9; ++i) {
                     store_once(A.H + i * A.ne + e, H[i]);
-                    store_once(A.P + i * A.ne + e, P[i]);
+                    if (A.keep) store_once(A.P + i * A.ne + e, P[i]);
                 }
             }
         };
@@ -671,7 +717,7 @@ __global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KI
                 add8(reinterpret_cast<const uint4 *>(L.ent)[ln], f);
                 const uint32_t csr = L.csr[ln];
                 if (csr & 0xffffu) add_more(csr, A.hx_base[t], f);
-                finish_node<MODE>(A, L, ln, nint, ibase, f);
+                finish_node<MODE, UL>(A, L, ln, nint, ibase, f);
             }
         } else {
             const int64_t tr = t * (int64_t)rounds + r;
@@ -682,7 +728,7 @@ __global__ __launch_bounds__(MULTI || hex_wide<KIND>() ? 512 : 1024, hex_wide<KI
                 const uint32_t csr = A.hx_csr[tr * A.tpad + ln];
                 if (csr & 0xffffu) add_more(csr, A.hx_base[tr], f);
                 if (r + 1 < rounds) st3(acc, ln, f);
-                else finish_node<MODE>(A, L, ln, nint, ibase, f);
+                else finish_node<MODE, UL>(A, L, ln, nint, ibase, f);
             }
             if (r + 1 < rounds) __syncthreads();
         }
@@ -998,9 +1044,13 @@ struct BoundArgs {
     double dt;
     double *upred;  // mode 2: store the next step's predicted displacement (same dt), or null
     int keep;       // 0: an inner step, f is not stored
+    // updated / semi-Lagrangian: the configuration integrated over, and as in TileArgs
+    const double *xn;
+    double *dinc, *xnp1;
+    int semi;
 };
 
-template <int MODE>
+template <int MODE, bool UL = false>
 __global__ __launch_bounds__(256) void k_boundary(BoundArgs A) {
     const int64_t b_raw = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool live = b_raw < A.nb;
@@ -1045,7 +1095,17 @@ __global__ __launch_bounds__(256) void k_boundary(BoundArgs A) {
         double vh[3], u1[3], a1[3], v1[3];
         cd_predict(u, v, a, fx, dt, vh, u1);
         cd_correct(f, m, fx, dt, vh, a1, v1);
-        st3(A.u, g, u1);
+        if constexpr (UL) {
+#pragma clang fp contract(off)
+            double x[3], acc[3];
+            ld3(A.xn, g, x);
+            ld3(A.dinc, g, acc);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) acc[d] = acc[d] + dt * vh[d];
+            ul_store(A.u, A.dinc, A.xnp1, A.semi, g, dt, vh, x, acc);
+        } else {
+            st3(A.u, g, u1);
+        }
         st3(A.v, g, v1);
         st3(A.a, g, a1);
         if (A.upred) {  // the predictor of the next step from the values just stored
@@ -1066,6 +1126,13 @@ void launch_tile(Ctx &c, const TileArgs &A) {
             APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(threads), lds, c.stream, A);
     };
+    if constexpr (MODE == 2) {
+        if (c.formulation != APHIP_TOTAL_LAGRANGIAN) {
+            if constexpr (NPE == 4) go(k_tile<4, KIND, 2, true>, P.threads, P.lds_bytes);
+            else go(k_hex_tile<KIND, PER_QP, 2, false, true>, hex_threads<KIND, true>(P.te, 1), P.lds_bytes);
+            return;
+        }
+    }
     if constexpr (NPE == 4) {
         go(k_tile<4, KIND, MODE>, P.threads, P.lds_bytes);
     } else {
@@ -1111,7 +1178,7 @@ bool stream_eligible(const Ctx &c) {
 template <int NPE, int MODE>
 void dispatch_kind(Ctx &c, const TileArgs &A) {
     if constexpr (NPE == 4 && MODE == 2) {
-        if (stream_eligible(c)) {
+        if (stream_eligible(c) && c.formulation == APHIP_TOTAL_LAGRANGIAN) {
             switch (c.mat.kind) {
                 case APHIP_LINEAR_ELASTIC: launch_stream<APHIP_LINEAR_ELASTIC>(c, A); return;
                 case APHIP_NEO_HOOKEAN: launch_stream<APHIP_NEO_HOOKEAN>(c, A); return;
@@ -1403,8 +1470,10 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     const bool cells8 = c.npe == 8 && c.cells.ready;
     APHIP_REQUIRE(!cells8 || (mode == 0 && P.threads == P.te), "Hex8 cells: force mode, one cell per thread");
     if (c.ne == 0) return;
+    const bool ul = c.formulation != APHIP_TOTAL_LAGRANGIAN;
+    APHIP_REQUIRE(!ul || (mode == 2 && !pred_in && !pred_out && P.hx_rounds == 1), "updated formulation: step mode");
     TileArgs A;
-    A.X = c.X.p;
+    A.X = ul ? c.xcn().p : c.X.p;
     A.u = run.u_in ? const_cast<double *>(run.u_in) : c.u.p;
     A.v = c.v.p;
     A.a = c.a.p;
@@ -1434,7 +1503,7 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     A.bpart = P.bpart.p;
     A.H = c.Hnp1().p;
     A.P = c.Pnp1().p;
-    A.Hn = c.mat.rate_form() ? c.Hn().p : nullptr;
+    A.Hn = c.formulation == APHIP_SEMI_LAGRANGIAN ? c.Href.p : c.h_pair() ? c.Hn().p : nullptr;
     A.Pn = c.mat.rate_form() ? c.Pn().p : nullptr;
     A.rate_dt = mode == 2 ? dt : c.rate_dt;
     A.state_n = c.state[1 - c.state_np1].p;
@@ -1458,7 +1527,11 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     A.upred = pred_in ? P.upred.p : nullptr;
     A.first_shared = P.n_interior;
     A.cell_marker = c.cells.ready;
+    A.dinc = c.dinc.p;
+    A.xnp1 = c.formulation == APHIP_UPDATED_LAGRANGIAN ? c.xcnp1().p : nullptr;
+    A.semi = c.formulation == APHIP_SEMI_LAGRANGIAN;
     A.keep = run.keep || c.mat.rate_form();  // (the rate-form materials read the previous H and P)
+    A.keep_h = A.keep || c.h_pair();
     prof_begin(c, 1);
     if (c.npe == 4) {
         if (mode == 0) dispatch_kind<4, 0>(c, A);
@@ -1474,11 +1547,13 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     if (P.nb > 0) {
         BoundArgs B{P.nb, P.n_interior, P.bstart.p, P.bpart.p, c.u.p, c.v.p, c.a.p, A.f, c.mass.p,
                     c.has_fixed ? c.fixed.p : nullptr, c.node_dt.p, P.zero.p, dt,
-                    pred_out ? P.upred.p : nullptr, A.keep};
+                    pred_out ? P.upred.p : nullptr, A.keep,
+                    A.X, A.dinc, A.xnp1, A.semi};
         const dim3 grid((unsigned)((P.nb + 255) / 256));
         prof_begin(c, 2);
         if (mode == 0) hipLaunchKernelGGL(k_boundary<0>, grid, dim3(256), 0, c.stream, B);
         else if (mode == 1) hipLaunchKernelGGL(k_boundary<1>, grid, dim3(256), 0, c.stream, B);
+        else if (ul) hipLaunchKernelGGL((k_boundary<2, true>), grid, dim3(256), 0, c.stream, B);
         else hipLaunchKernelGGL(k_boundary<2>, grid, dim3(256), 0, c.stream, B);
         APHIP_HIP(hipGetLastError());
         prof_end(c, 2);

@@ -182,3 +182,43 @@ def test_semi_refuses_rate_form(gpu_available):
         s.set_material(A.POWER_LAW_CREEP, RHO, E, NU, creep=CREEP)
         with pytest.raises(A.AphipError, match="rate-form"):
             s.set_semi_lagrangian(5)
+
+
+# tile steps against the element-partial steps (FLAG_TWO_PASS): one tile and several, partial
+# tiles, a fixed face, several calls with a reference update inside one.  Both paths are within
+# the 1e-10 of the oracle that the runs above allow, so twice that between them.
+@pytest.mark.parametrize("n", [1, 3, 9], ids=lambda n: f"n{n}")
+@pytest.mark.parametrize("formulation", [A.UPDATED_LAGRANGIAN, A.SEMI_LAGRANGIAN], ids=["updated", "semi"])
+@pytest.mark.parametrize("etype,mat,per_qp", [(A.TET4, "nh", False), (A.TET4, "j2", False), (A.TET4, "creep", False),
+                                              (A.HEX8, "nh", False), (A.HEX8, "j2", False), (A.HEX8, "j2", True),
+                                              (A.HEX8, "creep", False)])
+def test_tile_steps_match_element_partials(gpu_available, etype, mat, per_qp, formulation, n):
+    kind, kw = KINDS[mat]
+    if kind == A.POWER_LAW_CREEP and formulation == A.SEMI_LAGRANGIAN:
+        pytest.skip("the semi-Lagrangian formulation does not take the rate-form materials")
+    X, hc, conn = _block(etype, n)
+    dt = 0.5 * M.stable_dt_estimate(X, M.split_tets(X, hc), E, NU, RHO)
+    v0 = _v0(X, dt)
+    fixed = np.zeros(X.shape, dtype=np.uint8)
+    fixed[X[:, 2] < 0.01] = (1, 0, 1)
+    print(f"tile steps etype={etype} mat={mat} formulation={formulation} n={n}", flush=True)
+    out = []
+    for flags in (0, A.FLAG_TWO_PASS):
+        with A.Solver(flags=flags) as s:
+            s.set_mesh(etype, X, conn)
+            s.set_material(kind, RHO, E, NU, kw.get("yield_stress", 0.0), kw.get("hardening", 0.0), per_qp,
+                           creep=CREEP if kind == A.POWER_LAW_CREEP else None)
+            if formulation == A.SEMI_LAGRANGIAN:
+                s.set_semi_lagrangian(3)
+            else:
+                s.set_formulation(formulation)
+            s.compute_mass()
+            s.set_fixed(fixed)
+            s.set_field(A.FIELD_V, v0)
+            s.initialize()
+            for k in (4, 1, 5):
+                s.step(dt, k)
+            fields = [A.FIELD_U, A.FIELD_V, A.FIELD_A, A.FIELD_F, A.FIELD_H, A.FIELD_P]
+            out.append([s.get(f) for f in fields + ([A.FIELD_STATE] if kind != A.NEO_HOOKEAN else [])])
+    for i, (a, b) in enumerate(zip(*out)):
+        assert rel_err(a, b) < 2e-10, i
