@@ -459,18 +459,18 @@ static void setup_mesh(Ctx &c, int32_t elem_type, int64_t n_nodes, const double 
     APHIP_HIP(hipStreamSynchronize(c.stream));
 }
 
-static void force_pass(Ctx &c, bool keep = true) {
+static void force_pass(Ctx &c, bool keep = true, bool raw = false, bool keep_local = true) {
     prof_begin(c, 1);
-    if (c.cells.ready) rk_cell_force(c, keep);
+    if (c.cells.ready) rk_cell_force(c, keep, raw, keep_local);
     else fem_element_force(c);
     prof_end(c, 1);
 }
 
 static void step_once(Ctx &c, double dt, bool pred_in = false, bool pred_out = false, bool keep = true);
 
-static void node_pass(Ctx &c, double dt, int mode, bool more = false) {
+static void node_pass(Ctx &c, double dt, int mode, bool more = false, bool raw = false, bool keep = true) {
     prof_begin(c, 2);
-    if (c.cells.ready) rk_node_update(c, dt, mode, more);
+    if (c.cells.ready) rk_node_update(c, dt, mode, more, raw, keep);
     else fem_node_update(c, dt, mode);
     prof_end(c, 2);
 }
@@ -496,9 +496,10 @@ static void step_once(Ctx &c, double dt, bool pred_in, bool pred_out, bool keep)
     } else {
         // (ensembles keep their own increment per node, which only the predictor kernel reads)
         const bool chain = c.cells.ready && !c.node_dt.p;
-        if (!(chain && pred_in)) fem_predict(c, dt);
-        force_pass(c, keep);
-        node_pass(c, dt, 2, chain && pred_out);
+        const bool raw = !(chain && pred_in) && rk_fused(c);  // both passes take the predictor themselves
+        if (!(chain && pred_in) && !raw) fem_predict(c, dt);
+        force_pass(c, keep, raw, keep);
+        node_pass(c, dt, 2, chain && pred_out, raw, keep);
     }
 }
 
@@ -793,6 +794,7 @@ int aphip_set_tiling(aphip_ctx *c, int32_t te, int32_t threads) {
     APHIP_HIP(hipStreamSynchronize(c->stream));
     c->graph_reset();
     tile_build(*c, te, threads);
+    c->tiles.by_user = true;
     APHIP_API_END
 }
 
@@ -1389,6 +1391,7 @@ int aphip_autotune(aphip_ctx *c, double dt, int32_t trial_steps, int32_t *chosen
     (void)hipEventDestroy(e1);
     c->prof.enabled = was_prof;
     tile_build(*c, best.te, best.threads);
+    c->tiles.by_user = true;
     c->tiles.use_stream = best.pipelined;
     set_node_field(*c, c->u, su.data());
     set_node_field(*c, c->v, sv.data());

@@ -187,6 +187,8 @@ struct CellData {
 // Element-tile plan of the fused step (tile.hip), internal numbering.  The plan
 // renumbers nodes: interior nodes of each tile are contiguous, shared nodes follow.
 struct TilePlan {
+    bool by_user = false;  // shape set by aphip_set_tiling or aphip_autotune
+    bool orphans = false;  // some node belongs to no element
     bool ready = false;
     int te = 0;                       // elements per tile (= threads)
     int threads = 0;                  // workgroup size
@@ -408,11 +410,26 @@ void tile_build(Ctx &c, int te, int threads);
 // node-indexed array of the context (capi.hip).
 void renumber_nodes(Ctx &c, const std::vector<int32_t> &old_of_new);
 // One tiled pass (MODE 0 force only, 1 force and a = f/m, 2 the full step).
+constexpr int kMaxNbr = 40;  // neighbors of a node (include/Constants.h:15)
+
+// Rows of Phi, by which a force evaluation takes the displacements it stages.
+struct PhiRows {
+    const int32_t *num, *nbr;  // neighbors of a node, kMaxNbr to a row
+    const double *phi;
+    int copy_lonely;  // a node without neighbors takes its own coefficient (else zero)
+    int raw;          // the coefficients are predicted on the way (central difference, dt)
+    double *out;      // also store Phi u, or null; a shared node's by the tile of its first slot
+    const int32_t *bstart;
+};
 struct TileRun {
     // MODE 0: displacement read and force written when not the context's u and f (RKPM
     // element cells: physical displacement in, local force out)
     const double *u_in = nullptr;
     double *f_out = nullptr;
+    // MODE 0, Tet4: the displacement staged is Phi u of the context's u
+    const PhiRows *phi = nullptr;
+    // MODE 0: the shared nodes' partial sums stay in their slots, no shared-node pass
+    bool park = false;
     // MODE 2: shared nodes take the displacement predicted by the previous step's shared-node
     // pass (it must have run with pred_out and the same dt in this same call); pred_out: the
     // shared-node pass stores that prediction for the next step
@@ -447,10 +464,14 @@ void step_once_tiles(Ctx &c, double dt, bool keep);
 void rk_setup(Ctx &c, double scale, bool two_pass, bool fe_cells = false, int nodal_subdomains = -1,
               bool fbar = false);
 // keep = false: H and P may be left unwritten (see TileRun)
-void rk_cell_force(Ctx &c, bool keep);
+// keep_local = false: an inner step, Phi u may be left unwritten
+void rk_cell_force(Ctx &c, bool keep, bool raw = false, bool keep_local = true);
 // more (mode 2): another step of the same call with the same dt follows; its predictor is
 // taken here and fem_predict is not called for it
-void rk_node_update(Ctx &c, double dt, int mode, bool more);
+// raw: the step's predictor has not been taken; both passes of a fused step (rk_fused) take it.
+// keep = false: an inner step, the local force may be left unwritten
+void rk_node_update(Ctx &c, double dt, int mode, bool more, bool raw = false, bool keep = true);
+bool rk_fused(const Ctx &c);
 void rk_mass(Ctx &c, double *total);
 
 // ---- profiling helpers (capi.hip) ----

@@ -53,8 +53,8 @@ namespace aphip {
 
 namespace {
 
-constexpr int kMaxNbr = 40;  // include/Constants.h:15
 constexpr int kSearchBlock = 64;
+constexpr int kFusedNodes = 12000;  // element cells: two launches a step (rk_fused)
 constexpr int kCellBlock = 64;
 
 __device__ __forceinline__ void ld3(const double *p, int64_t i, double *o) {
@@ -538,6 +538,7 @@ struct RkNodeArgs {
     // also takes that step's predictor (u and v are what k_predict would leave) and stores
     // neither f nor a, which that step overwrites unread
     int more;
+    int raw;  // mode 2: the step's predictor has not been taken yet
 };
 
 // Node i's force f is complete: store it and finish the node (MODE 0: force only,
@@ -545,13 +546,19 @@ struct RkNodeArgs {
 template <int MODE>
 __device__ __forceinline__ void rk_finish(const RkNodeArgs &A, int64_t i, const double (&f)[3]) {
     if constexpr (MODE == 2) {
-        double vh[3], a1[3], v1[3];
+        double u[3], vh[3], a1[3], v1[3];
         ld3(A.v, i, vh);
         const unsigned fx = A.fixed ? A.fixed[i] : 0u;
+        if (A.more || A.raw) ld3(A.u, i, u);
+        if (A.raw) {
+            double v0[3] = {vh[0], vh[1], vh[2]}, a0[3], u0[3] = {u[0], u[1], u[2]};
+            ld3(A.a, i, a0);
+            cd_predict(u0, v0, a0, fx, A.dt, vh, u);
+            if (!A.more) st3(A.u, i, u);
+        }
         cd_correct(f, A.mass[i], fx, A.dt, vh, a1, v1);
         if (A.more) {
-            double u[3], u1[3];
-            ld3(A.u, i, u);
+            double u1[3];
             cd_predict(u, v1, a1, fx, A.dt, vh, u1);
             st3(A.u, i, u1);
             st3(A.v, i, vh);
@@ -973,14 +980,29 @@ struct RkGatherArgs {
     const double *src;  // coefficients [nn * 3]
     double *dst;        // physical values [nn * 3]
     int copy_lonely;    // two-pass: a node without neighbors copies its coefficient (one-pass: zero)
+    // RAW: the coefficients are predicted on the way
+    const double *v, *a;
+    const uint8_t *fixed;
+    double dt;
 };
 
 // dst_i = sum_k phi_ik src_(nbr_ik): LANES lanes per node, lane l takes entries
 // l, l + LANES, ... of the node's row (contiguous across the lanes), the partial
 // sums are combined by the xor butterfly.
 // (8 lanes, five entries each for a full row of 40: 3 % faster than 16 lanes.)
-template <int LANES>
+template <int LANES, bool RAW>
 __global__ __launch_bounds__(256) void k_rk_gather(RkGatherArgs A) {
+    auto coefficient = [&](int64_t j, double (&x)[3]) {
+        if constexpr (RAW) {
+            double u[3], v[3], a[3], vh[3];
+            ld3(A.src, j, u);
+            ld3(A.v, j, v);
+            ld3(A.a, j, a);
+            cd_predict(u, v, a, A.fixed ? A.fixed[j] : 0u, A.dt, vh, x);
+        } else {
+            ld3(A.src, j, x);
+        }
+    };
     constexpr int R = (kMaxNbr + LANES - 1) / LANES;
     const int l = threadIdx.x & (LANES - 1);
     const int64_t i_raw = xcd_block(A.nblocks) * (256 / LANES) + (threadIdx.x / LANES);
@@ -1002,7 +1024,7 @@ __global__ __launch_bounds__(256) void k_rk_gather(RkGatherArgs A) {
     double s[3] = {0.0, 0.0, 0.0};
     double x[R][3];
 #pragma unroll
-    for (int r = 0; r < R; ++r) ld3(A.src, j[r], x[r]);
+    for (int r = 0; r < R; ++r) coefficient(j[r], x[r]);
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -1010,7 +1032,7 @@ __global__ __launch_bounds__(256) void k_rk_gather(RkGatherArgs A) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) s[d] = group_sum<LANES>(s[d]);
     if (!live || l != 0) return;
-    if (n == 0 && A.copy_lonely) ld3(A.src, i, s);
+    if (n == 0 && A.copy_lonely) coefficient(i, s);
     A.dst[3 * i] = s[0];
     A.dst[3 * i + 1] = s[1];
     A.dst[3 * i + 2] = s[2];
@@ -1024,14 +1046,57 @@ struct RkScatterArgs {
     const double *rphi;      // phi_iJ of each reverse entry
     const double *src;       // local (physical) force [nn * 3]
     int copy_lonely;         // two-pass: a node without neighbors takes src_J
+    // SLOTS: the local force of the nodes from first_shared on is the sum of their slots
+    // bstart[j - first_shared] .. (ascending, as the shared-node pass adds them)
+    const int32_t *bstart;
+    const double *bpart;
+    int64_t first_shared;
+    double *local;  // also store the shared nodes' local force, or null
 };
 
 // f_J = sum over points i that list J of phi_iJ src_i (the transpose of the
 // gather), LANES lanes per node over its contiguous reverse entries, NB per lane at a
 // time (16 x 3: a reverse list of about 40 entries in one round with little padding;
 // 6 % faster than 16 x 4, and than 8 x 5), then the node update.
-template <int MODE, int LANES, int NB>
+template <int MODE, int LANES, int NB, bool SLOTS = false>
 __global__ __launch_bounds__(256) void k_rk_scatter(RkScatterArgs A) {
+    // local force of NB nodes
+    auto local = [&](auto &src, auto &x) {
+        constexpr int M = sizeof(src) / sizeof(src[0]);
+        if constexpr (!SLOTS) {
+#pragma unroll
+            for (int r = 0; r < M; ++r) ld3(A.src, src[r], x[r]);
+        } else {
+            const double *p[M];
+            int left[M], most = 1;
+#pragma unroll
+            for (int r = 0; r < M; ++r) {
+                p[r] = A.src + 3 * (int64_t)src[r];
+                left[r] = 1;
+                if (const int64_t b = src[r] - A.first_shared; b >= 0) {
+                    const int32_t s0 = A.bstart[b];
+                    left[r] = A.bstart[b + 1] - s0;
+                    if (left[r] > 0) p[r] = A.bpart + 3 * (int64_t)s0;  // (a node of no element has no slot)
+                }
+                most = max(most, left[r]);
+                x[r][0] = x[r][1] = x[r][2] = 0.0;
+            }
+            constexpr int Q = 2;
+            for (int q = 0; q < most; q += Q) {
+                double y[M][Q][3];
+#pragma unroll
+                for (int r = 0; r < M; ++r)
+#pragma unroll
+                    for (int k = 0; k < Q; ++k) ld3(p[r], max(min(q + k, left[r] - 1), 0), y[r][k]);
+#pragma unroll
+                for (int r = 0; r < M; ++r)
+#pragma unroll
+                    for (int k = 0; k < Q; ++k)
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) x[r][d] += q + k < left[r] ? y[r][k][d] : 0.0;
+            }
+        }
+    };
     const int l = threadIdx.x & (LANES - 1);
     const int64_t i_raw = xcd_block(A.out.nblocks) * (256 / LANES) + (threadIdx.x / LANES);
     const bool live = i_raw < A.out.nn;
@@ -1047,8 +1112,7 @@ __global__ __launch_bounds__(256) void k_rk_scatter(RkScatterArgs A) {
             src[r] = A.rsrc[t];
             w[r] = tb + r * LANES < t1 ? A.rphi[t] : 0.0;
         }
-#pragma unroll
-        for (int r = 0; r < NB; ++r) ld3(A.src, src[r], x[r]);
+        local(src, x);
 #pragma unroll
         for (int r = 0; r < NB; ++r)
 #pragma unroll
@@ -1057,7 +1121,17 @@ __global__ __launch_bounds__(256) void k_rk_scatter(RkScatterArgs A) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) f[d] = group_sum<LANES>(f[d]);
     if (!live || l != 0) return;
-    if (A.copy_lonely && A.num[i] == 0) ld3(A.src, i, f);
+    const bool lonely = A.copy_lonely && A.num[i] == 0;
+    if (lonely || (SLOTS && A.local && i >= A.first_shared)) {
+        const int32_t self[1] = {(int32_t)i};
+        double x[1][3];
+        local(self, x);
+        if (SLOTS && A.local && i >= A.first_shared) st3(A.local, i, x[0]);
+        if (lonely) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) f[d] = x[0][d];
+        }
+    }
     rk_finish<MODE>(A.out, i, f);
 }
 
@@ -1275,13 +1349,19 @@ static void nodal_subcells(Ctx &c, const std::vector<int64_t> &sub_start, const 
 
 // The element cells' force runs on the element tile plan, one element per thread: built
 // here when the context has none (APHIP_FLAG_TWO_PASS, a nodal set-up before this one) or
-// has the eight-lanes-per-Hex8 shape.  64 elements always fit a CU's LDS.
-static void ensure_element_tiles(Ctx &c) {
+// has the eight-lanes-per-Hex8 shape.  64 elements always fit a CU's LDS.  RKPM cells on Tet4
+// take smaller tiles than the mesh's default unless the caller set them: 256 elements on the
+// small meshes, where a workgroup of 1024 keeps its CU's issue slots busy four times as long
+// (alone, 10 steps of 16k cells in two launches: 291 -> 218 us), else 512, whose workgroups
+// leave room for a second one on the CU (10 steps of 750k cells: 742 -> 719 us).
+static void ensure_element_tiles(Ctx &c, bool fe_cells) {
     auto fits = [&] {
         return c.tiles.ready && c.tiles.threads == c.tiles.te && c.tiles.cell_lds_bytes <= 160 * 1024;
     };
-    if (c.ne == 0 || fits()) return;
-    for (int te = c.npe == 4 ? 1024 : 128;; te /= 2) {
+    int te0 = c.npe == 4 ? 1024 : 128;
+    if (c.npe == 4 && !fe_cells && !c.tiles.by_user) te0 = c.nn <= kFusedNodes ? 256 : 512;
+    if (c.ne == 0 || (fits() && c.tiles.te <= te0)) return;
+    for (int te = te0;; te /= 2) {
         try {
             tile_build(c, te, te);
             if (fits()) return;
@@ -1296,7 +1376,7 @@ void rk_setup(Ctx &c, double scale, bool two_pass, bool fe_cells, int nodal_subd
     D.reset();
     c.n_dof = c.nn;
     const int64_t nn = c.nn;
-    if (nodal_subdomains < 0) ensure_element_tiles(c);  // (renumbers the nodes: before anything refers to them)
+    if (nodal_subdomains < 0) ensure_element_tiles(c, fe_cells);  // (renumbers the nodes: before anything refers to them)
     if (fe_cells) {
         fe_smoothing_setup(c);
         return;
@@ -1708,7 +1788,20 @@ static void rk_tile_force(Ctx &c) {
     APHIP_HIP(hipGetLastError());
 }
 
-void rk_cell_force(Ctx &c, bool keep) {
+// Small meshes: fewer launches a step.  The passes take the first step's predictor themselves,
+// the scatter sums the shared nodes' slots itself (once for each list that holds them), and Tet4
+// tiles gather u = Phi d as they stage their nodes (a shared node's row in each of its tiles): two
+// launches a step, whose added work stays below the launches saved up to about 12k nodes.  10
+// one-pass steps at kernel scale 1.3 with three streams in turn, four launches / two: 343 nodes
+// 161 / 105 us, 9261 162 / 118, 19683 164 / 201.  Hex8 cells keep the gather pass (their tile
+// workgroups of two waves take longer over it than a launch costs: 9261 nodes 113 / 166 us).
+bool rk_fused(const Ctx &c) {
+    const CellData &D = c.cells;
+    return D.ready && !D.nodal && !D.fbar && D.ncells > 0 && !c.node_dt.p && c.n_dof == c.nn &&
+           !c.tiles.orphans && c.nn <= kFusedNodes;
+}
+
+void rk_cell_force(Ctx &c, bool keep, bool raw, bool keep_local) {
     CellData &D = c.cells;
     if (D.ncells == 0) return;  // no cells: f_local stays zero
     if (D.fbar) {
@@ -1721,9 +1814,26 @@ void rk_cell_force(Ctx &c, bool keep) {
     }
     // physical displacement = Phi d (ExplicitSolver::ComputeForce, Explicit.cpp:148-152), then
     // the element tiles
+    const bool fused = rk_fused(c);
+    if (fused && c.npe == 4) {
+        const PhiRows phi{D.num_nbr.p, D.nbr.p, D.phi.p, D.two_pass, raw, keep_local ? D.u_phys.p : nullptr,
+                          c.tiles.bstart.p};
+        TileRun run;
+        run.phi = &phi;
+        run.park = true;
+        run.f_out = D.f_local.p;
+        run.keep = keep;
+        const bool prof = c.prof.enabled;  // timed as this force pass, not as tile launches
+        c.prof.enabled = false;
+        tile_run(c, c.rate_dt, 0, run);
+        c.prof.enabled = prof;
+        return;
+    }
     const int64_t nbg = padded_groups(c.nn, kGsLanes);
-    RkGatherArgs G{c.nn, nbg, D.num_nbr.p, D.nbr.p, D.phi.p, c.u.p, D.u_phys.p, D.two_pass};
-    hipLaunchKernelGGL(k_rk_gather<kGsLanes>, dim3((unsigned)nbg), dim3(256), 0, c.stream, G);
+    const RkGatherArgs G{c.nn, nbg, D.num_nbr.p, D.nbr.p, D.phi.p, c.u.p, D.u_phys.p, D.two_pass,
+                         c.v.p, c.a.p, c.has_fixed ? c.fixed.p : nullptr, c.rate_dt};
+    if (raw) hipLaunchKernelGGL((k_rk_gather<kGsLanes, true>), dim3((unsigned)nbg), dim3(256), 0, c.stream, G);
+    else hipLaunchKernelGGL((k_rk_gather<kGsLanes, false>), dim3((unsigned)nbg), dim3(256), 0, c.stream, G);
     APHIP_HIP(hipGetLastError());
     const bool prof = c.prof.enabled;  // timed as this force pass, not as tile launches
     c.prof.enabled = false;
@@ -1731,27 +1841,34 @@ void rk_cell_force(Ctx &c, bool keep) {
     run.u_in = D.u_phys.p;
     run.f_out = D.f_local.p;
     run.keep = keep;
+    run.park = fused;
     tile_run(c, 0.0, 0, run);
     c.prof.enabled = prof;
 }
 
-void rk_node_update(Ctx &c, double dt, int mode, bool more) {
+void rk_node_update(Ctx &c, double dt, int mode, bool more, bool raw, bool keep) {
     CellData &D = c.cells;
     // nodes with degrees of freedom only (nodal cells put them first; the others keep
     // their values, as the reference's integrator runs over the active part)
     const int lanes = D.nodal ? kSlotLanes : kCellLanes;
     const int64_t nb = padded_groups(c.n_dof, lanes);
     const dim3 g((unsigned)nb);
-    const RkNodeArgs A{c.n_dof, nb, c.mass.p, c.has_fixed ? c.fixed.p : nullptr, c.f.p, c.a.p, c.v.p, c.u.p, dt, more};
+    const RkNodeArgs A{c.n_dof, nb, c.mass.p, c.has_fixed ? c.fixed.p : nullptr, c.f.p, c.a.p, c.v.p, c.u.p, dt, more,
+                       raw};
     if (D.nodal) {
         const RkSlotNodeArgs N{A, D.nslot_start.p, D.nslot.p, D.slots.p};
         if (mode == 0) hipLaunchKernelGGL((k_rk_slot_nodes<0, kSlotLanes>), g, dim3(256), 0, c.stream, N);
         else if (mode == 1) hipLaunchKernelGGL((k_rk_slot_nodes<1, kSlotLanes>), g, dim3(256), 0, c.stream, N);
         else hipLaunchKernelGGL((k_rk_slot_nodes<2, kSlotLanes>), g, dim3(256), 0, c.stream, N);
     } else {  // f = Phi^T f_local with the node update (ScatterValues, Explicit.cpp:181-186)
-        const RkScatterArgs S{A, D.num_nbr.p, D.rstart.p, D.rsrc.p, D.rphi.p, D.f_local.p, D.two_pass};
+        const RkScatterArgs S{A, D.num_nbr.p, D.rstart.p, D.rsrc.p, D.rphi.p, D.f_local.p, D.two_pass,
+                              c.tiles.bstart.p, c.tiles.bpart.p, c.tiles.n_interior, mode != 2 || keep ? D.f_local.p : nullptr};
         constexpr int NB = (kMaxNbr + kCellLanes - 1) / kCellLanes;
-        if (mode == 0) hipLaunchKernelGGL((k_rk_scatter<0, kCellLanes, NB>), g, dim3(256), 0, c.stream, S);
+        if (rk_fused(c)) {
+            if (mode == 0) hipLaunchKernelGGL((k_rk_scatter<0, kCellLanes, NB, true>), g, dim3(256), 0, c.stream, S);
+            else if (mode == 1) hipLaunchKernelGGL((k_rk_scatter<1, kCellLanes, NB, true>), g, dim3(256), 0, c.stream, S);
+            else hipLaunchKernelGGL((k_rk_scatter<2, kCellLanes, NB, true>), g, dim3(256), 0, c.stream, S);
+        } else if (mode == 0) hipLaunchKernelGGL((k_rk_scatter<0, kCellLanes, NB>), g, dim3(256), 0, c.stream, S);
         else if (mode == 1) hipLaunchKernelGGL((k_rk_scatter<1, kCellLanes, NB>), g, dim3(256), 0, c.stream, S);
         else hipLaunchKernelGGL((k_rk_scatter<2, kCellLanes, NB>), g, dim3(256), 0, c.stream, S);
     }

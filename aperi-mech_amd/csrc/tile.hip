@@ -105,6 +105,7 @@ struct TileArgs {
     double *dinc, *xnp1;
     int semi;
     int cell_marker;  // smoothed cells turn a new failure's marker into the maximum damage
+    PhiRows phi;      // GATHER
 };
 
 // LDS carve-up (bytes), sized on the host (tile_lds_bytes) from the tile's rows.  X and U (the
@@ -208,6 +209,60 @@ __device__ __forceinline__ void stage_predict(const TileArgs &A, const double *u
     }
 }
 
+// U rows of tile t's nodes: Phi u, eight lanes a node, each with its share of the row (the
+// entries past the row weighted by zero), combined by a xor butterfly.
+__device__ __forceinline__ void stage_phi(const TileArgs &A, const TileLds &L, int64_t t, int tn) {
+    constexpr int LANES = 8, R = (kMaxNbr + LANES - 1) / LANES;
+    const int l = threadIdx.x & (LANES - 1), step = blockDim.x / LANES;
+    const int rounds = (tn + step - 1) / step;
+    for (int r0 = 0; r0 < rounds; ++r0) {
+        const int ln_raw = r0 * step + (int)threadIdx.x / LANES, ln = min(ln_raw, tn - 1);
+        const int64_t i = A.tnp_node[t * (int64_t)A.tpad + ln];
+        const int n = A.phi.num[i];
+        const int64_t row = i * kMaxNbr;
+        int32_t j[R];
+        double w[R], x[R][3], s[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            // (a row holds kMaxNbr places: loaded without waiting for its length)
+            const int k = l + r * LANES, kk = min(k, kMaxNbr - 1);
+            const int32_t jl = A.phi.nbr[row + kk];
+            const double wl = A.phi.phi[row + kk];
+            j[r] = k < n ? jl : (int32_t)i;
+            w[r] = k < n ? wl : 0.0;
+        }
+        if (n == 0 && A.phi.copy_lonely && l == 0) w[0] = 1.0;
+        if (A.phi.raw) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                double u[3], v[3], a[3], vh[3];
+                ld3(A.u, j[r], u);
+                ld3(A.v, j[r], v);
+                ld3(A.a, j[r], a);
+                cd_predict(u, v, a, load_fixed(A, j[r]), A.dt, vh, x[r]);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) ld3(A.u, j[r], x[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) s[d] += x[r][d] * w[r];
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int m = LANES / 2; m >= 1; m >>= 1) s[d] += __shfl_xor(s[d], m, LANES);
+        if (l == 0 && ln_raw < tn) {
+            st3(L.U, ln, s);
+            if (A.phi.out) {
+                const int32_t slot = A.tnp_bdst[t * (int64_t)A.tpad + ln];
+                if (slot < 0 || slot == A.phi.bstart[i - A.first_shared]) st3(A.phi.out, i, s);
+            }
+        }
+    }
+}
+
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt at their maxima: not waited on).  At a
 // point where no store is outstanding this costs nothing beyond the loads' latency.
 __device__ __forceinline__ void wait_vmem_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
@@ -265,9 +320,10 @@ __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L,
 // MODE 0: force only; 1: force + a = f/m (initial); 2: full central-difference step.
 // One element per thread: Tet4 (NPE 4), or smoothed Hex8 cells (NPE 8, MODE 0); the 2x2x2 Gauss
 // Hex8 has k_hex_tile.
-// UL: updated / semi-Lagrangian step.
-template <int NPE, int KIND, int MODE, bool UL = false>
+// UL: updated / semi-Lagrangian step.  GATHER: the displacement staged is Phi u.
+template <int NPE, int KIND, int MODE, bool UL = false, bool GATHER = false>
 __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_tile(TileArgs A) {
+    static_assert(!GATHER || (NPE == 4 && MODE == 0), "Tet4 in force mode");
     static_assert(NPE == 4 || MODE == 0, "smoothed Hex8 cells are evaluated in force mode");
     extern __shared__ __align__(16) char lds_raw[];
     const int64_t t = xcd_tile(A.nblocks);
@@ -390,7 +446,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
             if (!pre) stage_predict<UL>(A, u, v, a, fx, nd, vh, u1);
             st3(L.U, ln, u1);
             if (interior) st3(L.V, ln, vh);
-        } else {
+        } else if constexpr (!GATHER) {
             st3(L.U, ln, u);
         }
     };
@@ -415,6 +471,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
         }
         stage(ln, A.tn_csr[tb + ln], A.tn_bdst[tb + ln], x, u, v, a, fx, mm, nd, false);
     }
+    if constexpr (GATHER) stage_phi(A, L, t, tn);
     // Every load of the wave completes here, on every path (a wave whose lanes all
     // skip the staging loop still has its element prefetch in flight).  Otherwise the
     // join after the element phase merges a path with pending loads into the path
@@ -1134,6 +1191,12 @@ void launch_tile(Ctx &c, const TileArgs &A) {
         }
     }
     if constexpr (NPE == 4) {
+        if constexpr (MODE == 0) {
+            if (A.phi.num) {
+                go(k_tile<4, KIND, 0, false, true>, P.threads, P.lds_bytes);
+                return;
+            }
+        }
         go(k_tile<4, KIND, MODE>, P.threads, P.lds_bytes);
     } else {
         if constexpr (MODE == 0 && !PER_QP) {
@@ -1336,6 +1399,9 @@ void tile_build(Ctx &c, int te, int threads) {
     P.maxtn = maxtn;
     P.nb = nb;
     P.n_interior = n_interior;
+    P.by_user = false;
+    P.orphans = false;
+    for (int64_t b = 0; b < nb; ++b) P.orphans |= bstart[b] == bstart[b + 1];
     P.total_tile_nodes = (int64_t)tnodes.size();
     P.tn_start.upload(tstart.data(), tstart.size(), c.stream);
     P.tile_e0.upload(te0v.data(), te0v.size(), c.stream);
@@ -1462,12 +1528,13 @@ void tile_build(Ctx &c, int te, int threads) {
 void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     TilePlan &P = c.tiles;
     APHIP_REQUIRE(P.ready, "tile plan not built");
-    APHIP_REQUIRE(mode == 0 || (run.u_in == nullptr && run.f_out == nullptr),
+    APHIP_REQUIRE(mode == 0 || (run.u_in == nullptr && run.f_out == nullptr && !run.phi && !run.park),
                   "displacement / force arrays only in force mode");
     APHIP_REQUIRE(mode == 2 || !(run.pred_in || run.pred_out), "predicted displacements only in step mode");
     const bool pred_in = run.pred_in && P.nb > 0, pred_out = run.pred_out && P.nb > 0;
     // smoothed Hex8 cells have a B of their own (a smoothed Tet4's is its gradient)
     const bool cells8 = c.npe == 8 && c.cells.ready;
+    APHIP_REQUIRE(!run.phi || c.npe == 4, "Phi rows are staged by Tet4 tiles");
     APHIP_REQUIRE(!cells8 || (mode == 0 && P.threads == P.te), "Hex8 cells: force mode, one cell per thread");
     if (c.ne == 0) return;
     const bool ul = c.formulation != APHIP_TOTAL_LAGRANGIAN;
@@ -1527,6 +1594,7 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     A.upred = pred_in ? P.upred.p : nullptr;
     A.first_shared = P.n_interior;
     A.cell_marker = c.cells.ready;
+    A.phi = run.phi ? *run.phi : PhiRows{};
     A.dinc = c.dinc.p;
     A.xnp1 = c.formulation == APHIP_UPDATED_LAGRANGIAN ? c.xcnp1().p : nullptr;
     A.semi = c.formulation == APHIP_SEMI_LAGRANGIAN;
@@ -1544,7 +1612,7 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     }
     APHIP_HIP(hipGetLastError());
     prof_end(c, 1);
-    if (P.nb > 0) {
+    if (P.nb > 0 && !run.park) {
         BoundArgs B{P.nb, P.n_interior, P.bstart.p, P.bpart.p, c.u.p, c.v.p, c.a.p, A.f, c.mass.p,
                     c.has_fixed ? c.fixed.p : nullptr, c.node_dt.p, P.zero.p, dt,
                     pred_out ? P.upred.p : nullptr, A.keep,

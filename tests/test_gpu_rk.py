@@ -463,6 +463,48 @@ def test_element_cells_force_from_every_plan(gpu_available, etype, route, one_pa
             assert rel_err(s.get(fld), ref) < 1e-12, fld
 
 
+@pytest.mark.parametrize("etype,one_pass,dims", [(A.TET4, True, (1, 1, 1)), (A.TET4, True, (20, 20, 20)),
+                                                 (A.TET4, False, (9, 22, 20)), (A.HEX8, True, (20, 20, 20)),
+                                                 (A.HEX8, False, (9, 22, 20))])
+def test_small_mesh_passes_match_separate_ones(gpu_available, etype, one_pass, dims):
+    """Small meshes gather, sum the shared nodes and predict inside the tile and scatter passes;
+    the same block as one of several apart in a larger mesh (separate passes) moves the same.
+    Bar: sums of up to 40 x 24 terms in another order, about 1e-14 of the largest element force
+    a step, and up to 1e2 of cancellation in a nodal force, over five steps."""
+    n = max(dims)
+    X, hc = M.hex_lattice(*dims, *(d / n for d in dims))
+    X = M.jitter(X, 1 / n, 0.1, 3, 1)
+    conn = M.split_tets(X, hc) if etype == A.TET4 else hc
+    nn, copies = len(X), 12000 // len(X) + 1
+    assert nn <= 12000 < nn * copies
+    rng = np.random.default_rng(2)
+    v0 = rng.uniform(-1.0, 1.0, X.shape)
+    fixed = np.zeros(X.shape, dtype=np.uint8)
+    fixed[X[:, 2] < 0.01] = (1, 0, 1)
+    dt = 0.2 * M.stable_dt_estimate(X, M.split_tets(X, hc), J2["E"], J2["nu"], J2["rho"])
+    k = np.arange(copies)  # (apart: 4 a copy, its size 1 and the kernel radius at most 2.3)
+    shift = 4.0 * np.stack([k % 30, k // 30 % 30, k // 900], axis=1)
+    out = []
+    for c in (1, copies):
+        print(f"small passes etype={etype} one_pass={one_pass}: {c} x {nn} nodes", flush=True)
+        with A.Solver() as s:
+            s.set_mesh(etype, (X[None] + shift[:c, None]).reshape(-1, 3),
+                       (conn[None] + (nn * k[:c])[:, None, None]).reshape(-1, conn.shape[1]))
+            s.set_material(A.J2, J2["rho"], J2["E"], J2["nu"], J2["yield_stress"], J2["hardening"])
+            s.rk_setup(1.3, one_pass=one_pass)
+            s.compute_mass()
+            s.set_fixed(np.tile(fixed, (c, 1)))
+            s.set_field(A.FIELD_V, np.tile(v0, (c, 1)))
+            s.initialize()
+            s.step(dt, 1)
+            s.step(dt, 4)
+            two = () if one_pass else (A.FIELD_RK_DISPLACEMENT, A.FIELD_RK_FORCE_LOCAL)
+            out.append([s.get(f)[:nn] for f in (A.FIELD_U, A.FIELD_V, A.FIELD_A, A.FIELD_F, *two)]
+                       + [s.get(A.FIELD_P)[:len(conn)]])
+    for i, (a, b) in enumerate(zip(*out)):
+        assert rel_err(a, b) < 1e-11, i
+
+
 @pytest.mark.parametrize("cells", ["one-pass", "two-pass", "fe", "nodal", "f-bar"])
 def test_cell_steps_of_one_call_match_single_steps(gpu_available, cells):
     """A call's steps hand the next step's predictor on and store H, P, f and a at the last
