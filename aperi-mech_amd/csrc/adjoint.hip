@@ -18,8 +18,7 @@
 #include <cmath>
 #include <vector>
 
-#include "element.hpp"
-#include "internal.hpp"
+#include "patch.hpp"
 
 namespace aphip {
 
@@ -408,6 +407,223 @@ __global__ __launch_bounds__(NPE == 4 ? 512 : 128) void k_tile_adj(AdjArgs A) {
     }
 }
 
+// hex8_vjp with one lane per Gauss point (see hex8_lanes; sB: f_bar, row2: 21 doubles more for its
+// modes).  On return the corners' u_bar stands in row; lb, mb: the element's sums, in every lane.
+template <int KIND>
+__device__ __forceinline__ void hex8_vjp_lanes(int lane, const uint32_t (&cn)[4], const double *sX, const double *sU,
+                                               const double *sB, double *row, double *row2, const MatParams &m,
+                                               double ga, double &lb, double &mb) {
+    const int x = hex8_lane_label(lane);
+    const bool b0 = x & 1, b1 = x & 2, b2 = x & 4;
+    const int q = x == 2 ? 3 : x == 3 ? 2 : x == 6 ? 7 : x == 7 ? 6 : x;  // point (and corner) index
+    {
+        const double *src = lane < 3 ? sX + lane : lane < 6 ? sU + (lane - 3) : sB + (lane - 6);
+        hex8_field_modes(cn, src, ga, lane < 6 ? row + 7 * lane : row2 + 7 * (lane - 6));
+        if (lane == 0) hex8_field_modes(cn, sB + 2, ga, row2 + 14);
+    }
+    __builtin_amdgcn_wave_barrier();  // (LDS operations of a wave stay in order)
+    const double s0 = b0 ? -1.0 : 1.0, s1 = b1 ? -1.0 : 1.0, s2 = b2 ? -1.0 : 1.0;
+    const double s01 = s0 * s1, s02 = s0 * s2, s12 = s1 * s2;
+    auto grad = [&](const double *r, double *g) {
+        double w[8];
+        w[0] = 0.0;
+#pragma unroll
+        for (int S = 1; S < 8; ++S) w[S] = r[S - 1];
+        double h[3];
+        hex8_grad(w, -s0, -s1, -s2, s01, s02, s12, h);
+        g[0] = h[0];
+        g[1] = h[1];
+        g[2] = h[2];
+    };
+    double Ad[9], H[9], Pb[9], Hb[9];
+    double id;
+    {
+        double J[9];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) grad(row + 7 * i, J + 3 * i);
+        id = 1.0 / adjugate3(J, Ad);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        double g[3], b[3];
+        grad(row + 7 * (i + 3), g);
+        grad(row2 + 7 * i, b);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            H[3 * i + j] = dot3(g[0], Ad[j], g[1], Ad[3 + j], g[2], Ad[6 + j]) * id;
+            // P_bar = -w FG J^-1: w J^-1 is the adjugate up to exact powers of two
+            Pb[3 * i + j] = dot3(b[0], Ad[j], b[1], Ad[3 + j], b[2], Ad[6 + j]) * (-1.0 / 512.0);
+        }
+    }
+    stress_vjp<KIND>(H, Pb, m, Hb, lb, mb);
+    auto sum8 = [](double v) {
+        v += hex8_partner<0>(v);
+        v += hex8_partner<1>(v);
+        return v + hex8_partner<2>(v);
+    };
+    lb = sum8(lb);
+    mb = sum8(mb);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) Hb[i] *= id;
+    hex8_to_corners(x, b0, b1, b2, s0, s1, s2, ga, 1.0, Ad, Hb, row + 3 * q);
+}
+
+// ---- node patches: a reverse step in one launch -----------------------------------
+// The reverse step needs f_bar on the nodes around an element only, which a patch (patch.hip)
+// computes from vb and ab as it stages its ring of neighbours; vb and ab are read from one set
+// of buffers and written to another, ub and the parameter sums belong to the owned nodes and
+// elements.  No shared-node pass, eight lanes per Hex8, and small workgroups: the 128-element
+// tiles put two waves on half the CUs, one Hex8 in 390 VGPRs a thread.
+struct PatchAdjArgs {
+    const double *X, *u1, *fbar;     // as in AdjArgs
+    const double *vb, *ab;           // adjoint state read
+    double *ub, *vb1, *ab1;          // ... and written
+    const double *mass;
+    const uint8_t *fixed;
+    const double *zero;
+    const int32_t *meta, *node, *elem;  // the plan's lists (PatchArgs)
+    const uint32_t *csr;
+    const uint16_t *conn, *ent;
+    double *lam_bar, *mu_bar;
+    MatParams mat;
+    const double *elem_lambda, *elem_mu;
+    double gauss_a, dt;
+    int64_t npatch, nblocks;
+    int npad, cpad, epad, entpad;
+};
+
+struct PatchAdjLds {
+    double *X, *U, *B, *F, *F2;
+    uint32_t *csr;
+    uint16_t *conn, *ent;
+    size_t bytes;
+};
+
+__host__ __device__ __forceinline__ PatchAdjLds carve_adj(char *base, int npe, int npad, int cpad, int epad, int entpad) {
+    PatchAdjLds L;
+    char *p = base;
+    auto take = [&](size_t n) {
+        char *q = p;
+        p += (n + 15) & ~(size_t)15;
+        return q;
+    };
+    L.X = reinterpret_cast<double *>(take(24 * (size_t)npad));
+    L.U = reinterpret_cast<double *>(take(24 * (size_t)npad));
+    L.B = reinterpret_cast<double *>(take(24 * (size_t)npad));
+    L.F = reinterpret_cast<double *>(take(npe == 4 ? 96 * (size_t)patch_stride(epad) : 8 * kHexRow * (size_t)epad));
+    L.F2 = reinterpret_cast<double *>(take(npe == 4 ? 0 : 168 * (size_t)epad));
+    L.csr = reinterpret_cast<uint32_t *>(take(4 * (size_t)cpad));
+    L.conn = reinterpret_cast<uint16_t *>(take(2 * (size_t)npe * epad));
+    L.ent = reinterpret_cast<uint16_t *>(take(2 * (size_t)entpad));
+    L.bytes = (size_t)(p - base);
+    return L;
+}
+
+template <int NPE, int KIND, int MODE>
+__global__ __launch_bounds__(NPE == 4 ? 512 : 256) void k_patch_adj(PatchAdjArgs A) {
+    extern __shared__ __align__(16) char lds_raw[];
+    const int64_t b = blockIdx.x;
+    const int64_t p = (b % kNumXcd) * (A.nblocks / kNumXcd) + b / kNumXcd;  // neighbours share an XCD's L2
+    if (p >= A.npatch) return;
+    const PatchAdjLds L = carve_adj(lds_raw, NPE, A.npad, A.cpad, A.epad, A.entpad);
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int32_t *node = A.node + p * A.npad;
+    const int32_t *elem = A.elem + p * A.epad;
+    const int32_t *meta = A.meta + 16 * p;
+    const int nN = meta[1], nE = meta[9], nC = meta[0], nown = meta[8];  // one ring
+    for (int i = tid; i < nN; i += nt) {
+        const int64_t g = node[i];
+        double x[3], u[3], fb[3];
+        ld3(A.X, g, x);
+        ld3(A.u1, g, u);
+        if constexpr (MODE == 0) {
+            ld3(A.fbar, g, fb);
+        } else {
+            double a[3];
+            ld3(A.ab, g, a);
+            const double m = A.mass[g];
+            if constexpr (MODE == 1) {
+                double v[3];
+                ld3(A.vb, g, v);
+                const uint8_t *pf = A.fixed ? A.fixed : reinterpret_cast<const uint8_t *>(A.zero);
+                const unsigned f8 = pf[A.fixed ? g : 0], fx = A.fixed ? f8 : 0u;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) fb[d] = (fx & (1u << d)) ? 0.0 : __fma_rn(0.5 * A.dt, v[d], a[d]) / m;
+            } else {
+#pragma unroll
+                for (int d = 0; d < 3; ++d) fb[d] = a[d] / m;
+            }
+        }
+        st3(L.X, i, x);
+        st3(L.U, i, u);
+        st3(L.B, i, fb);
+    }
+    for (int i = tid; i < A.cpad; i += nt) L.csr[i] = A.csr[p * A.cpad + i];
+    {
+        const uint4 *src = reinterpret_cast<const uint4 *>(A.ent + p * A.entpad);
+        uint4 *dst = reinterpret_cast<uint4 *>(L.ent);
+        for (int i = tid; i < A.entpad / kBatch; i += nt) dst[i] = src[i];
+    }
+    for (int i = tid; i < A.epad; i += nt) {
+#pragma unroll
+        for (int k = 0; k < NPE / 4; ++k)
+            reinterpret_cast<ushort4 *>(L.conn)[NPE / 4 * i + k] =
+                reinterpret_cast<const ushort4 *>(A.conn + p * A.epad * NPE)[NPE / 4 * i + k];
+    }
+    __syncthreads();
+    const int fs = patch_stride(A.epad);
+    constexpr int LPE = NPE == 8 ? 8 : 1;  // lanes per element
+    for (int le = tid / LPE; le < nE; le += nt / LPE) {
+        MatParams m = A.mat;
+        const int64_t e = elem[le];
+        if (A.elem_lambda) {
+            m.lambda = A.elem_lambda[e];
+            m.mu = A.elem_mu[e];
+        }
+        double lb, mb;
+        if constexpr (NPE == 8) {
+            const uint4 c = reinterpret_cast<const uint4 *>(L.conn)[le];
+            const uint32_t cn[4] = {c.x, c.y, c.z, c.w};
+            hex8_vjp_lanes<KIND>(tid & 7, cn, L.X, L.U, L.B, L.F + kHexRow * le, L.F2 + 21 * le, m, A.gauss_a, lb, mb);
+        } else {
+            const ushort4 c = reinterpret_cast<const ushort4 *>(L.conn)[le];
+            const int lc[4] = {c.x, c.y, c.z, c.w};
+            double X[4][3], U[4][3], Fb[4][3], ub[4][3];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                ld3(L.X, lc[k], X[k]);
+                ld3(L.U, lc[k], U[k]);
+                ld3(L.B, lc[k], Fb[k]);
+            }
+            tet4_vjp<KIND>(X, U, Fb, m, ub, lb, mb);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) st3(L.F, k * fs + le, ub[k]);
+        }
+        if (le < nown && tid % LPE == 0) {
+            A.lam_bar[e] += lb;
+            A.mu_bar[e] += mb;
+        }
+    }
+    if constexpr (MODE == 2) return;
+    __syncthreads();
+    for (int t4 = tid; t4 < 4 * nC; t4 += nt) {  // four lanes per node, one per component
+        const int ln = t4 >> 2, d = t4 & 3;
+        if (d == 3) continue;
+        const int64_t n = node[ln], g = 3 * n + d;
+        if constexpr (MODE == 0) {
+            A.ub[g] = patch_sum(L.F + d, L.ent, L.csr[ln]);
+        } else {
+            const double u0 = A.ub[g], v = A.vb[g];
+            const unsigned fx = A.fixed ? A.fixed[n] : 0u;
+            const double u = u0 + patch_sum(L.F + d, L.ent, L.csr[ln]);
+            const double vh = (fx & (1u << d)) ? 0.0 : __fma_rn(A.dt, u, v);
+            A.ub[g] = u;
+            A.vb1[g] = vh;
+            A.ab1[g] = (0.5 * A.dt) * vh;
+        }
+    }
+}
+
 struct AdjBoundArgs {
     int64_t nb, first;
     const int32_t *bstart;
@@ -462,8 +678,54 @@ void launch_adj(Ctx &c, const AdjArgs &A, size_t lds) {
     else run(k_tile_adj<NPE, APHIP_NEO_HOOKEAN, MODE>);
 }
 
+// Whether this context's adjoints, and the steps they record, run on node patches: decided by
+// the mesh and its plan alone, so that a backward pass takes the numbering of its forward pass.
+bool on_patches(Ctx &c) {
+    if (!c.tiles.ready || c.tiles.use_stream || c.n_specimens != 0 || c.formulation != APHIP_TOTAL_LAGRANGIAN ||
+        !patch_planned(c))
+        return false;
+    const PatchPlan &P = c.patch;
+    return carve_adj(nullptr, c.npe, P.npad, P.cpad, P.epad, P.entpad).bytes <= 160 * 1024;
+}
+
+template <int NPE, int KIND>
+void launch_patch_adj(Ctx &c, const PatchAdjArgs &A, int mode) {
+    const PatchPlan &P = c.patch;
+    const size_t lds = carve_adj(nullptr, NPE, P.npad, P.cpad, P.epad, P.entpad).bytes;
+    auto go = [&](auto kern) {
+        if (lds > 65536)
+            APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(std::min(P.threads, NPE == 4 ? 512 : 256)), lds, c.stream, A);
+        APHIP_HIP(hipGetLastError());
+    };
+    if (mode == 0) go(k_patch_adj<NPE, KIND, 0>);
+    else if (mode == 1) go(k_patch_adj<NPE, KIND, 1>);
+    else go(k_patch_adj<NPE, KIND, 2>);
+}
+
+void patch_adj_run(Ctx &c, const double *u1, const double *fbar, int mode, double dt) {
+    const PatchPlan &P = c.patch;
+    AdjointData &D = c.adj;
+    const PatchAdjArgs A{c.X.p, u1, fbar, D.vb.p, D.ab.p, D.ub.p, D.vb1.p, D.ab1.p, c.mass.p,
+                         c.has_fixed ? c.fixed.p : nullptr, c.tiles.zero.p, P.meta, P.node, P.elem, P.csr, P.conn, P.ent,
+                         D.lam_bar.p, D.mu_bar.p, c.mat.params(), c.has_fields ? c.elem_lambda.p : nullptr,
+                         c.has_fields ? c.elem_mu.p : nullptr, 1.0 / std::sqrt(3.0), dt, P.npatch, padded(P.npatch),
+                         P.npad, P.cpad, P.epad, P.entpad};
+    const bool le = c.mat.kind == APHIP_LINEAR_ELASTIC;
+    if (c.npe == 4) le ? launch_patch_adj<4, APHIP_LINEAR_ELASTIC>(c, A, mode) : launch_patch_adj<4, APHIP_NEO_HOOKEAN>(c, A, mode);
+    else le ? launch_patch_adj<8, APHIP_LINEAR_ELASTIC>(c, A, mode) : launch_patch_adj<8, APHIP_NEO_HOOKEAN>(c, A, mode);
+    if (mode == 1) {
+        std::swap(D.vb.p, D.vb1.p);
+        std::swap(D.ab.p, D.ab1.p);
+    }
+}
+
 // mode: 0 force VJP, 1 reverse step, 2 initial-acceleration parameter adjoint
 void adj_run(Ctx &c, const double *u1, const double *fbar, int mode, double dt) {
+    if (on_patches(c)) {
+        patch_adj_run(c, u1, fbar, mode, dt);
+        return;
+    }
     TilePlan &P = c.tiles;
     APHIP_REQUIRE(P.threads == P.te && (c.npe == 4 || P.te <= 128), "adjoint needs a one-element-per-thread tiling");
     AdjointData &D = c.adj;
@@ -527,8 +789,9 @@ void require_adjoint_ready(Ctx &c) {
     APHIP_REQUIRE(c.mat.kind == APHIP_LINEAR_ELASTIC || c.mat.kind == APHIP_NEO_HOOKEAN,
                   "adjoints are provided for linear elastic and neo-Hookean materials");
     APHIP_REQUIRE(c.tiles.ready && !c.cells.ready, "adjoints run on the tiled Gaussian element path");
-    // the adjoint kernels evaluate one element per thread, at most 512 Tet4 or 128 Hex8
+    // the tile adjoint kernels evaluate one element per thread, at most 512 Tet4 or 128 Hex8
     // per workgroup
+    if (on_patches(c)) return;
     if (c.tiles.threads != c.tiles.te || c.tiles.te > (c.npe == 8 ? 128 : 512)) tile_build(c, 64, 64);
 }
 
@@ -537,6 +800,10 @@ void alloc_adjoint(Ctx &c) {
     for (DevBuf<double> *b : {&D.ub, &D.vb, &D.ab}) {
         b->alloc(3 * c.nn);
         b->zero(c.stream);
+    }
+    if (on_patches(c)) {
+        D.vb1.alloc(3 * c.nn);
+        D.ab1.alloc(3 * c.nn);
     }
     D.lam_bar.alloc(std::max<int64_t>(c.ne, 1));
     D.mu_bar.alloc(std::max<int64_t>(c.ne, 1));
@@ -562,18 +829,42 @@ void parameter_gradients(Ctx &c, double *E_bar, double *nu_bar) {
     }
 }
 
+// u, v, a to or from one record of 9 doubles per node: one launch, not three copies
+__global__ __launch_bounds__(256) void k_state_copy(int64_t n3, const double *u, const double *v, const double *a,
+                                                    double *u1, double *v1, double *a1) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n3) return;
+    u1[i] = u[i];
+    v1[i] = v[i];
+    a1[i] = a[i];
+}
+
 void copy_state(Ctx &c, double *dst) {
-    const size_t n3 = 3 * (size_t)c.nn * sizeof(double);
-    APHIP_HIP(hipMemcpyAsync(dst, c.u.p, n3, hipMemcpyDeviceToDevice, c.stream));
-    APHIP_HIP(hipMemcpyAsync(dst + 3 * c.nn, c.v.p, n3, hipMemcpyDeviceToDevice, c.stream));
-    APHIP_HIP(hipMemcpyAsync(dst + 6 * c.nn, c.a.p, n3, hipMemcpyDeviceToDevice, c.stream));
+    const int64_t n3 = 3 * c.nn;
+    hipLaunchKernelGGL(k_state_copy, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, c.stream, n3, c.u.p, c.v.p, c.a.p,
+                       dst, dst + n3, dst + 2 * n3);
+    APHIP_HIP(hipGetLastError());
 }
 
 void restore_state(Ctx &c, const double *src) {
-    const size_t n3 = 3 * (size_t)c.nn * sizeof(double);
-    APHIP_HIP(hipMemcpyAsync(c.u.p, src, n3, hipMemcpyDeviceToDevice, c.stream));
-    APHIP_HIP(hipMemcpyAsync(c.v.p, src + 3 * c.nn, n3, hipMemcpyDeviceToDevice, c.stream));
-    APHIP_HIP(hipMemcpyAsync(c.a.p, src + 6 * c.nn, n3, hipMemcpyDeviceToDevice, c.stream));
+    const int64_t n3 = 3 * c.nn;
+    hipLaunchKernelGGL(k_state_copy, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, c.stream, n3, src, src + n3,
+                       src + 2 * n3, c.u.p, c.v.p, c.a.p);
+    APHIP_HIP(hipGetLastError());
+}
+
+// Step k of a segment, its displacement to seg_u.
+void recorded_step(Ctx &c, double dt, int k, bool keep) {
+    const int64_t n3 = 3 * c.nn;
+    double *rec = c.adj.seg_u.p + (size_t)k * n3;
+    if (on_patches(c)) {
+        c.state_np1 = 1 - c.state_np1;
+        c.rate_dt = dt;
+        patch_run(c, dt, 1, keep, rec);
+    } else {
+        step_once_tiles(c, dt, keep);
+        APHIP_HIP(hipMemcpyAsync(rec, c.u.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    }
 }
 
 }  // namespace
@@ -607,10 +898,28 @@ void adjoint_forward(Ctx &c, double dt, int n_steps, int interval) {
         D.ckpt.back()->alloc(9 * c.nn);
     }
     D.final_state.alloc(9 * c.nn);
-    for (int s = 0; s < n_steps; ++s) {
+    // the backward pass begins with the last segment: its displacements are recorded here
+    const int last = (nck - 1) * interval;
+    D.seg_u.alloc((size_t)std::min(interval, n_steps) * 3 * c.nn);
+    const bool patches = on_patches(c);
+    if (patches) c.graph_reset();  // (a patch launch exchanges the buffers a graph was captured with)
+    for (int s = 0; s < n_steps;) {
         if (s % interval == 0) copy_state(c, D.ckpt[s / interval]->p);
-        step_once_tiles(c, dt, s + 1 == n_steps);
+        if (s >= last) {
+            recorded_step(c, dt, s - last, s + 1 == n_steps);
+            ++s;
+        } else if (patches) {
+            const int k = std::min(c.patch.rings, interval - s % interval);
+            c.state_np1 = 1 - c.state_np1;
+            c.rate_dt = dt;
+            patch_run(c, dt, k, false);
+            s += k;
+        } else {
+            step_once_tiles(c, dt, false);
+            ++s;
+        }
     }
+    D.seg_held = nck - 1;
     copy_state(c, D.final_state.p);
     APHIP_HIP(hipStreamSynchronize(c.stream));
     D.dt = dt;
@@ -637,15 +946,15 @@ void adjoint_backward(Ctx &c, const double *ub_T, const double *vb_T, double *E_
         D.vb.upload(h.data(), n3, c.stream);
     }
     const int K = D.interval;
-    D.seg_u.alloc((size_t)K * n3);
+    if (on_patches(c)) c.graph_reset();
     const int nseg = (int)D.ckpt.size();
     for (int sg = nseg - 1; sg >= 0; --sg) {
         const int s0 = sg * K, len = std::min(K, D.n_steps - s0);
-        restore_state(c, D.ckpt[sg]->p);
-        for (int k = 0; k < len; ++k) {
-            step_once_tiles(c, D.dt, false);
-            APHIP_HIP(hipMemcpyAsync(D.seg_u.p + (size_t)k * n3, c.u.p, sizeof(double) * n3, hipMemcpyDeviceToDevice,
-                                     c.stream));
+        if (D.seg_held != sg) {
+            D.seg_held = -1;
+            restore_state(c, D.ckpt[sg]->p);
+            for (int k = 0; k < len; ++k) recorded_step(c, D.dt, k, false);
+            D.seg_held = sg;
         }
         for (int k = len - 1; k >= 0; --k) adj_run(c, D.seg_u.p + (size_t)k * n3, nullptr, 1, D.dt);
     }

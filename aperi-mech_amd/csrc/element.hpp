@@ -291,6 +291,55 @@ APHIP_DEV int hex8_lane_label(int lane) {
     return x0 | (x1 << 1) | (x2 << 2);
 }
 
+// One field's modes to the seven doubles of out (src: the field's component of node 0).
+APHIP_DEV void hex8_field_modes(const uint32_t (&cn)[4], const double *src, double ga, double *out) {
+#pragma clang fp contract(off)
+    double v[8], w[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = src[k & 1 ? cn[k >> 1] >> 16 : cn[k >> 1] & 0xffffu];
+    hex8_modes(v, w);
+    // a mode of |S| axes is only ever used times ga^(|S| - 1) and signs
+    w[3] *= ga;
+    w[5] *= ga;
+    w[6] *= ga;
+    w[7] *= ga * ga;
+#pragma unroll
+    for (int S = 1; S < 8; ++S) out[S - 1] = w[S];
+}
+
+// The lanes' nodal vectors of a stress-like P: scale sum over the points and axes n of the
+// derivative along n of a corner's function times (Ad P^T)_n, to out of every lane's corner.
+APHIP_DEV void hex8_to_corners(int x, bool b0, bool b1, bool b2, double s0, double s1, double s2, double ga, double scale,
+                               const double *Ad, const double *P, double *out) {
+#pragma clang fp contract(off)
+    // W_nj[x] = sum over the points of sign_(x without n)(point) Q_nj by butterflies: lane x keeps
+    // pattern x of the other axes, along axis n both partners take the plain sum
+    double W[3][3];
+#pragma unroll
+    for (int n = 0; n < 3; ++n)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            double v = dot3(Ad[3 * n], P[3 * j], Ad[3 * n + 1], P[3 * j + 1], Ad[3 * n + 2], P[3 * j + 2]);
+            v = n == 0 ? v + hex8_partner<0>(v) : __fma_rn(s0, hex8_partner<0>(v), v);
+            v = n == 1 ? v + hex8_partner<1>(v) : __fma_rn(s1, hex8_partner<1>(v), v);
+            W[n][j] = n == 2 ? v + hex8_partner<2>(v) : __fma_rn(s2, hex8_partner<2>(v), v);
+        }
+    // mode x: R_xj = c sum_{n in x} W_nj, c = ga^(|x| - 1); then to the corners
+    const int nx = (x & 1) + ((x >> 1) & 1) + (x >> 2);
+    const double c = (nx == 3 ? ga * ga : nx == 2 ? ga : 1.0) * scale;
+    const double c0 = b0 ? c : 0.0, c1 = b1 ? c : 0.0, c2 = b2 ? c : 0.0;
+    double f[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        double v = __fma_rn(c2, W[2][j], __fma_rn(c1, W[1][j], c0 * W[0][j]));
+        v = __fma_rn(-s0, hex8_partner<0>(v), v);
+        v = __fma_rn(-s1, hex8_partner<1>(v), v);
+        f[j] = __fma_rn(-s2, hex8_partner<2>(v), v);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) out[j] = f[j];
+}
+
 // lane: 0..7 within the element (all eight active); cn: the offsets (3 x local node) of corners
 // 2 i and 2 i + 1 in cn[i]; sX, sU: 3 doubles per local node; row: the element's kHexRow doubles, on
 // return the corner forces (corner k at 3 k).  H, P and the state of the last point are valid
@@ -306,20 +355,7 @@ APHIP_DEV bool hex8_lanes(int lane, const uint32_t (&cn)[4], const double *sX, c
     int x = hex8_lane_label(lane);
     bool b0 = x & 1, b1 = x & 2, b2 = x & 4;
     const int q = x == 2 ? 3 : x == 3 ? 2 : x == 6 ? 7 : x == 7 ? 6 : x;  // point (and corner) index
-    if (lane < 6) {
-        const double *src = (lane < 3 ? sX : sU) + (lane < 3 ? lane : lane - 3);
-        double v[8], w[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = src[k & 1 ? cn[k >> 1] >> 16 : cn[k >> 1] & 0xffffu];
-        hex8_modes(v, w);
-        // a mode of |S| axes is only ever used times ga^(|S| - 1) and signs
-        w[3] *= ga;
-        w[5] *= ga;
-        w[6] *= ga;
-        w[7] *= ga * ga;
-#pragma unroll
-        for (int S = 1; S < 8; ++S) row[7 * lane + S - 1] = w[S];
-    }
+    if (lane < 6) hex8_field_modes(cn, (lane < 3 ? sX : sU) + (lane < 3 ? lane : lane - 3), ga, row + 7 * lane);
     __builtin_amdgcn_wave_barrier();  // (LDS operations of a wave stay in order)
     double s0 = b0 ? -1.0 : 1.0, s1 = b1 ? -1.0 : 1.0, s2 = b2 ? -1.0 : 1.0;
     const double s01 = s0 * s1, s02 = s0 * s2, s12 = s1 * s2;
@@ -373,32 +409,7 @@ APHIP_DEV bool hex8_lanes(int lane, const uint32_t (&cn)[4], const double *sX, c
         s1 = b1 ? -1.0 : 1.0;
         s2 = b2 ? -1.0 : 1.0;
     }
-    // W_nj[x] = sum over the points of sign_(x without n)(point) Q_nj by butterflies: lane x keeps
-    // pattern x of the other axes, along axis n both partners take the plain sum
-    double W[3][3];
-#pragma unroll
-    for (int n = 0; n < 3; ++n)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            double v = dot3(Ad[3 * n], Pf[3 * j], Ad[3 * n + 1], Pf[3 * j + 1], Ad[3 * n + 2], Pf[3 * j + 2]);
-            v = n == 0 ? v + hex8_partner<0>(v) : __fma_rn(s0, hex8_partner<0>(v), v);
-            v = n == 1 ? v + hex8_partner<1>(v) : __fma_rn(s1, hex8_partner<1>(v), v);
-            W[n][j] = n == 2 ? v + hex8_partner<2>(v) : __fma_rn(s2, hex8_partner<2>(v), v);
-        }
-    // mode x: R_xj = c sum_{n in x} W_nj, c = ga^(|x| - 1); then to the corners
-    const int nx = (x & 1) + ((x >> 1) & 1) + (x >> 2);
-    const double c = (nx == 3 ? ga * ga : nx == 2 ? ga : 1.0) * (-1.0 / 512.0);  // (-1/512 = -w det^-1, exact)
-    const double c0 = b0 ? c : 0.0, c1 = b1 ? c : 0.0, c2 = b2 ? c : 0.0;
-    double f[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        double v = __fma_rn(c2, W[2][j], __fma_rn(c1, W[1][j], c0 * W[0][j]));
-        v = __fma_rn(-s0, hex8_partner<0>(v), v);
-        v = __fma_rn(-s1, hex8_partner<1>(v), v);
-        f[j] = __fma_rn(-s2, hex8_partner<2>(v), v);
-    }
-#pragma unroll
-    for (int j = 0; j < 3; ++j) row[3 * q + j] = f[j];
+    hex8_to_corners(x, b0, b1, b2, s0, s1, s2, ga, -1.0 / 512.0, Ad, Pf, row + 3 * q);  // (exact: -w det^-1)
     return last;
 }
 

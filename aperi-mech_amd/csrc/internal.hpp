@@ -100,15 +100,18 @@ struct AdjointData {
     int n_steps = 0, interval = 0;
     std::vector<DevBuf<double> *> ckpt;  // (u, v, a) at steps 0, K, 2K, ...; 9 doubles per node
     DevBuf<double> final_state;          // (u, v, a) at the last step
-    DevBuf<double> seg_u;                // recomputed u of one segment, K x 3 x nn
+    DevBuf<double> seg_u;                // u of one segment's steps, K x 3 x nn
+    int seg_held = -1;                   // the segment it holds (the last one after a forward run)
     DevBuf<double> ub, vb, ab;           // adjoint node state
+    DevBuf<double> vb1, ab1;             // on patches: the vb, ab that the next launch writes
     DevBuf<double> lam_bar, mu_bar;      // per-element parameter adjoints
     void reset() {
         for (auto *b : ckpt) delete b;
         ckpt.clear();
         final_state.release();
         seg_u.release();
-        ub.release(); vb.release(); ab.release(); lam_bar.release(); mu_bar.release();
+        seg_held = -1;
+        ub.release(); vb.release(); ab.release(); vb1.release(); ab1.release(); lam_bar.release(); mu_bar.release();
         ready = false;
     }
     ~AdjointData() { reset(); }
@@ -447,8 +450,10 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run = TileRun());
 bool patch_eligible(Ctx &c);
 int patch_steps(const Ctx &c, int left);
 // `steps` steps in one launch (the state buffers' roles were swapped once by the caller);
-// keep: store H, P and f of the last one
-void patch_run(Ctx &c, double dt, int steps, bool keep);
+// keep: store H, P and f of the last one; u_rec: store its displacement there as well
+void patch_run(Ctx &c, double dt, int steps, bool keep, double *u_rec = nullptr);
+// whether the mesh has a plan (built on first use), for passes with conditions of their own
+bool patch_planned(Ctx &c);
 
 // ---- adjoint (adjoint.hip) ----
 void adjoint_forward(Ctx &c, double dt, int n_steps, int interval);

@@ -27,8 +27,7 @@
 #include <thread>
 #include <vector>
 
-#include "element.hpp"
-#include "internal.hpp"
+#include "patch.hpp"
 
 namespace aphip {
 
@@ -36,8 +35,6 @@ namespace {
 
 constexpr int kNumXcd = 8;
 constexpr int kRings = PatchPlan::kRings;
-constexpr uint16_t kNewTile = 0x8000;   // entry flag: the node's first element of another tile
-constexpr int kBatch = 8;               // entries of a node are padded to a multiple of this
 
 __device__ __forceinline__ void ld3(const double *p, int64_t i, double *o) {
     o[0] = p[3 * i];
@@ -55,6 +52,7 @@ struct PatchArgs {
     const double *X;
     const double *u, *v, *a;     // state read
     double *u1, *v1, *a1, *f;    // state written (other buffers)
+    double *u_rec;               // the displacement once more, or null
     const double *mass;
     const uint8_t *fixed;
     const double *zero;          // 8 zero doubles: stands in for an absent optional array
@@ -85,16 +83,6 @@ struct PatchLds {
     size_t bytes;
 };
 
-// rows between the slot blocks of the force rows (as in the tile kernel: the slots of one
-// element sit 24 banks apart)
-__host__ __device__ __forceinline__ int f_stride(int n) { return n + ((4 - n) & 31); }
-
-// force row of (local element, slot), in rows of three doubles: Tet4 slot-major, Hex8 in the
-// element's LDS row
-__host__ __device__ __forceinline__ int force_row(int npe, int epad, int le, int k) {
-    return npe == 4 ? k * f_stride(epad) + le : (kHexRow / 3) * le + k;
-}
-
 __host__ __device__ __forceinline__ PatchLds carve(char *base, int npe, int npad, int cpad, int epad, int entpad) {
     PatchLds L;
     char *p = base;
@@ -108,7 +96,7 @@ __host__ __device__ __forceinline__ PatchLds carve(char *base, int npe, int npad
     L.V = reinterpret_cast<double *>(take(24 * (size_t)npad));
     L.M = reinterpret_cast<double *>(take(8 * (size_t)cpad));
     L.S = reinterpret_cast<double *>(take(8 * (size_t)epad));
-    L.F = reinterpret_cast<double *>(take(npe == 4 ? 96 * (size_t)f_stride(epad) : 8 * kHexRow * (size_t)epad));
+    L.F = reinterpret_cast<double *>(take(npe == 4 ? 96 * (size_t)patch_stride(epad) : 8 * kHexRow * (size_t)epad));
     L.csr = reinterpret_cast<uint32_t *>(take(4 * (size_t)cpad));
     L.conn = reinterpret_cast<uint16_t *>(take(2 * (size_t)npe * epad));
     L.ent = reinterpret_cast<uint16_t *>(take(2 * (size_t)entpad));
@@ -164,7 +152,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 512, NPE == 4 ? 1 : 3) void k_pat
         if constexpr (state_width<KIND>() > 0) L.S[i] = load_state<KIND>(A.state_n, elem[i]);
     }
     __syncthreads();
-    const int fs = f_stride(A.epad);
+    const int fs = patch_stride(A.epad);
     int ne_now = nE, nn_now = nC;
     for (int s = 1;; ++s) {
         const bool last = s == A.steps;
@@ -232,31 +220,11 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 512, NPE == 4 ? 1 : 3) void k_pat
             }
         }
         __syncthreads();
-        // four lanes per node, one per component (the fourth idles): the sums stay in order and
-        // the LDS latency is paid once per kBatch entries
+        // four lanes per node, one per component (the fourth idles)
         for (int t4 = tid; t4 < 4 * nn_now; t4 += nt) {
             const int ln = t4 >> 2, d = t4 & 3;
             if (d == 3) continue;
-            const uint32_t pk = L.csr[ln];
-            const int st = (int)(pk >> 16) * kBatch, cnt = (int)(pk & 0xffffu);
-            const double *F = L.F + d;
-            double f = 0.0, t = 0.0;
-            for (int j = 0; j < cnt; j += kBatch) {
-                const uint4 w = *reinterpret_cast<const uint4 *>(L.ent + st + j);
-                const unsigned en[kBatch] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16,
-                                             w.z & 0xffffu, w.z >> 16, w.w & 0xffffu, w.w >> 16};
-                double r[kBatch];
-#pragma unroll
-                for (int q = 0; q < kBatch; ++q) r[q] = F[3 * (en[q] & 0x7fffu)];
-#pragma unroll
-                for (int q = 0; q < kBatch; ++q) {
-                    const bool fresh = en[q] & kNewTile;
-                    f = fresh ? f + t : f;
-                    t = fresh ? 0.0 : t;
-                    t = j + q < cnt ? t + r[q] : t;
-                }
-            }
-            f += t;
+            const double f = patch_sum(L.F + d, L.ent, L.csr[ln]);
             const bool fx = L.fx[ln] & (1u << d);
             double a1, v1;
             const double u1 = L.U[3 * ln + d];
@@ -264,6 +232,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 512, NPE == 4 ? 1 : 3) void k_pat
             if (last) {
                 const int64_t g = 3 * (int64_t)node[ln] + d;
                 A.u1[g] = u1;
+                if (A.u_rec) A.u_rec[g] = u1;
                 A.v1[g] = v1;
                 A.a1[g] = a1;
                 if (A.keep) A.f[g] = f;
@@ -489,14 +458,18 @@ static void patch_build(Ctx &c) {
     P.ready = true;
 }
 
-bool patch_eligible(Ctx &c) {
+bool patch_planned(Ctx &c) {
     if (c.tiles.ready && !c.patch.tried) patch_build(c);
-    return c.patch.ready && !c.node_dt.p && !c.tiles.use_stream && !c.mat.state_per_qp &&
+    return c.patch.ready;
+}
+
+bool patch_eligible(Ctx &c) {
+    return patch_planned(c) && !c.node_dt.p && !c.tiles.use_stream && !c.mat.state_per_qp &&
            (c.mat.kind == APHIP_LINEAR_ELASTIC || c.mat.kind == APHIP_NEO_HOOKEAN || c.mat.kind == APHIP_J2 ||
             c.mat.kind == APHIP_SVK);
 }
 
-void patch_run(Ctx &c, double dt, int steps, bool keep) {
+void patch_run(Ctx &c, double dt, int steps, bool keep, double *u_rec) {
     PatchPlan &P = c.patch;
     APHIP_REQUIRE(P.ready && steps >= 1 && steps <= P.rings, "patch plan does not cover these steps");
     PatchArgs A;
@@ -507,6 +480,7 @@ void patch_run(Ctx &c, double dt, int steps, bool keep) {
     A.u1 = P.u.p;
     A.v1 = P.v.p;
     A.a1 = P.a.p;
+    A.u_rec = u_rec;
     A.f = c.f.p;
     A.mass = c.mass.p;
     A.fixed = c.has_fixed ? c.fixed.p : nullptr;
