@@ -23,7 +23,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
-#include <cstring>
+#include <memory>
 #include <thread>
 #include <vector>
 
@@ -282,7 +282,7 @@ static void patch_build(Ctx &c) {
     PatchPlan &P = c.patch;
     P.tried = true;
     const int64_t nn = c.nn, ne = c.ne;
-    const int npe = c.npe;
+    const int npe = c.npe, sh = npe == 4 ? 2 : 3;
     // The lines, from calls of 20 steps on n^3 x 6 Tet4 lattices (neo-Hookean; us a call, three
     // meshes in turn / one alone; T the tile path, k x s: k rings, s owned elements):
     //     750 T 71/177  2x64 59/149          24,576 T 119/275  1x128 70/174  2x128 88/169
@@ -310,7 +310,7 @@ static void patch_build(Ctx &c) {
     const int64_t np = (ne + target - 1) / target;
     std::vector<std::vector<int32_t>> own(np);
     for (int64_t i = 0; i < nn; ++i)
-        own[start[i] < start[i + 1] ? (inc[start[i]] / npe) / target : i % np].push_back((int32_t)i);
+        own[start[i] < start[i + 1] ? (inc[start[i]] >> sh) / target : i % np].push_back((int32_t)i);
     // tile of every element (the grouping of the sums)
     const int te = c.tiles.te;
     struct Patch {
@@ -331,6 +331,10 @@ static void patch_build(Ctx &c) {
                 q.elems.push_back((int32_t)e);
             }
             q.ne[0] = (int)q.elems.size();
+            q.elems.reserve(4 * target);
+            q.nodes.reserve(4 * target);
+            q.conn.reserve(4 * npe * target);
+            q.ent.reserve(2 * npe * target);
             for (size_t i = 0; i < q.nodes.size(); ++i) nloc[q.nodes[i]] = (int32_t)i;
             q.nn[0] = (int)q.nodes.size();
             size_t n_from = 0;
@@ -338,7 +342,7 @@ static void patch_build(Ctx &c) {
                 const size_t n_to = q.nodes.size(), e_from = q.elems.size(), e_new = r == 1 ? 0 : e_from;
                 for (size_t i = n_from; i < n_to; ++i)
                     for (int32_t t = start[q.nodes[i]]; t < start[q.nodes[i] + 1]; ++t) {
-                        const int32_t e = inc[t] / npe;
+                        const int32_t e = inc[t] >> sh;
                         if (eloc[e] < 0) {
                             eloc[e] = 0;
                             q.elems.push_back(e);
@@ -365,7 +369,7 @@ static void patch_build(Ctx &c) {
                 const size_t s0 = q.ent.size();
                 int32_t tile = -1;
                 for (int32_t t = start[q.nodes[i]]; t < start[q.nodes[i] + 1]; ++t) {
-                    const int32_t e = inc[t] / npe, k = inc[t] % npe;
+                    const int32_t e = inc[t] >> sh, k = inc[t] & (npe - 1);
                     const bool fresh = tile >= 0 && e / te != tile;
                     tile = e / te;
                     // (local element and slot; the force row once the row stride is known)
@@ -384,13 +388,14 @@ static void patch_build(Ctx &c) {
             for (int32_t e : q.elems) eloc[e] = -1;
         }
     };
-    {
-        const int nw = (int)std::max<int64_t>(1, std::min<int64_t>({16, (int64_t)std::thread::hardware_concurrency(), np / 6}));
+    auto parallel = [np](int most, auto &fn) {  // (a thread costs some 20 us)
+        const int nw = (int)std::max<int64_t>(1, std::min<int64_t>({most, (int64_t)std::thread::hardware_concurrency(), np / 6}));
         std::vector<std::thread> pool;
-        for (int w = 1; w < nw; ++w) pool.emplace_back(work, w, nw);
-        work(0, nw);
+        for (int w = 1; w < nw; ++w) pool.emplace_back([&fn, w, nw] { fn(w, nw); });
+        fn(0, nw);
         for (auto &t : pool) t.join();
-    }
+    };
+    parallel(16, work);
     if (!fits) return;
     size_t npad = 1, cpad = 1, epad = 1, entpad = kBatch;
     for (const Patch &q : pt) {
@@ -402,39 +407,45 @@ static void patch_build(Ctx &c) {
     if (force_row(npe, (int)epad, (int)epad, npe) > 0x7fff) return;
     const size_t lds = carve(nullptr, npe, (int)npad, (int)cpad, (int)epad, (int)entpad).bytes;
     if (lds > 160 * 1024) return;
-    std::vector<int32_t> meta((size_t)np * 16, 0), node(np * npad);
-    std::vector<int32_t> elem(np * epad);
-    std::vector<uint32_t> csr(np * cpad, 0);
-    std::vector<uint16_t> lconn(np * epad * npe), ent(np * entpad, 0);
-    for (int64_t p = 0; p < np; ++p) {
-        const Patch &q = pt[p];
-        for (int r = 0; r <= K; ++r) {
-            meta[16 * p + r] = q.nn[r];
-            meta[16 * p + 8 + r] = q.ne[r];
-        }
-        for (size_t i = 0; i < npad; ++i) node[p * npad + i] = q.nodes[std::min(i, q.nodes.size() - 1)];
-        std::copy(q.csr.begin(), q.csr.end(), csr.begin() + p * cpad);
-        for (size_t i = 0; i < q.ent.size(); ++i) {
-            const int le = q.ent[i] & ~kNewTile;
-            ent[p * entpad + i] = (uint16_t)force_row(npe, (int)epad, le / npe, le % npe) | (q.ent[i] & kNewTile);
-        }
-        for (size_t i = 0; i < epad; ++i) {
-            const size_t j = std::min(i, q.elems.size() - 1);
-            elem[p * epad + i] = q.elems[j];
-            for (int k = 0; k < npe; ++k) lconn[(p * epad + i) * npe + k] = (uint16_t)((npe == 8 ? 3 : 1) * q.conn[j * npe + k]);
-        }
-    }
-    // one allocation and one copy for the six lists (each on a 16-byte boundary)
-    std::vector<unsigned char> bytes;
-    auto put = [&](const auto &v) {
-        const size_t at = (bytes.size() + 15) & ~(size_t)15;
-        bytes.resize(at + sizeof(v[0]) * v.size());
-        std::memcpy(bytes.data() + at, v.data(), sizeof(v[0]) * v.size());
+    // the six lists (each on a 16-byte boundary) in one allocation and one copy
+    size_t total = 0;
+    auto put = [&](size_t bytes) {
+        const size_t at = total;
+        total += (bytes + 15) & ~(size_t)15;
         return at;
     };
-    const size_t o_meta = put(meta), o_node = put(node), o_csr = put(csr), o_elem = put(elem), o_conn = put(lconn),
-                 o_ent = put(ent);
-    P.lists.upload(bytes.data(), bytes.size(), c.stream);
+    const size_t o_meta = put(64 * np), o_node = put(4 * np * npad), o_csr = put(4 * np * cpad),
+                 o_elem = put(4 * np * epad), o_conn = put(2 * np * epad * npe), o_ent = put(2 * np * entpad);
+    std::unique_ptr<unsigned char[]> bytes(new unsigned char[total]);
+    auto pack = [&](int w, int nw) {
+        for (int64_t p = w; p < np; p += nw) {
+            const Patch &q = pt[p];
+            int32_t *meta = reinterpret_cast<int32_t *>(bytes.get() + o_meta) + 16 * p;
+            int32_t *node = reinterpret_cast<int32_t *>(bytes.get() + o_node) + p * npad;
+            uint32_t *csr = reinterpret_cast<uint32_t *>(bytes.get() + o_csr) + p * cpad;
+            int32_t *elem = reinterpret_cast<int32_t *>(bytes.get() + o_elem) + p * epad;
+            uint16_t *lconn = reinterpret_cast<uint16_t *>(bytes.get() + o_conn) + p * epad * npe;
+            uint16_t *ent = reinterpret_cast<uint16_t *>(bytes.get() + o_ent) + p * entpad;
+            std::fill(meta, meta + 16, 0);
+            for (int r = 0; r <= K; ++r) {
+                meta[r] = q.nn[r];
+                meta[8 + r] = q.ne[r];
+            }
+            for (size_t i = 0; i < npad; ++i) node[i] = q.nodes[std::min(i, q.nodes.size() - 1)];
+            for (size_t i = 0; i < cpad; ++i) csr[i] = i < q.csr.size() ? q.csr[i] : 0;
+            for (size_t i = 0; i < entpad; ++i) {
+                const int le = i < q.ent.size() ? q.ent[i] & ~kNewTile : 0;
+                ent[i] = i < q.ent.size() ? (uint16_t)force_row(npe, (int)epad, le >> sh, le & (npe - 1)) | (q.ent[i] & kNewTile) : 0;
+            }
+            for (size_t i = 0; i < epad; ++i) {
+                const size_t j = std::min(i, q.elems.size() - 1);
+                elem[i] = q.elems[j];
+                for (int k = 0; k < npe; ++k) lconn[i * npe + k] = (uint16_t)((npe == 8 ? 3 : 1) * q.conn[j * npe + k]);
+            }
+        }
+    };
+    parallel(4, pack);
+    P.lists.upload(bytes.get(), total, c.stream);
     P.meta = reinterpret_cast<const int32_t *>(P.lists.p + o_meta);
     P.node = reinterpret_cast<const int32_t *>(P.lists.p + o_node);
     P.csr = reinterpret_cast<const uint32_t *>(P.lists.p + o_csr);
