@@ -496,7 +496,7 @@ static void step_once(Ctx &c, double dt, bool pred_in, bool pred_out, bool keep)
     } else {
         // (ensembles keep their own increment per node, which only the predictor kernel reads)
         const bool chain = c.cells.ready && !c.node_dt.p;
-        const bool raw = !(chain && pred_in) && rk_fused(c);  // both passes take the predictor themselves
+        const bool raw = !(chain && pred_in) && rk_takes_predictor(c);  // both passes take the predictor themselves
         if (!(chain && pred_in) && !raw) fem_predict(c, dt);
         force_pass(c, keep, raw, keep);
         node_pass(c, dt, 2, chain && pred_out, raw, keep);

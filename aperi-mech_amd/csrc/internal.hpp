@@ -473,10 +473,11 @@ void rk_setup(Ctx &c, double scale, bool two_pass, bool fe_cells = false, int no
 void rk_cell_force(Ctx &c, bool keep, bool raw = false, bool keep_local = true);
 // more (mode 2): another step of the same call with the same dt follows; its predictor is
 // taken here and fem_predict is not called for it
-// raw: the step's predictor has not been taken; both passes of a fused step (rk_fused) take it.
+// raw: the step's predictor has not been taken; both passes take it (rk_takes_predictor).
 // keep = false: an inner step, the local force may be left unwritten
 void rk_node_update(Ctx &c, double dt, int mode, bool more, bool raw = false, bool keep = true);
 bool rk_fused(const Ctx &c);
+bool rk_takes_predictor(const Ctx &c);
 void rk_mass(Ctx &c, double *total);
 
 // ---- profiling helpers (capi.hip) ----

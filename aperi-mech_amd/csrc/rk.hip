@@ -613,7 +613,43 @@ struct RkTileArgs {
     const double *elem_lambda, *elem_mu;
     const double *Hn, *Pn;
     double rate_dt;
+    int keep;  // 0: an inner step, H and P are not stored
+    // raw: u is predicted on the way (the nodes below n_dof; dt is rate_dt)
+    int raw;
+    int64_t n_dof;
+    const double *v, *a;
+    const uint8_t *fixed;
 };
+
+// u of the tile's nodes tb .. tb + tn - 1 to U, by blockDim threads, in batches of kStage rows a
+// thread, every load of a batch issued before its first LDS write (a load and its write per
+// iteration would cost a latency each).
+__device__ __forceinline__ void stage_tile_u(const RkTileArgs &A, int tb, int tn, double *U) {
+    constexpr int kStage = 4;
+    const int nt = blockDim.x;
+    for (int l0 = threadIdx.x; l0 < tn; l0 += nt * kStage) {
+        int64_t gi[kStage];
+#pragma unroll
+        for (int r = 0; r < kStage; ++r) gi[r] = A.t_node[tb + min(l0 + nt * r, tn - 1)];
+        double ur[kStage][3];
+#pragma unroll
+        for (int r = 0; r < kStage; ++r) ld3(A.u, gi[r], ur[r]);
+        if (A.raw) {
+#pragma unroll
+            for (int r = 0; r < kStage; ++r) {
+                double v[3], a[3], vh[3], u1[3];
+                ld3(A.v, gi[r], v);
+                ld3(A.a, gi[r], a);
+                cd_predict(ur[r], v, a, A.fixed ? A.fixed[gi[r]] : 0u, A.rate_dt, vh, u1);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) ur[r][d] = gi[r] < A.n_dof ? u1[d] : ur[r][d];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kStage; ++r)
+            if (l0 + nt * r < tn) st3(U, l0 + nt * r, ur[r]);
+    }
+}
 
 template <int KIND, int LPC, int K>
 __global__ __launch_bounds__(64) void k_rk_tile(RkTileArgs A) {
@@ -625,28 +661,8 @@ __global__ __launch_bounds__(64) void k_rk_tile(RkTileArgs A) {
     if (t >= A.ntiles) return;
     const int lane = threadIdx.x;
     const int tb = A.t_nstart[t], tn = A.t_nstart[t + 1] - tb;
-    // staging in batches of kStage rows per lane, every load of a batch issued before its
-    // first LDS write (a load and its write per iteration would cost a latency each)
-    constexpr int kStage = 8;
-    for (int l0 = lane; l0 < tn; l0 += 64 * kStage) {
-        int64_t gi[kStage];
-#pragma unroll
-        for (int r = 0; r < kStage; ++r) gi[r] = A.t_node[tb + min(l0 + 64 * r, tn - 1)];
-        double ur[kStage][3];
-#pragma unroll
-        for (int r = 0; r < kStage; ++r) ld3(A.u, gi[r], ur[r]);
-#pragma unroll
-        for (int r = 0; r < kStage; ++r) {
-            const int ln = l0 + 64 * r;
-            if (ln < tn) {
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    U[3 * ln + d] = ur[r][d];
-                    F[3 * ln + d] = 0.0;
-                }
-            }
-        }
-    }
+    stage_tile_u(A, tb, tn, U);
+    for (int k = lane; k < 3 * tn; k += 64) F[k] = 0.0;
     __syncthreads();
     constexpr int G = 64 / LPC;
     const int grp = lane / LPC, j = lane % LPC;
@@ -705,10 +721,12 @@ __global__ __launch_bounds__(64) void k_rk_tile(RkTileArgs A) {
             store_state<KIND>(A.state_np1, c, snp1, aux);
             // plain stores: one lane per cell writes H and P, a sparse stream that
             // measured 2 % faster through the L2 than as non-temporal stores
+            if (A.keep) {
 #pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                A.H[i * A.ncells + c] = H[i];
-                A.P[i * A.ncells + c] = P[i];
+                for (int i = 0; i < 9; ++i) {
+                    A.H[i * A.ncells + c] = H[i];
+                    A.P[i * A.ncells + c] = P[i];
+                }
             }
         }
         if (!live) continue;
@@ -740,16 +758,21 @@ __global__ __launch_bounds__(64) void k_rk_tile(RkTileArgs A) {
 }
 
 // F-bar on cell tiles (ComputeInternalForceSmoothedCell.h:120-413): a tile holds whole
-// nodal cells, so every pass of the F-bar force runs inside one wave with the subcell
+// nodal cells, so every pass of the F-bar force runs inside one workgroup with the subcell
 // rows in LDS: (1) subcell H (LPC lanes per subcell, butterfly) and J = DetApIm1(H) + 1;
 // (2) one lane per subcell: J-bar of its cell (the cell's J_k V_k summed in order over
 // V_cell, :120-175), H-bar = H cbrt(J-bar / J) + (cbrt(.) - 1) I unless the ratio is
 // within 3 eps of 1, the stress of H-bar (:177-213) and the subcell's term of the dual
 // pressure; (3) one lane per subcell: the dual pressure (the cell's terms in order) and
 // the un-barred P = P-bar s + (p - s / (3 J) P-bar : F) J F^-T (UnBarStress, :215-309);
-// (4) the entry forces -V P grad phi added into the tile's LDS rows, as in k_rk_tile.
-// The entries are read twice (H needs every subcell of a cell before any stress), the
-// second time right after the first by the same wave.
+// (4) the entry forces -V P grad phi added into LDS rows as in k_rk_tile, one set of rows per
+// wave (a wave's adds are in program order), and the waves' rows summed in wave order.
+// The entries are read twice, in (1) and (4).  A tile is one nodal cell of some twenty subcells;
+// bound by latency and by the entries' loads (26 B each).  Loading a lane's entries together
+// and summing J-bar from volumes in LDS (not one global load after the other) took the kernel
+// from 31 to 24.6 us on 41k subcells, and 20 steps with three streams in turn from 400 to 303;
+// holding the entries in registers from (1) to (4) (152 VGPRs: 422 us) or loading the next
+// subcell's ahead (316 us) did not pay.
 constexpr int kFbarSubRow = 29;  // LDS doubles per subcell: H 9, J 1, P-bar 9, dual term 1, P 9
 
 struct FbarTileArgs {
@@ -762,98 +785,98 @@ struct FbarTileArgs {
 };
 
 template <int KIND, int LPC>
-__global__ __launch_bounds__(64) void k_fbar_tile(FbarTileArgs B) {
+__global__ __launch_bounds__(256) void k_fbar_tile(FbarTileArgs B) {
 #pragma clang fp contract(off)
     constexpr double kEps = 2.2204460492503131e-16;
     const RkTileArgs &A = B.T;
     extern __shared__ __align__(16) double rk_lds[];
+    const int tid = threadIdx.x, nt = blockDim.x, nw = nt / 64;
     double *U = rk_lds;
-    double *F = U + 3 * (size_t)A.maxtn;
-    double *SH = F + 3 * (size_t)A.maxtn;  // [maxsub * 9]
+    double *F = U + 3 * (size_t)A.maxtn;         // a set of rows per wave
+    double *SH = F + 3 * (size_t)A.maxtn * nw;   // [maxsub * 9]
     double *SJ = SH + 9 * (size_t)B.maxsub;
-    double *SPb = SJ + B.maxsub;           // [maxsub * 9]
+    double *SPb = SJ + B.maxsub;                 // [maxsub * 9]
     double *SD = SPb + 9 * (size_t)B.maxsub;
-    double *SP = SD + B.maxsub;            // [maxsub * 9]
+    // [maxsub * 9] P; before (3) its place 0 holds the subcell's volume, 1 and 2 J-bar and cbrt
+    double *SP = SD + B.maxsub;
     const int64_t t = xcd_block(A.nblocks);
     if (t >= A.ntiles) return;
-    const int lane = threadIdx.x;
     const int tb = A.t_nstart[t], tn = A.t_nstart[t + 1] - tb;
-    constexpr int kStage = 8;
-    for (int l0 = lane; l0 < tn; l0 += 64 * kStage) {
-        int64_t gi[kStage];
+    const int64_t c0 = A.t_cstart[t], c1 = A.t_cstart[t + 1];
+    const int grp = tid / LPC, j = tid % LPC, G = nt / LPC;
+    // a subcell's entries, K per lane in flight together (those past the end weighted by zero)
+    constexpr int K = LPC == 4 ? 1 : 5;
+    auto entries = [&](int64_t e0, int64_t e1, int (&li)[K], double (&g)[K][3]) {
 #pragma unroll
-        for (int r = 0; r < kStage; ++r) gi[r] = A.t_node[tb + min(l0 + 64 * r, tn - 1)];
-        double ur[kStage][3];
+        for (int r = 0; r < K; ++r) {
+            const int64_t e = min(e0 + r * LPC, e1 - 1);
+            li[r] = A.lidx[e];
+            ld3(A.dphi, e, g[r]);
+        }
+    };
+    stage_tile_u(A, tb, tn, U);
+    for (int k = tid; k < 3 * A.maxtn * nw; k += nt) F[k] = 0.0;
+    for (int64_t s = c0 + tid; s < c1; s += nt) SP[9 * (int)(s - c0)] = A.volume[s];
+    __syncthreads();
+    // (1) subcell H and J
+    for (int64_t cb = c0; cb < c1; cb += G) {
+        const int64_t c = cb + grp;
+        const bool live = c < c1;  // (a lane group is live or idle as a whole)
+        if (!live) break;
+        double H[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        const int64_t s0 = A.start[c], s1 = A.start[c + 1];
+        for (int64_t e = s0 + j; e < s1; e += K * LPC) {
+            int li[K];
+            double g[K][3];
+            entries(e, s1, li, g);
 #pragma unroll
-        for (int r = 0; r < kStage; ++r) ld3(A.u, gi[r], ur[r]);
+            for (int r = 0; r < K; ++r) {
+                const bool in = e + r * LPC < s1;
+                double uj[3];
+                ld3(U, li[r], uj);
 #pragma unroll
-        for (int r = 0; r < kStage; ++r) {
-            const int ln = l0 + 64 * r;
-            if (ln < tn) {
+                for (int b = 0; b < 3; ++b) {
+                    const double gb = in ? g[r][b] : 0.0;
 #pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    U[3 * ln + d] = ur[r][d];
-                    F[3 * ln + d] = 0.0;
+                    for (int a = 0; a < 3; ++a) H[3 * a + b] = __fma_rn(uj[a], gb, H[3 * a + b]);
                 }
             }
         }
-    }
-    __syncthreads();
-    constexpr int G = 64 / LPC;
-    const int grp = lane / LPC, j = lane % LPC;
-    const int64_t c0 = A.t_cstart[t], c1 = A.t_cstart[t + 1];
-    // (1) subcell H and J
-    for (int64_t cb = c0; cb < c1; cb += G) {
-        const int64_t c_raw = cb + grp;
-        const bool live = c_raw < c1;
-        const int64_t c = live ? c_raw : c1 - 1;
-        const int64_t t0 = A.start[c], t1 = A.start[c + 1];
-        double H[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        for (int64_t e = t0 + j; e < t1; e += LPC) {
-            double uj[3], g[3];
-            ld3(U, A.lidx[e], uj);
-            ld3(A.dphi, e, g);
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-#pragma unroll
-                for (int b = 0; b < 3; ++b) H[3 * a + b] = __fma_rn(uj[a], g[b], H[3 * a + b]);
-        }
 #pragma unroll
         for (int i = 0; i < 9; ++i) H[i] = group_sum<LPC>(H[i]);
-        if (live && j == 0) {
+        if (j == 0) {
             const int sl = (int)(c - c0);
 #pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                SH[9 * sl + i] = H[i];
-                store_once(A.H + i * A.ncells + c, H[i]);
+            for (int i = 0; i < 9; ++i) SH[9 * sl + i] = H[i];
+            if (A.keep) {
+#pragma unroll
+                for (int i = 0; i < 9; ++i) store_once(A.H + i * A.ncells + c, H[i]);
             }
             SJ[sl] = det_ap_im1(H) + 1.0;
         }
     }
     __syncthreads();
-    auto jbar_of = [&](int64_t r) {
-        double jb = 0.0;
-        for (int64_t k = B.fcell_sub[r]; k < B.fcell_sub[r + 1]; ++k) jb = jb + SJ[k - c0] * A.volume[k];
-        return jb / B.fcell_volume[r];
-    };
     // (2) H-bar, its stress, the dual-pressure term
-    for (int64_t s = c0 + lane; s < c1; s += 64) {
+    for (int64_t s = c0 + tid; s < c1; s += nt) {
         const int sl = (int)(s - c0);
-        const double jbar = jbar_of(B.sub_fcell[s]);
+        const int64_t r = B.sub_fcell[s];
+        const int k0 = (int)(B.fcell_sub[r] - c0), k1 = (int)(B.fcell_sub[r + 1] - c0);
+        double jbar = 0.0;
+        for (int k = k0; k < k1; ++k) jbar = jbar + SJ[k] * SP[9 * k];
+        jbar = jbar / B.fcell_volume[r];
         double H[9], Hb[9], Pb[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) H[i] = SH[9 * sl + i];
         const double ratio = jbar / SJ[sl];
-        if (fabs(ratio - 1.0) < 3.0 * kEps) {
+        const double js = cbrt(ratio);
+        const bool same = fabs(ratio - 1.0) < 3.0 * kEps;
 #pragma unroll
-            for (int i = 0; i < 9; ++i) Hb[i] = H[i];
-        } else {
-            const double js = cbrt(ratio);
-#pragma unroll
-            for (int i = 0; i < 9; ++i) Hb[i] = H[i] * js;
-            Hb[0] += js - 1.0;
-            Hb[4] += js - 1.0;
-            Hb[8] += js - 1.0;
+        for (int i = 0; i < 9; ++i) Hb[i] = same ? H[i] : H[i] * js;
+        const double add = same ? 0.0 : js - 1.0;
+        if (!same) {
+            Hb[0] += add;
+            Hb[4] += add;
+            Hb[8] += add;
         }
         double snp1 = 0.0, aux = 0.0;
         const double sn = load_state<KIND>(A.state_n, s);
@@ -861,25 +884,24 @@ __global__ __launch_bounds__(64) void k_fbar_tile(FbarTileArgs B) {
         store_state<KIND>(A.state_np1, s, snp1, aux);
 #pragma unroll
         for (int i = 0; i < 9; ++i) SPb[9 * sl + i] = Pb[i];
-        const double js = cbrt(jbar / SJ[sl]);
         const double djb = js / (3.0 * jbar);
         double ph = 0.0;
 #pragma unroll
         for (int i = 0; i < 9; ++i) ph += Pb[i] * H[i];
         const double tr = Pb[0] + Pb[4] + Pb[8];
-        SD[sl] = djb * A.volume[s] * (ph + tr);
+        SD[sl] = djb * SP[9 * sl] * (ph + tr);
+        SP[9 * sl + 1] = js;
     }
     __syncthreads();
     // (3) the dual pressure and the un-barred stress
-    for (int64_t s = c0 + lane; s < c1; s += 64) {
+    for (int64_t s = c0 + tid; s < c1; s += nt) {
         const int sl = (int)(s - c0);
         const int64_t r = B.sub_fcell[s];
-        const double jbar = jbar_of(r);
+        const int k0 = (int)(B.fcell_sub[r] - c0), k1 = (int)(B.fcell_sub[r + 1] - c0);
         double dual = 0.0;
-        for (int64_t k = B.fcell_sub[r]; k < B.fcell_sub[r + 1]; ++k) dual += SD[k - c0];
+        for (int k = k0; k < k1; ++k) dual += SD[k];
         dual = dual / B.fcell_volume[r];
-        const double Js = SJ[sl];
-        const double js = cbrt(jbar / Js);
+        const double Js = SJ[sl], js = SP[9 * sl + 1];
         double Fm[9], Fi[9], Pb[9], pf = 0.0;
 #pragma unroll
         for (int i = 0; i < 9; ++i) {
@@ -900,37 +922,32 @@ __global__ __launch_bounds__(64) void k_fbar_tile(FbarTileArgs B) {
             for (int b = 0; b < 3; ++b) {
                 const double p = Pb[3 * a + b] * js + scalar * Fi[3 * b + a];
                 SP[9 * sl + 3 * a + b] = p;
-                store_once(A.P + (3 * a + b) * A.ncells + s, p);
+                if (A.keep) store_once(A.P + (3 * a + b) * A.ncells + s, p);
             }
     }
     __syncthreads();
     // (4) entry forces
-    constexpr int BQ = 4;  // entries per lane whose loads are issued together
+    double *Fw = F + 3 * (size_t)A.maxtn * (tid / 64);
     for (int64_t cb = c0; cb < c1; cb += G) {
         const int64_t c = cb + grp;
-        if (c >= c1) continue;
+        if (c >= c1) break;
         const int sl = (int)(c - c0);
         double P[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) P[i] = SP[9 * sl + i];
         const double mv = -A.volume[c];
-        const int64_t t0 = A.start[c], t1 = A.start[c + 1];
-        for (int64_t eb = t0 + j; eb < t1; eb += BQ * LPC) {
-            int li[BQ];
-            double g[BQ][3];
+        const int64_t s0 = A.start[c], s1 = A.start[c + 1];
+        for (int64_t e = s0 + j; e < s1; e += K * LPC) {
+            int li[K];
+            double g[K][3];
+            entries(e, s1, li, g);
 #pragma unroll
-            for (int r = 0; r < BQ; ++r) {
-                const int64_t e = min(eb + r * LPC, t1 - 1);
-                li[r] = A.lidx[e];
-                ld3(A.dphi, e, g[r]);
-            }
-#pragma unroll
-            for (int r = 0; r < BQ; ++r) {
-                if (eb + r * LPC < t1) {
+            for (int r = 0; r < K; ++r) {
+                if (e + r * LPC < s1) {
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
                         const double fa = mv * dot3(P[3 * a], g[r][0], P[3 * a + 1], g[r][1], P[3 * a + 2], g[r][2]);
-                        __hip_atomic_fetch_add(F + 3 * li[r] + a, fa, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                        __hip_atomic_fetch_add(Fw + 3 * li[r] + a, fa, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     }
                 }
             }
@@ -938,7 +955,11 @@ __global__ __launch_bounds__(64) void k_fbar_tile(FbarTileArgs B) {
     }
     __syncthreads();
     double *dst = A.slots + 3 * (int64_t)tb;
-    for (int k = lane; k < 3 * tn; k += 64) dst[k] = F[k];
+    for (int k = tid; k < 3 * tn; k += nt) {
+        double f = F[k];
+        for (int q = 1; q < nw; ++q) f += F[3 * (size_t)A.maxtn * q + k];
+        dst[k] = f;
+    }
 }
 
 struct RkSlotNodeArgs {
@@ -1733,45 +1754,55 @@ static void launch_rk_tile(const RkTileArgs &T, int lpc, dim3 g, size_t lds, hip
     else hipLaunchKernelGGL((k_rk_tile<KIND, 16, 8>), g, dim3(64), lds, s, T);
 }
 
-static RkTileArgs rk_tile_args(Ctx &c) {
+static RkTileArgs rk_tile_args(Ctx &c, bool keep, bool raw) {
     CellData &D = c.cells;
     const int64_t nbt = ((D.ntiles + kNumXcd - 1) / kNumXcd) * kNumXcd;
     return RkTileArgs{D.ncells, D.ntiles, nbt, D.tile_maxtn, D.start.p, D.lidx.p, D.dphi.p,
                       D.volume.p, c.u.p, D.t_nstart.p, D.t_node.p, D.t_cstart.p, D.slots.p, c.Hnp1().p, c.Pnp1().p,
                       c.state[1 - c.state_np1].p, c.state[c.state_np1].p, c.mat.params(),
                       c.has_fields ? c.elem_lambda.p : nullptr, c.has_fields ? c.elem_mu.p : nullptr,
-                      c.mat.rate_form() ? c.Hn().p : nullptr, c.mat.rate_form() ? c.Pn().p : nullptr, c.rate_dt};
+                      c.mat.rate_form() ? c.Hn().p : nullptr, c.mat.rate_form() ? c.Pn().p : nullptr, c.rate_dt,
+                      keep || c.mat.rate_form(), raw, c.n_dof, c.v.p, c.a.p, c.has_fixed ? c.fixed.p : nullptr};
 }
 
 template <int KIND>
-static void launch_fbar_tile(const FbarTileArgs &B, int lpc, dim3 g, size_t lds, hipStream_t s) {
-    if (lpc == 4) hipLaunchKernelGGL((k_fbar_tile<KIND, 4>), g, dim3(64), lds, s, B);
-    else if (lpc == 8) hipLaunchKernelGGL((k_fbar_tile<KIND, 8>), g, dim3(64), lds, s, B);
-    else hipLaunchKernelGGL((k_fbar_tile<KIND, 16>), g, dim3(64), lds, s, B);
+static void launch_fbar_tile(const FbarTileArgs &B, int lpc, dim3 g, int threads, size_t lds, hipStream_t s) {
+    if (lpc == 4) hipLaunchKernelGGL((k_fbar_tile<KIND, 4>), g, dim3(threads), lds, s, B);
+    else if (lpc == 8) hipLaunchKernelGGL((k_fbar_tile<KIND, 8>), g, dim3(threads), lds, s, B);
+    else hipLaunchKernelGGL((k_fbar_tile<KIND, 16>), g, dim3(threads), lds, s, B);
 }
 
-static void rk_fbar_tiles(Ctx &c) {
+static void rk_fbar_tiles(Ctx &c, bool keep, bool raw) {
     CellData &D = c.cells;
     if (D.ntiles == 0) return;
-    const FbarTileArgs B{rk_tile_args(c), D.t_fstart.p, D.fcell_sub.p, D.fcell_volume.p, D.sub_fcell.p,
+    const FbarTileArgs B{rk_tile_args(c, keep, raw), D.t_fstart.p, D.fcell_sub.p, D.fcell_volume.p, D.sub_fcell.p,
                          std::max(D.tile_maxsub, 1)};
     const dim3 g((unsigned)B.T.nblocks);
-    const size_t lds = (size_t)tile_lds(D.tile_maxtn, D.tile_maxsub, true);
     const int lpc = D.tile_lpc;
+    // Meshes of few tiles: as many waves as give every subcell of the largest tile a lane group, up
+    // to four and to what the LDS budget leaves for their rows (10 steps of 719 tiles in turn, 1 /
+    // 3 waves: 91 / 83 us; 20 steps of 2183 tiles: 303 / 381 us)
+    size_t lds = (size_t)tile_lds(D.tile_maxtn, D.tile_maxsub, true);
+    const size_t row = 24 * (size_t)std::max(D.tile_maxtn, 1);
+    int waves = 1;
+    while (D.ntiles <= 1024 && waves < 4 && waves * 64 / lpc < D.tile_maxsub && lds + row <= (size_t)kTileLdsMax) {
+        ++waves;
+        lds += row;
+    }
     switch (c.mat.kind) {
-        case APHIP_LINEAR_ELASTIC: launch_fbar_tile<APHIP_LINEAR_ELASTIC>(B, lpc, g, lds, c.stream); break;
-        case APHIP_NEO_HOOKEAN: launch_fbar_tile<APHIP_NEO_HOOKEAN>(B, lpc, g, lds, c.stream); break;
-        case APHIP_J2: launch_fbar_tile<APHIP_J2>(B, lpc, g, lds, c.stream); break;
-        case APHIP_SVK: launch_fbar_tile<APHIP_SVK>(B, lpc, g, lds, c.stream); break;
+        case APHIP_LINEAR_ELASTIC: launch_fbar_tile<APHIP_LINEAR_ELASTIC>(B, lpc, g, 64 * waves, lds, c.stream); break;
+        case APHIP_NEO_HOOKEAN: launch_fbar_tile<APHIP_NEO_HOOKEAN>(B, lpc, g, 64 * waves, lds, c.stream); break;
+        case APHIP_J2: launch_fbar_tile<APHIP_J2>(B, lpc, g, 64 * waves, lds, c.stream); break;
+        case APHIP_SVK: launch_fbar_tile<APHIP_SVK>(B, lpc, g, 64 * waves, lds, c.stream); break;
         default: throw Error(APHIP_ERR_UNSUPPORTED, "F-bar takes the linear elastic, neo-Hookean, J2 and SVK materials");
     }
     APHIP_HIP(hipGetLastError());
 }
 
-static void rk_tile_force(Ctx &c) {
+static void rk_tile_force(Ctx &c, bool keep, bool raw) {
     CellData &D = c.cells;
     if (D.ntiles == 0) return;
-    const RkTileArgs T = rk_tile_args(c);
+    const RkTileArgs T = rk_tile_args(c, keep, raw);
     const dim3 g((unsigned)T.nblocks);
     const size_t lds = 48 * (size_t)std::max(D.tile_maxtn, 1);
     const int lpc = D.tile_lpc;
@@ -1801,15 +1832,17 @@ bool rk_fused(const Ctx &c) {
            !c.tiles.orphans && c.nn <= kFusedNodes;
 }
 
+bool rk_takes_predictor(const Ctx &c) { return rk_fused(c) || (c.cells.ready && c.cells.nodal && !c.node_dt.p); }
+
 void rk_cell_force(Ctx &c, bool keep, bool raw, bool keep_local) {
     CellData &D = c.cells;
     if (D.ncells == 0) return;  // no cells: f_local stays zero
     if (D.fbar) {
-        rk_fbar_tiles(c);
+        rk_fbar_tiles(c, keep, raw);
         return;
     }
     if (D.nodal) {
-        rk_tile_force(c);
+        rk_tile_force(c, keep, raw);
         return;
     }
     // physical displacement = Phi d (ExplicitSolver::ComputeForce, Explicit.cpp:148-152), then

@@ -186,3 +186,31 @@ def test_fbar_tiles_are_deterministic_and_size_independent(gpu_available, monkey
     for g, r in ((u, ref.u), (v, ref.v), (f, ref.f)):
         assert rel_err(g, r) < 1e-10
     assert rel_err(P, ref.P[es]) < 1e-10 and rel_err(st, ref.state[es]) < 1e-10
+
+
+@pytest.mark.parametrize("kind", [A.NEO_HOOKEAN, A.J2], ids=["nh", "j2"])
+def test_fbar_waves_per_tile(gpu_available, kind):
+    """Meshes of at most 1024 cell tiles give a tile several waves, larger ones one: a block
+    alone and as one of four far apart moves the same.  Bar: entry forces summed in another
+    order, about 1e-14 of the largest a step and up to 1e2 of cancellation, over five steps."""
+    Xh, hx = _thex(6, 23)
+    nn, ne = len(Xh), len(hx)
+    dt = 0.3 * M.stable_dt_estimate(Xh, hx, E, NU, RHO)
+    v0 = np.random.default_rng(3).uniform(-1.0, 1.0, Xh.shape)
+    fixed = np.zeros(Xh.shape, dtype=np.uint8)
+    fixed[Xh[:, 2] < 0.01] = (1, 0, 1)
+    out = []
+    for copies in (1, 4):
+        print(f"F-bar waves kind={kind}: {copies} x {ne} subcells", flush=True)
+        k = np.arange(copies)[:, None, None]
+        X = (Xh[None] + 3.0 * k * np.array([1.0, 0.0, 0.0])).reshape(-1, 3)
+        with _gpu(X, (hx[None] + nn * k).reshape(-1, hx.shape[1]), kind, 0, True) as s:
+            s.compute_mass()
+            s.set_fixed(np.tile(fixed, (copies, 1)))
+            s.set_field(A.FIELD_V, np.tile(v0, (copies, 1)))
+            s.initialize()
+            s.step(dt, 1)
+            s.step(dt, 4)
+            out.append([s.get(f)[:nn] for f in (A.FIELD_U, A.FIELD_V, A.FIELD_F)] + [s.get(A.FIELD_P)[:ne]])
+    for i, (a, b) in enumerate(zip(*out)):
+        assert rel_err(a, b) < 1e-11, i
