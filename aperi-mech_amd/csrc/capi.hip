@@ -348,12 +348,10 @@ static bool steps_on_patches(Ctx &c) {
 static void default_tiling(Ctx &c) {
     if (c.ne == 0 || (c.flags & APHIP_FLAG_TWO_PASS)) return;
     if (c.etype == APHIP_TET4) {
-        // 1024-element tiles (fewer shared nodes) when the mesh's tiles fit a CU's LDS
-        try {
-            tile_build(c, 1024, 1024);
-        } catch (const Error &) {
-            tile_build(c, 512, 512);
-        }
+        // 512 elements: two workgroups share a CU, so that one's loads overlap the other's element
+        // phase (a step with inner stores left out, 1024 / 512 / 256 elements: 6M Tet4 208 / 193 /
+        // 196 us, 664k 20.3 / 17.9 / 17.3 with three streams in turn, 197k 7.9 / 6.9 / 6.9)
+        tile_build(c, 512, 512);
     } else {
         tile_build(c, 128, 128);
     }
@@ -477,12 +475,10 @@ static void node_pass(Ctx &c, double dt, int mode, bool more = false, bool raw =
 
 // one step of the explicit loop body (src/Solvers/Explicit.cpp:391-452).  Steps of one
 // aphip_step call hand the next one's predictor on, so nothing between calls can leave it
-// stale (the same arithmetic on the same values: bitwise the same steps).  On the tile path,
-// pred_out has the shared-node pass also store the shared nodes' predicted displacement for
-// the next step, and pred_in has the tile kernel take it instead of predicting from u, v and
-// a (57 B less per shared tile-node row); on smoothed cells the node pass leaves u and v as
-// the next step's predictor would.  keep = false: H, P and f (smoothed cells: a too) are not
-// stored, for the steps of a call after which another follows.
+// stale (the same arithmetic on the same values: bitwise the same steps): pred_out leaves u
+// and v as the next step's predictor would and does not store a, pred_in takes them so (48 B a
+// node read less, 24 written; 6M Tet4: 193 -> 168 us a step).  keep = false: H, P and f
+// (smoothed cells: a too) are not stored, for the steps of a call after which another follows.
 static void step_once(Ctx &c, double dt, bool pred_in, bool pred_out, bool keep) {
     c.state_np1 = 1 - c.state_np1;  // UpdateFieldStates (Explicit.cpp:393)
     c.rate_dt = dt;                 // SetTimeIncrement (ElementTetrahedron4.h:187)

@@ -215,7 +215,6 @@ struct TilePlan {
     DevBuf<uint16_t> lcsr;            // [ntiles * te * npe] local element * npe + slot
     DevBuf<uint16_t> lconn;           // [ne * npe] local node of each element slot
     DevBuf<double> bpart;             // [slots * 3] tile sums of shared nodes
-    DevBuf<double> upred;             // [nb * 3] shared nodes' predicted displacement for the next step
     DevBuf<int32_t> bstart;           // [nb + 1] slot range of each shared node
     DevBuf<double> zero;              // [8] zeros: stands in for absent optional arrays
     DevBuf<int32_t> meta;             // [ntiles * 8] packed per-tile scalars of the pipelined step
@@ -240,7 +239,7 @@ struct TilePlan {
         lds_bytes = 0;
         for (int &g : stream_grid) g = 0;
         tn_start.release(); tile_e0.release(); tn_ninterior.release(); int_base.release(); tn_node.release(); tn_csr.release();
-        tn_bdst.release(); lcsr.release(); lconn.release(); bpart.release(); bstart.release(); upred.release();
+        tn_bdst.release(); lcsr.release(); lconn.release(); bpart.release(); bstart.release();
         zero.release(); meta.release();
         tpad = 0;
         tnp_node.release(); tnp_csr.release(); tnp_bdst.release(); lconn_p.release();
@@ -433,9 +432,8 @@ struct TileRun {
     const PhiRows *phi = nullptr;
     // MODE 0: the shared nodes' partial sums stay in their slots, no shared-node pass
     bool park = false;
-    // MODE 2: shared nodes take the displacement predicted by the previous step's shared-node
-    // pass (it must have run with pred_out and the same dt in this same call); pred_out: the
-    // shared-node pass stores that prediction for the next step
+    // MODE 2: u and v hold the step's predicted displacement and v1/2 (the previous step ran
+    // with pred_out and the same dt in this same call); pred_out: leave the next step's there
     bool pred_in = false, pred_out = false;
     // false: H, P (and in MODE 2 f) of this evaluation are not stored: an inner step of one
     // call, whose values the next step overwrites before anything can read them, or a force

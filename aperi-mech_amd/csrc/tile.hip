@@ -93,9 +93,9 @@ struct TileArgs {
     int te, maxtn;
     int max_nint;  // most interior nodes in one tile (Hex8: LDS rows of the corrector data)
     double dt;
-    // mode 2: the shared nodes' displacement predicted by the previous step's shared-node
-    // pass (row first_shared + b at upred[3 b]), or null: predicted here from u, v, a
-    const double *upred;
+    // mode 2, steps of one call: pred: u and v hold this step's predicted displacement and
+    // v1/2 (else predicted here from u, v, a); more: leave the next step's there, and no a
+    int pred, more;
     int64_t first_shared;
     // 0: an inner step of one call, whose H, P and f the next step overwrites unread
     int keep;
@@ -270,18 +270,13 @@ __device__ __forceinline__ void wait_vmem_loads() { __builtin_amdgcn_s_waitcnt(0
 // Updated / semi-Lagrangian node update (ExplicitTimeIntegrator.h:193-226): with the step's
 // increment inc = dt v1/2, u += inc; updated: x_{n+1} = x_n + inc and the increment itself is
 // kept; semi: the accumulated increment acc.
-__device__ __forceinline__ void ul_store(double *u, double *dinc, double *xnp1, int semi, int64_t g, double dt,
-                                         const double *vh, const double *x, const double *acc) {
+__device__ __forceinline__ void ul_store1(double *u, double *dinc, double *xnp1, int semi, int64_t k, double dt,
+                                          double vh, double x, double acc) {
 #pragma clang fp contract(off)
-    double un[3];
-    ld3(u, g, un);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const double inc = dt * vh[d];
-        u[3 * g + d] = un[d] + inc;
-        dinc[3 * g + d] = semi ? acc[d] : inc;
-        if (!semi) xnp1[3 * g + d] = x[d] + inc;
-    }
+    const double inc = dt * vh;
+    u[k] = u[k] + inc;
+    dinc[k] = semi ? acc : inc;
+    if (!semi) xnp1[k] = x + inc;
 }
 
 // Node ln's force f is complete: an interior node is finished and written (MODE 0: f;
@@ -305,7 +300,14 @@ __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L,
             if constexpr (UL) {
                 double x[3];
                 ld3(L.X, ln, x);
-                ul_store(A.u, A.dinc, A.xnp1, A.semi, g, A.dt, vh, x, u1);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) ul_store1(A.u, A.dinc, A.xnp1, A.semi, 3 * g + d, A.dt, vh[d], x[d], u1[d]);
+            } else if (A.more) {
+                double u2[3], v2[3];
+                cd_predict(u1, v1, a1, L.fx[ln], L.DT[ln], v2, u2);
+                st3(A.u, g, u2);
+                st3(A.v, g, v2);
+                return;
             } else {
                 st3(A.u, g, u1);
             }
@@ -373,26 +375,24 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
     }
     double xq[NPT][3], uq[NPT][3], vq[NPT][3], aq[NPT][3], mq[NPT], dq[NPT];
     unsigned fq[NPT];
-    bool pq[NPT];  // shared row with a stored prediction: X and the predicted u only
+    bool pq[NPT];  // shared row of a predicted state: X and u only
 #pragma unroll
     for (int q = 0; q < NPT; ++q) {
         const int64_t g = gq[q];
-        pq[q] = MODE == 2 && A.upred != nullptr && bdq[q] >= 0;
+        pq[q] = MODE == 2 && !UL && A.pred && bdq[q] >= 0;
         ld3(A.X, g, xq[q]);
+        ld3(UL ? A.dinc : A.u, g, uq[q]);
         mq[q] = 1.0;
         dq[q] = A.dt;
-        if (pq[q]) {
-            ld3(A.upred, g - A.first_shared, uq[q]);
-            fq[q] = 0u;
+        fq[q] = 0u;
 #pragma unroll
-            for (int d = 0; d < 3; ++d) vq[q][d] = aq[q][d] = 0.0;
-        } else {
-            ld3(UL ? A.dinc : A.u, g, uq[q]);
+        for (int d = 0; d < 3; ++d) vq[q][d] = aq[q][d] = 0.0;
+        if (!pq[q]) {
             fq[q] = load_fixed(A, g);
             if constexpr (MODE >= 1) mq[q] = A.mass[g];
             if constexpr (MODE == 2) {
                 ld3(A.v, g, vq[q]);
-                ld3(A.a, g, aq[q]);
+                if (UL || !A.pred) ld3(A.a, g, aq[q]);
                 dq[q] = load_node_dt(A, g);
             }
         }
@@ -428,10 +428,9 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
     }
     // Hex8 keeps the corrector data of interior nodes only (the only ones it finishes);
     // Tet4 writes it for every node (measured faster with its 512-element tiles).
-    // pre: u is already the predicted displacement (a shared row; the corrector data
-    // written for it are never read)
+    // (the corrector data written for a shared row are never read)
     auto stage = [&](int ln, uint32_t csr, int32_t bdst, const double *x, const double *u, const double *v,
-                     const double *a, unsigned fx, double mm, double nd, bool pre) {
+                     const double *a, unsigned fx, double mm, double nd) {
         L.csr[ln] = csr;
         L.bdst[ln] = bdst;
         st3(L.X, ln, x);
@@ -442,8 +441,8 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
             L.DT[ln] = nd;
         }
         if constexpr (MODE == 2) {
-            double vh[3] = {0.0, 0.0, 0.0}, u1[3] = {u[0], u[1], u[2]};
-            if (!pre) stage_predict<UL>(A, u, v, a, fx, nd, vh, u1);
+            double vh[3] = {v[0], v[1], v[2]}, u1[3] = {u[0], u[1], u[2]};
+            if (UL || !A.pred) stage_predict<UL>(A, u, v, a, fx, nd, vh, u1);
             st3(L.U, ln, u1);
             if (interior) st3(L.V, ln, vh);
         } else if constexpr (!GATHER) {
@@ -453,7 +452,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
 #pragma unroll
     for (int q = 0; q < NPT; ++q) {
         const int ln = tid + q * (int)blockDim.x;
-        if (ln < tn) stage(ln, csrq[q], bdq[q], xq[q], uq[q], vq[q], aq[q], fq[q], mq[q], dq[q], pq[q]);
+        if (ln < tn) stage(ln, csrq[q], bdq[q], xq[q], uq[q], vq[q], aq[q], fq[q], mq[q], dq[q]);
     }
     // rows past NPT x blockDim (tiles with unusually many nodes)
     for (int ln = tid + NPT * (int)blockDim.x; ln < tn; ln += blockDim.x) {
@@ -469,7 +468,7 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
             ld3(A.a, g, a);
             nd = load_node_dt(A, g);
         }
-        stage(ln, A.tn_csr[tb + ln], A.tn_bdst[tb + ln], x, u, v, a, fx, mm, nd, false);
+        stage(ln, A.tn_csr[tb + ln], A.tn_bdst[tb + ln], x, u, v, a, fx, mm, nd);
     }
     if constexpr (GATHER) stage_phi(A, L, t, tn);
     // Every load of the wave completes here, on every path (a wave whose lanes all
@@ -636,7 +635,6 @@ __global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_
     double x0[3], u0[3], v0[3], a0[3], m0 = 1.0, d0 = A.dt;
     unsigned f0 = 0u;
     int32_t bd0 = 0;
-    bool pre0 = false;
     uint4 en0{};
     uint32_t csr0 = 0;
     if (wave0 < A.tpad) {
@@ -647,19 +645,16 @@ __global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_
             en0 = A.hx_first[row];
             csr0 = A.hx_csr[row];
         }
-        pre0 = MODE == 2 && A.upred != nullptr && bd0 >= 0;  // X and the predicted u only
         ld3(A.X, g0, x0);
-        if (pre0) {
-            ld3(A.upred, g0 - A.first_shared, u0);
+        ld3(UL ? A.dinc : A.u, g0, u0);
 #pragma unroll
-            for (int d = 0; d < 3; ++d) v0[d] = a0[d] = 0.0;
-        } else {
-            ld3(UL ? A.dinc : A.u, g0, u0);
+        for (int d = 0; d < 3; ++d) v0[d] = a0[d] = 0.0;
+        if (!(MODE == 2 && !UL && A.pred && bd0 >= 0)) {  // (a shared row of a predicted state: X and u only)
             f0 = load_fixed(A, g0);
             if constexpr (MODE >= 1) m0 = A.mass[g0];
             if constexpr (MODE == 2) {
                 ld3(A.v, g0, v0);
-                ld3(A.a, g0, a0);
+                if (UL || !A.pred) ld3(A.a, g0, a0);
                 d0 = load_node_dt(A, g0);
             }
         }
@@ -671,7 +666,7 @@ __global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_
     const int nel = A.tile_e0[t + 1] - (int)te0;
     if (tid < 3) L.F[kHexRow * rw + tid] = 0.0;  // the row of padding entries
     auto stage = [&](int ln, uint4 en, uint32_t csr, int32_t bdst, const double *x, const double *u, const double *v,
-                     const double *a, unsigned fx, double mm, double nd, bool pre) {
+                     const double *a, unsigned fx, double mm, double nd) {
         if constexpr (!MULTI) {
             reinterpret_cast<uint4 *>(L.ent)[ln] = en;
             L.csr[ln] = csr;
@@ -684,15 +679,15 @@ __global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_
             L.DT[ln] = nd;
         }
         if constexpr (MODE == 2) {
-            double vh[3] = {0.0, 0.0, 0.0}, u1[3] = {u[0], u[1], u[2]};
-            if (!pre) stage_predict<UL>(A, u, v, a, fx, nd, vh, u1);
+            double vh[3] = {v[0], v[1], v[2]}, u1[3] = {u[0], u[1], u[2]};
+            if (UL || !A.pred) stage_predict<UL>(A, u, v, a, fx, nd, vh, u1);
             st3(L.U, ln, u1);
             if (ln < nint) st3(L.V, ln, vh);
         } else {
             st3(L.U, ln, u);
         }
     };
-    if (tid < tn) stage(tid, en0, csr0, bd0, x0, u0, v0, a0, f0, m0, d0, pre0);
+    if (tid < tn) stage(tid, en0, csr0, bd0, x0, u0, v0, a0, f0, m0, d0);
     for (int ln = tid + nt; ln < tn; ln += nt) {  // tiles with more nodes than threads
         const int64_t row = t * (int64_t)A.tpad + ln, g = A.tnp_node[row];
         double x[3], u[3], v[3], a[3], mm = 1.0, nd = A.dt;
@@ -706,7 +701,7 @@ __global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_
             nd = load_node_dt(A, g);
         }
         stage(ln, MULTI ? uint4{} : A.hx_first[row], MULTI ? 0u : A.hx_csr[row], A.tnp_bdst[row], x, u, v, a, fx, mm,
-              nd, false);
+              nd);
     }
     __syncthreads();
 
@@ -1099,7 +1094,7 @@ struct BoundArgs {
     const double *node_dt;
     const double *zero;  // 8 zero doubles: stands in for an absent optional array
     double dt;
-    double *upred;  // mode 2: store the next step's predicted displacement (same dt), or null
+    int pred, more;  // as in TileArgs
     int keep;       // 0: an inner step, f is not stored
     // updated / semi-Lagrangian: the configuration integrated over, and as in TileArgs
     const double *xn;
@@ -1107,68 +1102,64 @@ struct BoundArgs {
     int semi;
 };
 
+// One thread per component of a node: a wave's accesses to u, v, a, f and (the slots of
+// consecutive nodes being consecutive) to the slots are contiguous runs.  Bound by memory; one
+// thread per node, three strided accesses each, took 36 us where this took 34.8 (6M Tet4 in tiles of
+// 512: memory-bound there, 73k Tet4: 14.1 -> 12.2 us a step alone), and 23.1 once the steps of a call left
+// the next predictor in u and v instead of u, v, a and a copy of the predicted displacement.
+constexpr int kBoundNodes = 64;  // nodes per workgroup
 template <int MODE, bool UL = false>
-__global__ __launch_bounds__(256) void k_boundary(BoundArgs A) {
-    const int64_t b_raw = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(3 * kBoundNodes) void k_boundary(BoundArgs A) {
+#pragma clang fp contract(off)
+    const int64_t b_raw = (int64_t)blockIdx.x * kBoundNodes + threadIdx.x / 3;
+    const int d = threadIdx.x % 3;
     const bool live = b_raw < A.nb;
     const int64_t b = live ? b_raw : A.nb - 1;  // idle lanes redo the last node and store nothing
-    const int64_t g = A.first + b;
+    const int64_t g = A.first + b, k = 3 * g + d;
     const int32_t s0 = A.bstart[b], s1 = A.bstart[b + 1];
     // node data first: independent of the slot sums, so its loads overlap them
-    double u[3], v[3], a[3], m = 1.0, dt = A.dt;
-    unsigned fx = 0u;
+    double u = 0.0, v = 0.0, a = 0.0, m = 1.0, dt = A.dt;
+    bool fx = false;
     if constexpr (MODE >= 1) m = A.mass[g];
     if constexpr (MODE == 2) {
-        ld3(A.u, g, u);
-        ld3(A.v, g, v);
-        ld3(A.a, g, a);
+        u = A.u[k];
+        v = A.v[k];
+        if (UL || !A.pred) a = A.a[k];
         const uint8_t *pf = A.fixed ? A.fixed : reinterpret_cast<const uint8_t *>(A.zero);
         const double *pd = A.node_dt ? A.node_dt : A.zero;
         const unsigned f8 = pf[A.fixed ? g : 0];
         const double d8 = pd[A.node_dt ? g : 0];
-        fx = A.fixed ? f8 : 0u;
+        fx = A.fixed && (f8 & (1u << d));
         dt = A.node_dt ? d8 : A.dt;
     }
     // slot sums in ascending tile order, four slots' loads at a time (clamped; an
     // absent slot adds zero)
-    double f[3] = {0.0, 0.0, 0.0};
+    double f = 0.0;
     for (int32_t sb = s0; sb < s1; sb += 4) {
-        double p[4][3];
+        double p[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ld3(A.bpart, min(sb + r, s1 - 1), p[r]);
+        for (int r = 0; r < 4; ++r) p[r] = A.bpart[3 * (int64_t)min(sb + r, s1 - 1) + d];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const bool in = sb + r < s1;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) f[d] += in ? p[r][d] : 0.0;
-        }
+        for (int r = 0; r < 4; ++r) f += sb + r < s1 ? p[r] : 0.0;
     }
     if (!live) return;
-    if (MODE != 2 || A.keep) st3(A.f, g, f);
+    if (MODE != 2 || A.keep) A.f[k] = f;
     if constexpr (MODE == 1) {
-        const double acc[3] = {f[0] / m, f[1] / m, f[2] / m};
-        st3(A.a, g, acc);
+        A.a[k] = f / m;
     } else if constexpr (MODE == 2) {
-        double vh[3], u1[3], a1[3], v1[3];
-        cd_predict(u, v, a, fx, dt, vh, u1);
-        cd_correct(f, m, fx, dt, vh, a1, v1);
-        if constexpr (UL) {
-#pragma clang fp contract(off)
-            double x[3], acc[3];
-            ld3(A.xn, g, x);
-            ld3(A.dinc, g, acc);
-#pragma unroll
-            for (int d = 0; d < 3; ++d) acc[d] = acc[d] + dt * vh[d];
-            ul_store(A.u, A.dinc, A.xnp1, A.semi, g, dt, vh, x, acc);
+        double vh = v, u1 = u, a1, v1;
+        if (UL || !A.pred) cd_predict1(u, v, a, fx, dt, vh, u1);
+        cd_correct1(f, m, fx, dt, vh, a1, v1);
+        if constexpr (UL) ul_store1(A.u, A.dinc, A.xnp1, A.semi, k, dt, vh, A.xn[k], A.dinc[k] + dt * vh);
+        if (!UL && A.more) {
+            double vh2, u2;
+            cd_predict1(u1, v1, a1, fx, dt, vh2, u2);
+            A.u[k] = u2;
+            A.v[k] = vh2;
         } else {
-            st3(A.u, g, u1);
-        }
-        st3(A.v, g, v1);
-        st3(A.a, g, a1);
-        if (A.upred) {  // the predictor of the next step from the values just stored
-            double vh2[3], u2[3];
-            cd_predict(u1, v1, a1, fx, dt, vh2, u2);
-            st3(A.upred, b, u2);
+            if constexpr (!UL) A.u[k] = u1;
+            A.v[k] = v1;
+            A.a[k] = a1;
         }
     }
 }
@@ -1236,6 +1227,10 @@ bool stream_eligible(const Ctx &c) {
     return P.use_stream && c.npe == 4 && P.te == P.threads && P.threads <= 256 && P.maxtn <= P.threads &&
            stream_lds_bytes(P.te, P.maxtn) <= 160 * 1024 && 72 * c.ne < lim && 24 * c.nn < lim &&
            24 * P.nslot < lim;
+}
+
+bool stream_kind(int kind) {
+    return kind == APHIP_LINEAR_ELASTIC || kind == APHIP_NEO_HOOKEAN || kind == APHIP_J2 || kind == APHIP_SVK;
 }
 
 template <int NPE, int MODE>
@@ -1482,7 +1477,6 @@ void tile_build(Ctx &c, int te, int threads) {
     }
     P.nslot = bstart[nb];
     P.bpart.alloc(3 * std::max<int64_t>(1, (int64_t)bstart[nb]));
-    P.upred.alloc(3 * std::max<int64_t>(1, nb));
     P.bstart.upload(bstart.data(), bstart.size(), c.stream);
     P.zero.alloc(8);
     P.zero.zero(c.stream);
@@ -1531,7 +1525,9 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     APHIP_REQUIRE(mode == 0 || (run.u_in == nullptr && run.f_out == nullptr && !run.phi && !run.park),
                   "displacement / force arrays only in force mode");
     APHIP_REQUIRE(mode == 2 || !(run.pred_in || run.pred_out), "predicted displacements only in step mode");
-    const bool pred_in = run.pred_in && P.nb > 0, pred_out = run.pred_out && P.nb > 0;
+    // (the pipelined kernel predicts from u, v and a in every step)
+    const bool chain = !(c.npe == 4 && stream_eligible(c) && stream_kind(c.mat.kind));
+    const bool pred_in = run.pred_in && chain, pred_out = run.pred_out && chain;
     // smoothed Hex8 cells have a B of their own (a smoothed Tet4's is its gradient)
     const bool cells8 = c.npe == 8 && c.cells.ready;
     APHIP_REQUIRE(!run.phi || c.npe == 4, "Phi rows are staged by Tet4 tiles");
@@ -1591,7 +1587,8 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     A.maxtn = P.maxtn;
     A.max_nint = P.max_nint;
     A.dt = dt;
-    A.upred = pred_in ? P.upred.p : nullptr;
+    A.pred = pred_in;
+    A.more = pred_out;
     A.first_shared = P.n_interior;
     A.cell_marker = c.cells.ready;
     A.phi = run.phi ? *run.phi : PhiRows{};
@@ -1615,14 +1612,14 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     if (P.nb > 0 && !run.park) {
         BoundArgs B{P.nb, P.n_interior, P.bstart.p, P.bpart.p, c.u.p, c.v.p, c.a.p, A.f, c.mass.p,
                     c.has_fixed ? c.fixed.p : nullptr, c.node_dt.p, P.zero.p, dt,
-                    pred_out ? P.upred.p : nullptr, A.keep,
+                    A.pred, A.more, A.keep,
                     A.X, A.dinc, A.xnp1, A.semi};
-        const dim3 grid((unsigned)((P.nb + 255) / 256));
+        const dim3 grid((unsigned)((P.nb + kBoundNodes - 1) / kBoundNodes)), block(3 * kBoundNodes);
         prof_begin(c, 2);
-        if (mode == 0) hipLaunchKernelGGL(k_boundary<0>, grid, dim3(256), 0, c.stream, B);
-        else if (mode == 1) hipLaunchKernelGGL(k_boundary<1>, grid, dim3(256), 0, c.stream, B);
-        else if (ul) hipLaunchKernelGGL((k_boundary<2, true>), grid, dim3(256), 0, c.stream, B);
-        else hipLaunchKernelGGL(k_boundary<2>, grid, dim3(256), 0, c.stream, B);
+        if (mode == 0) hipLaunchKernelGGL(k_boundary<0>, grid, block, 0, c.stream, B);
+        else if (mode == 1) hipLaunchKernelGGL(k_boundary<1>, grid, block, 0, c.stream, B);
+        else if (ul) hipLaunchKernelGGL((k_boundary<2, true>), grid, block, 0, c.stream, B);
+        else hipLaunchKernelGGL(k_boundary<2>, grid, block, 0, c.stream, B);
         APHIP_HIP(hipGetLastError());
         prof_end(c, 2);
     }
