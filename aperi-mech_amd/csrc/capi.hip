@@ -434,6 +434,7 @@ static void setup_mesh(Ctx &c, int32_t elem_type, int64_t n_nodes, const double 
         b->zero(c.stream);
     }
     c.pm_eig.alloc(3 * n_nodes);  // the power method's eigenvector, kept between its calls
+    c.pm_total.alloc(1);
     c.pm_l.alloc(n_nodes);        // and its max edge lengths
     c.H.alloc(9 * std::max<int64_t>(n_elem, 1));
     c.P.alloc(9 * std::max<int64_t>(n_elem, 1));
@@ -532,11 +533,13 @@ struct PowerMethodResult {
 // the final eigenvector and starts the next call from it (:350-361, :468-469); only the
 // first call after the mesh is set draws the random start.  The force evaluations write H, P
 // and the NP1 state into the call's work buffers (the context's pointers are exchanged for
-// the call and exchanged back on every exit), and u and f are restored afterwards, so the
-// call leaves the simulation state untouched.  The max edge lengths are the context's.
+// the call and exchanged back on every exit).  On the tile path the perturbed displacement and
+// its force are work buffers too; the other paths evaluate on u and f, which are restored
+// afterwards.  Either way the call leaves the simulation state untouched.  The max edge lengths
+// are the context's.
 // Device buffers of one power-method call (internal numbering): the displacement and
-// force on entry, F(u), the iterate, the targets of H / P / state and the norm's partial
-// sums.
+// force on entry (tiles: the perturbed ones), F(u), an unused one (the iterate is the context's
+// eigenvector), the targets of H / P / state and the norm's partial sums.
 struct PowerMethodWork {
     double *u_in, *f_in, *f0, *v, *H, *P, *st, *partial;
 };
@@ -579,8 +582,11 @@ static PowerMethodResult power_method(Ctx &c, const PowerMethodWork &w, double p
                   "All nodes are in the essential boundary set. Cannot run the power method. Use the "
                   "direct_time_stepper instead.");
     const int64_t ns = c.state_count();
-    APHIP_HIP(hipMemcpyAsync(w.u_in, c.u.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
-    APHIP_HIP(hipMemcpyAsync(w.f_in, c.f.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    const bool tiles = use_tiles(c);
+    if (!tiles) {
+        APHIP_HIP(hipMemcpyAsync(w.u_in, c.u.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+        APHIP_HIP(hipMemcpyAsync(w.f_in, c.f.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    }
     Redirect redirect;
     if (c.ne) {
         redirect.to(c.Hnp1().p, w.H);
@@ -593,12 +599,24 @@ static PowerMethodResult power_method(Ctx &c, const PowerMethodWork &w, double p
         c.pm_l_valid = true;
     }
     const double *l = c.pm_l.p;
-    if (c.pm_eig_valid)
-        APHIP_HIP(hipMemcpyAsync(w.v, c.pm_eig.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
-    else
-        pm_start(c, c.d_node_iperm.p, seed, eps, l, w.v);
-    internal_force_eval(c, false);  // F(u)
-    APHIP_HIP(hipMemcpyAsync(w.f0, c.f.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    double *v = c.pm_eig.p;
+    if (!c.pm_eig_valid) {
+        pm_start(c, c.d_node_iperm.p, seed, eps, l, v);
+        c.pm_norm = 1.0;
+    }
+    c.pm_eig_valid = false;  // (until this call's iterate is complete)
+    TileRun eval;
+    eval.keep = false;
+    if (tiles) {  // F(u)
+        eval.f_out = w.f0;
+        tile_run(c, 0.0, 0, eval);
+        eval.u_in = w.u_in;
+        eval.f_out = w.f_in;
+        eval.park = true;
+    } else {
+        internal_force_eval(c, false);
+        APHIP_HIP(hipMemcpyAsync(w.f0, c.f.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    }
 
     constexpr int window = 5;
     std::array<double, window> recent{};
@@ -607,10 +625,11 @@ static PowerMethodResult power_method(Ctx &c, const PowerMethodWork &w, double p
     int used = n_iter;
     for (int k = 0; k < n_iter; ++k) {
         dt_n = dt_np1;
-        pm_perturb(c, w.u_in, w.v, l, eps);
-        internal_force_eval(c, false);
-        const double lambda = pm_next(c, w.f0, l, eps, w.v, w.partial);
-        pm_scale(c, lambda, w.v);
+        pm_perturb(c, tiles ? c.u.p : w.u_in, v, c.pm_norm, l, eps, tiles ? w.u_in : c.u.p, w.partial);
+        if (tiles) tile_run(c, 0.0, 0, eval);
+        else internal_force_eval(c, false);
+        const double lambda = pm_next(c, tiles ? w.f_in : c.f.p, tiles, w.f0, l, eps, v, w.partial);
+        c.pm_norm = lambda;
         dt_np1 = 2.0 / std::sqrt(lambda);
         recent[k % window] = dt_np1;
         if (std::fabs(dt_np1 - dt_n) < tol * dt_np1) {
@@ -647,12 +666,12 @@ static PowerMethodResult power_method(Ctx &c, const PowerMethodWork &w, double p
     }
     const double wmin = *std::min_element(recent.begin(), recent.end());
     const double dt = converged ? (oscillating ? wmin : dt_np1) : wmin;
-    APHIP_HIP(hipMemcpyAsync(c.pm_eig.p, w.v, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
     c.pm_eig_valid = true;
-
-    APHIP_HIP(hipMemcpyAsync(c.u.p, w.u_in, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
-    APHIP_HIP(hipMemcpyAsync(c.f.p, w.f_in, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
-    APHIP_HIP(hipStreamSynchronize(c.stream));
+    if (!tiles) {
+        APHIP_HIP(hipMemcpyAsync(c.u.p, w.u_in, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+        APHIP_HIP(hipMemcpyAsync(c.f.p, w.f_in, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+        APHIP_HIP(hipStreamSynchronize(c.stream));
+    }
     return PowerMethodResult{dt, used, converged};
 }
 

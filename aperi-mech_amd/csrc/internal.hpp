@@ -68,6 +68,25 @@ struct DevBuf {
     }
 };
 
+// Host memory that the device writes to.
+template <typename T>
+struct PinnedBuf {
+    T *p = nullptr;
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf &) = delete;
+    PinnedBuf &operator=(const PinnedBuf &) = delete;
+    ~PinnedBuf() {
+        if (p) (void)hipHostFree(p);
+    }
+    void alloc(size_t count) {
+        if (p) return;
+        if (hipHostMalloc(reinterpret_cast<void **>(&p), sizeof(T) * count, hipHostMallocDefault) != hipSuccess) {
+            p = nullptr;
+            throw Error(APHIP_ERR_ALLOC, "hipHostMalloc of " + std::to_string(sizeof(T) * count) + " bytes failed");
+        }
+    }
+};
+
 // Material constants resolved on the host (Lame form).
 struct MaterialConst {
     int kind = -1;
@@ -378,6 +397,8 @@ struct Ctx {
     // depends on X and the connectivity only; a node renumbering permutes it); the work
     // buffers of the allocating entry point, kept between its calls
     DevBuf<double> pm_eig;               // 3 nn, internal numbering, allocated with the mesh
+    double pm_norm = 1.0;                // by which pm_eig is still to be divided
+    PinnedBuf<double> pm_total;          // the norm's square, written by the device; allocated with the mesh
     DevBuf<double> pm_l;                 // nn, internal numbering, allocated with the mesh
     DevBuf<double> pm_work[8];
     bool pm_eig_valid = false;
@@ -485,12 +506,15 @@ void prof_end(Ctx &c, int which);
 // ---- power-method stable increment (power.hip) ----
 void pm_max_edge(Ctx &c, double *l);
 void pm_start(Ctx &c, const int32_t *caller_id, uint64_t seed, double eps, const double *l, double *v);
-void pm_perturb(Ctx &c, const double *u_in, const double *v, const double *l, double eps);
-// doubles of the partial-sum buffer pm_next needs (one per block of nodes, plus the total)
+// u = u_in + v / norm l eps (partial: as for the pm_next that follows)
+void pm_perturb(Ctx &c, const double *u_in, const double *v, double norm, const double *l, double eps, double *u,
+                double *partial);
+// doubles of the partial-sum buffer pm_next needs (one per block of nodes, plus their count)
 int64_t pm_partials(const Ctx &c);
-// v = (f - f0) / (l eps m), returns |v|_2 (partial: pm_partials(c) doubles)
-double pm_next(Ctx &c, const double *f0, const double *l, double eps, double *v, double *partial);
-void pm_scale(Ctx &c, double norm, double *v);  // v /= norm
+// v = (f - f0) / (l eps m), returns |v|_2 (partial: pm_partials(c) doubles); parked: the shared
+// nodes' f stands in the tile plan's slots
+double pm_next(Ctx &c, const double *f, bool parked, const double *f0, const double *l, double eps, double *v,
+               double *partial);
 
 // ---- field transfer with caller device arrays (field.hip) ----
 // dst[i, :] = src[iperm[i], :] / dst[iperm[i], :] = src[i, :], w doubles per entity

@@ -2,7 +2,10 @@
 // PowerMethodProcessor, include/PowerMethodProcessor.h:150-470): per-node max edge
 // length, the seeded start vector, the perturbation u + v l eps, the next iterate
 // (F(u + v l eps) - F(u)) / (l eps m) and its L2 norm (deterministic block partial
-// sums, added in a fixed order by one workgroup).  The driver is in capi.hip.
+// sums, added in a fixed order by the workgroup that ends last).  The driver is in capi.hip.
+// An iteration waits for its norm, so it is a chain of launches and their gaps: three of them
+// (perturb with the previous norm, the element tiles, the next iterate with the shared nodes'
+// sums and the norm, which goes straight to pinned host memory).
 #include <cmath>
 
 #include "internal.hpp"
@@ -53,63 +56,72 @@ __global__ __launch_bounds__(kBlock) void k_pm_start(int64_t nn, const int32_t *
     }
 }
 
-// u_eps = u_in + v l eps on free DOFs, u_in on fixed ones (PerturbDisplacementCoefficients, :230-260).
-__global__ __launch_bounds__(kBlock) void k_pm_perturb(int64_t nn, const double *u_in, const double *v,
-                                                       const double *l, const uint8_t *fixed, double eps, double *u) {
+// u_eps = u_in + v / norm l eps on free DOFs, u_in on fixed ones (PerturbDisplacementCoefficients,
+// :230-260); clears the count of finished workgroups of the k_pm_next that follows.
+__global__ __launch_bounds__(kBlock) void k_pm_perturb(int64_t nn, const double *u_in, const double *v, double norm,
+                                                       const double *l, const uint8_t *fixed, double eps, double *u,
+                                                       unsigned *done) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i == 0) *done = 0;
     if (i >= nn) return;
     const unsigned fx = fixed ? fixed[i] : 0u;
     for (int d = 0; d < 3; ++d) {
         const double ui = u_in[3 * i + d];
-        u[3 * i + d] = (fx & (1u << d)) ? ui : __fma_rn(v[3 * i + d] * l[i], eps, ui);
+        u[3 * i + d] = (fx & (1u << d)) ? ui : __fma_rn(v[3 * i + d] / norm * l[i], eps, ui);
     }
 }
 
 // v = (F1 - F0) / (l eps m) on free DOFs, 0 on fixed ones (ComputeNextEigenvector, :262-330);
-// each block writes the sum of squares of its DOFs (tree order fixed by the block size).
+// each block writes the sum of squares of its DOFs (tree order fixed by the block size), and
+// the last one to end adds them up, thread t partial[t], partial[t + kBlock], ... in turn, then
+// a tree, to *total.  The nodes from first_shared on take F1 as the sum of their slots.
 __global__ __launch_bounds__(kBlock) void k_pm_next(int64_t nn, const double *f1, const double *f0,
                                                     const double *mass, const double *l, const uint8_t *fixed,
-                                                    double eps, double *v, double *partial) {
+                                                    double eps, double *v, double *partial, unsigned *done,
+                                                    double *total, int64_t first_shared, const int32_t *bstart,
+                                                    const double *bpart) {
     __shared__ double red[kBlock];
+    __shared__ bool last;
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     double s = 0.0;
     if (i < nn) {
         const unsigned fx = fixed ? fixed[i] : 0u;
         const double le = l[i] * eps;
+        double f[3] = {0.0, 0.0, 0.0};
+        if (i >= first_shared) {
+            for (int32_t k = bstart[i - first_shared]; k < bstart[i - first_shared + 1]; ++k)
+                for (int d = 0; d < 3; ++d) f[d] += bpart[3 * (int64_t)k + d];
+        } else {
+            for (int d = 0; d < 3; ++d) f[d] = f1[3 * i + d];
+        }
         for (int d = 0; d < 3; ++d) {
-            const double w = (fx & (1u << d)) ? 0.0 : (f1[3 * i + d] - f0[3 * i + d]) / (le * mass[i]);
+            const double w = (fx & (1u << d)) ? 0.0 : (f[d] - f0[3 * i + d]) / (le * mass[i]);
             v[3 * i + d] = w;
             s = __fma_rn(w, w, s);
         }
     }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    auto tree = [&](double x) {
+        red[threadIdx.x] = x;
         __syncthreads();
+        for (int w = kBlock / 2; w > 0; w >>= 1) {
+            if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+            __syncthreads();
+        }
+    };
+    tree(s);
+    if (threadIdx.x == 0) {
+        // (device scope: the workgroups run on several XCDs, each with its own L2)
+        __hip_atomic_store(partial + blockIdx.x, red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-// partial[nb] = the sum of partial[0 .. nb-1] in a fixed order: lane t of one workgroup adds
-// partial[t], partial[t + kSumLanes], ... in turn, then a tree over the lanes
-constexpr int kSumLanes = 1024;
-__global__ __launch_bounds__(kSumLanes) void k_pm_sum(int64_t nb, double *partial) {
-    __shared__ double red[kSumLanes];
-    double s = 0.0;
-    for (int64_t b = threadIdx.x; b < nb; b += kSumLanes) s += partial[b];
-    red[threadIdx.x] = s;
     __syncthreads();
-    for (int w = kSumLanes / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[nb] = red[0];
-}
-
-__global__ __launch_bounds__(kBlock) void k_pm_scale(int64_t n, double norm, double *v) {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) v[i] /= norm;
+    if (!last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    s = 0.0;
+    for (unsigned b = threadIdx.x; b < gridDim.x; b += kBlock)
+        s += __hip_atomic_load(partial + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    tree(s);
+    if (threadIdx.x == 0) __hip_atomic_store(total, red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 inline dim3 blocks(int64_t n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
@@ -127,30 +139,26 @@ void pm_start(Ctx &c, const int32_t *caller_id, uint64_t seed, double eps, const
     APHIP_HIP(hipGetLastError());
 }
 
-void pm_perturb(Ctx &c, const double *u_in, const double *v, const double *l, double eps) {
-    hipLaunchKernelGGL(k_pm_perturb, blocks(c.nn), dim3(kBlock), 0, c.stream, c.nn, u_in, v, l,
-                       c.has_fixed ? c.fixed.p : nullptr, eps, c.u.p);
+// the count of finished workgroups lies behind the partial sums
+static unsigned *pm_done(const Ctx &c, double *partial) { return reinterpret_cast<unsigned *>(partial + blocks(c.nn).x); }
+
+void pm_perturb(Ctx &c, const double *u_in, const double *v, double norm, const double *l, double eps, double *u,
+                double *partial) {
+    hipLaunchKernelGGL(k_pm_perturb, blocks(c.nn), dim3(kBlock), 0, c.stream, c.nn, u_in, v, norm, l,
+                       c.has_fixed ? c.fixed.p : nullptr, eps, u, pm_done(c, partial));
     APHIP_HIP(hipGetLastError());
 }
 
 int64_t pm_partials(const Ctx &c) { return (int64_t)blocks(c.nn).x + 1; }
 
-double pm_next(Ctx &c, const double *f0, const double *l, double eps, double *v, double *partial) {
-    const dim3 g = blocks(c.nn);
-    hipLaunchKernelGGL(k_pm_next, g, dim3(kBlock), 0, c.stream, c.nn, c.f.p, f0, c.mass.p, l,
-                       c.has_fixed ? c.fixed.p : nullptr, eps, v, partial);
+double pm_next(Ctx &c, const double *f, bool parked, const double *f0, const double *l, double eps, double *v,
+               double *partial) {
+    hipLaunchKernelGGL(k_pm_next, blocks(c.nn), dim3(kBlock), 0, c.stream, c.nn, f, f0, c.mass.p, l,
+                       c.has_fixed ? c.fixed.p : nullptr, eps, v, partial, pm_done(c, partial), c.pm_total.p,
+                       parked ? c.tiles.n_interior : c.nn, c.tiles.bstart.p, c.tiles.bpart.p);
     APHIP_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_pm_sum, dim3(1), dim3(kSumLanes), 0, c.stream, (int64_t)g.x, partial);
-    APHIP_HIP(hipGetLastError());
-    double s = 0.0;
-    APHIP_HIP(hipMemcpyAsync(&s, partial + g.x, sizeof(double), hipMemcpyDeviceToHost, c.stream));
     APHIP_HIP(hipStreamSynchronize(c.stream));
-    return sqrt(s);
-}
-
-void pm_scale(Ctx &c, double norm, double *v) {
-    hipLaunchKernelGGL(k_pm_scale, blocks(3 * c.nn), dim3(kBlock), 0, c.stream, 3 * c.nn, norm, v);
-    APHIP_HIP(hipGetLastError());
+    return sqrt(*c.pm_total.p);
 }
 
 }  // namespace aphip
