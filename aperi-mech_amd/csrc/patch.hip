@@ -277,26 +277,12 @@ int patch_steps(const Ctx &c, int left) {
     return c.mat.state_width() > 0 && left > 1 && k == left ? left - 1 : k;
 }
 
-// Plan for the current tile plan and numbering; none when the mesh is too large for it.
-static void patch_build(Ctx &c) {
+// Plan of K rings and runs of `target` owned elements for the current tile plan and numbering;
+// false when a patch's rows do not fit a CU's LDS (or the lists' 16-bit fields).
+static bool patch_plan(Ctx &c, int K, int64_t target) {
     PatchPlan &P = c.patch;
-    P.tried = true;
     const int64_t nn = c.nn, ne = c.ne;
     const int npe = c.npe, sh = npe == 4 ? 2 : 3;
-    // The lines, from calls of 20 steps on n^3 x 6 Tet4 lattices (neo-Hookean; us a call, three
-    // meshes in turn / one alone; T the tile path, k x s: k rings, s owned elements):
-    //     750 T 71/177  2x64 59/149          24,576 T 119/275  1x128 70/174  2x128 88/169
-    //   3,072 T 169/294 2x64 46/137  1x64 95/203   48,000 T 168/280  1x256 114/211  1x128 119/229
-    //  10,368 T 120/264 2x128 54/165 2x64 69/146   93,750 T 167/288  1x256 209/344
-    // n^3 Hex8 (the tile path costs 163-175 in turn from launches alone, on this host):
-    //     125 T 96/192  2x8 59/171  1x16 94/181    8,000 T 175/286  1x32 103/248  1x64 138/336
-    //   1,000 T 172/265 1x16 93/178 2x8 74/216    17,576 T 168/337  1x32 153/322
-    //   2,744 T 175/267 1x16 97/181 1x32 92/211   32,768 T 163/292  1x64 231/340
-    // A second ring pays while the chip idles (it evaluates some four times the elements), the
-    // whole scheme until the elements evaluated twice cost what a launch does.
-    if (ne == 0 || ne > (npe == 4 ? 64000 : 20000) || c.tiles.threads != c.tiles.te || c.elem_seg.size() != 2) return;
-    const int K = ne <= (npe == 4 ? 16000 : 500) ? 2 : 1;
-    const int64_t target = npe == 4 ? (ne <= 6500 ? 64 : ne <= 32000 ? 128 : 256) : (ne <= 500 ? 8 : ne <= 4000 ? 16 : 32);
     const std::vector<int32_t> &conn = c.conn_h;
     // node -> (element, slot), ascending
     std::vector<int32_t> start(nn + 1, 0), inc((size_t)ne * npe);
@@ -396,7 +382,7 @@ static void patch_build(Ctx &c) {
         for (auto &t : pool) t.join();
     };
     parallel(16, work);
-    if (!fits) return;
+    if (!fits) return false;
     size_t npad = 1, cpad = 1, epad = 1, entpad = kBatch;
     for (const Patch &q : pt) {
         npad = std::max(npad, q.nodes.size());
@@ -404,9 +390,9 @@ static void patch_build(Ctx &c) {
         epad = std::max(epad, q.elems.size());
         entpad = std::max(entpad, q.ent.size());
     }
-    if (force_row(npe, (int)epad, (int)epad, npe) > 0x7fff) return;
+    if (force_row(npe, (int)epad, (int)epad, npe) > 0x7fff) return false;
     const size_t lds = carve(nullptr, npe, (int)npad, (int)cpad, (int)epad, (int)entpad).bytes;
-    if (lds > 160 * 1024) return;
+    if (lds > 160 * 1024) return false;
     // the six lists (each on a 16-byte boundary) in one allocation and one copy
     size_t total = 0;
     auto put = [&](size_t bytes) {
@@ -467,6 +453,34 @@ static void patch_build(Ctx &c) {
     // several patches share a CU (8,000 Hex8, 50 steps: 216 us in turn, 312 us with 512)
     P.threads = npe == 4 ? std::max(128, std::min(1024, (int)(epad + 63) / 64 * 64)) : 256;
     P.ready = true;
+    return true;
+}
+
+// Plan for the current tile plan; none when the mesh is too large for it.
+static void patch_build(Ctx &c) {
+    PatchPlan &P = c.patch;
+    P.tried = true;
+    const int64_t ne = c.ne;
+    const int npe = c.npe;
+    // The lines, from calls of 20 steps on n^3 x 6 Tet4 lattices (neo-Hookean; us a call, three
+    // meshes in turn / one alone; T the tile path, k x s: k rings, s owned elements):
+    //     750 T 71/177  2x64 59/149          24,576 T 119/275  1x128 70/174  2x128 88/169
+    //   3,072 T 169/294 2x64 46/137  1x64 95/203   48,000 T 168/280  1x256 114/211  1x128 119/229
+    //  10,368 T 120/264 2x128 54/165 2x64 69/146   93,750 T 167/288  1x256 209/344
+    // n^3 Hex8 (the tile path costs 163-175 in turn from launches alone, on this host):
+    //     125 T 96/192  2x8 59/171  1x16 94/181    8,000 T 175/286  1x32 103/248  1x64 138/336
+    //   1,000 T 172/265 1x16 93/178 2x8 74/216    17,576 T 168/337  1x32 153/322
+    //   2,744 T 175/267 1x16 97/181 1x32 92/211   32,768 T 163/292  1x64 231/340
+    // A second ring pays while the chip idles (it evaluates some four times the elements), the
+    // whole scheme until the elements evaluated twice cost what a launch does.  That line, in us a
+    // step against the tile path as it is now (the T above are of its 1024-element tiles):
+    //   48,000 Tet4 T 6.2/13.1 patches 5.5/9.2    63,888 Tet4 T 6.1/13.0 patches 7.1/9.3
+    //   13,824 Hex8 T 6.5/13.1 patches 6.2/12.7   19,683 Hex8 T 6.5/13.2 patches 8.4/15.6
+    if (ne == 0 || ne > (npe == 4 ? 54000 : 15000) || c.tiles.threads != c.tiles.te || c.elem_seg.size() != 2) return;
+    const int K = ne <= (npe == 4 ? 16000 : 500) ? 2 : 1;
+    const int64_t target = npe == 4 ? (ne <= 6500 ? 64 : ne <= 32000 ? 128 : 256) : (ne <= 500 ? 8 : ne <= 4000 ? 16 : 32);
+    for (int k = K; k >= 1 && !patch_plan(c, k, target); --k) {  // (some mesh shapes have larger second rings)
+    }
 }
 
 bool patch_planned(Ctx &c) {

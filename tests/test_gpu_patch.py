@@ -67,3 +67,19 @@ def test_hex8_patches_match_tiles(gpu_available, n, kind, fields, tiling):
         got = _run(X, conn, kind, calls, False, fields, tiling, A.HEX8)
         for a, b in zip(want, got):
             assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+# elongated and flat meshes, whose second rings may not fit a CU's LDS: the plan takes one
+@pytest.mark.parametrize("etype,n", [(A.TET4, (24, 11, 9)), (A.TET4, (40, 30, 2)), (A.TET4, (220, 3, 4)),
+                                     (A.HEX8, (1, 20, 25)), (A.HEX8, (120, 2, 2)), (A.HEX8, (50, 50, 5))])
+def test_patches_of_uneven_meshes_match_tiles(gpu_available, etype, n):
+    X, conn = M.hex_lattice(*n, *(k / max(n) for k in n))
+    X = M.jitter(X, 1.0 / max(n), 0.1, 7, 1)
+    if etype == A.TET4:
+        conn = M.split_tets(X, conn)
+    print(f"patches {len(conn)} of {n}", flush=True)
+    want = _run(X, conn, A.SVK, [2, 2, 2], True, False, 0, etype)
+    for calls in ([1] * 6, [6]):
+        got = _run(X, conn, A.SVK, calls, False, False, 0, etype)
+        for a, b in zip(want, got):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
