@@ -670,8 +670,7 @@ inline int64_t padded(int64_t n) { return ((n + kNumXcd - 1) / kNumXcd) * kNumXc
 template <int NPE, int MODE>
 void launch_adj(Ctx &c, const AdjArgs &A, size_t lds) {
     auto run = [&](auto kern) {
-        if (lds > 65536)
-            APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        allow_lds(c, (const void *)kern, lds);
         hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(c.tiles.threads), lds, c.stream, A);
     };
     if (c.mat.kind == APHIP_LINEAR_ELASTIC) run(k_tile_adj<NPE, APHIP_LINEAR_ELASTIC, MODE>);
@@ -693,8 +692,7 @@ void launch_patch_adj(Ctx &c, const PatchAdjArgs &A, int mode) {
     const PatchPlan &P = c.patch;
     const size_t lds = carve_adj(nullptr, NPE, P.npad, P.cpad, P.epad, P.entpad).bytes;
     auto go = [&](auto kern) {
-        if (lds > 65536)
-            APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        allow_lds(c, (const void *)kern, lds);
         hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(std::min(P.threads, NPE == 4 ? 512 : 256)), lds, c.stream, A);
         APHIP_HIP(hipGetLastError());
     };

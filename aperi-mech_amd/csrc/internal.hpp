@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <memory>
 #include <stdexcept>
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -396,6 +397,7 @@ struct Ctx {
     // per-node max edge length, computed on the first call after the mesh is set (it
     // depends on X and the connectivity only; a node renumbering permutes it); the work
     // buffers of the allocating entry point, kept between its calls
+    std::vector<const void *> big_lds;   // kernels that may take a CU's whole LDS (allow_lds)
     DevBuf<double> pm_eig;               // 3 nn, internal numbering, allocated with the mesh
     double pm_norm = 1.0;                // by which pm_eig is still to be divided
     PinnedBuf<double> pm_total;          // the norm's square, written by the device; allocated with the mesh
@@ -462,6 +464,16 @@ struct TileRun {
     bool keep = true;
 };
 void tile_run(Ctx &c, double dt, int mode, const TileRun &run = TileRun());
+
+// A launch of kern with more than 64 KiB of dynamic LDS needs an attribute of the kernel: set
+// once per context and kernel, to all of a CU's LDS (contexts of several threads launch the same
+// kernels with different sizes).
+inline void allow_lds(Ctx &c, const void *kern, size_t lds) {
+    constexpr size_t kCuLds = 160 * 1024;
+    if (lds <= 65536 || (lds <= kCuLds && std::find(c.big_lds.begin(), c.big_lds.end(), kern) != c.big_lds.end())) return;
+    APHIP_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)std::max(lds, kCuLds)));
+    c.big_lds.push_back(kern);
+}
 
 // ---- small-mesh step on node patches (patch.hip) ----
 // Whether this context's total-Lagrangian steps run on patches (builds the plan on first use:

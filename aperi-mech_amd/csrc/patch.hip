@@ -253,9 +253,7 @@ template <int NPE>
 void launch(Ctx &c, const PatchArgs &A) {
     const PatchPlan &P = c.patch;
     auto go = [&](auto kern) {
-        if (P.lds_bytes > 65536)
-            APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)P.lds_bytes));
+        allow_lds(c, (const void *)kern, P.lds_bytes);
         hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(P.threads), P.lds_bytes, c.stream, A);
         APHIP_HIP(hipGetLastError());
     };

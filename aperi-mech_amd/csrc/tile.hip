@@ -1170,8 +1170,7 @@ template <int NPE, int KIND, bool PER_QP, int MODE>
 void launch_tile(Ctx &c, const TileArgs &A) {
     const TilePlan &P = c.tiles;
     auto go = [&](auto kern, int threads, size_t lds) {
-        if (lds > 65536)
-            APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        allow_lds(c, (const void *)kern, lds);
         hipLaunchKernelGGL(kern, dim3((unsigned)A.nblocks), dim3(threads), lds, c.stream, A);
     };
     if constexpr (MODE == 2) {
@@ -1208,8 +1207,7 @@ void launch_stream(Ctx &c, const TileArgs &A) {
     const size_t lds = stream_lds_bytes(P.te, P.maxtn);
     int &grid = P.stream_grid[KIND];
     if (grid == 0) {
-        if (lds > 65536)
-            APHIP_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        allow_lds(c, (const void *)kern, lds);
         int per_cu = 0, cus = 0;
         APHIP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, P.threads, lds));
         APHIP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
