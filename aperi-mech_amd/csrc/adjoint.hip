@@ -809,24 +809,6 @@ void alloc_adjoint(Ctx &c) {
     D.mu_bar.zero(c.stream);
 }
 
-// d(lambda, mu)/d(E, nu) chain rule per element, in caller element order
-void parameter_gradients(Ctx &c, double *E_bar, double *nu_bar) {
-    std::vector<double> lb(c.ne), mb(c.ne);
-    c.adj.lam_bar.download(lb.data(), c.ne, c.stream);
-    c.adj.mu_bar.download(mb.data(), c.ne, c.stream);
-    APHIP_HIP(hipStreamSynchronize(c.stream));
-    for (int64_t e = 0; e < c.ne; ++e) {
-        const double E = c.has_fields && !c.elem_E_h.empty() ? c.elem_E_h[e] : c.mat.E;
-        const double nu = c.has_fields && !c.elem_nu_h.empty() ? c.elem_nu_h[e] : c.mat.nu;
-        const double q = (1 + nu) * (1 - 2 * nu);
-        const double dl_dE = nu / q, dm_dE = 1.0 / (2 * (1 + nu));
-        const double dl_dnu = E * (1 + 2 * nu * nu) / (q * q), dm_dnu = -E / (2 * (1 + nu) * (1 + nu));
-        const int64_t ce = c.elem_iperm[e];
-        if (E_bar) E_bar[ce] = lb[e] * dl_dE + mb[e] * dm_dE;
-        if (nu_bar) nu_bar[ce] = lb[e] * dl_dnu + mb[e] * dm_dnu;
-    }
-}
-
 // u, v, a to or from one record of 9 doubles per node: one launch, not three copies
 __global__ __launch_bounds__(256) void k_state_copy(int64_t n3, const double *u, const double *v, const double *a,
                                                     double *u1, double *v1, double *a1) {
@@ -881,7 +863,7 @@ void force_vjp(Ctx &c, const double *f_bar, double *u_bar, double *E_bar, double
     if (u_bar)
         for (int64_t i = 0; i < c.nn; ++i)
             for (int d = 0; d < 3; ++d) u_bar[3 * (int64_t)c.node_iperm[i] + d] = h[3 * i + d];
-    parameter_gradients(c, E_bar, nu_bar);
+    parameter_gradients_to_host(c, c.adj.lam_bar.p, c.adj.mu_bar.p, E_bar, nu_bar);
 }
 
 void adjoint_forward(Ctx &c, double dt, int n_steps, int interval) {
@@ -964,7 +946,7 @@ void adjoint_backward(Ctx &c, const double *ub_T, const double *vb_T, double *E_
         for (int64_t i = 0; i < c.nn; ++i)
             for (int d = 0; d < 3; ++d) v0_bar[3 * (int64_t)c.node_iperm[i] + d] = h[3 * i + d];
     }
-    parameter_gradients(c, E_bar, nu_bar);
+    parameter_gradients_to_host(c, c.adj.lam_bar.p, c.adj.mu_bar.p, E_bar, nu_bar);
     restore_state(c, D.final_state.p);
     APHIP_HIP(hipStreamSynchronize(c.stream));
 }

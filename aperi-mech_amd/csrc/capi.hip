@@ -449,6 +449,8 @@ static void setup_mesh(Ctx &c, int32_t elem_type, int64_t n_nodes, const double 
     c.has_fields = false;
     c.elem_lambda.release();
     c.elem_mu.release();
+    c.elem_E.release();
+    c.elem_nu.release();
     c.elem_rho.release();
     c.node_dt.release();
     fem_volumes(c);
@@ -900,29 +902,17 @@ int aphip_set_material_fields(aphip_ctx *c, const double *E, const double *nu) {
     c->graph_reset();
     if (!E && !nu) {
         c->has_fields = false;
-        c->elem_E_h.clear();
-        c->elem_nu_h.clear();
+        c->elem_E.release();
+        c->elem_nu.release();
         c->elem_lambda.release();
         c->elem_mu.release();
         return APHIP_OK;
     }
     APHIP_REQUIRE(E && nu, "E and nu must both be given");
-    std::vector<double> lam(c->ne), mu(c->ne);
-    c->elem_E_h.assign(c->ne, 0.0);
-    c->elem_nu_h.assign(c->ne, 0.0);
-    for (int64_t e = 0; e < c->ne; ++e) {
-        const int64_t src = c->elem_iperm[e];
-        const double Ee = E[src], ne = nu[src];
-        APHIP_REQUIRE(ne >= -1.0 && ne < 0.5 && Ee > 0.0, "per-element E/nu out of bounds");
-        mu[e] = Ee / (2 * (1 + ne));
-        lam[e] = (Ee * ne) / ((1 + ne) * (1 - 2 * ne));
-        c->elem_E_h[e] = Ee;
-        c->elem_nu_h[e] = ne;
-    }
-    c->elem_lambda.upload(lam.data(), lam.size(), c->stream);
-    c->elem_mu.upload(mu.data(), mu.size(), c->stream);
+    for (int64_t e = 0; e < c->ne; ++e)
+        APHIP_REQUIRE(nu[e] >= -1.0 && nu[e] < 0.5 && E[e] > 0.0, "per-element E/nu out of bounds");
+    material_fields_from_host(*c, E, nu);
     c->has_fields = true;
-    APHIP_HIP(hipStreamSynchronize(c->stream));
     APHIP_API_END
 }
 

@@ -373,7 +373,8 @@ struct Ctx {
     bool has_fields = false;             // per-element lambda / mu
     DevBuf<double> elem_lambda, elem_mu;
     DevBuf<double> elem_rho;             // per-element density (ensembles), else mat.density
-    std::vector<double> elem_E_h, elem_nu_h;  // per-element E / nu (internal order) when fields are set
+    DevBuf<double> elem_E, elem_nu;      // per-element E / nu (internal order) when fields are set
+    DevBuf<double> stage;                // E and nu, or their adjoints, in caller order (field.hip)
     DevBuf<double> node_dt;              // per-node time increment (ensembles), else the step argument
 
     // captured step sequences (aphip_set_graph)
@@ -531,6 +532,8 @@ double pm_next(Ctx &c, const double *f, bool parked, const double *f0, const dou
 // ---- field transfer with caller device arrays (field.hip) ----
 // dst[i, :] = src[iperm[i], :] / dst[iperm[i], :] = src[i, :], w doubles per entity
 void field_gather_rows(Ctx &c, int64_t n, int w, const int32_t *iperm, const double *src, double *dst);
+void material_fields_from_host(Ctx &c, const double *E, const double *nu);
+void parameter_gradients_to_host(Ctx &c, const double *lam_bar, const double *mu_bar, double *E_bar, double *nu_bar);
 void field_scatter_rows(Ctx &c, int64_t n, int w, const int32_t *iperm, const double *src, double *dst);
 // SoA 9 x ne tensor planes -> caller row-major n_elem x 9
 void field_scatter_tensor(Ctx &c, const double *planes, double *dst);
