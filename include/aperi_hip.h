@@ -226,7 +226,8 @@ int aphip_initialize(aphip_ctx *ctx);
 
 /* n_steps of the explicit loop body (src/Solvers/Explicit.cpp:383-452) with a fixed
  * increment (DirectTimeStepper, include/TimeStepper.h:97-128): state swap, v += dt/2 a,
- * velocity BC, u += dt v, internal force, a = f/m, acceleration BC, v += dt/2 a. */
+ * velocity BC, u += dt v, internal force, a = f/m, acceleration BC, v += dt/2 a.  H, P and f
+ * are those of the last step. */
 int aphip_step(aphip_ctx *ctx, double time_increment, int32_t n_steps);
 
 /* Stable time increment 2 / sqrt(lambda_max(M^-1 K)) by the power method about the
@@ -281,10 +282,11 @@ int aphip_results_write(aphip_ctx *ctx, double time);
 int aphip_results_close(aphip_ctx *ctx);
 
 /* Element-tile shape of the fused step: elements per tile and workgroup size.
- * Tet4: one element per thread (64, 128, 256, 512 or 1024).  Hex8: one element per
- * thread (64, 128 or 256), or eight lanes per element, one per Gauss point
- * (threads = 8 x elements, 8..64 elements).  Rebuilds the tile plan; results do
- * not depend on it beyond the rounding of the summation grouping.  No reference
+ * Tet4: one element per thread (64, 128, 256, 512 or 1024; 512 by default).  Hex8: 64, 128
+ * or 256 elements given as one per thread (128 by default), or 8..64 elements with threads =
+ * 8 x elements; every shape runs eight lanes per element, one per Gauss point.  Rebuilds the
+ * tile plan; results do not depend on it beyond the rounding of the summation grouping.  Small
+ * meshes step on node patches, whose sums are grouped by this plan too.  No reference
  * counterpart. */
 int aphip_set_tiling(aphip_ctx *ctx, int32_t elems_per_tile, int32_t threads);
 
@@ -414,7 +416,8 @@ int aphip_adjoint_backward(aphip_ctx *ctx, const double *u_bar_T, const double *
 
 /* ---- profiling ----------------------------------------------------------- */
 
-/* Record HIP events around every launch of the step kernels on the context's stream. */
+/* Record HIP events around every launch of the step kernels on the context's stream (on small
+ * meshes a launch may be two steps of a call, counted as one). */
 int aphip_set_profiling(aphip_ctx *ctx, int32_t enable);
 /* Accumulated launches and device milliseconds of kernel class `which`
  * (0 = whole step, 1 = element/force kernel, 2 = node update kernel) since the last reset. */
