@@ -36,12 +36,12 @@ def step_bytes(npe, nn, ne, steps, material_fields=False):
 # scaled by the same counters on a 1 GiB device copy (fetch x 2.0, write x 1.0); summed
 # over the step's two launches.  profiles/tile_step_tet4_6M_neohookean_hbm_traffic.txt
 # holds the commands and per-kernel figures.  Keyed by (material, hexes per edge).
-MEASURED_TRAFFIC = {}
+MEASURED_TRAFFIC = {("nh", 100): 411.0e6, ("le", 100): 411.0e6}
 # FP64 flops per step of the same workload from rocprofv3 --pmc SQ_INSTS_VALU_{FMA,MUL,ADD,
 # TRANS}_F64 on the tile kernel (64 lanes x (2 FMA + MUL + ADD + TRANS) per wave
 # instruction) on the tile and shared-node kernels; profiles/tile_step_tet4_6M_neohookean_
 # fp64_valu.txt.  FP64 vector peak of the MI355X: 78.6 TFLOP/s.
-MEASURED_FP64_FLOPS = {("nh", 100): 3.30e9, ("le", 100): 1.64e9}
+MEASURED_FP64_FLOPS = {("nh", 100): 2.78e9, ("le", 100): 1.70e9}
 FP64_PEAK_TFLOPS = 78.6
 
 
@@ -719,7 +719,7 @@ def main():
         "kernels_ms": {"step": r["step_ms"], "tile_kernel": r["force_ms"], "shared_node_kernel": r["node_ms"]},
         "fp64_valu": fp64_line(MEASURED_FP64_FLOPS.get((args.material, args.n)), r["step_ms"]),
         "launch": {"mode": r["mode"], "ms_per_step": {k: 1e3 * v / args.steps for k, v in r["walls"].items()},
-                   "tiling": "1024 Tet4 per workgroup, one per thread (default plan)"},
+                   "tiling": "512 Tet4 per workgroup, one per thread (default plan)"},
     }
     if not r["finite"]:
         line["error"] = "non-finite displacement"
