@@ -832,7 +832,7 @@ int aphip_set_material(aphip_ctx *c, int32_t kind, const aphip_material_params *
                   "the semi-Lagrangian formulation does not take the rate-form materials");
     APHIP_HIP(hipSetDevice(c->device));
     APHIP_HIP(hipStreamSynchronize(c->stream));
-    c->graph_reset();
+    c->model_changed();
     c->mat = m;
     if (c->etype >= 0) alloc_state(*c);
     APHIP_HIP(hipStreamSynchronize(c->stream));
@@ -853,7 +853,7 @@ static void set_formulation(Ctx &c, int formulation, int64_t interval) {
     APHIP_REQUIRE(interval >= 1, "the reference update interval must be at least 1");
     APHIP_HIP(hipSetDevice(c.device));
     APHIP_HIP(hipStreamSynchronize(c.stream));
-    c.graph_reset();
+    c.model_changed();
     c.formulation = formulation;
     c.semi_interval = interval;
     c.steps_done = 0;
@@ -899,7 +899,7 @@ int aphip_set_material_fields(aphip_ctx *c, const double *E, const double *nu) {
     APHIP_REQUIRE(!(c->cells.ready && c->cells.nodal), "nodal cells take one material per block");
     APHIP_HIP(hipSetDevice(c->device));
     APHIP_HIP(hipStreamSynchronize(c->stream));
-    c->graph_reset();
+    c->model_changed();
     if (!E && !nu) {
         c->has_fields = false;
         c->elem_E.release();
@@ -922,7 +922,7 @@ int aphip_compute_mass(aphip_ctx *c, double *total) {
     require_ready(*c, false);
     APHIP_HIP(hipSetDevice(c->device));
     APHIP_HIP(hipStreamSynchronize(c->stream));
-    c->graph_reset();
+    c->model_changed();
     double tot = 0.0;
     if (c->cells.ready) {
         rk_mass(*c, &tot);
@@ -944,7 +944,7 @@ int aphip_set_fixed(aphip_ctx *c, const uint8_t *mask) {
     APHIP_REQUIRE(c->etype >= 0, "mesh not set");
     APHIP_HIP(hipSetDevice(c->device));
     APHIP_HIP(hipStreamSynchronize(c->stream));
-    c->graph_reset();
+    c->model_changed();
     if (!mask) {
         c->fixed.release();
         c->has_fixed = false;
@@ -981,6 +981,7 @@ int aphip_set_field(aphip_ctx *c, int32_t field, const double *data) {
             for (int d = 0; d < 3; ++d) h[3 * i + d] = data[3 * (int64_t)c->node_iperm[i] + d];
         b->upload(h.data(), h.size(), c->stream);
     } else if (field == APHIP_FIELD_MASS) {
+        c->model_changed();
         std::vector<double> h(c->nn);
         for (int64_t i = 0; i < c->nn; ++i) {
             h[i] = data[c->node_iperm[i]];
@@ -1116,6 +1117,7 @@ int aphip_set_field_device(aphip_ctx *c, int32_t field, const double *data) {
         field_gather_rows(*c, c->nn, 3, c->d_node_iperm.p, data, node_vector(*c, field).p);
     } else if (field == APHIP_FIELD_MASS) {
         require_device_array(*c, data, sizeof(double) * c->nn);
+        c->model_changed();
         c->mass.alloc(c->nn);
         c->has_mass = false;
         APHIP_REQUIRE(field_gather_mass(*c, data) == 0, "nodal mass must be positive");

@@ -121,7 +121,8 @@ struct AdjointData {
     std::vector<DevBuf<double> *> ckpt;  // (u, v, a) at steps 0, K, 2K, ...; 9 doubles per node
     DevBuf<double> final_state;          // (u, v, a) at the last step
     DevBuf<double> seg_u;                // u of one segment's steps, K x 3 x nn
-    int seg_held = -1;                   // the segment it holds (the last one after a forward run)
+    int seg_held = -1;                   // the segment it holds (the last one after a forward run);
+                                         // -1: none, or recorded with another model (model_changed)
     DevBuf<double> ub, vb, ab;           // adjoint node state
     DevBuf<double> vb1, ab1;             // on patches: the vb, ab that the next launch writes
     DevBuf<double> lam_bar, mu_bar;      // per-element parameter adjoints
@@ -412,6 +413,13 @@ struct Ctx {
     PatchPlan patch;
     AdjointData adj;
     Profile prof;
+
+    // Material, fields, mass or constraints were set: captured sequences hold their old values, and
+    // recorded displacements of a segment are recomputed from its checkpoint with the new ones
+    void model_changed() {
+        graph_reset();
+        adj.seg_held = -1;
+    }
 
     int64_t state_count() const {
         return mat.state_width() * ne * ((etype == APHIP_HEX8 && mat.state_per_qp) ? 8 : 1);

@@ -407,7 +407,9 @@ int aphip_adjoint_forward(aphip_ctx *ctx, double time_increment, int32_t n_steps
 
 /* Reverse sweep of the last aphip_adjoint_forward: given the adjoint of the final
  * displacement (and optionally velocity), returns dL/dE_e, dL/dnu_e (n_elem, caller
- * order) and dL/dv0 (n_nodes x 3), recomputing each segment from its checkpoint.
+ * order) and dL/dv0 (n_nodes x 3), recomputing each segment from its checkpoint (the last
+ * one's displacements stand from the forward run, unless the material, the fields, the mass or
+ * the fixed mask were set since: then every segment is recomputed with the new ones).
  * The initial acceleration is taken as f(u0)/m.  Leaves the final forward state.  A new
  * tile plan (aphip_set_tiling, aphip_autotune) renumbers the nodes and drops the recording:
  * the call then fails until aphip_adjoint_forward runs again. */

@@ -263,3 +263,63 @@ def test_patch_adjoint_matches_tiles(gpu_available, etype, kind, n):
             out.append(res)
     for i, (a, b) in enumerate(zip(*out)):
         assert np.abs(a - b).max() <= 1e-11 * np.abs(b).max(), i
+
+
+def _change_model(s, what, X, conn):
+    E, nu = _fields(len(conn), 31)
+    mass = 1.5 * s.get(A.FIELD_MASS)
+    if what == "material":
+        s.set_material(A.NEO_HOOKEAN, RHO, 120e9, 0.2)
+    elif what == "fields":
+        s.set_material_fields(E, nu)
+    elif what == "fixed":
+        fixed = np.zeros(X.shape, dtype=np.uint8)
+        fixed[X[:, 0] > 0.99] = (0, 1, 1)
+        s.set_fixed(fixed)
+    elif what == "density":
+        s.set_material(A.NEO_HOOKEAN, 1.5 * RHO, 200e9, 0.3)
+        s.compute_mass()
+    elif what == "mass":
+        s.set_field(A.FIELD_MASS, mass)
+    else:
+        from test_gpu_device_fields import DeviceArray
+        d = DeviceArray(mass.size).upload(mass)
+        s.set_field_device(A.FIELD_MASS, d.address)
+        s.synchronize()
+        d.free()
+
+
+@pytest.mark.parametrize("what", ["material", "fields", "fixed", "density", "mass", "mass_device"])
+@pytest.mark.parametrize("flags", [0, A.FLAG_PIPELINED], ids=["patches", "tiles"])
+def test_backward_takes_the_model_of_its_call(gpu_available, what, flags):
+    """A model set between the forward and the backward pass holds for every segment: the
+    displacements that the forward run left of its last segment are recomputed, as those of the
+    others are.  u0 = 0, so the initial acceleration is zero under either model: with one segment
+    the gradients are those of a run under the new model alone; with three, those after a
+    backward pass that left another segment's displacements."""
+    X, conn = _mesh(A.HEX8, 4, 12)
+    v0 = 40.0 * M.normal(4, 3, X.size).reshape(X.shape)
+    ub = M.normal(5, 5, X.size).reshape(X.shape)
+    dt = 0.3 * M.stable_dt_estimate(X, M.split_tets(X, conn), 200e9, 0.3, RHO)
+
+    def grads(interval, before=False, after=False, between=False):
+        print(f"backward after {what} flags={flags} interval={interval}", flush=True)
+        with A.Solver(flags=flags) as s:
+            s.set_mesh(A.HEX8, X, conn)
+            s.set_material(A.NEO_HOOKEAN, RHO, 200e9, 0.3)
+            s.compute_mass()
+            if before:
+                _change_model(s, what, X, conn)
+            s.set_field(A.FIELD_V, v0)
+            s.initialize()
+            s.adjoint_forward(dt, 9, interval)
+            if between:
+                s.adjoint_backward(ub)
+            if after:
+                _change_model(s, what, X, conn)
+            return s.adjoint_backward(ub)
+
+    for got, want in ((grads(20, after=True), grads(20, before=True)),
+                      (grads(4, after=True), grads(4, after=True, between=True))):
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b)
