@@ -12,6 +12,7 @@
 #include <utility>
 
 #include "internal.hpp"
+#include "workers.hpp"
 
 namespace aphip {
 
@@ -162,9 +163,11 @@ static std::vector<int32_t> rcb_order(const std::vector<double> &pts, int64_t n)
             return px != py ? px < py : x < y;
         });
         if (depth < par_depth && m > 65536) {
-            std::thread left([&, b, k, depth] { split(b, b + k, depth + 1); });
+            // (split itself throws nothing: neither half allocates)
+            std::thread left = try_thread([&, b, k, depth] { split(b, b + k, depth + 1); });
+            if (!left.joinable()) split(b, b + k, depth + 1);
             split(b + k, e, depth + 1);
-            left.join();
+            if (left.joinable()) left.join();
         } else {
             split(b, b + k, depth + 1);
             split(b + k, e, depth + 1);

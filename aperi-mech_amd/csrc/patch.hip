@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "patch.hpp"
+#include "workers.hpp"
 
 namespace aphip {
 
@@ -305,9 +306,10 @@ static bool patch_plan(Ctx &c, int K, int64_t target) {
     };
     std::vector<Patch> pt(np);
     std::atomic<bool> fits{true};
-    auto work = [&](int w, int nw) {
+    std::atomic<int64_t> next{0};
+    auto work = [&] {
         std::vector<int32_t> nloc(nn, -1), eloc(ne, -1);
-        for (int64_t p = w; p < np; p += nw) {
+        for (int64_t p; (p = next++) < np;) {
             Patch &q = pt[p];
             q.nodes = own[p];
             for (int64_t e = p * target; e < std::min(ne, (p + 1) * target); ++e) {
@@ -372,12 +374,9 @@ static bool patch_plan(Ctx &c, int K, int64_t target) {
             for (int32_t e : q.elems) eloc[e] = -1;
         }
     };
-    auto parallel = [np](int most, auto &fn) {  // (a thread costs some 20 us)
-        const int nw = (int)std::max<int64_t>(1, std::min<int64_t>({most, (int64_t)std::thread::hardware_concurrency(), np / 6}));
-        std::vector<std::thread> pool;
-        for (int w = 1; w < nw; ++w) pool.emplace_back([&fn, w, nw] { fn(w, nw); });
-        fn(0, nw);
-        for (auto &t : pool) t.join();
+    auto parallel = [&](int most, auto &fn) {  // (a thread costs some 20 us)
+        next = 0;
+        run_workers((int)std::min<int64_t>({most, (int64_t)std::thread::hardware_concurrency(), np / 6}), fn);
     };
     parallel(16, work);
     if (!fits) return false;
@@ -401,8 +400,8 @@ static bool patch_plan(Ctx &c, int K, int64_t target) {
     const size_t o_meta = put(64 * np), o_node = put(4 * np * npad), o_csr = put(4 * np * cpad),
                  o_elem = put(4 * np * epad), o_conn = put(2 * np * epad * npe), o_ent = put(2 * np * entpad);
     std::unique_ptr<unsigned char[]> bytes(new unsigned char[total]);
-    auto pack = [&](int w, int nw) {
-        for (int64_t p = w; p < np; p += nw) {
+    auto pack = [&] {
+        for (int64_t p; (p = next++) < np;) {
             const Patch &q = pt[p];
             int32_t *meta = reinterpret_cast<int32_t *>(bytes.get() + o_meta) + 16 * p;
             int32_t *node = reinterpret_cast<int32_t *>(bytes.get() + o_node) + p * npad;
@@ -429,6 +428,9 @@ static bool patch_plan(Ctx &c, int K, int64_t target) {
         }
     };
     parallel(4, pack);
+    P.u.alloc(3 * nn);
+    P.v.alloc(3 * nn);
+    P.a.alloc(3 * nn);
     P.lists.upload(bytes.get(), total, c.stream);
     P.meta = reinterpret_cast<const int32_t *>(P.lists.p + o_meta);
     P.node = reinterpret_cast<const int32_t *>(P.lists.p + o_node);
@@ -436,9 +438,6 @@ static bool patch_plan(Ctx &c, int K, int64_t target) {
     P.elem = reinterpret_cast<const int32_t *>(P.lists.p + o_elem);
     P.conn = reinterpret_cast<const uint16_t *>(P.lists.p + o_conn);
     P.ent = reinterpret_cast<const uint16_t *>(P.lists.p + o_ent);
-    P.u.alloc(3 * nn);
-    P.v.alloc(3 * nn);
-    P.a.alloc(3 * nn);
     APHIP_HIP(hipStreamSynchronize(c.stream));
     P.rings = K;
     P.npatch = np;
@@ -477,7 +476,20 @@ static void patch_build(Ctx &c) {
     if (ne == 0 || ne > (npe == 4 ? 54000 : 15000) || c.tiles.threads != c.tiles.te || c.elem_seg.size() != 2) return;
     const int K = ne <= (npe == 4 ? 16000 : 500) ? 2 : 1;
     const int64_t target = npe == 4 ? (ne <= 6500 ? 64 : ne <= 32000 ? 128 : 256) : (ne <= 500 ? 8 : ne <= 4000 ? 16 : 32);
-    for (int k = K; k >= 1 && !patch_plan(c, k, target); --k) {  // (some mesh shapes have larger second rings)
+    // without the memory for a plan the steps stay on the tiles
+    auto none = [&] {
+        (void)hipGetLastError();
+        P.reset();
+        P.tried = true;
+    };
+    try {
+        for (int k = K; k >= 1 && !patch_plan(c, k, target); --k) {  // (some mesh shapes have larger second rings)
+        }
+    } catch (const Error &e) {
+        if (e.code != APHIP_ERR_ALLOC) throw;
+        none();
+    } catch (const std::bad_alloc &) {
+        none();
     }
 }
 

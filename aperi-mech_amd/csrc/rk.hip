@@ -40,6 +40,7 @@
 //   scatter kernel      ScatterValues (:130-181) as a gather over reverse neighbor lists (points that
 //                       list the node, ascending), fused with the central-difference node update
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <numeric>
@@ -48,6 +49,7 @@
 
 #include "element.hpp"
 #include "internal.hpp"
+#include "workers.hpp"
 
 namespace aphip {
 
@@ -1648,25 +1650,23 @@ static void rk_tile_plan(Ctx &c) {
         maxsub = 0;
         for (int64_t t = 0; t < nt; ++t) maxsub = std::max<int64_t>(maxsub, cst[t + 1] - cst[t]);
         sets.assign(nt, {});
-        std::vector<int> tile_max(nthreads, 0);
-        auto work = [&](int w) {
+        std::vector<int> tile_max(std::max<int64_t>(nt, 1), 0);
+        std::atomic<int64_t> next{0};
+        auto work = [&] {
             std::vector<int32_t> loc(nn, 0);
-            for (int64_t t = w; t < nt; t += nthreads) {
+            for (int64_t t; (t = next++) < nt;) {
                 const int64_t e0 = hs[cst[t]], e1 = hs[cst[t + 1]];
                 std::vector<int32_t> &u = sets[t];
                 u.assign(hn.begin() + e0, hn.begin() + e1);
                 std::sort(u.begin(), u.end());
                 u.erase(std::unique(u.begin(), u.end()), u.end());
-                tile_max[w] = std::max(tile_max[w], (int)u.size());
+                tile_max[t] = (int)u.size();
                 if (u.size() > 65535) continue;  // too large: the caller halves the tile
                 for (size_t k = 0; k < u.size(); ++k) loc[u[k]] = (int32_t)k;
                 for (int64_t e = e0; e < e1; ++e) lidx[e] = (uint16_t)loc[hn[e]];
             }
         };
-        std::vector<std::thread> pool;
-        for (int w = 1; w < nthreads; ++w) pool.emplace_back(work, w);
-        work(0);
-        for (auto &th : pool) th.join();
+        run_workers(nthreads, work);
         maxtn = *std::max_element(tile_max.begin(), tile_max.end());
         if (tile_lds(maxtn, maxsub, D.fbar) <= kTileLdsMax || tc == 1) break;
         tc = std::max(1, tc / 2);
