@@ -815,6 +815,7 @@ int aphip_set_tiling(aphip_ctx *c, int32_t te, int32_t threads) {
     c->graph_reset();
     tile_build(*c, te, threads);
     c->tiles.by_user = true;
+    (void)steps_on_patches(*c);  // (the new plan's patches here, not inside the next step)
     APHIP_API_END
 }
 
@@ -1326,6 +1327,7 @@ int aphip_set_graph(aphip_ctx *c, int32_t enable) {
     APHIP_HIP(hipStreamSynchronize(c->stream));
     c->graph_reset();
     c->graph_enabled = enable != 0;
+    (void)steps_on_patches(*c);  // (a plan that graph replay had no use for)
     APHIP_API_END
 }
 

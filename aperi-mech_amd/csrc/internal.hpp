@@ -486,7 +486,7 @@ inline void allow_lds(Ctx &c, const void *kern, size_t lds) {
 
 // ---- small-mesh step on node patches (patch.hip) ----
 // Whether this context's total-Lagrangian steps run on patches (builds the plan on first use:
-// aphip_initialize, or the first step without it).
+// aphip_initialize or aphip_set_tiling, or the first step without them).
 bool patch_eligible(Ctx &c);
 int patch_steps(const Ctx &c, int left);
 // `steps` steps in one launch (the state buffers' roles were swapped once by the caller);

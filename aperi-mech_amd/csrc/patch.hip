@@ -499,9 +499,10 @@ bool patch_planned(Ctx &c) {
 }
 
 bool patch_eligible(Ctx &c) {
-    return patch_planned(c) && !c.node_dt.p && !c.tiles.use_stream && !c.mat.state_per_qp &&
+    return !c.node_dt.p && !c.tiles.use_stream && !c.mat.state_per_qp &&
            (c.mat.kind == APHIP_LINEAR_ELASTIC || c.mat.kind == APHIP_NEO_HOOKEAN || c.mat.kind == APHIP_J2 ||
-            c.mat.kind == APHIP_SVK);
+            c.mat.kind == APHIP_SVK) &&
+           patch_planned(c);  // (last: builds the plan, 0.6 to 2 ms of host time)
 }
 
 void patch_run(Ctx &c, double dt, int steps, bool keep, double *u_rec) {

@@ -83,3 +83,50 @@ def test_patches_of_uneven_meshes_match_tiles(gpu_available, etype, n):
         got = _run(X, conn, A.SVK, calls, False, False, 0, etype)
         for a, b in zip(want, got):
             assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+def _free_bytes():
+    import ctypes
+    A.load_library()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+# a plan of this mesh takes some MiB of device memory, so that its allocation shows
+@pytest.mark.parametrize("case", ["damage", "creep", "per_qp", "pipelined", "graph", "plan"])
+def test_patch_plans_are_built_where_they_are_used(gpu_available, case):
+    """A context that never steps on patches builds no plan; one that does has it after
+    initialize, and after a new tiling without waiting for a step."""
+    hexes = case == "per_qp"
+    X, conn = M.hex_lattice(*((24, 24, 24) if hexes else (20, 20, 20)))
+    if not hexes:
+        conn = M.split_tets(X, conn)
+    damage = dict(I1_critical=3.1, I1_failure=4.0, alpha=0.5, maximum_damage=0.9, maximum_damage_increment=0.1)
+    creep = dict(A=1e-18, n=3.0, m=0.0, constant_temperature=0.0)
+    kind, more = dict(damage=(A.NEO_HOOKEAN_DAMAGE, dict(damage=damage)), creep=(A.POWER_LAW_CREEP, dict(creep=creep)),
+                      per_qp=(A.J2, dict(state_per_qp=1))).get(case, (A.NEO_HOOKEAN, {}))
+    for warm in (True, False):  # (the first launches load code)
+        with A.Solver(flags=A.FLAG_PIPELINED if case == "pipelined" else 0) as s:
+            s.set_mesh(A.HEX8 if hexes else A.TET4, X, conn)
+            s.set_material(kind, 2700.0, 70e9, 0.33, 30e6, 1e9, **more)
+            s.compute_mass()
+            free = [_free_bytes()]
+            s.set_graph(case == "graph")
+            s.initialize()
+            free.append(_free_bytes())
+            s.step(1e-9, 1)
+            s.synchronize()
+            free.append(_free_bytes())
+            if case == "plan":
+                s.set_tiling(256, 256)
+                free.append(_free_bytes())
+                s.step(1e-9, 1)
+                s.synchronize()
+                free.append(_free_bytes())
+    print(case, [f - free[0] for f in free], flush=True)
+    if case == "plan":
+        assert free[1] < free[0] - (1 << 20) and free[1] == free[2] and free[3] == free[4]
+    else:
+        assert free[0] == free[1] == free[2]
