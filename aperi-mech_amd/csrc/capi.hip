@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <functional>
 #include <array>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -696,6 +697,61 @@ static void set_node_field(Ctx &c, DevBuf<double> &b, const double *in) {
     APHIP_HIP(hipStreamSynchronize(c.stream));
 }
 
+// n_steps of the loop body with a fixed increment, as aphip_step runs them: replayed from a graph,
+// on node patches, or on the tiles with the predictor handed on.
+static void run_steps(Ctx &c, double dt, int n_steps) {
+    int done = 0;
+    if (c.graph_enabled && !c.prof.enabled && n_steps >= 2 && c.formulation != APHIP_SEMI_LAGRANGIAN) {
+        // two steps per graph: the N/NP1 state buffers swap twice and return to their roles
+        if (!c.graph_exec || c.graph_dt != dt || c.graph_parity != c.state_np1) {
+            c.graph_reset();
+            const int parity = c.state_np1;
+            hipGraph_t g = nullptr;
+            APHIP_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal));
+            try {  // the second step takes the first one's prediction
+                step_once(c, dt, false, true, false);
+                step_once(c, dt, true, false, true);
+            } catch (...) {
+                (void)hipStreamEndCapture(c.stream, &g);
+                if (g) (void)hipGraphDestroy(g);
+                c.state_np1 = parity;
+                throw;
+            }
+            APHIP_HIP(hipStreamEndCapture(c.stream, &g));
+            const hipError_t ie = hipGraphInstantiate(&c.graph_exec, g, nullptr, nullptr, 0);
+            (void)hipGraphDestroy(g);
+            APHIP_HIP(ie);
+            c.graph_dt = dt;
+            c.graph_parity = parity;
+        }
+        for (; done + 2 <= n_steps; done += 2) APHIP_HIP(hipGraphLaunch(c.graph_exec, c.stream));
+    }
+    if (steps_on_patches(c)) {  // small meshes: several steps per launch
+        while (done < n_steps) {
+            const int k = patch_steps(c, n_steps - done);
+            prof_begin(c, 0);
+            c.state_np1 = 1 - c.state_np1;
+            c.rate_dt = dt;
+            prof_begin(c, 1);
+            patch_run(c, dt, k, done + k == n_steps);
+            prof_end(c, 1);
+            prof_end(c, 0);
+            done += k;
+        }
+    }
+    for (bool pred = false; done < n_steps; ++done) {
+        const bool more = done + 1 < n_steps;
+        // (a semi-Lagrangian reference update after this step reads H)
+        const bool update = c.formulation == APHIP_SEMI_LAGRANGIAN && (c.steps_done + 1) % c.semi_interval == 0;
+        prof_begin(c, 0);
+        step_once(c, dt, pred, more, !more || update);
+        prof_end(c, 0);
+        pred = more;
+        // the reference's StepScheduler(interval, interval) after step n (Explicit.cpp:195-212)
+        if (c.formulation == APHIP_SEMI_LAGRANGIAN && ++c.steps_done % c.semi_interval == 0) fem_semi_update(c);
+    }
+}
+
 }  // namespace aphip
 
 using namespace aphip;
@@ -1267,56 +1323,7 @@ int aphip_step(aphip_ctx *c, double dt, int32_t n_steps) {
     APHIP_REQUIRE(n_steps >= 0, "n_steps must be non-negative");
     APHIP_REQUIRE(std::isfinite(dt) && dt >= 0.0, "time increment must be finite and non-negative");
     APHIP_HIP(hipSetDevice(c->device));
-    int32_t done = 0;
-    if (c->graph_enabled && !c->prof.enabled && n_steps >= 2 && c->formulation != APHIP_SEMI_LAGRANGIAN) {
-        // two steps per graph: the N/NP1 state buffers swap twice and return to their roles
-        if (!c->graph_exec || c->graph_dt != dt || c->graph_parity != c->state_np1) {
-            c->graph_reset();
-            const int parity = c->state_np1;
-            hipGraph_t g = nullptr;
-            APHIP_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-            try {  // the second step takes the first one's prediction
-                step_once(*c, dt, false, true, false);
-                step_once(*c, dt, true, false, true);
-            } catch (...) {
-                (void)hipStreamEndCapture(c->stream, &g);
-                if (g) (void)hipGraphDestroy(g);
-                c->state_np1 = parity;
-                throw;
-            }
-            APHIP_HIP(hipStreamEndCapture(c->stream, &g));
-            const hipError_t ie = hipGraphInstantiate(&c->graph_exec, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
-            APHIP_HIP(ie);
-            c->graph_dt = dt;
-            c->graph_parity = parity;
-        }
-        for (; done + 2 <= n_steps; done += 2) APHIP_HIP(hipGraphLaunch(c->graph_exec, c->stream));
-    }
-    if (steps_on_patches(*c)) {  // small meshes: several steps per launch
-        while (done < n_steps) {
-            const int k = patch_steps(*c, n_steps - done);
-            prof_begin(*c, 0);
-            c->state_np1 = 1 - c->state_np1;
-            c->rate_dt = dt;
-            prof_begin(*c, 1);
-            patch_run(*c, dt, k, done + k == n_steps);
-            prof_end(*c, 1);
-            prof_end(*c, 0);
-            done += k;
-        }
-    }
-    for (bool pred = false; done < n_steps; ++done) {
-        const bool more = done + 1 < n_steps;
-        // (a semi-Lagrangian reference update after this step reads H)
-        const bool update = c->formulation == APHIP_SEMI_LAGRANGIAN && (c->steps_done + 1) % c->semi_interval == 0;
-        prof_begin(*c, 0);
-        step_once(*c, dt, pred, more, !more || update);
-        prof_end(*c, 0);
-        pred = more;
-        // the reference's StepScheduler(interval, interval) after step n (Explicit.cpp:195-212)
-        if (c->formulation == APHIP_SEMI_LAGRANGIAN && ++c->steps_done % c->semi_interval == 0) fem_semi_update(*c);
-    }
+    run_steps(*c, dt, n_steps);
     APHIP_API_END
 }
 
@@ -1374,37 +1381,46 @@ int aphip_autotune(aphip_ctx *c, double dt, int32_t trial_steps, int32_t *chosen
         cand = {{64, 64, false}, {128, 128, false}, {256, 256, false}, {16, 128, false}, {32, 256, false},
                 {64, 512, false}};
     const bool was_prof = c->prof.enabled;
-    Cand best{prev_te, c->tiles.threads, c->tiles.use_stream};
-    double best_ms = 1e300;
-    hipEvent_t e0, e1;
-    APHIP_HIP(hipEventCreate(&e0));
-    APHIP_HIP(hipEventCreate(&e1));
     c->prof.enabled = false;
+    Cand best{prev_te, c->tiles.threads, c->tiles.use_stream};
+    // A call as aphip_step runs it (node patches or graph replay where its steps take them, else the
+    // predictor handed on and one store of H, P and f), by the host's clock: launches count.  The
+    // shortest of three, after a call that warms up and lays out or captures what is made once.
+    // Patches are out of reach for the pipelined and the eight-lane shapes.
+    auto time_calls = [&](const Cand &tt) {
+        c->tiles.use_stream = tt.pipelined;
+        run_steps(*c, dt, std::min(trial_steps, 2));
+        double least = 1e300;
+        for (int k = 0; k < 3; ++k) {
+            APHIP_HIP(hipStreamSynchronize(c->stream));
+            const auto t0 = std::chrono::steady_clock::now();
+            run_steps(*c, dt, trial_steps);
+            APHIP_HIP(hipStreamSynchronize(c->stream));
+            least = std::min(least, std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
+        }
+        return least;
+    };
+    double best_s = c->tiles.ready ? time_calls(best) : 1e300;
     for (const auto &tt : cand) {
         try {
             tile_build(*c, tt.te, tt.threads);
         } catch (const Error &) {
             continue;  // this shape does not fit the mesh (e.g. a tile needs more LDS than a CU has)
         }
-        c->tiles.use_stream = tt.pipelined;
-        step_once(*c, dt);  // warm-up
-        APHIP_HIP(hipEventRecord(e0, c->stream));
-        for (int k = 0; k < trial_steps; ++k) step_once(*c, dt);
-        APHIP_HIP(hipEventRecord(e1, c->stream));
-        APHIP_HIP(hipEventSynchronize(e1));
-        float ms = 0.0f;
-        APHIP_HIP(hipEventElapsedTime(&ms, e0, e1));
-        if (ms < best_ms) {
-            best_ms = ms;
+        const double t = time_calls(tt);
+        // within 5 % the earlier one stays, the present plan first of all: launches cost the host
+        // more or less from one process to the next (729 Hex8, 40 steps: patches 321 us, one launch a
+        // step; 16-element tiles, two launches, 310 here and 345 to 397 a minute later)
+        if (t < 0.95 * best_s) {
+            best_s = t;
             best = tt;
         }
     }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
     c->prof.enabled = was_prof;
     tile_build(*c, best.te, best.threads);
     c->tiles.by_user = true;
     c->tiles.use_stream = best.pipelined;
+    (void)steps_on_patches(*c);
     set_node_field(*c, c->u, su.data());
     set_node_field(*c, c->v, sv.data());
     set_node_field(*c, c->a, sa.data());

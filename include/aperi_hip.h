@@ -298,8 +298,9 @@ int aphip_set_tiling(aphip_ctx *ctx, int32_t elems_per_tile, int32_t threads);
 int aphip_set_graph(aphip_ctx *ctx, int32_t enable);
 
 /* Times the candidate tile shapes (and, for Tet4, the pipelined kernel) on the
- * context's own workload (trial_steps steps each, the simulation state is restored
- * afterwards) and keeps the fastest.  Writes elements_per_tile * 10000 + threads
+ * context's own workload (calls of trial_steps steps as aphip_step runs them, on small meshes
+ * on node patches, with the GPU otherwise idle; the simulation state is restored afterwards) and
+ * keeps the fastest.  Writes elements_per_tile * 10000 + threads
  * (+ 100000000 for the pipelined kernel) of the choice to *chosen.  No reference
  * counterpart. */
 int aphip_autotune(aphip_ctx *ctx, double time_increment, int32_t trial_steps, int32_t *chosen);
