@@ -252,6 +252,7 @@ struct TilePlan {
     DevBuf<uint4> hx_first, hx_more;  // [ntiles * rounds * tpad] first eight entries of a row; the rest
     DevBuf<uint32_t> hx_csr;          // [ntiles * rounds * tpad] (first further batch << 16) | batches
     DevBuf<int32_t> hx_base;          // [ntiles * rounds] origin of the batches in hx_more
+    DevBuf<double> hx_part;           // several rounds: [ntiles * tpad * 3] the rows' sums so far
     size_t cell_lds_bytes = 0;        // LDS of the smoothed Hex8 cell kernel
     void reset() {
         ready = false;
@@ -264,7 +265,7 @@ struct TilePlan {
         zero.release(); meta.release();
         tpad = 0;
         tnp_node.release(); tnp_csr.release(); tnp_bdst.release(); lconn_p.release();
-        hx_conn.release(); hx_first.release(); hx_more.release(); hx_csr.release(); hx_base.release();
+        hx_conn.release(); hx_first.release(); hx_more.release(); hx_csr.release(); hx_base.release(); hx_part.release();
         hx_rounds = 1;
         cell_lds_bytes = 0;
     }

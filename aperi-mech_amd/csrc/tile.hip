@@ -75,6 +75,7 @@ struct TileArgs {
     const uint4 *hx_first, *hx_more;
     const uint32_t *hx_csr;
     const int32_t *hx_base;
+    double *hx_part;  // several rounds: [ntiles * tpad * 3] the rows' sums so far
     int hx_rounds;
     double *bpart;
     double *H, *P;
@@ -112,6 +113,9 @@ struct TileArgs {
 // predicted displacement) are kept for every tile node; v_half, m, dt and the fixed mask for
 // max_nint rows (Hex8: the interior nodes, the only ones the kernel finishes; Tet4: every
 // tile node); F holds nf doubles: the element forces of one round or the Hex8 element rows.
+// LEAN: a Hex8 tile in rounds, which reads m, dt, the mask and the entries from global memory when
+// it needs them (the freed LDS saves rounds: 76,800 Hex8 in bars of three, tiles of 256, 58 to
+// 61 us a step in four rounds, 47 to 51 in two).
 struct TileLds {
     double *X, *U, *V, *F, *M, *DT;
     uint32_t *csr;
@@ -126,16 +130,18 @@ struct TileLds {
 // read at the same time in the gather, never share a bank.
 __host__ __device__ __forceinline__ int f_stride(int te_round) { return te_round + ((4 - te_round) & 31); }
 
-__host__ __device__ __forceinline__ TileLds carve(char *base, int maxtn, int max_nint, int nent, size_t nf) {
+__host__ __device__ __forceinline__ TileLds carve(char *base, int maxtn, int max_nint, int nent, size_t nf,
+                                                  bool lean = false) {
     TileLds L;
+    const int fin = lean ? 0 : max_nint;
     L.X = reinterpret_cast<double *>(base);
     L.U = L.X + 3 * maxtn;
     L.V = L.U + 3 * maxtn;
     L.M = L.V + 3 * max_nint;
-    L.DT = L.M + max_nint;
-    L.F = L.DT + max_nint;
+    L.DT = L.M + fin;
+    L.F = L.DT + fin;
     L.csr = reinterpret_cast<uint32_t *>(L.F + nf);
-    L.bdst = reinterpret_cast<int32_t *>(L.csr + maxtn);
+    L.bdst = reinterpret_cast<int32_t *>(L.csr + (lean ? 0 : maxtn));
     // (16-byte aligned: entries are read eight at a time)
     L.ent = reinterpret_cast<uint16_t *>((reinterpret_cast<uintptr_t>(L.bdst + maxtn) + 15) & ~(uintptr_t)15);
     L.fx = reinterpret_cast<uint8_t *>(L.ent + nent);
@@ -149,10 +155,13 @@ __host__ __device__ __forceinline__ size_t tile_f_doubles(int npe, int te, bool 
     return npe == 4 ? 12 * (size_t)f_stride(te) : cell ? 24 * (size_t)f_stride(te / 2) : kHexRow * (size_t)te + 4;
 }
 
-// nent: entries kept in LDS
-__host__ inline size_t tile_lds_bytes(int maxtn, int max_nint, int te, int npe, int nent, bool cell) {
-    return sizeof(double) * (6 * (size_t)maxtn + 5 * (size_t)max_nint + tile_f_doubles(npe, te, cell)) +
-           8 * (size_t)maxtn + 2 * (size_t)nent + (size_t)max_nint + 16 + 16;
+// Entries of a Hex8 tile kept in LDS: eight a row, or none in rounds.
+__host__ __device__ __forceinline__ int hex_entries(int maxtn, int rounds) { return rounds == 1 ? 8 * maxtn : 0; }
+
+// nent: entries kept in LDS; lean: as carve's
+__host__ inline size_t tile_lds_bytes(int maxtn, int max_nint, int te, int npe, int nent, bool cell, bool lean = false) {
+    return sizeof(double) * (6 * (size_t)maxtn + (lean ? 3 : 5) * (size_t)max_nint + tile_f_doubles(npe, te, cell)) +
+           (lean ? 4 : 8) * (size_t)maxtn + 2 * (size_t)nent + (lean ? 0 : (size_t)max_nint) + 16 + 16;
 }
 
 // Materials whose Hex8 kernel needs more than the 128 VGPRs of four waves per SIMD (it would
@@ -282,21 +291,23 @@ __device__ __forceinline__ void ul_store1(double *u, double *dinc, double *xnp1,
 // Node ln's force f is complete: an interior node is finished and written (MODE 0: f;
 // 1: f and a = f/m; 2: the corrector); a shared node parks f in its slot for the
 // shared-node pass.
-template <int MODE, bool UL = false>
+template <int MODE, bool UL = false, bool LEAN = false>
 __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L, int ln, int nint, int64_t ibase,
                                             const double (&f)[3]) {
     if (ln < nint) {
         const int64_t g = ibase + ln;
         if (MODE != 2 || A.keep) st3(A.f, g, f);
+        const double mm = MODE == 0 ? 1.0 : LEAN ? A.mass[g] : L.M[ln];
         if constexpr (MODE == 1) {
-            const double mm = L.M[ln];
             const double acc[3] = {f[0] / mm, f[1] / mm, f[2] / mm};
             st3(A.a, g, acc);
         } else if constexpr (MODE == 2) {
             double vh[3], u1[3], a1[3], v1[3];
+            const unsigned fx = LEAN ? load_fixed(A, g) : L.fx[ln];
+            const double nd = LEAN ? load_node_dt(A, g) : L.DT[ln];
             ld3(L.V, ln, vh);
             ld3(L.U, ln, u1);
-            cd_correct(f, L.M[ln], L.fx[ln], L.DT[ln], vh, a1, v1);
+            cd_correct(f, mm, fx, nd, vh, a1, v1);
             if constexpr (UL) {
                 double x[3];
                 ld3(L.X, ln, x);
@@ -304,7 +315,7 @@ __device__ __forceinline__ void finish_node(const TileArgs &A, const TileLds &L,
                 for (int d = 0; d < 3; ++d) ul_store1(A.u, A.dinc, A.xnp1, A.semi, 3 * g + d, A.dt, vh[d], x[d], u1[d]);
             } else if (A.more) {
                 double u2[3], v2[3];
-                cd_predict(u1, v1, a1, L.fx[ln], L.DT[ln], v2, u2);
+                cd_predict(u1, v1, a1, fx, nd, v2, u2);
                 st3(A.u, g, u2);
                 st3(A.v, g, v2);
                 return;
@@ -611,17 +622,15 @@ __global__ __launch_bounds__(NPE == 4 ? 1024 : 256, NPE == 8 ? 2 : 1) void k_til
 // four waves per SIMD (the wide materials two).  20^3 Hex8, a step: 21.6 -> 12.5 us alone; the
 // 1.3M-Hex8 ensemble, where issue slots alone count, 0.20 ms of tile kernel either way.  The
 // elements' forces and, before them, the modes share the element's LDS row; a tile whose rows
-// do not fit the LDS passes them through in rounds (MULTI), whose sums a node's thread adds up
-// in an LDS row: the same sequence for every number of rounds.
+// do not fit the LDS passes them through in rounds (MULTI), between which a node's thread keeps
+// its row's sum in global memory: the same sequence for every number of rounds.
 template <int KIND, bool PER_QP, int MODE, bool MULTI, bool UL = false>
-__global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_wide<KIND, UL>()) ? 2 : 4) void k_hex_tile(TileArgs A) {
+__global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (MULTI || hex_wide<KIND, UL>()) ? 2 : 4) void k_hex_tile(TileArgs A) {
     extern __shared__ __align__(16) char lds_raw[];
     const int64_t t = xcd_tile(A.nblocks);
     if (t >= A.ntiles) return;
     const int rounds = MULTI ? A.hx_rounds : 1, rw = A.te / rounds;
-    // (MULTI: 12 entry halves a row are the 24 bytes of its partial sum)
-    const TileLds L = carve(lds_raw, A.maxtn, A.max_nint, (MULTI ? 12 : 8) * A.maxtn, tile_f_doubles(8, rw, false));
-    double *acc = reinterpret_cast<double *>(L.ent);
+    const TileLds L = carve(lds_raw, A.maxtn, A.max_nint, hex_entries(A.maxtn, rounds), tile_f_doubles(8, rw, false), MULTI);
     const int tid = threadIdx.x, nt = blockDim.x;
     // A: every global load of the stage before the first LDS write (see k_tile)
     constexpr int PASSES = hex_wide<KIND, UL>() ? 4 : 2;  // te <= PASSES * blockDim / 8
@@ -673,7 +682,7 @@ __global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_
         }
         L.bdst[ln] = bdst;
         st3(L.X, ln, x);
-        if (ln < nint) {
+        if (!MULTI && ln < nint) {
             L.fx[ln] = (uint8_t)fx;
             L.M[ln] = mm;
             L.DT[ln] = nd;
@@ -775,12 +784,13 @@ __global__ __launch_bounds__((MULTI || hex_wide<KIND, UL>()) ? 512 : 1024, (hex_
             const int64_t tr = t * (int64_t)rounds + r;
             for (int ln = tid; ln < tn; ln += nt) {
                 double f[3] = {0.0, 0.0, 0.0};
-                if (r > 0) ld3(acc, ln, f);
+                const int64_t row = t * (int64_t)A.tpad + ln;
+                if (r > 0) ld3(A.hx_part, row, f);
                 add8(A.hx_first[tr * A.tpad + ln], f);
                 const uint32_t csr = A.hx_csr[tr * A.tpad + ln];
                 if (csr & 0xffffu) add_more(csr, A.hx_base[tr], f);
-                if (r + 1 < rounds) st3(acc, ln, f);
-                else finish_node<MODE, UL>(A, L, ln, nint, ibase, f);
+                if (r + 1 < rounds) st3(A.hx_part, row, f);
+                else finish_node<MODE, UL, true>(A, L, ln, nint, ibase, f);
             }
             if (r + 1 < rounds) __syncthreads();
         }
@@ -1434,7 +1444,7 @@ void tile_build(Ctx &c, int te, int threads) {
             // one round unless the rows do not fit the LDS beside the tile's nodes
             int max_int = 0;
             for (int64_t t = 0; t < nt; ++t) max_int = std::max(max_int, ninterior[t]);
-            auto lds_of = [&](int r) { return tile_lds_bytes(maxtn, max_int, te / r, 8, (r == 1 ? 8 : 12) * maxtn, false); };
+            auto lds_of = [&](int r) { return tile_lds_bytes(maxtn, max_int, te / r, 8, hex_entries(maxtn, r), false, r > 1); };
             int R = 1;
             while (te / R > 16 && lds_of(R) > 160 * 1024) R *= 2;
             const int rw = te / R;
@@ -1471,6 +1481,7 @@ void tile_build(Ctx &c, int te, int threads) {
             P.hx_more.upload(reinterpret_cast<const uint4 *>(more.data()), more.size() / 8, c.stream);
             P.hx_csr.upload(hcsr.data(), hcsr.size(), c.stream);
             P.hx_base.upload(base.data(), base.size(), c.stream);
+            P.hx_part.alloc(R > 1 ? 3 * (size_t)nt * P.tpad : 0);
         }
     }
     P.nslot = bstart[nb];
@@ -1501,9 +1512,9 @@ void tile_build(Ctx &c, int te, int threads) {
     APHIP_REQUIRE(P.lds_bytes <= 160 * 1024, "tile needs more LDS than a CU has; use a smaller tile");
     for (const bool cell : {false, true}) {  // the kernels' carve-up must end inside the allocation
         const int R = npe == 8 && !cell ? P.hx_rounds : 1;
-        const int nent = npe == 8 && !cell ? (R == 1 ? 8 : 12) * P.maxtn : te * npe;
-        const TileLds L = carve(nullptr, P.maxtn, P.max_nint, nent, tile_f_doubles(npe, te / R, cell));
-        APHIP_REQUIRE((size_t)(reinterpret_cast<const char *>(L.fx + P.max_nint) - static_cast<const char *>(nullptr)) <=
+        const int nent = npe == 8 && !cell ? hex_entries(P.maxtn, R) : te * npe;
+        const TileLds L = carve(nullptr, P.maxtn, P.max_nint, nent, tile_f_doubles(npe, te / R, cell), R > 1);
+        APHIP_REQUIRE((size_t)(reinterpret_cast<const char *>(L.fx + (R > 1 ? 0 : P.max_nint)) - static_cast<const char *>(nullptr)) <=
                           (cell ? P.cell_lds_bytes : P.lds_bytes),
                       "tile LDS layout exceeds its allocation");
     }
@@ -1560,6 +1571,7 @@ void tile_run(Ctx &c, double dt, int mode, const TileRun &run) {
     A.hx_more = P.hx_more.p;
     A.hx_csr = P.hx_csr.p;
     A.hx_base = P.hx_base.p;
+    A.hx_part = P.hx_part.p;
     A.hx_rounds = P.hx_rounds;
     A.bpart = P.bpart.p;
     A.H = c.Hnp1().p;

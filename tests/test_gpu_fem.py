@@ -311,3 +311,50 @@ def test_pipelined_step_matches_one_tile_per_workgroup(gpu_available, mat, te):
             print(f"field {fld}: {np.count_nonzero(d)} differ, max {d.max():.3e} at {i}")
         assert np.array_equal(a, b), fld
     assert np.abs(outs[0][0]).max() > 0.0
+
+
+def _bars(n, length):
+    """n x n unconnected bars of 1 x 1 x length hexes."""
+    X, conn = M.hex_lattice(1, 1, length, 0.1, 0.1, 0.1 * length)
+    Xs = [X + (0.2 * i, 0.2 * j, 0.0) for i in range(n) for j in range(n)]
+    return np.concatenate(Xs), np.concatenate([conn + k * len(X) for k in range(n * n)])
+
+
+# A 256-element tile's rows pass the LDS in rounds where it has many nodes: one long bar (1028 nodes
+# of 256 hexes: two rounds) and bars of three hexes (1366 nodes: four; a shape that fitted when the
+# force rows alone passed in rounds); the last tile is partial
+@pytest.mark.parametrize("mesh", ["long", "short"])
+@pytest.mark.parametrize("mat,per_qp", [("nh", 0), ("j2", 1), ("creep", 0), ("creep", 1)])
+def test_hex8_tiles_in_rounds(gpu_available, mesh, mat, per_qp):
+    X, conn = _bars(1, 300) if mesh == "long" else _bars(10, 3)
+    X = M.jitter(X, 0.1, 0.1, 31, 1)
+    creep = dict(A=1e-18, n=3.0, m=0.0, constant_temperature=0.0)
+    kind, p = (A.POWER_LAW_CREEP, dict(E=1e9, nu=0.3, rho=1000.0)) if mat == "creep" else MATS[mat]
+    lam, mu = O.lame(p["E"], p["nu"])
+    v0 = (30.0 if mat == "j2" else 5.0) * (2.0 * M.uniform01(4, 2, X.size).reshape(X.shape) - 1.0)
+    mass = O.lumped_mass(A.HEX8, X, conn, p["rho"])
+    dt = 0.3 * M.stable_dt_estimate(X, M.split_tets(X, conn), p["E"], p["nu"], p["rho"])
+    ref = O.Solver(A.HEX8, X, conn, O.CREEP if mat == "creep" else kind, lam, mu, mass, None, p.get("yield_stress", 0.0),
+                   p.get("hardening", 0.0), state_per_qp=per_qp,
+                   creep=dict(creep, bulk=p["E"] / (3 * (1 - 2 * p["nu"]))) if mat == "creep" else None)
+    ref.v[:] = v0
+    print(f"hex8 rounds mesh={mesh} mat={mat} per_qp={per_qp}", flush=True)
+    with A.Solver() as s:
+        s.set_mesh(A.HEX8, X, conn)
+        s.set_material(kind, p["rho"], p["E"], p["nu"], p.get("yield_stress", 0.0), p.get("hardening", 0.0), per_qp,
+                       creep=creep if mat == "creep" else None)
+        s.set_tiling(256, 256)
+        s.compute_mass()
+        s.set_field(A.FIELD_V, v0)
+        s.set_graph(True)  # (the tile kernel, where an eager call would take node patches)
+        s.initialize()
+        for n in (1, 12, 7):
+            s.step(dt, n)
+            ref.run(dt, n)
+            for fld, r in ((A.FIELD_U, ref.u), (A.FIELD_V, ref.v), (A.FIELD_A, ref.a), (A.FIELD_F, ref.f),
+                           (A.FIELD_H, ref.H), (A.FIELD_P, ref.P)):
+                assert rel_err(s.get(fld), r) < (TOL_STEP if n == 1 else 1e-11), (n, fld)
+            if mat != "nh":
+                assert rel_err(s.get(A.FIELD_STATE), ref.state) < 1e-11
+        s.internal_force(0.0, dt)
+        assert rel_err(s.get(A.FIELD_F), ref.f) < 1e-11 or mat != "nh"  # (rate forms and J2 read the N state)
