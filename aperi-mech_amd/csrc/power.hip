@@ -113,6 +113,8 @@ __global__ __launch_bounds__(kBlock) void k_pm_next(int64_t nn, const double *f1
         // The workgroups run on several XCDs, each with its own L2: the partial sum goes to memory
         // by a device-scope exchange, whose return the count waits for, and is read back past the
         // L2s. (A release here would write back the XCD's whole L2: 8.8 us a launch, against 6.2.)
+        // The order is this chip's, not the language's: a device-scope exchange has taken place in
+        // memory when its old value is back, and the asm keeps the count behind that.
         const unsigned long long was =
             __hip_atomic_exchange(reinterpret_cast<unsigned long long *>(partial) + blockIdx.x,
                                   (unsigned long long)__double_as_longlong(red[0]), __ATOMIC_RELAXED,
