@@ -154,3 +154,115 @@ def test_autotune_keeps_patches(gpu_available, etype, n):
         s.synchronize()
         steps, shared = s.profile(0)[0], s.profile(2)[0]
     assert steps <= 40 and shared == 0  # a patch launch has no shared-node pass
+
+
+def _block(etype, n, seed=7):
+    X, conn = M.hex_lattice(*n, *(k / max(n) for k in n))
+    X = M.jitter(X, 1.0 / max(n), 0.1, seed, 1)
+    return X, (M.split_tets(X, conn) if etype == A.TET4 else conn)
+
+
+def _start(s, X, conn, etype, kind, seed=9):
+    s.set_mesh(etype, X, conn)
+    s.set_material(kind, 2700.0, 70e9, 0.33, 30e6, 1e9)
+    s.compute_mass()
+    mass = s.get(A.FIELD_MASS)
+    s.set_field(A.FIELD_MASS, np.where(mass > 0.0, mass, mass.max()))  # (nodes of no element)
+    s.set_field(A.FIELD_V, 30.0 * (2 * M.uniform01(seed, 4, X.size).reshape(X.shape) - 1))
+    return 0.3 * M.stable_dt_estimate(X, conn if etype == A.TET4 else M.split_tets(X, conn), 70e9, 0.33, 2700.0)
+
+
+BLOCKS = [(A.TET4, (6, 7, 5)), (A.TET4, (14, 13, 12)), (A.HEX8, (6, 7, 8)), (A.HEX8, (12, 11, 10))]
+
+
+@pytest.mark.parametrize("etype,n", BLOCKS)
+def test_graph_replay_between_patch_calls(gpu_available, etype, n):
+    """Patch launches exchange the buffers of u, v and a; replay captured before or after them
+    reads the right ones."""
+    X, conn = _block(etype, n)
+    out = []
+    for toggle in (False, True):
+        print(f"graph between patches {etype} {n} {toggle}", flush=True)
+        with A.Solver() as s:
+            dt = _start(s, X, conn, etype, A.J2)
+            s.set_graph(True)
+            s.initialize()
+            for k, calls in enumerate((4, 3, 1, 2, 5, 4, 6)):
+                s.set_graph(not toggle or k % 2 == 0)
+                s.step(dt, calls)
+            out.append([s.get(f) for f in (*FIELDS, A.FIELD_STATE)])
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("etype,n", BLOCKS)
+def test_power_method_between_patch_steps(gpu_available, etype, n):
+    X, conn = _block(etype, n)
+    out = []
+    for graph in (True, False):
+        print(f"power method between patches {etype} {n} {graph}", flush=True)
+        with A.Solver() as s:
+            _start(s, X, conn, etype, A.NEO_HOOKEAN)
+            s.set_graph(graph)
+            s.initialize()
+            res = []
+            for calls in (3, 4, 1):
+                inc = s.power_method_time_increment()
+                s.step(0.3 * inc[0], calls)
+                res += [np.array(inc, dtype=float), *(s.get(f) for f in FIELDS)]
+            out.append(res)
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("etype", [A.TET4, A.HEX8])
+@pytest.mark.parametrize("parts,n,lonely", [(3, (4, 4, 4), 5), (60, (1, 1, 1), 0), (1, (1, 1, 1), 40), (8, (7, 5, 6), 300)])
+def test_patches_of_parts_and_lonely_nodes(gpu_available, etype, parts, n, lonely):
+    """Unconnected parts, and nodes of no element before and between theirs."""
+    Xs, cs, at = [], [], 0
+    for k in range(parts):
+        X, conn = _block(etype, n, 7 + k)
+        extra = np.array([[2.0 * k, -1.0, 0.1 * j] for j in range(lonely // parts + (k == 0))]).reshape(-1, 3)
+        Xs += [extra, X + (2.0 * k, 0.0, 0.0)]
+        cs.append(conn + at + len(extra))
+        at += len(extra) + len(X)
+    X, conn = np.concatenate(Xs), np.concatenate(cs)
+    out = []
+    for graph in (True, False):
+        print(f"parts {etype} {parts} {n} {lonely} {graph}", flush=True)
+        with A.Solver() as s:
+            dt = _start(s, X, conn, etype, A.J2)
+            s.set_graph(graph)
+            s.initialize()
+            for calls in (4, 2):
+                s.step(dt, calls)
+            out.append([s.get(f) for f in (*FIELDS, A.FIELD_STATE)])
+    for a, b in zip(*out):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+def test_patches_from_two_threads(gpu_available):
+    import threading
+    jobs = [(et, *_block(et, n, 3 + k)) for k, (et, n) in enumerate(BLOCKS)]
+
+    def job(k, out):
+        et, X, conn = jobs[k]
+        with A.Solver() as s:
+            dt = _start(s, X, conn, et, A.SVK, 11 + k)
+            s.initialize()
+            for calls in [5] * 40:
+                s.step(dt, calls)
+            out[k] = [s.get(f) for f in FIELDS]
+
+    alone, together = {}, {}
+    for k in range(len(jobs)):
+        job(k, alone)
+    print("threads", flush=True)
+    threads = [threading.Thread(target=lambda ks=ks: [job(k, together) for k in ks]) for ks in ((0, 3), (2, 1))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in alone:
+        for a, b in zip(alone[k], together[k]):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
