@@ -468,6 +468,10 @@ static void patch_build(Ctx &c) {
     //     125 T 96/192  2x8 59/171  1x16 94/181    8,000 T 175/286  1x32 103/248  1x64 138/336
     //   1,000 T 172/265 1x16 93/178 2x8 74/216    17,576 T 168/337  1x32 153/322
     //   2,744 T 175/267 1x16 97/181 1x32 92/211   32,768 T 163/292  1x64 231/340
+    // 64 or 128 owned Tet4 where two rings fit (both measured again; a second ring of 128 that does not
+    // fit leaves one):
+    //     4,374 2x64 60/141 2x128 72/160     7,986 2x64 60/142 2x128 96/174 (one ring)
+    //     6,000 2x64 60/143 2x128 60/156    10,368 2x64 66/140 2x128 59/154
     // A second ring pays while the chip idles (it evaluates some four times the elements), the
     // whole scheme until the elements evaluated twice cost what a launch does.  That line, in us a
     // step against the tile path as it is now (the T above are of its 1024-element tiles):
@@ -475,7 +479,7 @@ static void patch_build(Ctx &c) {
     //   13,824 Hex8 T 6.5/13.1 patches 6.2/12.7   19,683 Hex8 T 6.5/13.2 patches 8.4/15.6
     if (ne == 0 || ne > (npe == 4 ? 54000 : 15000) || c.tiles.threads != c.tiles.te || c.elem_seg.size() != 2) return;
     const int K = ne <= (npe == 4 ? 16000 : 500) ? 2 : 1;
-    const int64_t target = npe == 4 ? (ne <= 6500 ? 64 : ne <= 32000 ? 128 : 256) : (ne <= 500 ? 8 : ne <= 4000 ? 16 : 32);
+    const int64_t target = npe == 4 ? (ne <= 9000 ? 64 : ne <= 32000 ? 128 : 256) : (ne <= 500 ? 8 : ne <= 4000 ? 16 : 32);
     // without the memory for a plan the steps stay on the tiles
     auto none = [&] {
         (void)hipGetLastError();
