@@ -17,11 +17,14 @@
 //   RK mass             src/MassUtils.cpp:79-112 via FunctionEvaluationProcessor::ScatterValues
 //   two-pass cells      include/SmoothedCellDataProcessor.h:474-486, :637-648 (the element's own
 //                       nodes, derivative (B_k V)/V)
-// Per step:
-//   cell kernel         include/ComputeInternalForceSmoothedCell.h:86-117, :186-224 (H = sum u (x) grad phi,
-//                       stress; the stress term -V P^T of :325-326 is kept per cell)
-//   node kernel         :328-349 as a node gather over the cell entries that name the node, in ascending
-//                       (cell, entry) order, fused with the central-difference node update
+// Per step, element cells (both methods; src/Solvers/Explicit.cpp:148-186):
+//   gather kernel       FunctionEvaluationProcessor::ComputeValues (include/FunctionEvaluationProcessor.h:
+//                       70-117): u = Phi d
+//   element tiles       include/ComputeInternalForceSmoothedCell.h:86-117, :186-224, :325-349 on u, the
+//                       cell of an element being the element (tile.hip, force mode)
+//   scatter kernel      ScatterValues (:130-181) as a gather over reverse neighbor lists (points that
+//                       list the node, ascending), fused with the central-difference node update
+//                       (small meshes: gather and scatter in the tile's and the node's launch)
 // Nodal smoothing cells on a thex mesh (each tet split into four hexes):
 //   active nodes        include/MeshLabelerProcessor.h:227-330 (each hex's node of lowest
 //                       caller id; exactly one per hex), cells and subcells :690-827 (one cell
@@ -34,11 +37,8 @@
 //   F-bar force         include/ComputeInternalForceSmoothedCell.h:120-413 (subcell J, cell
 //                       J-bar, stress of F-bar, dual pressure, un-barred stress), used when a
 //                       cell has more subcells than one (:458-459)
-// Per step, two-pass method (src/Solvers/Explicit.cpp:148-186):
-//   gather kernel       FunctionEvaluationProcessor::ComputeValues (include/FunctionEvaluationProcessor.h:
-//                       70-117): physical displacement = Phi d before the cell kernel
-//   scatter kernel      ScatterValues (:130-181) as a gather over reverse neighbor lists (points that
-//                       list the node, ascending), fused with the central-difference node update
+// Per step, nodal cells: one kernel over cell tiles (forces to the tiles' node slots) and one over
+// the nodes (slots in ascending tile order, node update).
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -1588,7 +1588,7 @@ static int64_t tile_lds(int maxtn, int maxsub, bool fbar) {
     return 48 * (int64_t)std::max(maxtn, 1) + (fbar ? 8 * (int64_t)kFbarSubRow * std::max(maxsub, 1) : 0);
 }
 
-// Cell tiles of the one-pass force: runs of tile_cells consecutive cells, the sorted
+// Cell tiles of the nodal cells: runs of tile_cells consecutive cells, the sorted
 // union of their node lists, every entry's index in it, and every node's slots (its
 // positions in the tile-major node sets, ascending tile).  The tile size starts at 64
 // cells (256 for cells of at most four entries), is halved while the mesh gives fewer
