@@ -1408,10 +1408,10 @@ int aphip_autotune(aphip_ctx *c, double dt, int32_t trial_steps, int32_t *chosen
             continue;  // this shape does not fit the mesh (e.g. a tile needs more LDS than a CU has)
         }
         const double t = time_calls(tt);
-        // within 5 % the earlier one stays, the present plan first of all: launches cost the host
+        // within 10 % the earlier one stays, the present plan first of all: launches cost the host
         // more or less from one process to the next (729 Hex8, 40 steps: patches 321 us, one launch a
         // step; 16-element tiles, two launches, 310 here and 345 to 397 a minute later)
-        if (t < 0.95 * best_s) {
+        if (t < 0.90 * best_s) {
             best_s = t;
             best = tt;
         }

@@ -133,7 +133,7 @@ def test_patch_plans_are_built_where_they_are_used(gpu_available, case):
 
 
 # patches against the best tile shape, 40 steps alone: 321 and 310..385 us (729 Hex8; the present plan stays
-# unless another is 5 % faster), 240 and 387 (6000 Tet4)
+# unless another is 10 % faster), 240 and 387 (6000 Tet4)
 @pytest.mark.parametrize("etype,n", [(A.HEX8, 9), (A.TET4, 10)])
 def test_autotune_keeps_patches(gpu_available, etype, n):
     """Autotuning times what a call of many steps runs, so a mesh whose steps are fastest on
